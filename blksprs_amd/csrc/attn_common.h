@@ -49,6 +49,7 @@ int attn_fwd_records(const bsa_attn_args &a, const int32_t *entries, int32_t *re
 int attn_bwd_generic(const bsa_attn_args &a, hipStream_t s);
 // MFMA paths; return 1 if the configuration is not covered (caller falls back to the generic kernels)
 int attn_fwd_mfma(const bsa_attn_args &a, hipStream_t s);
+int attn_fwd_small(const bsa_attn_args &a, hipStream_t s);
 int attn_fwd_f32mma(const bsa_attn_args &a, hipStream_t s);
 int attn_bwd_f32mma(const bsa_attn_args &a, hipStream_t s);
 int attn_bwd_mfma(const bsa_attn_args &a, hipStream_t s);
