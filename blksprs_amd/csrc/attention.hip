@@ -107,6 +107,7 @@ extern "C" int bsa_attn_bwd(const bsa_attn_args *args, bsa_stream_t stream) {
   }
   hipStream_t s = bsa::as_stream(stream);
   int rc = bsa::attn_bwd_mfma(*args, s);
+  if (rc == 1) rc = bsa::attn_bwd_small(*args, s);
   if (rc == 1) rc = bsa::attn_bwd_f32mma(*args, s);
   if (rc == 1) rc = bsa::attn_bwd_generic(*args, s);
   return rc;

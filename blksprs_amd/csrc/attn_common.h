@@ -51,6 +51,7 @@ int attn_bwd_generic(const bsa_attn_args &a, hipStream_t s);
 int attn_fwd_mfma(const bsa_attn_args &a, hipStream_t s);
 int attn_fwd_small(const bsa_attn_args &a, hipStream_t s);
 int attn_fwd_f32mma(const bsa_attn_args &a, hipStream_t s);
+int attn_bwd_small(const bsa_attn_args &a, hipStream_t s);
 int attn_bwd_f32mma(const bsa_attn_args &a, hipStream_t s);
 int attn_bwd_mfma(const bsa_attn_args &a, hipStream_t s);
 int attn_mask_dead(const void *mask, int64_t n_mask_blocks, uint8_t *dead, hipStream_t s);

@@ -1,0 +1,458 @@
+// Block-sparse flash attention backward for 16-bit operands in blocks of 16 and 32, on the 16-bit matrix cores (the
+// forward kernel: attn_small_fwd.hip; tiles, fragments and the walk over a list: attn_small_common.h).
+//
+// Two launches, no atomics, fixed summation order.  The first gives a wave a query block: delta = rowsum(o * dO) from the
+// fragments of o and dO it holds anyway, then dQ (and dBias) over the block's key list.  The second gives a wave a key
+// block: dK and dV over its query list.  Both form scores, probabilities and dP of every pair themselves, so no
+// intermediate of the size of the attention layout exists; a wave walks alone, without barriers.  A lane owns one
+// row of the own block in every product, so P and dS pass from the accumulators of one product into the operands of
+// the next without leaving registers:
+//
+//   dQ kernel, lane owns a query i, registers run over keys j:
+//     dP^T = V dO^T, S^T = K Q^T    rows of V, K from LDS, dO and Q in registers
+//     dQ^T += K^T dS^T              columns of K from LDS
+//   dK / dV kernel, lane owns a key j, registers run over queries i:
+//     S = Q K^T, dP = dO V^T        rows of Q, dO from LDS, K and V in registers
+//     dV^T += dO^T P, dK^T += Q^T dS columns of dO, Q from LDS
+//
+// What bounds it: the chain of a step (tiles awaited, products, exponentials, products) with two to four waves per SIMD
+// to overlap it; matrix cores 21 % busy in the second kernel.  Against the fp32 matrix-core kernels that ran these shapes
+// before (48 x 4096 queries, sbs 32, head dimension 64, fp16, 33 key blocks per query block): delta + zero fill
+// 0.071 -> 0, dK / dV 1.89 -> 0.125 ms, dQ 1.24 -> 0.096 ms (delta included); bf16, sbs 16, 32 causal sequences of 1032 to
+// 2064: dK / dV 0.067, dQ 0.065 ms.
+//
+// Scores as in the forward kernel; p = exp2(s - lse), 0 where lse = -inf; P and dS are rounded to the operand type
+// before they enter a product (blksprs/ops/flash_attention.py:1452, :1468, :1692).
+#include <type_traits>
+
+#include "attn_small_common.h"
+
+namespace bsa {
+namespace {
+
+using namespace small;
+
+constexpr int kWaves = 4;
+
+template <int SBS, int NS>
+struct BwdShape {
+  static constexpr int NB = SBS == 32 ? 1 : 2;  // partner blocks per step
+  using T = Tile<SBS, NS, NB>;
+  static constexpr int kRegs = SBS == 32 ? 16 : 4;
+  static constexpr int kScores = kRegs * NB;
+  static constexpr int kPartial = SBS * SBS * NS * 4;
+  static constexpr int kStats = 256;  // lse and delta of the 32 queries of a step
+  // dK / dV kernel: Q and dO of two steps where registers allow two waves per SIMD anyway (sbs 32: 133 against 137 us);
+  // at sbs 16 one step's tiles and twice the waves are faster (67 against 92 us)
+  static constexpr int kBufs = SBS == 32 && NS <= 2 ? 2 : 1;
+  static constexpr int kKvBuf = 2 * T::kBytes + kStats;
+  // the last row fragment of an odd number of slices of 16 reads (and drops) a slice beyond its tile
+  static constexpr int kPad = T::kHalfLast ? T::kPiece : 0;
+  static constexpr int kKvLds = kPad + (kBufs * kKvBuf > 2 * kPartial ? kBufs * kKvBuf : 2 * kPartial);
+  static constexpr int kQLds = kPad + (2 * T::kBytes > kPartial ? 2 * T::kBytes : kPartial);
+  static constexpr int kQMinWaves = SBS == 32 ? (NS <= 2 ? 3 : 2) : (NS <= 4 ? 4 : 2);
+  static constexpr int kKvMinWaves = SBS == 32 ? (NS <= 3 ? 2 : 1) : (NS <= 4 ? 3 : 2);
+};
+
+// 4 bytes per lane, global -> LDS: lane l's value lands at dst + 4 l
+__device__ inline void copy_words_to_lds(const float *addr, char *dst) {
+  const uint32_t lds_addr = (uint32_t)(uintptr_t)(lds_ptr_t)dst;
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(addr), "s"(lds_addr) : "memory");
+}
+
+template <typename Tr, int kScores>
+__device__ inline void pack_scores(u32x4 (&w)[kScores / 8], const float *v) {
+#pragma unroll
+  for (int m = 0; m < kScores / 8; ++m)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[m][i] = Tr::pack2(v[8 * m + 2 * i], v[8 * m + 2 * i + 1]);
+}
+
+// the partial sums of the waves that share a row, added up in order into those of the first
+template <int NS, int kRegs, typename Acc>
+__device__ inline void leave_partial(const Acc (&acc)[NS], float *mine, int lane) {
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
+#pragma unroll
+    for (int r = 0; r < kRegs; r += 4)
+      *reinterpret_cast<f32x4 *>(mine + ((h * kRegs + r) / 4 * 64 + lane) * 4) =
+          f32x4{acc[h][r], acc[h][r + 1], acc[h][r + 2], acc[h][r + 3]};
+}
+template <int NS, int kRegs, typename Acc>
+__device__ inline void add_partial(Acc (&acc)[NS], const float *other, int lane) {
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
+#pragma unroll
+    for (int r = 0; r < kRegs; r += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4 *>(other + ((h * kRegs + r) / 4 * 64 + lane) * 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[h][r + i] += v[i];
+    }
+}
+
+// gradient blocks of the own row, eight bytes of a row per lane: columns 2 r + 4 group .. + 3
+template <typename Tr, int SBS, int NS, typename Acc>
+__device__ inline void store_gradient(const Acc (&acc)[NS], float scale, void *out, const int64_t *pidx, int n_slices,
+                                      int64_t n_blocks, int me, int group) {
+  constexpr int kRegs = SBS == 32 ? 16 : 4;
+#pragma unroll
+  for (int h = 0; h < NS; ++h) {
+    if (h >= n_slices) break;
+    const int64_t p = pidx[h];
+    if (p < 0 || p >= n_blocks) continue;
+    char *blk = static_cast<char *>(out) + p * (SBS * SBS * 2) + me * (2 * SBS) + 8 * group;
+#pragma unroll
+    for (int r = 0; r < kRegs; r += 4) {
+      u32x2 w;
+      w[0] = Tr::pack2(acc[h][r] * scale, acc[h][r + 1] * scale);
+      w[1] = Tr::pack2(acc[h][r + 2] * scale, acc[h][r + 3] * scale);
+      *reinterpret_cast<u32x2 *>(blk + 4 * r) = w;
+    }
+  }
+}
+
+template <typename Tr, int SBS, int NS>
+__global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kQMinWaves)) void attn_small_dq_kernel(bsa_attn_args a, int split) {
+  using Shape = BwdShape<SBS, NS>;
+  using T = typename Shape::T;
+  using W = Walk<SBS, NS, Shape::NB, true>;
+  constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs;
+  using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
+  extern __shared__ __attribute__((aligned(1024))) char small_smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = first_lane(threadIdx.x >> 6);
+  char *lds_k = small_smem + wave * Shape::kQLds, *lds_v = lds_k + T::kBytes;
+
+  const RowOfWave me(a.B, a.nq, true, wave, kWaves, split);
+  const int64_t row = me.b * a.nq + me.own;
+  const int qi = lane % SBS, kq = lane / SBS;
+  W walk;
+  walk.start(a, me.b, me.own, me.there, me.part, split);
+
+  OwnRows<SBS, NS> qf, gf;
+  qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, lane);
+  gf.load(a.d_o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, lane);
+  float delta = 0.f, neg_lse = -a.lse[row * SBS + qi];
+  if (neg_lse == INFINITY) neg_lse = -INFINITY;  // a query that sees nothing: p = 0
+  {
+    OwnRows<SBS, NS> of;
+    of.load(a.o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, lane);
+#pragma unroll
+    for (int f = 0; f < T::kFrags; ++f)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) delta = Tr::dot2(of.fr[f][i], gf.fr[f][i], delta);
+    delta = row_sum<SBS>(delta);
+    if (me.there && me.part == 0 && kq == 0) a.delta[row * SBS + qi] = delta;
+  }
+  acc_t dq[NS];
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
+#pragma unroll
+    for (int r = 0; r < kRegs; ++r) dq[h][r] = 0.f;
+
+  const float qk_scale = a.scale * kLog2e;
+  const float cc = a.bias ? 1.f : qk_scale;
+  const uint32_t source = T::source_offset(lane);
+  const char *const tensor_k = static_cast<const char *>(a.k), *const tensor_v = static_cast<const char *>(a.v);
+  const typename T::RowReader k_rows(lds_k, lane), v_rows(lds_v, lane);
+  const typename T::ColReader k_cols(lds_k, lane);
+  typename W::Step now, next;
+  walk.take(now, lane);
+  settle(qf);
+  settle(gf);
+  bool counted = false;  // exactly kCopies copies were issued after the tile that is needed next
+  if (now.count) {
+    walk.template copy<true>(now, tensor_v, lds_v, source, lane);
+    counted = walk.template copy<false>(now, tensor_k, lds_k, source, lane);
+  }
+  while (now.count) {
+    // ---- dP^T = V dO^T.  In flight at most: V and K of this step, in that order.
+    if (counted) wait_vmem<T::kCopies>();
+    else wait_vmem<0>();
+    acc_t dp[NB], sacc[NB];
+    product_rows<Tr, SBS, NS, NB>(dp, v_rows, gf);
+    wait_lds();
+    walk.take(next, lane);
+    counted = false;
+    if (next.count) counted = walk.template copy<true>(next, tensor_v, lds_v, source, lane);
+
+    // ---- S^T = K Q^T.  In flight at most: K of this step, V of the next.
+    if (counted) wait_vmem<T::kCopies>();
+    else wait_vmem<0>();
+    product_rows<Tr, SBS, NS, NB>(sacc, k_rows, qf);
+    float sv[kScores];
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
+    if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, qi, kq);
+
+    // ---- dS = P (dP - delta)
+#pragma unroll
+    for (int x = 0; x < kScores; ++x)
+      sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], cc, neg_lse)) * (dp[x / kRegs][x % kRegs] - delta);
+    if (now.special) {
+      const late_args_t p = late_args();
+      if (p->dbias) {  // every pair is visited once: plain stores
+#pragma unroll
+        for (int t = 0; t < NB; ++t)
+          if (now.bias[t] >= 0) {
+            float *out = p->dbias + ((int64_t)now.bias[t] * SBS + qi) * SBS + 4 * kq;
+#pragma unroll
+            for (int r = 0; r < kRegs; r += 4) {
+              const float *v = sv + kRegs * t + r;
+              *reinterpret_cast<f32x4 *>(out + 2 * r) = f32x4{v[0], v[1], v[2], v[3]};
+            }
+          }
+      }
+    }
+    u32x4 w[kScores / 8];
+    pack_scores<Tr, kScores>(w, sv);
+
+    // ---- dQ^T += K^T dS^T
+    product_cols<Tr, SBS, NS, NB>(dq, k_cols, w);
+    wait_lds();
+    counted = false;
+    if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
+    now = next;
+  }
+  if (split > 1) {
+    float *mine = reinterpret_cast<float *>(lds_k);
+    if (me.part != 0) leave_partial<NS, kRegs>(dq, mine, lane);
+    __syncthreads();
+    if (me.part != 0) return;
+    for (int p = 1; p < split; ++p) add_partial<NS, kRegs>(dq, mine + p * (Shape::kQLds / 4), lane);
+  }
+  if (!me.there) return;
+  const late_args_t p = late_args();
+  store_gradient<Tr, SBS, NS>(dq, p->scale, p->dq, p->pidx_q + row * p->nh, (int)p->nh, p->n_q_blocks, qi, kq);
+}
+
+template <typename Tr, int SBS, int NS>
+__global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kKvMinWaves)) void attn_small_dkv_kernel(bsa_attn_args a, int split) {
+  using Shape = BwdShape<SBS, NS>;
+  using T = typename Shape::T;
+  using W = Walk<SBS, NS, Shape::NB, false>;
+  constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs, kBufs = Shape::kBufs;
+  using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
+  extern __shared__ __attribute__((aligned(1024))) char small_smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = first_lane(threadIdx.x >> 6);
+  char *lds = small_smem + wave * Shape::kKvLds;  // per buffer: Q tile, dO tile, lse and delta
+
+  const RowOfWave me(a.B, a.nk, false, wave, kWaves, split);
+  const int64_t row = me.b * a.nk + me.own;
+  const int kj = lane % SBS, kq = lane / SBS;  // key row; which queries of a block this lane's registers hold
+  W walk;
+  walk.start(a, me.b, me.own, me.there, me.part, split);
+
+  OwnRows<SBS, NS> kf, vf;
+  kf.load(a.k, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, lane);
+  vf.load(a.v, a.pidx_v + row * a.nhv, (int)a.nhv, a.n_v_blocks, lane);
+  acc_t dk[NS], dv[NS];
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
+#pragma unroll
+    for (int r = 0; r < kRegs; ++r) dk[h][r] = dv[h][r] = 0.f;
+
+  const float qk_scale = a.scale * kLog2e;
+  const float cc = a.bias ? 1.f : qk_scale;
+  const uint32_t source = T::source_offset(lane);
+  const char *const tensor_q = static_cast<const char *>(a.q), *const tensor_g = static_cast<const char *>(a.d_o);
+  // this lane's share of the statistics copy: lanes 0 .. 31 lse, 32 .. 63 delta of the step's 32 queries
+  const float *const stats = (lane < 32 ? a.lse : a.delta) + me.b * a.nq * SBS + lane % SBS;
+  const int stats_block = SBS == 16 ? (lane >> 4) & 1 : 0;
+  auto copy_stats = [&](const typename W::Step &s, char *dst) {
+    int other = __builtin_amdgcn_readlane(walk.other, s.slot[0]);
+    if constexpr (NB > 1) {
+      const int second = s.count > 1 ? __builtin_amdgcn_readlane(walk.other, s.slot[1]) : other;
+      other = stats_block ? second : other;
+    }
+    copy_words_to_lds(stats + (int64_t)other * SBS, dst);
+  };
+  auto copy_all = [&](const typename W::Step &s, char *buf) {
+    const bool q_whole = walk.template copy<false>(s, tensor_q, buf, source, lane);
+    const bool g_whole = walk.template copy<true>(s, tensor_g, buf + T::kBytes, source, lane);
+    copy_stats(s, buf + 2 * T::kBytes);
+    return q_whole && g_whole;
+  };
+
+  const typename T::RowReader q_rows0(lds, lane), g_rows0(lds + T::kBytes, lane);
+  const typename T::ColReader q_cols0(lds, lane), g_cols0(lds + T::kBytes, lane);
+  typename W::Step now, next;
+  walk.take(now, lane);
+  settle(kf);
+  settle(vf);
+  int buf = 0;
+  if (now.count) copy_all(now, lds);
+  while (now.count) {
+    const int at = kBufs == 2 ? buf * Shape::kKvBuf : 0;
+    if constexpr (kBufs == 2) {
+      // the next step's tiles into the other buffer, then wait for everything but them
+      wait_lds();
+      walk.take(next, lane);
+      bool counted = false;
+      if (next.count) counted = copy_all(next, lds + (buf ^ 1) * Shape::kKvBuf);
+      if (counted) wait_vmem<2 * T::kCopies + 1>();
+      else wait_vmem<0>();
+    } else {
+      wait_vmem<0>();
+    }
+    typename T::RowReader q_rows = q_rows0, g_rows = g_rows0;
+    typename T::ColReader q_cols = q_cols0, g_cols = g_cols0;
+    if constexpr (kBufs == 2) {
+      q_rows.base0 += at, q_rows.base1 += at, g_rows.base0 += at, g_rows.base1 += at;
+      q_cols.base0 += at, q_cols.base1 += at, g_cols.base0 += at, g_cols.base1 += at;
+    }
+    const float *lse = reinterpret_cast<const float *>(lds + at + 2 * T::kBytes), *delta = lse + 32;
+
+    // ---- S = Q K^T, P = exp2(S - lse)
+    acc_t sacc[NB], dp[NB];
+    product_rows<Tr, SBS, NS, NB>(sacc, q_rows, kf);
+    float sv[kScores], ls[kScores];
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
+    if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, kj, kq);
+#pragma unroll
+    for (int x = 0; x < kScores; x += 4) {
+      const f32x4 l4 = *reinterpret_cast<const f32x4 *>(lse + (x / kRegs) * SBS + 2 * (x % kRegs) + 4 * kq);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ls[x + i] = l4[i];
+    }
+    product_rows<Tr, SBS, NS, NB>(dp, g_rows, vf);
+    float lowest = ls[0];
+#pragma unroll
+    for (int x = 1; x < kScores; ++x) lowest = fminf(lowest, ls[x]);
+    if (__any(lowest == -INFINITY)) {  // a query that sees nothing: p = 0
+#pragma unroll
+      for (int x = 0; x < kScores; ++x)
+        if (ls[x] == -INFINITY) ls[x] = INFINITY;
+    }
+#pragma unroll
+    for (int x = 0; x < kScores; ++x) sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], cc, -ls[x]));
+    u32x4 w[kScores / 8];
+    pack_scores<Tr, kScores>(w, sv);
+
+    // ---- dS = P (dP - delta)
+#pragma unroll
+    for (int x = 0; x < kScores; x += 4) {
+      const f32x4 d4 = *reinterpret_cast<const f32x4 *>(delta + (x / kRegs) * SBS + 2 * (x % kRegs) + 4 * kq);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sv[x + i] *= dp[x / kRegs][x % kRegs + i] - d4[i];
+    }
+    // ---- dV^T += dO^T P
+    product_cols<Tr, SBS, NS, NB>(dv, g_cols, w);
+    if constexpr (kBufs == 1) {
+      wait_lds();
+      walk.take(next, lane);
+      if (next.count) {
+        walk.template copy<true>(next, tensor_g, lds + T::kBytes, source, lane);
+        copy_stats(next, lds + 2 * T::kBytes);
+      }
+    }
+    // ---- dK^T += Q^T dS
+    pack_scores<Tr, kScores>(w, sv);
+    product_cols<Tr, SBS, NS, NB>(dk, q_cols, w);
+    if constexpr (kBufs == 1) {
+      wait_lds();
+      if (next.count) walk.template copy<false>(next, tensor_q, lds, source, lane);
+    }
+    now = next;
+    buf ^= 1;
+  }
+  if (split > 1) {
+    float *mine = reinterpret_cast<float *>(lds);
+    if (me.part != 0) {
+      leave_partial<NS, kRegs>(dk, mine, lane);
+      leave_partial<NS, kRegs>(dv, mine + Shape::kPartial / 4, lane);
+    }
+    __syncthreads();
+    if (me.part != 0) return;
+    for (int p = 1; p < split; ++p) {
+      add_partial<NS, kRegs>(dk, mine + p * (Shape::kKvLds / 4), lane);
+      add_partial<NS, kRegs>(dv, mine + p * (Shape::kKvLds / 4) + Shape::kPartial / 4, lane);
+    }
+  }
+  if (!me.there) return;
+  const late_args_t p = late_args();
+  store_gradient<Tr, SBS, NS>(dk, p->scale, p->dk, p->pidx_k + row * p->nh, (int)p->nh, p->n_k_blocks, kj, kq);
+  store_gradient<Tr, SBS, NS>(dv, 1.f, p->dv, p->pidx_v + row * p->nhv, (int)p->nhv, p->n_v_blocks, kj, kq);
+}
+
+// bias blocks outside the attention layout, and pairs the causal predicate rules out, have no wave that writes them
+__global__ void small_zero_kernel(f32x4 *out, int64_t n) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) out[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+template <typename K>
+int raise_lds(K kernel, int bytes) {
+  if (bytes > 64 * 1024)
+    BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  return BSA_OK;
+}
+
+template <typename Tr, int SBS, int NS>
+int launch(const bsa_attn_args &a, hipStream_t s) {
+  using Shape = BwdShape<SBS, NS>;
+  constexpr int q_lds = Shape::kQLds * kWaves, kv_lds = Shape::kKvLds * kWaves;
+  static_assert(q_lds <= 160 * 1024 && kv_lds <= 160 * 1024, "LDS");
+  static const int raised = [] {
+    const int rc = raise_lds(&attn_small_dq_kernel<Tr, SBS, NS>, q_lds);
+    return rc ? rc : raise_lds(&attn_small_dkv_kernel<Tr, SBS, NS>, kv_lds);
+  }();
+  if (raised) return raised;
+  if (a.dbias && a.n_bias_blocks > 0) {
+    const int64_t n = a.n_bias_blocks * SBS * SBS / 4, blocks = cdiv(n, (int64_t)256);
+    small_zero_kernel<<<(unsigned)(blocks < 65536 ? blocks : 65536), 256, 0, s>>>(reinterpret_cast<f32x4 *>(a.dbias), n);
+    if (int rc = check_launch("small_zero_kernel")) return rc;
+  }
+  if (const int64_t rows = a.B * a.nq) {
+    const int split = waves_per_row(rows);
+    attn_small_dq_kernel<Tr, SBS, NS><<<row_groups(rows, kWaves, split), 64 * kWaves, q_lds, s>>>(a, split);
+    if (int rc = check_launch("attn_small_dq_kernel")) return rc;
+  }
+  if (const int64_t rows = a.B * a.nk) {
+    const int split = waves_per_row(rows);
+    attn_small_dkv_kernel<Tr, SBS, NS><<<row_groups(rows, kWaves, split), 64 * kWaves, kv_lds, s>>>(a, split);
+    if (int rc = check_launch("attn_small_dkv_kernel")) return rc;
+  }
+  return BSA_OK;
+}
+
+template <typename Tr>
+int dispatch(const bsa_attn_args &a, hipStream_t s) {
+  const int64_t slices = a.nh > a.nhv ? a.nh : a.nhv;
+  if (a.sbs == 32) {
+    switch (slices) {
+      case 1: return launch<Tr, 32, 1>(a, s);
+      case 2: return launch<Tr, 32, 2>(a, s);
+      case 3: return launch<Tr, 32, 3>(a, s);
+      case 4: return launch<Tr, 32, 4>(a, s);
+    }
+    return 1;
+  }
+  switch (slices) {
+    case 1: return launch<Tr, 16, 1>(a, s);
+    case 2: return launch<Tr, 16, 2>(a, s);
+    case 3: return launch<Tr, 16, 3>(a, s);
+    case 4: return launch<Tr, 16, 4>(a, s);
+    case 5: return launch<Tr, 16, 5>(a, s);
+    case 6: return launch<Tr, 16, 6>(a, s);
+    case 7: return launch<Tr, 16, 7>(a, s);
+    case 8: return launch<Tr, 16, 8>(a, s);
+  }
+  return 1;
+}
+
+}  // namespace
+
+// 1: not covered
+int attn_bwd_small(const bsa_attn_args &a, hipStream_t s) {
+  if (!small_applies(a)) return 1;
+  return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, s) : dispatch<SF16>(a, s);
+}
+
+}  // namespace bsa

@@ -287,5 +287,242 @@ __device__ static inline float row_sum(float v) {
   return sum_across32(v);
 }
 
+// One wave's walk over the list of partner blocks of one block of its own: key blocks of a query block, or (kOwnIsQuery
+// false) query blocks of a key block.
+//
+// The list is read 64 entries at a time, one per lane: the partner block, the packed indices of its first slices (of K
+// and V, or of Q and dO), its mask and bias block.  Entries the causal predicate rules out as a whole are left out of
+// `live`; `special` marks those whose scores need more than the scale; `apart` says that some block's slices are
+// missing or do not lie one behind the other.
+template <int SBS, int NS, int NB, bool kOwnIsQuery>
+struct Walk {
+  using T = Tile<SBS, NS, NB>;
+  int64_t b, own;          // batch entry, own block
+  int end, base, seq_len;  // end of the list, first entry of the window; valid length of a causal sequence
+  int other, first_a, first_b, mask, bias;  // of this lane's entry
+  uint64_t live, special;
+  bool apart;
+
+  // a step: how many entries it takes and their places in the window, and, if special, their facts (the window may be
+  // another one by the time the scores are formed)
+  struct Step {
+    int count, slot[NB], other[NB], mask[NB], bias[NB];
+    bool special, apart;
+  };
+
+  // part of parts: the contiguous share of the list that this wave walks
+  __device__ inline void start(const bsa_attn_args &a, int64_t b_, int64_t own_, bool there, int part, int parts) {
+    b = b_, own = own_;
+    seq_len = 0x7fffffff;
+    if (a.causal_lengths) {
+      const int64_t len = a.causal_lengths[b];
+      seq_len = len < 0 ? 0 : (len > 0x7fffffffLL ? 0x7fffffff : (int)len);
+    }
+    const int32_t *offsets = (kOwnIsQuery ? a.key_offsets : a.query_offsets) + b * (kOwnIsQuery ? a.nq : a.nk) + own;
+    int begin = first_lane(offsets[0]);
+    end = first_lane(offsets[1]);
+    if (parts > 1) {
+      const int64_t n = end - begin;
+      end = begin + (int)(n * (part + 1) / parts);
+      begin += (int)(n * part / parts);
+    }
+    if (!there || (int)own * SBS >= seq_len) end = begin;
+    base = begin - 64;
+    other = first_a = first_b = 0;
+    mask = bias = -1;
+    live = special = 0;
+    apart = false;
+  }
+
+  __device__ inline void refill(int lane) {
+    const late_args_t p = late_args();
+    base += 64;
+    const int e = base + lane;
+    bool in = e < end;
+    other = in ? (kOwnIsQuery ? p->key_indices : p->query_indices)[e] : 0;
+    const bool causal = p->causal_lengths != nullptr;
+    in = in && !(causal && ((kOwnIsQuery ? other > (int)own : other < (int)own) || other * SBS >= seq_len));
+    const int64_t place = b * (kOwnIsQuery ? p->nk : p->nq) + other;
+    bool far = p->nh != NS || p->nhv != NS;
+    if (in && !far) {
+      const int64_t *pa = (kOwnIsQuery ? p->pidx_k : p->pidx_q) + place * NS;
+      const int64_t *pb = (kOwnIsQuery ? p->pidx_v : p->pidx_o) + place * NS;
+      const int64_t a0 = pa[0], b0 = pb[0];
+      far = a0 < 0 || b0 < 0 || a0 + NS > (kOwnIsQuery ? p->n_k_blocks : p->n_q_blocks) ||
+            b0 + NS > (kOwnIsQuery ? p->n_v_blocks : p->n_o_blocks);
+#pragma unroll
+      for (int h = 1; h < NS; ++h) far = far || pa[h] != a0 + h || pb[h] != b0 + h;
+      first_a = (int)a0;
+      first_b = (int)b0;
+    }
+    apart = __any(in && far);
+    bool extra = causal && (other == (int)own || ((int)own + 1) * SBS > seq_len || (other + 1) * SBS > seq_len);
+    const int64_t pair = kOwnIsQuery ? (b * p->nq + own) * p->nk + other : (b * p->nq + other) * p->nk + own;
+    if (p->mask) {
+      const int64_t m = in ? p->pidx_mask[pair] : -1;
+      mask = m < p->n_mask_blocks ? (int)m : -1;
+      extra = extra || mask >= 0;
+    }
+    if (p->bias) {
+      const int64_t m = in ? p->pidx_bias[pair] : -1;
+      bias = m < p->n_bias_blocks ? (int)m : -1;
+      extra = true;
+    }
+    live = __ballot(in);
+    special = __ballot(in && extra);
+  }
+
+  __device__ inline void take(Step &s, int lane) {
+    while (live == 0 && base + 64 < end) refill(lane);
+    s.count = 0;
+    uint64_t taken = 0;
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      const uint64_t lowest = live & -live;
+      s.slot[t] = lowest ? __builtin_ctzll(lowest) : 0;
+      s.count += lowest ? 1 : 0;
+      live ^= lowest;
+      taken |= lowest;
+    }
+    s.apart = apart;
+    s.special = (taken & special) != 0 || (NB > 1 && s.count < NB);
+    if (s.special) {
+#pragma unroll
+      for (int t = 0; t < NB; ++t) {
+        s.other[t] = __builtin_amdgcn_readlane(other, s.slot[t]);
+        s.mask[t] = t < s.count ? __builtin_amdgcn_readlane(mask, s.slot[t]) : -1;
+        s.bias[t] = t < s.count ? __builtin_amdgcn_readlane(bias, s.slot[t]) : -1;
+      }
+    }
+  }
+
+  // Requests the step's blocks of the first (K or Q) or second (V or dO) tensor; returns whether exactly T::kCopies
+  // asynchronous copies are on their way.  To be called before the next take().  Blocks that are not there (the last
+  // step of a list) become zeros.
+  template <bool kSecond>
+  __device__ inline bool copy(const Step &s, const char *tensor, char *dst, uint32_t offset, int lane) const {
+    if (!s.apart) {
+#pragma unroll
+      for (int t = 0; t < NB; ++t)
+        if (NB == 1 || t < s.count)
+          T::copy_block(tensor, __builtin_amdgcn_readlane(kSecond ? first_b : first_a, s.slot[t]), dst + t * T::kBlock, offset, lane);
+      if (NB == 1 || s.count == NB) return true;
+    }
+    const late_args_t p = late_args();
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      if (!s.apart && t < s.count) continue;
+      const int n = t < s.count ? (int)(kSecond ? p->nhv : p->nh) : 0;
+      const int64_t place = b * (kOwnIsQuery ? p->nk : p->nq) + __builtin_amdgcn_readlane(other, s.slot[t]);
+      const int64_t *pidx = kSecond ? (kOwnIsQuery ? p->pidx_v : p->pidx_o) : (kOwnIsQuery ? p->pidx_k : p->pidx_q);
+      const int64_t count = kSecond ? (kOwnIsQuery ? p->n_v_blocks : p->n_o_blocks) : (kOwnIsQuery ? p->n_k_blocks : p->n_q_blocks);
+      T::gather_block(tensor, pidx + place * n, n, count, dst + t * T::kBlock, offset, lane);
+    }
+    return false;
+  }
+
+  // Bias, mask, causal predicate and missing blocks of a special step, in this order (blksprs/ops/flash_attention.py
+  // :1110-1150).  sv: the step's scores up to the factor cc of the exponential, block after block; with a bias they leave
+  // multiplied by qk_scale and complete, and cc is 1.  me: this lane's own row; group: lane / SBS.
+  template <typename Tr>
+  __device__ inline void finish_scores(const Step &s, float *sv, float qk_scale, int me, int group) const {
+    constexpr int kRegs = SBS == 32 ? 16 : 4;
+    const late_args_t p = late_args();
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      float *v = sv + kRegs * t;
+      // registers 4 w .. 4 w + 3 belong to partner rows 8 w + 4 group .. + 3
+      if (p->bias) {
+        const char *blk = static_cast<const char *>(p->bias) + (int64_t)s.bias[t] * T::kPiece;
+#pragma unroll
+        for (int w = 0; w < kRegs / 4; ++w) {
+          u32x2 bw{0u, 0u};
+          if (s.bias[t] >= 0) {
+            if constexpr (kOwnIsQuery) {
+              bw = *reinterpret_cast<const u32x2 *>(blk + me * (2 * SBS) + 16 * w + 8 * group);
+            } else {
+              const uint16_t *col = reinterpret_cast<const uint16_t *>(blk) + (8 * w + 4 * group) * SBS + me;
+              bw = u32x2{col[0] | (uint32_t)col[SBS] << 16, col[2 * SBS] | (uint32_t)col[3 * SBS] << 16};
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            v[4 * w + i] = v[4 * w + i] * qk_scale + Tr::widen((uint16_t)(bw[i / 2] >> (16 * (i % 2)))) * kLog2e;
+        }
+      }
+      if (s.mask[t] >= 0) {
+        const uint8_t *blk = static_cast<const uint8_t *>(p->mask) + (int64_t)s.mask[t] * (SBS * SBS);
+        uint32_t mw[kRegs / 4];
+#pragma unroll
+        for (int w = 0; w < kRegs / 4; ++w) {
+          if constexpr (kOwnIsQuery) {
+            mw[w] = *reinterpret_cast<const uint32_t *>(blk + me * SBS + 8 * w + 4 * group);
+          } else {
+            const uint8_t *col = blk + (8 * w + 4 * group) * SBS + me;
+            mw[w] = col[0] | (uint32_t)col[SBS] << 8 | (uint32_t)col[2 * SBS] << 16 | (uint32_t)col[3 * SBS] << 24;
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < kRegs; ++r)
+          if ((mw[r / 4] >> (8 * (r % 4))) & 0xffu) v[r] = -INFINITY;
+      }
+      if (p->causal_lengths) {
+        const int mine = (int)own * SBS + me;
+#pragma unroll
+        for (int r = 0; r < kRegs; ++r) {
+          const int theirs = s.other[t] * SBS + 8 * (r / 4) + 4 * group + r % 4;
+          if ((kOwnIsQuery ? theirs > mine : theirs < mine) || mine >= seq_len || theirs >= seq_len) v[r] = -INFINITY;
+        }
+      }
+      if (t >= s.count) {
+#pragma unroll
+        for (int r = 0; r < kRegs; ++r) v[r] = -INFINITY;
+      }
+    }
+  }
+};
+
+// Whether the kernels for blocks of 16 and 32 take these arguments (up to the head slices they are built for)
+inline bool small_applies(const bsa_attn_args &a) {
+  if (a.sbs != 16 && a.sbs != 32) return false;
+  if (a.dtype != BSA_BF16 && a.dtype != BSA_F16) return false;
+  // the forward kernel takes the row maximum before the scale is applied
+  if (!(a.scale > 0.f) || a.scale > 3.0e38f) return false;
+  const int64_t most = 0x7fffffffLL;  // indices and positions are 32-bit numbers
+  if (a.n_q_blocks > most || a.n_k_blocks > most || a.n_v_blocks > most || a.n_o_blocks > most ||
+      a.n_mask_blocks > most || a.n_bias_blocks > most || a.nq * a.sbs > most || a.nk * a.sbs > most)
+    return false;
+  const int64_t slices = a.nh > a.nhv ? a.nh : a.nhv;
+  return slices >= 1 && slices <= 128 / a.sbs;
+}
+
+// Waves that share one row of a launch of `rows` rows, each walking a contiguous part of its list.  A launch lasts as
+// long as the serial walk of its longest lists, and the last round of a launch of few rounds is mostly empty: shorter
+// shares help until their prologue (four dependent loads) costs more than the walk.  Forward, 64 rows (8 key blocks
+// each, sbs 32): 9.6 us with two waves per row, 8.1 with four; 4128 rows (sbs 16, causal, up to 65 steps): 80 / 60 / 61 us
+// with one, two, four; 6144 rows (sbs 32, 33 steps): 83 / 75 / 82.
+inline int waves_per_row(int64_t rows) { return rows <= 512 ? 4 : rows <= 8192 ? 2 : 1; }
+
+// The row of a wave.  XCD c (workgroup g runs on XCD g % 8) takes a contiguous eighth of the rows, so that the waves in
+// flight on one L2 share few batch entries' partner blocks; inside a batch entry the long rows of a causal layout (the
+// last query blocks, the first key blocks) come first.
+struct RowOfWave {
+  int64_t b, own;
+  int part;
+  bool there;
+  __device__ inline RowOfWave(int64_t batches, int64_t rows_per_batch, bool last_first, int wave, int waves, int split) {
+    const int64_t group = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const int64_t item = group * (waves / split) + wave / split;
+    part = wave % split;
+    there = item < batches * rows_per_batch;
+    b = there ? item / rows_per_batch : 0;
+    own = there ? item % rows_per_batch : 0;
+    if (last_first) own = rows_per_batch - 1 - own;
+  }
+};
+inline unsigned row_groups(int64_t rows, int waves, int split) {
+  return (unsigned)(cdiv(cdiv(rows, (int64_t)(waves / split)), (int64_t)8) * 8);
+}
+
 }  // namespace small
 }  // namespace bsa

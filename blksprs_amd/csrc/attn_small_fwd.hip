@@ -2,7 +2,7 @@
 //
 // A wave owns one query block (or a share of its key list, below) and walks the list alone: no barrier, no tile
 // shared between waves, so waves of a compute unit drift apart and fill each other's waits.  A step takes one key
-// block of 32 or up to four of 16.  The products are formed transposed (S^T = K Q^T, O^T = V^T P^T): a lane owns one
+// block of 32 or two of 16.  The products are formed transposed (S^T = K Q^T, O^T = V^T P^T): a lane owns one
 // query row, the statistics of the softmax are in-lane reductions plus one or two lane swaps, and the probabilities
 // are, as they sit in the accumulators of the score product, the second operand of the value product.
 //
@@ -17,7 +17,7 @@
 // wave at a time; matrix cores 16 % busy, 113 vector and 63 scalar instructions per step of 32 x 32 at head dimension 64.
 // Against the fp32 matrix-core kernel that ran these shapes before: 48 x 4096 queries, sbs 32, head dimension 64, fp16,
 // 33 key blocks per query block: 0.65 -> 0.075 ms (443 TFLOP/s); 32 prompts of 1032 to 2064 tokens, sbs 16, bf16, causal:
-// 0.54 -> 0.076 ms.
+// 0.54 -> 0.060 ms.
 //
 // Score pipeline (log2 domain), in the reference's order (blksprs/ops/flash_attention.py:1058-1224): scale * q k^T,
 // + bias, native causal predicate, explicit mask; probabilities are rounded to the operand type before they multiply
@@ -37,15 +37,16 @@ constexpr int kWaves = 4;
 template <int SBS, int NS>
 struct FwdShape {
   // Key blocks per step.  Two blocks of 32 leave registers for three waves per SIMD instead of four (97 against 84 us,
-  // 6144 rows of 33 blocks, head dimension 64); two blocks of 16 instead of four make no difference.
-  static constexpr int NB = SBS == 32 ? 1 : (NS <= 4 ? 4 : 2);
+  // 6144 rows of 33 blocks, head dimension 64); four blocks of 16 take twice the LDS, which leaves half the waves (76
+  // against 60 us, 4128 rows, causal, head dimension 64).
+  static constexpr int NB = SBS == 32 ? 1 : 2;
   using T = Tile<SBS, NS, NB>;
   static constexpr int kScores = SBS == 32 ? 16 * NB : 4 * NB;  // per lane and step
   static constexpr int kRegs = SBS == 32 ? 16 : 4;              // accumulator registers per block
   // K tile, V tile; at the end the partial output of a wave that shares a query block with others
   static constexpr int kPartial = SBS * SBS * NS * 4;
   static constexpr int kLds = (2 * T::kBytes > kPartial ? 2 * T::kBytes : kPartial) + 512;
-  static constexpr int kMinWaves = SBS == 32 ? (NS <= 2 ? 4 : 2) : (NS <= 2 ? 4 : 2);
+  static constexpr int kMinWaves = SBS == 32 ? (NS <= 2 ? 4 : 2) : (NS <= 4 ? 4 : 3);
 };
 
 // split: 1, 2 or 4 waves share one query block, each walking a contiguous part of its key list
@@ -53,6 +54,7 @@ template <typename Tr, int SBS, int NS>
 __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void attn_small_fwd_kernel(bsa_attn_args a, int split) {
   using Shape = FwdShape<SBS, NS>;
   using T = typename Shape::T;
+  using W = Walk<SBS, NS, Shape::NB, true>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs, kPiece = T::kPiece;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
@@ -60,17 +62,11 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
   const int wave = first_lane(threadIdx.x >> 6);
   char *lds_k = small_smem + wave * Shape::kLds, *lds_v = lds_k + T::kBytes;
 
-  // XCD c (workgroup g runs on XCD g % 8) takes a contiguous eighth of the query blocks, so that the waves in flight
-  // on one L2 share few batch entries' K and V; inside a batch entry the last query blocks, which are the long ones
-  // under a causal layout, come first.
-  const int per_group = kWaves / split;
-  const int64_t group = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const int64_t item = group * per_group + wave / split;
-  const int part = wave % split;
-  const bool has_row = item < a.B * a.nq;
-  const int64_t b = has_row ? item / a.nq : 0, qb = has_row ? a.nq - 1 - item % a.nq : 0;
-  const int64_t row = b * a.nq + qb;
+  const RowOfWave me(a.B, a.nq, true, wave, kWaves, split);
+  const int64_t row = me.b * a.nq + me.own;
   const int qi = lane % SBS, kq = lane / SBS;  // query row; which keys of a block this lane's registers hold
+  W walk;
+  walk.start(a, me.b, me.own, me.there, me.part, split);
 
   OwnRows<SBS, NS> qf;
   qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, lane);
@@ -83,125 +79,18 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
 
   const float qk_scale = a.scale * kLog2e;
   const float cc = a.bias ? 1.f : qk_scale;
-  int seq_len = 0x7fffffff;
-  if (a.causal_lengths) {
-    const int64_t len = a.causal_lengths[b];
-    seq_len = len < 0 ? 0 : (len > 0x7fffffffLL ? 0x7fffffff : (int)len);
-  }
-  int e_begin = first_lane(a.key_offsets[row]), e_end = first_lane(a.key_offsets[row + 1]);
-  if (split > 1) {
-    const int n = e_end - e_begin;
-    e_end = e_begin + (int)((int64_t)n * (part + 1) / split);
-    e_begin = e_begin + (int)((int64_t)n * part / split);
-  }
-  if (!has_row || (int)qb * SBS >= seq_len) e_end = e_begin;
-
-  // ---- The list, 64 entries at a time, one per lane: key block, packed index of the first K and V slice, mask and bias
-  // block.  Entries the causal predicate rules out are not in w_live; w_special marks those whose scores need more
-  // than the scale.  w_apart: some block's slices are missing or not one behind the other.
-  int w_base = e_begin - 64, w_kb = 0, w_pk = 0, w_pv = 0, w_pm = -1, w_pb = -1;
-  uint64_t w_live = 0, w_special = 0;
-  bool w_apart = false;
-  auto refill = [&]() {
-    const late_args_t p = late_args();
-    w_base += 64;
-    const int e = w_base + lane;
-    bool in = e < e_end;
-    w_kb = in ? p->key_indices[e] : 0;
-    const bool causal = p->causal_lengths != nullptr;
-    in = in && !(causal && (w_kb > (int)qb || w_kb * SBS >= seq_len));
-    const int64_t kv = b * p->nk + w_kb;
-    const int nh = (int)p->nh, nhv = (int)p->nhv;
-    bool apart = nh != NS || nhv != NS;
-    if (in && !apart) {
-      const int64_t *pk = p->pidx_k + kv * NS, *pv = p->pidx_v + kv * NS;
-      const int64_t k0 = pk[0], v0 = pv[0];
-      apart = k0 < 0 || v0 < 0 || k0 + NS > p->n_k_blocks || v0 + NS > p->n_v_blocks;
-#pragma unroll
-      for (int h = 1; h < NS; ++h) apart = apart || pk[h] != k0 + h || pv[h] != v0 + h;
-      w_pk = (int)k0;
-      w_pv = (int)v0;
-    }
-    w_apart = __any(in && apart);
-    bool special = causal && (w_kb == (int)qb || ((int)qb + 1) * SBS > seq_len || (w_kb + 1) * SBS > seq_len);
-    if (p->mask) {
-      const int64_t pm = in ? p->pidx_mask[row * p->nk + w_kb] : -1;
-      w_pm = pm < p->n_mask_blocks ? (int)pm : -1;
-      special = special || w_pm >= 0;
-    }
-    if (p->bias) {
-      const int64_t pb = in ? p->pidx_bias[row * p->nk + w_kb] : -1;
-      w_pb = pb < p->n_bias_blocks ? (int)pb : -1;
-      special = true;
-    }
-    w_live = __ballot(in);
-    w_special = __ballot(in && special);
-  };
-  // a step: how many entries it takes, their places in the window and whether their slices lie apart, and, if special,
-  // their facts (the window may be another one by the time the scores are formed)
-  struct Step {
-    int count, slot[NB], kb[NB], pm[NB], pb[NB];
-    bool special, apart;
-  };
-  auto take = [&](Step &s) {
-    while (w_live == 0 && w_base + 64 < e_end) refill();
-    s.count = 0;
-    uint64_t taken = 0;
-#pragma unroll
-    for (int t = 0; t < NB; ++t) {
-      const uint64_t lowest = w_live & -w_live;
-      s.slot[t] = lowest ? __builtin_ctzll(lowest) : 0;
-      s.count += lowest ? 1 : 0;
-      w_live ^= lowest;
-      taken |= lowest;
-    }
-    s.apart = w_apart;
-    s.special = (taken & w_special) != 0 || (NB > 1 && s.count < NB);
-    if (s.special) {
-#pragma unroll
-      for (int t = 0; t < NB; ++t) {
-        s.kb[t] = __builtin_amdgcn_readlane(w_kb, s.slot[t]);
-        s.pm[t] = t < s.count ? __builtin_amdgcn_readlane(w_pm, s.slot[t]) : -1;
-        s.pb[t] = t < s.count ? __builtin_amdgcn_readlane(w_pb, s.slot[t]) : -1;
-      }
-    }
-  };
   const uint32_t source = T::source_offset(lane);
   const char *const tensor_k = static_cast<const char *>(a.k), *const tensor_v = static_cast<const char *>(a.v);
-  // requests the step's K (V) blocks; returns whether exactly kCopies asynchronous copies are on their way
-  auto copy = [&](const Step &s, bool is_k) {
-    const char *tensor = is_k ? tensor_k : tensor_v;
-    char *dst = is_k ? lds_k : lds_v;
-    if (!s.apart) {
-#pragma unroll
-      for (int t = 0; t < NB; ++t) {
-        // a block that is not there: the copy of the one in front of it once more, its scores become -inf and its V zeros
-        if (NB == 1 || t < s.count)
-          T::copy_block(tensor, __builtin_amdgcn_readlane(is_k ? w_pk : w_pv, s.slot[t]), dst + t * T::kBlock, source, lane);
-      }
-      if (NB == 1 || s.count == NB) return true;
-    }
-    const late_args_t p = late_args();
-#pragma unroll
-    for (int t = 0; t < NB; ++t) {
-      if (!s.apart && t < s.count) continue;
-      const int n = t < s.count ? (int)(is_k ? p->nh : p->nhv) : 0;
-      const int64_t kv = b * p->nk + __builtin_amdgcn_readlane(w_kb, s.slot[t]);
-      T::gather_block(tensor, (is_k ? p->pidx_k : p->pidx_v) + kv * n, n, is_k ? p->n_k_blocks : p->n_v_blocks,
-                      dst + t * T::kBlock, source, lane);
-    }
-    return false;
-  };
 
   const typename T::RowReader k_rows(lds_k, lane);
   const typename T::ColReader v_cols(lds_v, lane);
-  Step now, next;
-  take(now);
+  typename W::Step now, next;
+  walk.take(now, lane);
   settle(qf);
   bool counted = false;  // exactly kCopies copies (the V tile's) were issued after the K tile's
   if (now.count) {
-    copy(now, true);
-    counted = copy(now, false);
+    walk.template copy<false>(now, tensor_k, lds_k, source, lane);
+    counted = walk.template copy<true>(now, tensor_v, lds_v, source, lane);
   }
   while (now.count) {
     // ---- S^T = K Q^T.  In flight at most: K and V of this step, in that order.
@@ -212,9 +101,9 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
 
     // ---- K of the next step
     wait_lds();
-    take(next);
+    walk.take(next, lane);
     counted = false;
-    if (next.count) counted = copy(next, true);
+    if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
 
     // ---- scores: sv holds them up to the positive factor cc, applied inside the exponential
     float sv[kScores];
@@ -222,47 +111,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
     for (int t = 0; t < NB; ++t)
 #pragma unroll
       for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
-    if (now.special) {
-      const late_args_t p = late_args();
-      const int qpos = (int)qb * SBS + qi;
-#pragma unroll
-      for (int t = 0; t < NB; ++t) {
-        float *s = sv + kRegs * t;
-        if (p->bias) {  // finished scores; the factor inside the exponential is 1 then
-          u32x2 bw[kRegs / 4];
-#pragma unroll
-          for (int w = 0; w < kRegs / 4; ++w) {
-            bw[w] = u32x2{0u, 0u};
-            if (now.pb[t] >= 0)
-              bw[w] = *reinterpret_cast<const u32x2 *>(static_cast<const char *>(p->bias) + (int64_t)now.pb[t] * kPiece +
-                                                       qi * (2 * SBS) + 16 * w + 8 * kq);
-          }
-#pragma unroll
-          for (int r = 0; r < kRegs; ++r)
-            s[r] = s[r] * qk_scale + Tr::widen((uint16_t)(bw[r / 4][(r % 4) / 2] >> (16 * (r % 2)))) * kLog2e;
-        }
-        if (now.pm[t] >= 0) {
-          const char *words = static_cast<const char *>(p->mask) + (int64_t)now.pm[t] * (SBS * SBS) + qi * SBS + 4 * kq;
-          uint32_t mw[kRegs / 4];
-#pragma unroll
-          for (int w = 0; w < kRegs / 4; ++w) mw[w] = *reinterpret_cast<const uint32_t *>(words + 8 * w);
-#pragma unroll
-          for (int r = 0; r < kRegs; ++r)
-            if ((mw[r / 4] >> (8 * (r % 4))) & 0xffu) s[r] = -INFINITY;
-        }
-        if (p->causal_lengths) {
-#pragma unroll
-          for (int r = 0; r < kRegs; ++r) {
-            const int kpos = now.kb[t] * SBS + 8 * (r / 4) + 4 * kq + r % 4;
-            if (kpos > qpos || qpos >= seq_len || kpos >= seq_len) s[r] = -INFINITY;
-          }
-        }
-        if (t >= now.count) {
-#pragma unroll
-          for (int r = 0; r < kRegs; ++r) s[r] = -INFINITY;
-        }
-      }
-    }
+    if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, qi, kq);
 
     // ---- online softmax of the row, the reference maximum following lazily (attn_mfma.hip)
     float m_blk = sv[0];
@@ -300,7 +149,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
     product_cols<Tr, SBS, NS, NB>(oacc, v_cols, pf);
     wait_lds();
     counted = false;
-    if (next.count) counted = copy(next, false);
+    if (next.count) counted = walk.template copy<true>(next, tensor_v, lds_v, source, lane);
     now = next;
   }
 
@@ -310,7 +159,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
     // every wave leaves (m, l, O) of its part; the first wave of a query block scales them to the common maximum and
     // adds them up, in order
     float *mine = reinterpret_cast<float *>(lds_k);
-    if (part != 0) {
+    if (me.part != 0) {
 #pragma unroll
       for (int h = 0; h < NS; ++h)
 #pragma unroll
@@ -323,7 +172,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
       }
     }
     __syncthreads();
-    if (part != 0) return;
+    if (me.part != 0) return;
     for (int p = 1; p < split; ++p) {
       const float *other = mine + p * (Shape::kLds / 4);
       const float m_o = other[Shape::kLds / 4 - 128 + 2 * qi], l_o = other[Shape::kLds / 4 - 128 + 2 * qi + 1];
@@ -343,7 +192,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
         }
     }
   }
-  if (!has_row) return;
+  if (!me.there) return;
   const late_args_t p = late_args();
   const int nhv = (int)p->nhv;
   const float inv_l = (l_i != 0.f) ? 1.f / l_i : 0.f;
@@ -368,12 +217,7 @@ template <typename Tr, int SBS, int NS>
 int launch(const bsa_attn_args &a, hipStream_t s) {
   using Shape = FwdShape<SBS, NS>;
   const int64_t rows = a.B * a.nq;
-  // A launch lasts as long as the serial walk of its longest lists, and the last round of a launch of few rounds is
-  // mostly empty: shorter shares of a list help until their prologue (four dependent loads) costs more than the walk.
-  // 64 rows (8 key blocks each, sbs 32): 9.6 us with two waves per row, 8.1 with four; 4128 rows (sbs 16, causal, up to
-  // 33 steps): 79 / 76 / 94 us with one, two, four; 6144 rows (sbs 32, 33 steps): 83 / 75 / 82.
-  const int split = rows <= 512 ? 4 : rows <= 8192 ? 2 : 1;
-  const int64_t groups = cdiv(cdiv(rows, (int64_t)(kWaves / split)), (int64_t)8) * 8;
+  const int split = waves_per_row(rows);
   constexpr int lds = Shape::kLds * kWaves;
   static_assert(lds <= 160 * 1024, "LDS");
   if (lds > 64 * 1024) {
@@ -381,7 +225,7 @@ int launch(const bsa_attn_args &a, hipStream_t s) {
         reinterpret_cast<const void *>(&attn_small_fwd_kernel<Tr, SBS, NS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     BSA_HIP(raised);
   }
-  attn_small_fwd_kernel<Tr, SBS, NS><<<(unsigned)groups, 64 * kWaves, lds, s>>>(a, split);
+  attn_small_fwd_kernel<Tr, SBS, NS><<<row_groups(rows, kWaves, split), 64 * kWaves, lds, s>>>(a, split);
   return check_launch("attn_small_fwd_kernel");
 }
 
@@ -414,15 +258,7 @@ int dispatch(const bsa_attn_args &a, hipStream_t s) {
 
 // 1: not covered
 int attn_fwd_small(const bsa_attn_args &a, hipStream_t s) {
-  if (a.sbs != 16 && a.sbs != 32) return 1;
-  if (a.dtype != BSA_BF16 && a.dtype != BSA_F16) return 1;
-  // the row maximum is taken before the scale is applied
-  if (!(a.scale > 0.f) || a.scale > 3.0e38f) return 1;
-  if (a.n_k_blocks > 0x7fffffffLL || a.n_v_blocks > 0x7fffffffLL || a.n_mask_blocks > 0x7fffffffLL ||
-      a.n_bias_blocks > 0x7fffffffLL)
-    return 1;
-  // positions are 32-bit numbers
-  if (a.nq * a.sbs > 0x7fffffffLL || a.nk * a.sbs > 0x7fffffffLL) return 1;
+  if (!small_applies(a)) return 1;
   if (a.B * a.nq == 0) return BSA_OK;
   return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, s) : dispatch<SF16>(a, s);
 }
