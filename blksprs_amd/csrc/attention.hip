@@ -1,7 +1,7 @@
-// C ABI of block-sparse flash attention: argument checks and the choice between the 16-bit matrix-core kernels (16-bit
-// operands; 64 x 64 blocks and at most two head slices in attn_mfma.hip, blocks of 16 and 32 and a head dimension of at
-// most 128 in attn_small_fwd.hip), the fp32 matrix-core kernels (the other operand types and head dimensions) and the
-// generic kernels (what neither takes: more head slices than fit LDS).
+// C ABI of block-sparse flash attention: argument checks and the choice of kernels: 16-bit operands in 64 x 64 blocks
+// with at most two head slices (attn_mfma.hip, attn_bwd_mfma.hip), blocks of 16 and 32 with head dimensions up to 128
+// (attn_small_fwd.hip, attn_small_bwd.hip), the rest on the fp32 matrix-core instruction (attn_f32mma.hip: fp32 blocks of
+// 64, longer head dimensions, scales that are not positive), and the generic kernels for more head slices than fit LDS.
 #include "attn_common.h"
 
 namespace {
@@ -48,7 +48,7 @@ extern "C" int bsa_attn_fwd(const bsa_attn_args *args, bsa_stream_t stream) {
   if (int rc = check_args("bsa_attn_fwd", args, false)) return rc;
   hipStream_t s = bsa::as_stream(stream);
   int rc = bsa::attn_fwd_mfma(*args, s);          // 16-bit operands, 64 x 64 blocks
-  if (rc == 1) rc = bsa::attn_fwd_small(*args, s);   // 16-bit operands, blocks of 16 and 32
+  if (rc == 1) rc = bsa::attn_fwd_small(*args, s);   // blocks of 16 and 32
   if (rc == 1) rc = bsa::attn_fwd_f32mma(*args, s);  // everything else, on the fp32 matrix-core instruction
   if (rc == 1) rc = bsa::attn_fwd_generic(*args, s);
   return rc;

@@ -1,4 +1,4 @@
-// Block-sparse flash attention backward for 16-bit operands in blocks of 16 and 32, on the 16-bit matrix cores (the
+// Block-sparse flash attention backward for blocks of 16 and 32 and head dimensions up to 128, fp16, bf16 and fp32 (the
 // forward kernel: attn_small_fwd.hip; tiles, fragments and the walk over a list: attn_small_common.h).
 //
 // Two launches, no atomics, fixed summation order.  The first gives a wave a query block: delta = rowsum(o * dO) from the
@@ -19,7 +19,8 @@
 // to overlap it; matrix cores 21 % busy in the second kernel.  Against the fp32 matrix-core kernels that ran these shapes
 // before (48 x 4096 queries, sbs 32, head dimension 64, fp16, 33 key blocks per query block): delta + zero fill
 // 0.071 -> 0, dK / dV 1.89 -> 0.125 ms, dQ 1.24 -> 0.096 ms (delta included); bf16, sbs 16, 32 causal sequences of 1032 to
-// 2064: dK / dV 0.067, dQ 0.065 ms.
+// 2064: dK / dV 0.067, dQ 0.065 ms; fp32, 8 x 2048 queries, sbs 32, half of the blocks, head dimension 64: dK / dV 0.238 -> 0.096,
+// dQ 0.198 -> 0.077 ms (89 and 84 TFLOP/s).
 //
 // Scores as in the forward kernel; p = exp2(s - lse), 0 where lse = -inf; P and dS are rounded to the operand type
 // before they enter a product (blksprs/ops/flash_attention.py:1452, :1468, :1692).
@@ -34,38 +35,30 @@ using namespace small;
 
 constexpr int kWaves = 4;
 
-template <int SBS, int NS>
+template <int ES, int SBS, int NS>
 struct BwdShape {
   static constexpr int NB = SBS == 32 ? 1 : 2;  // partner blocks per step
-  using T = Tile<SBS, NS, NB>;
+  using T = Tile<ES, SBS, NS, NB>;
   static constexpr int kRegs = SBS == 32 ? 16 : 4;
   static constexpr int kScores = kRegs * NB;
   static constexpr int kPartial = SBS * SBS * NS * 4;
   static constexpr int kStats = 256;  // lse and delta of the 32 queries of a step
   // dK / dV kernel: Q and dO of two steps where registers allow two waves per SIMD anyway (sbs 32: 133 against 137 us);
   // at sbs 16 one step's tiles and twice the waves are faster (67 against 92 us)
-  static constexpr int kBufs = SBS == 32 && NS <= 2 ? 2 : 1;
+  static constexpr int kBufs = ES == 2 && SBS == 32 && NS <= 2 ? 2 : 1;
   static constexpr int kKvBuf = 2 * T::kBytes + kStats;
   // the last row fragment of an odd number of slices of 16 reads (and drops) a slice beyond its tile
   static constexpr int kPad = T::kHalfLast ? T::kPiece : 0;
   static constexpr int kKvLds = kPad + (kBufs * kKvBuf > 2 * kPartial ? kBufs * kKvBuf : 2 * kPartial);
   static constexpr int kQLds = kPad + (2 * T::kBytes > kPartial ? 2 * T::kBytes : kPartial);
-  static constexpr int kQMinWaves = SBS == 32 ? (NS <= 2 ? 3 : 2) : (NS <= 4 ? 4 : 2);
-  static constexpr int kKvMinWaves = SBS == 32 ? (NS <= 3 ? 2 : 1) : (NS <= 4 ? 3 : 2);
+  static constexpr int kQMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS <= 2 ? 3 : 2) : (NS <= 4 ? 4 : 2);
+  static constexpr int kKvMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS <= 3 ? 2 : 1) : (NS <= 4 ? 3 : 2);
 };
 
 // 4 bytes per lane, global -> LDS: lane l's value lands at dst + 4 l
 __device__ inline void copy_words_to_lds(const float *addr, char *dst) {
   const uint32_t lds_addr = (uint32_t)(uintptr_t)(lds_ptr_t)dst;
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(addr), "s"(lds_addr) : "memory");
-}
-
-template <typename Tr, int kScores>
-__device__ inline void pack_scores(u32x4 (&w)[kScores / 8], const float *v) {
-#pragma unroll
-  for (int m = 0; m < kScores / 8; ++m)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w[m][i] = Tr::pack2(v[8 * m + 2 * i], v[8 * m + 2 * i + 1]);
 }
 
 // the partial sums of the waves that share a row, added up in order into those of the first
@@ -90,7 +83,7 @@ __device__ inline void add_partial(Acc (&acc)[NS], const float *other, int lane)
     }
 }
 
-// gradient blocks of the own row, eight bytes of a row per lane: columns 2 r + 4 group .. + 3
+// gradient blocks of the own row, columns 2 r + 4 group .. + 3 of a row per lane
 template <typename Tr, int SBS, int NS, typename Acc>
 __device__ inline void store_gradient(const Acc (&acc)[NS], float scale, void *out, const int64_t *pidx, int n_slices,
                                       int64_t n_blocks, int me, int group) {
@@ -100,22 +93,18 @@ __device__ inline void store_gradient(const Acc (&acc)[NS], float scale, void *o
     if (h >= n_slices) break;
     const int64_t p = pidx[h];
     if (p < 0 || p >= n_blocks) continue;
-    char *blk = static_cast<char *>(out) + p * (SBS * SBS * 2) + me * (2 * SBS) + 8 * group;
+    char *blk = static_cast<char *>(out) + (p * SBS * SBS + me * SBS + 4 * group) * Tr::kElem;
 #pragma unroll
-    for (int r = 0; r < kRegs; r += 4) {
-      u32x2 w;
-      w[0] = Tr::pack2(acc[h][r] * scale, acc[h][r + 1] * scale);
-      w[1] = Tr::pack2(acc[h][r + 2] * scale, acc[h][r + 3] * scale);
-      *reinterpret_cast<u32x2 *>(blk + 4 * r) = w;
-    }
+    for (int r = 0; r < kRegs; r += 4)
+      store4<Tr>(blk + 2 * r * Tr::kElem, acc[h][r] * scale, acc[h][r + 1] * scale, acc[h][r + 2] * scale, acc[h][r + 3] * scale);
   }
 }
 
 template <typename Tr, int SBS, int NS>
-__global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kQMinWaves)) void attn_small_dq_kernel(bsa_attn_args a, int split) {
-  using Shape = BwdShape<SBS, NS>;
+__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWaves)) void attn_small_dq_kernel(bsa_attn_args a, int split) {
+  using Shape = BwdShape<Tr::kElem, SBS, NS>;
   using T = typename Shape::T;
-  using W = Walk<SBS, NS, Shape::NB, true>;
+  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
@@ -129,18 +118,16 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kQMinWaves)) void 
   W walk;
   walk.start(a, me.b, me.own, me.there, me.part, split);
 
-  OwnRows<SBS, NS> qf, gf;
+  OwnRows<Tr::kElem, SBS, NS> qf, gf;
   qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, lane);
   gf.load(a.d_o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, lane);
   float delta = 0.f, neg_lse = -a.lse[row * SBS + qi];
   if (neg_lse == INFINITY) neg_lse = -INFINITY;  // a query that sees nothing: p = 0
   {
-    OwnRows<SBS, NS> of;
+    OwnRows<Tr::kElem, SBS, NS> of;
     of.load(a.o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, lane);
 #pragma unroll
-    for (int f = 0; f < T::kFrags; ++f)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) delta = Tr::dot2(of.fr[f][i], gf.fr[f][i], delta);
+    for (int f = 0; f < T::kFrags; ++f) delta = Tr::dot(of.fr[f], gf.fr[f], delta);
     delta = row_sum<SBS>(delta);
     if (me.there && me.part == 0 && kq == 0) a.delta[row * SBS + qi] = delta;
   }
@@ -206,11 +193,8 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kQMinWaves)) void 
           }
       }
     }
-    u32x4 w[kScores / 8];
-    pack_scores<Tr, kScores>(w, sv);
-
     // ---- dQ^T += K^T dS^T
-    product_cols<Tr, SBS, NS, NB>(dq, k_cols, w);
+    product_cols<Tr, SBS, NS, NB>(dq, k_cols, Weights<Tr, kScores>(sv));
     wait_lds();
     counted = false;
     if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
@@ -229,10 +213,10 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kQMinWaves)) void 
 }
 
 template <typename Tr, int SBS, int NS>
-__global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kKvMinWaves)) void attn_small_dkv_kernel(bsa_attn_args a, int split) {
-  using Shape = BwdShape<SBS, NS>;
+__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinWaves)) void attn_small_dkv_kernel(bsa_attn_args a, int split) {
+  using Shape = BwdShape<Tr::kElem, SBS, NS>;
   using T = typename Shape::T;
-  using W = Walk<SBS, NS, Shape::NB, false>;
+  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, false>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs, kBufs = Shape::kBufs;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
@@ -246,7 +230,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kKvMinWaves)) void
   W walk;
   walk.start(a, me.b, me.own, me.there, me.part, split);
 
-  OwnRows<SBS, NS> kf, vf;
+  OwnRows<Tr::kElem, SBS, NS> kf, vf;
   kf.load(a.k, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, lane);
   vf.load(a.v, a.pidx_v + row * a.nhv, (int)a.nhv, a.n_v_blocks, lane);
   acc_t dk[NS], dv[NS];
@@ -301,8 +285,8 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kKvMinWaves)) void
     typename T::RowReader q_rows = q_rows0, g_rows = g_rows0;
     typename T::ColReader q_cols = q_cols0, g_cols = g_cols0;
     if constexpr (kBufs == 2) {
-      q_rows.base0 += at, q_rows.base1 += at, g_rows.base0 += at, g_rows.base1 += at;
-      q_cols.base0 += at, q_cols.base1 += at, g_cols.base0 += at, g_cols.base1 += at;
+      q_rows.shift(at), g_rows.shift(at);
+      q_cols.shift(at), g_cols.shift(at);
     }
     const float *lse = reinterpret_cast<const float *>(lds + at + 2 * T::kBytes), *delta = lse + 32;
 
@@ -332,8 +316,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kKvMinWaves)) void
     }
 #pragma unroll
     for (int x = 0; x < kScores; ++x) sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], cc, -ls[x]));
-    u32x4 w[kScores / 8];
-    pack_scores<Tr, kScores>(w, sv);
+    const Weights<Tr, kScores> pw(sv);
 
     // ---- dS = P (dP - delta)
 #pragma unroll
@@ -343,7 +326,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kKvMinWaves)) void
       for (int i = 0; i < 4; ++i) sv[x + i] *= dp[x / kRegs][x % kRegs + i] - d4[i];
     }
     // ---- dV^T += dO^T P
-    product_cols<Tr, SBS, NS, NB>(dv, g_cols, w);
+    product_cols<Tr, SBS, NS, NB>(dv, g_cols, pw);
     if constexpr (kBufs == 1) {
       wait_lds();
       walk.take(next, lane);
@@ -353,8 +336,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<SBS, NS>::kKvMinWaves)) void
       }
     }
     // ---- dK^T += Q^T dS
-    pack_scores<Tr, kScores>(w, sv);
-    product_cols<Tr, SBS, NS, NB>(dk, q_cols, w);
+    product_cols<Tr, SBS, NS, NB>(dk, q_cols, Weights<Tr, kScores>(sv));
     if constexpr (kBufs == 1) {
       wait_lds();
       if (next.count) walk.template copy<false>(next, tensor_q, lds, source, lane);
@@ -396,7 +378,7 @@ int raise_lds(K kernel, int bytes) {
 
 template <typename Tr, int SBS, int NS>
 int launch(const bsa_attn_args &a, hipStream_t s) {
-  using Shape = BwdShape<SBS, NS>;
+  using Shape = BwdShape<Tr::kElem, SBS, NS>;
   constexpr int q_lds = Shape::kQLds * kWaves, kv_lds = Shape::kKvLds * kWaves;
   static_assert(q_lds <= 160 * 1024 && kv_lds <= 160 * 1024, "LDS");
   static const int raised = [] {
@@ -452,7 +434,7 @@ int dispatch(const bsa_attn_args &a, hipStream_t s) {
 // 1: not covered
 int attn_bwd_small(const bsa_attn_args &a, hipStream_t s) {
   if (!small_applies(a)) return 1;
-  return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, s) : dispatch<SF16>(a, s);
+  return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, s) : a.dtype == BSA_F16 ? dispatch<SF16>(a, s) : dispatch<SF32>(a, s);
 }
 
 }  // namespace bsa

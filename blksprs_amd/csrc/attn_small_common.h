@@ -1,11 +1,12 @@
-// Pieces shared by the 16-bit attention kernels for blocks of 16 and 32 (attn_small_fwd.hip, attn_small_bwd.hip):
-// LDS layout of a block slice, operand fragments, asynchronous copies of block slices, waits.
+// Pieces shared by the attention kernels for blocks of 16 and 32 (attn_small_fwd.hip, attn_small_bwd.hip): LDS layout of
+// a block slice, operand fragments, asynchronous copies of block slices, waits, the walk over a list of partner blocks.
 //
-// A block slice (SBS x SBS 16-bit elements, 512 or 2048 contiguous bytes in memory) lies row-major in LDS, the
-// 16-byte chunks of a row exchanged by chunk_swizzle(row).  It is read both ways: rows as they lie (contraction over
-// the head dimension: one 128-bit read per fragment) and columns through the transposing LDS read (contraction over
-// the sequence).  Products use v_mfma_f32_32x32x16 for blocks of 32 and v_mfma_f32_16x16x32 for blocks of 16, where
-// the 32 contracted values of a score product are two head slices and those of a value product two partner blocks.
+// A block slice (SBS x SBS elements, 512 bytes to 4 KiB, contiguous in memory) lies row-major in LDS, the 16-byte chunks
+// of a row exchanged by a function of the row.  It is read both ways: rows as they lie (contraction over the head
+// dimension: one 128-bit read per fragment) and columns (contraction over the sequence: the transposing LDS read for
+// 16-bit elements, 32-bit reads for fp32).  Products: 32x32x16 (blocks of 32) and 16x16x32 (blocks of 16, where the 32
+// contracted values of a score product are two head slices and those of a value product two partner blocks) for 16-bit
+// elements, 32x32x2 and 16x16x4 for fp32, whose contracted values are taken in an order that suits the 128-bit reads.
 #pragma once
 #include "attn_mfma_common.h"
 
@@ -15,13 +16,44 @@ namespace small {
 using namespace mfma;
 
 struct SBf16 : MBf16 {
-  __device__ static f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  static constexpr int kElem = 2;
+  // acc += fragment x fragment: 32 rows each, or 16
+  __device__ static void rows(f32x16 &acc, u32x4 a, u32x4 b) { acc = mfma(a, b, acc); }
+  __device__ static void rows(f32x4 &acc, u32x4 a, u32x4 b) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+  }
+  __device__ static float dot(u32x4 a, u32x4 b, float c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c = dot2(a[i], b[i], c);
+    return c;
   }
 };
 struct SF16 : MF16 {
-  __device__ static f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  static constexpr int kElem = 2;
+  __device__ static void rows(f32x16 &acc, u32x4 a, u32x4 b) { acc = mfma(a, b, acc); }
+  __device__ static void rows(f32x4 &acc, u32x4 a, u32x4 b) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0, 0, 0);
+  }
+  __device__ static float dot(u32x4 a, u32x4 b, float c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c = dot2(a[i], b[i], c);
+    return c;
+  }
+};
+struct SF32 {
+  static constexpr int kElem = 4;
+  __device__ static float as_float(uint32_t v) { return __builtin_bit_cast(float, v); }
+  __device__ static f32x16 one(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+  __device__ static f32x4 one(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+  template <typename Acc>
+  __device__ static void rows(Acc &acc, u32x4 a, u32x4 b) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = one(as_float(a[j]), as_float(b[j]), acc);
+  }
+  __device__ static float dot(u32x4 a, u32x4 b, float c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c = fmaf(as_float(a[i]), as_float(b[i]), c);
+    return c;
   }
 };
 
@@ -33,15 +65,22 @@ __device__ static inline void wait_vmem() {
 // LDS reads issued so far have returned: their buffer may be copied over
 __device__ static inline void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// XOR on the 16-byte chunk index of row r of a block slice.  Rows of 64 bytes (SBS 32): eight consecutive rows read at
-// one chunk index fall on different chunks of a 128-byte bank period and sixteen of a 256-byte one, and the four rows
-// r .. r + 3 (r a multiple of 4) of a transposing read use different halves of their rows.  Rows of 32 bytes (SBS 16):
-// the same for the row reads; a transposing read of four rows covers 128 consecutive bytes anyway.  Depends on
-// r % 16 only.
-template <int SBS>
+// XOR on the 16-byte chunk index of row r of a block slice.  Eight consecutive rows read at one chunk index must fall on
+// different chunks of a 128-byte bank period.  16-bit rows of 64 bytes (SBS 32): sixteen rows also spread over 256 bytes,
+// and the four rows r .. r + 3 (r a multiple of 4) of a transposing read use different halves of their rows.  16-bit rows
+// of 32 bytes: a transposing read of four rows covers 128 consecutive bytes anyway.  fp32 rows of 64 bytes (SBS 16) are
+// stored at row_place(r) so that the four rows r, r + 4, r + 8, r + 12 of a column read are neighbours.
+template <int ES, int SBS>
 __device__ static inline int chunk_swizzle(int r) {
-  if constexpr (SBS == 32) return ((((r >> 1) ^ (r >> 3)) & 1) << 1) | ((r >> 2) & 1);
+  if constexpr (ES == 4 && SBS == 32) return r & 7;
+  else if constexpr (ES == 4) return r & 3;
+  else if constexpr (SBS == 32) return ((((r >> 1) ^ (r >> 3)) & 1) << 1) | ((r >> 2) & 1);
   else return ((r >> 2) ^ (r >> 3)) & 1;
+}
+template <int ES, int SBS>
+__device__ static inline int row_place(int r) {
+  if constexpr (ES == 4 && SBS == 16) return 4 * (r & 3) + (r >> 2);
+  else return r;
 }
 
 // transposing LDS read of 8 bytes per lane
@@ -79,24 +118,22 @@ __device__ static inline void copy_kib_to_lds(const char *base, uint32_t off, ch
 }
 
 // Geometry of one wave's tile: NB partner blocks of NS head slices each, slice h of block t at piece t * NS + h.
-template <int SBS, int NS, int NB>
+template <int ES, int SBS, int NS, int NB>
 struct Tile {
-  static constexpr int kPiece = SBS * SBS * 2;
+  static constexpr int kPiece = SBS * SBS * ES;
+  static constexpr int kRowBytes = SBS * ES;
   static constexpr int kBlock = NS * kPiece;     // one partner block
   static constexpr int kBytes = NB * kBlock;
   static constexpr int kBlockCopies = (kBlock + 1023) / 1024;
   static constexpr int kCopies = NB * kBlockCopies;  // asynchronous copies per tile
 
-  // this lane's source offset for a copy that fills LDS linearly (all KiB of a block share it: the swizzle depends on
-  // row % 16 only, and a KiB holds 16 rows of 64 bytes or two slices of 16 rows of 32 bytes)
+  // This lane's source offset for a copy that fills LDS linearly.  All KiB of a block share it: a KiB holds eight rows
+  // of 128 bytes or sixteen of 64, or two slices of sixteen rows of 32 bytes.
   __device__ static inline uint32_t source_offset(int lane) {
-    if constexpr (SBS == 32) {
-      const int r = lane >> 2;
-      return (uint32_t)(r * 64 + (((lane & 3) ^ chunk_swizzle<32>(r)) << 4));
-    } else {
-      const int r = (lane & 31) >> 1;
-      return (uint32_t)((lane >> 5) * 512 + r * 32 + (((lane & 1) ^ chunk_swizzle<16>(r)) << 4));
-    }
+    constexpr int kChunks = kRowBytes / 16;
+    const int place = lane / kChunks % SBS;  // row_place is its own inverse
+    const int r = row_place<ES, SBS>(place);
+    return (uint32_t)((lane * 16 / kPiece) * kPiece + r * kRowBytes + (((lane % kChunks) ^ chunk_swizzle<ES, SBS>(r)) << 4));
   }
 
   // Requests block t of the tile, all of whose slices are there and lie one behind the other from packed index idx:
@@ -123,7 +160,7 @@ struct Tile {
 #pragma unroll
       for (int i = 0; i < kPiece; i += 1024) {
         u32x4 v{0u, 0u, 0u, 0u};
-        if (SBS == 32 || lane < 32) {
+        if (kPiece >= 1024 || lane < 32) {
           if (on) v = *reinterpret_cast<const u32x4 *>(tensor + idx * kPiece + i + offset);
           *reinterpret_cast<u32x4 *>(dst + h * kPiece + i + lane * 16) = v;
         }
@@ -131,140 +168,182 @@ struct Tile {
     }
   }
 
-  // ---- row fragments (contraction over the head dimension) ----
-  // SBS 32: fragment f of a block = values 16 f .. + 15 (2 per slice), this lane row lane % 32, values 8 (lane / 32) .. + 7.
-  // SBS 16: fragment f = slices 2 f, 2 f + 1, this lane row lane % 16, 8 values of slice 2 f + lane / 32 from
-  // 8 (lane / 16 % 2); behind the last slice of an odd count the upper half of the lanes hold zeros.  (The product of 16
-  // values for that slice is not used: its sum, fed by a product of 32 values right in front of it, came out without it.)
-  static constexpr int kFrags = SBS == 32 ? 2 * NS : (NS + 1) / 2;
-  static constexpr bool kHalfLast = SBS == 16 && (NS & 1);
+  // ---- row fragments (contraction over the head dimension): 16 bytes of a row per lane
+  // 16-bit, SBS 32: fragment f of a block = values 16 f .. + 15 (2 per slice), this lane row lane % 32, values
+  // 8 (lane / 32) .. + 7.  SBS 16: fragment f = slices 2 f, 2 f + 1, this lane row lane % 16, 8 values of slice
+  // 2 f + lane / 32 from 8 (lane / 16 % 2); behind the last slice of an odd count the upper half of the lanes hold zeros.
+  // (The product of 16 values for that slice is not used: its sum, fed by a product of 32 values right in front of it,
+  // came out without it.)
+  // fp32: fragment f = values 8 f .. + 7 (SBS 32) or 16 f .. + 15 (SBS 16), this lane row lane % SBS, the four values
+  // from 4 (lane / SBS); product j of the fragment contracts element j of every lane.
+  static constexpr int kFrags = ES == 4 ? NS * kRowBytes / 16 / (64 / SBS) : SBS == 32 ? 2 * NS : (NS + 1) / 2;
+  static constexpr int kSliceFrags = ES == 4 ? kFrags / NS : 2;  // of SBS 32 and fp32
+  static constexpr bool kHalfLast = ES == 2 && SBS == 16 && (NS & 1);
 
   struct RowReader {
-    const char *base0, *base1;  // SBS 32: even and odd fragments
-    bool beyond;                // SBS 16: this lane's half of the last fragment of an odd slice count is beyond the block
+    static constexpr int kBases = ES == 2 && SBS == 16 ? 1 : kSliceFrags;
+    const char *base[kBases];
+    bool beyond;  // 16-bit, SBS 16: this lane's half of the last fragment of an odd slice count is beyond the block
     __device__ RowReader(const char *lds, int lane) : beyond(lane >= 32) {
-      if constexpr (SBS == 32) {
-        const int r = lane & 31, c = (lane >> 5) ^ chunk_swizzle<32>(r);
-        base0 = lds + r * 64 + (c << 4);
-        base1 = lds + r * 64 + ((c ^ 2) << 4);
+      const int r = lane % SBS, g = lane / SBS, place = row_place<ES, SBS>(r) * kRowBytes, x = chunk_swizzle<ES, SBS>(r);
+      if constexpr (ES == 2 && SBS == 16) {
+        base[0] = lds + (g >> 1) * kPiece + place + (((g & 1) ^ x) << 4);
       } else {
-        const int r = lane & 15, g = lane >> 4;
-        base0 = base1 = lds + (g >> 1) * kPiece + r * 32 + (((g & 1) ^ chunk_swizzle<16>(r)) << 4);
+#pragma unroll
+        for (int i = 0; i < kBases; ++i) base[i] = lds + place + (((64 / SBS * i + g) ^ x) << 4);
       }
     }
+    __device__ void shift(int bytes) {
+#pragma unroll
+      for (int i = 0; i < kBases; ++i) base[i] += bytes;
+    }
     __device__ u32x4 frag(int t, int f) const {
-      if constexpr (SBS == 32) return *reinterpret_cast<const u32x4 *>(((f & 1) ? base1 : base0) + (t * NS + (f >> 1)) * kPiece);
-      u32x4 v = *reinterpret_cast<const u32x4 *>(base0 + (t * NS + 2 * f) * kPiece);
+      if constexpr (ES == 4 || SBS == 32)
+        return *reinterpret_cast<const u32x4 *>(base[f % kBases] + (t * NS + f / kBases) * kPiece);
+      u32x4 v = *reinterpret_cast<const u32x4 *>(base[0] + (t * NS + 2 * f) * kPiece);
       if (kHalfLast && f == kFrags - 1 && beyond) v = u32x4{0u, 0u, 0u, 0u};
       return v;
     }
   };
 
-  // ---- column fragments (contraction over the rows of the partner blocks) ----
-  // SBS 32: fragment m of block t, slice h: column lane % 32, rows 16 m + 4 kg .. + 3 and 16 m + 8 + 4 kg .. + 3
-  // (kg = lane / 32): the rows whose values a lane holds in accumulator registers 8 m .. 8 m + 7.
-  // SBS 16: fragment of blocks t and t + 1 (zeros for t + 1 == NB), slice h: column lane % 16, rows
-  // 4 (lane / 16) .. + 3 of either block: the rows of accumulator registers 0 .. 3 of the two blocks.
+  // ---- column fragments (contraction over the rows of the partner blocks)
+  // 16-bit, SBS 32: fragment m of block t, slice h: column lane % 32, rows 16 m + 4 kg .. + 3 and 16 m + 8 + 4 kg .. + 3
+  // (kg = lane / 32): the rows whose values a lane holds in accumulator registers 8 m .. 8 m + 7.  SBS 16: fragment of
+  // blocks t and t + 1, slice h: column lane % 16, rows 4 (lane / 16) .. + 3 of either block: the rows of accumulator
+  // registers 0 .. 3 of the two blocks.
+  // fp32: element (row of accumulator register r, column lane % SBS) of block t, slice h.
   struct ColReader {
-    const char *base0, *base1;  // SBS 32: first and second four rows of a fragment
+    static constexpr int kBases = ES == 4 ? 4 : SBS == 32 ? 2 : 1;
+    const char *base[kBases];
     __device__ ColReader(const char *lds, int lane) {
-      const int s = lane & 15;
-      if constexpr (SBS == 32) {
-        const int r = 4 * (lane >> 5) + (s >> 2), c = 2 * ((lane >> 4) & 1) + ((s & 3) >> 1);
-        base0 = lds + r * 64 + ((c ^ chunk_swizzle<32>(r)) << 4) + ((s & 1) << 3);
-        base1 = lds + (r + 8) * 64 + ((c ^ chunk_swizzle<32>(r + 8)) << 4) + ((s & 1) << 3);
+      if constexpr (ES == 4) {
+        const int c = lane % SBS, g = lane / SBS;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int r = 4 * g + j;
+          base[j] = lds + row_place<ES, SBS>(r) * kRowBytes + (((c >> 2) ^ chunk_swizzle<ES, SBS>(r)) << 4) + (c & 3) * 4;
+        }
       } else {
-        const int r = 4 * (lane >> 4) + (s >> 2), c = (s & 3) >> 1;
-        base0 = base1 = lds + r * 32 + ((c ^ chunk_swizzle<16>(r)) << 4) + ((s & 1) << 3);
+        const int s = lane & 15, half = SBS == 32 ? (lane >> 4) & 1 : 0;
+#pragma unroll
+        for (int i = 0; i < kBases; ++i) {
+          const int r = 8 * i + 4 * (lane / SBS) + (s >> 2), c = 2 * half + ((s & 3) >> 1);
+          base[i] = lds + r * kRowBytes + ((c ^ chunk_swizzle<ES, SBS>(r)) << 4) + ((s & 1) << 3);
+        }
       }
+    }
+    __device__ void shift(int bytes) {
+#pragma unroll
+      for (int i = 0; i < kBases; ++i) base[i] += bytes;
     }
     __device__ u32x4 frag(int t, int m, int h) const {
       u32x2 lo, hi;
       if constexpr (SBS == 32) {
-        lo = read_tr(base0 + (t * NS + h) * kPiece + m * 1024);
-        hi = read_tr(base1 + (t * NS + h) * kPiece + m * 1024);
+        lo = read_tr(base[0] + (t * NS + h) * kPiece + m * 1024);
+        hi = read_tr(base[kBases - 1] + (t * NS + h) * kPiece + m * 1024);
       } else {
-        lo = read_tr(base0 + ((t + 2 * m) * NS + h) * kPiece);
-        hi = read_tr(base0 + ((t + 2 * m + 1) * NS + h) * kPiece);
+        lo = read_tr(base[0] + ((t + 2 * m) * NS + h) * kPiece);
+        hi = read_tr(base[0] + ((t + 2 * m + 1) * NS + h) * kPiece);
       }
       return u32x4{lo[0], lo[1], hi[0], hi[1]};
+    }
+    __device__ float value(int t, int h, int r) const {
+      return *reinterpret_cast<const float *>(base[r % 4] + (t * NS + h) * kPiece + (r / 4) * 8 * kRowBytes);
     }
   };
 };
 
 // One block's own rows as the other operand of the score products, in registers for the whole walk (the same values
 // per lane as RowReader's fragments).
-template <int SBS, int NS>
+template <int ES, int SBS, int NS>
 struct OwnRows {
-  using T = Tile<SBS, NS, SBS == 32 ? 1 : 2>;
+  using T = Tile<ES, SBS, NS, 2>;
   u32x4 fr[T::kFrags];
 
   // pidx: packed indices of the block's slices, n_slices of them are there
   __device__ inline void load(const void *tensor, const int64_t *pidx, int n_slices, int64_t n_blocks, int lane) {
-    const char *p = static_cast<const char *>(tensor);
-    if constexpr (SBS == 32) {
+    const int r = lane % SBS, g = lane / SBS;
 #pragma unroll
-      for (int h = 0; h < NS; ++h) {
-        const int64_t idx = h < n_slices ? pidx[h] : -1;
-        const bool on = idx >= 0 && idx < n_blocks;
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-          fr[2 * h + m] = u32x4{0u, 0u, 0u, 0u};
-          if (on) fr[2 * h + m] = *reinterpret_cast<const u32x4 *>(p + idx * T::kPiece + (lane & 31) * 64 + (2 * m + (lane >> 5)) * 16);
-        }
-      }
-    } else {
-      const int g = lane >> 4;
-#pragma unroll
-      for (int f = 0; f < T::kFrags; ++f) {
-        const int h = 2 * f + (g >> 1);
-        const int64_t idx = h < n_slices ? pidx[h] : -1;
-        fr[f] = u32x4{0u, 0u, 0u, 0u};
-        if (idx >= 0 && idx < n_blocks)
-          fr[f] = *reinterpret_cast<const u32x4 *>(p + idx * T::kPiece + (lane & 15) * 32 + (g & 1) * 16);
-      }
+    for (int f = 0; f < T::kFrags; ++f) {
+      int h, chunk;
+      if constexpr (ES == 2 && SBS == 16) h = 2 * f + (g >> 1), chunk = g & 1;
+      else h = f / T::kSliceFrags, chunk = 64 / SBS * (f % T::kSliceFrags) + g;
+      const int64_t idx = h < n_slices ? pidx[h] : -1;
+      fr[f] = u32x4{0u, 0u, 0u, 0u};
+      if (idx >= 0 && idx < n_blocks)
+        fr[f] = *reinterpret_cast<const u32x4 *>(static_cast<const char *>(tensor) + idx * T::kPiece + r * T::kRowBytes + chunk * 16);
     }
   }
 };
 
 // Makes the compiler wait for the loads of the own rows here: left to their first use, the wait sits inside the loop and
 // is for every load in flight, each time round.
-template <int SBS, int NS>
-__device__ static inline void settle(OwnRows<SBS, NS> &own) {
+template <int ES, int SBS, int NS>
+__device__ static inline void settle(OwnRows<ES, SBS, NS> &own) {
 #pragma unroll
-  for (int f = 0; f < OwnRows<SBS, NS>::T::kFrags; ++f) asm volatile("" : "+v"(own.fr[f]));
+  for (int f = 0; f < OwnRows<ES, SBS, NS>::T::kFrags; ++f) asm volatile("" : "+v"(own.fr[f]));
 }
 
 // acc (per partner block t) = partner rows x own rows over all head slices: acc[t] belongs to this lane's own row
 // (lane % SBS) and partner rows 8 (r / 4) + 4 (lane / 32) + r % 4 (SBS 32) or 4 (lane / 16) + r (SBS 16).
 template <typename Tr, int SBS, int NS, int NB, typename Acc>
-__device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<SBS, NS, NB>::RowReader &rows,
-                                           const OwnRows<SBS, NS> &own) {
-  using T = Tile<SBS, NS, NB>;
+__device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<Tr::kElem, SBS, NS, NB>::RowReader &rows,
+                                           const OwnRows<Tr::kElem, SBS, NS> &own) {
 #pragma unroll
-  for (int t = 0; t < NB; ++t) {
+  for (int t = 0; t < NB; ++t)
 #pragma unroll
     for (int r = 0; r < (SBS == 32 ? 16 : 4); ++r) acc[t][r] = 0.f;
 #pragma unroll
-    for (int f = 0; f < T::kFrags; ++f) {
-      if constexpr (SBS == 32) acc[t] = Tr::mfma(rows.frag(t, f), own.fr[f], acc[t]);
-      else acc[t] = Tr::mfma16(rows.frag(t, f), own.fr[f], acc[t]);
-    }
+  for (int f = 0; f < Tile<Tr::kElem, SBS, NS, NB>::kFrags; ++f)
+#pragma unroll
+    for (int t = 0; t < NB; ++t) Tr::rows(acc[t], rows.frag(t, f), own.fr[f]);
+}
+
+// Probabilities (or dS) of a step, as the accumulators of its NB blocks hold them one after the other, made the second
+// operand of product_cols: rounded to the operand type and packed.
+template <typename Tr, int kScores>
+struct Weights {
+  u32x4 w[kScores / 8];
+  __device__ inline explicit Weights(const float *v) {
+#pragma unroll
+    for (int m = 0; m < kScores / 8; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[m][i] = Tr::pack2(v[8 * m + 2 * i], v[8 * m + 2 * i + 1]);
+  }
+};
+template <int kScores>
+struct Weights<SF32, kScores> {
+  float w[kScores];
+  __device__ inline explicit Weights(const float *v) {
+#pragma unroll
+    for (int x = 0; x < kScores; ++x) w[x] = v[x];
+  }
+};
+
+// out[h] += partner columns^T x weights
+template <typename Tr, int SBS, int NS, int NB, int kScores, typename Acc>
+__device__ static inline void product_cols(Acc (&out)[NS], const typename Tile<Tr::kElem, SBS, NS, NB>::ColReader &cols,
+                                           const Weights<Tr, kScores> &w) {
+  if constexpr (Tr::kElem == 4) {
+    constexpr int kRegs = kScores / NB;
+#pragma unroll
+    for (int x = 0; x < kScores; ++x)
+#pragma unroll
+      for (int h = 0; h < NS; ++h) out[h] = Tr::one(cols.value(x / kRegs, h, x % kRegs), w.w[x], out[h]);
+  } else {
+#pragma unroll
+    for (int h = 0; h < NS; ++h)
+#pragma unroll
+      for (int m = 0; m < kScores / 8; ++m)
+        Tr::rows(out[h], SBS == 32 ? cols.frag(m >> 1, m & 1, h) : cols.frag(0, m, h), w.w[m]);
   }
 }
 
-// out[h] += partner columns^T x weights, weights packed from accumulator registers: w[m] holds registers 8 m .. 8 m + 7
-// of the NB blocks' accumulators, one after the other
-template <typename Tr, int SBS, int NS, int NB, typename Acc>
-__device__ static inline void product_cols(Acc (&out)[NS], const typename Tile<SBS, NS, NB>::ColReader &cols,
-                                           const u32x4 (&w)[SBS == 32 ? 2 * NB : NB / 2]) {
-#pragma unroll
-  for (int h = 0; h < NS; ++h)
-#pragma unroll
-    for (int m = 0; m < (SBS == 32 ? 2 * NB : NB / 2); ++m) {
-      if constexpr (SBS == 32) out[h] = Tr::mfma(cols.frag(m >> 1, m & 1, h), w[m], out[h]);
-      else out[h] = Tr::mfma16(cols.frag(0, m, h), w[m], out[h]);
-    }
+// four consecutive values of an output row
+template <typename Tr>
+__device__ static inline void store4(char *p, float a, float b, float c, float d) {
+  if constexpr (Tr::kElem == 4) *reinterpret_cast<f32x4 *>(p) = f32x4{a, b, c, d};
+  else *reinterpret_cast<u32x2 *>(p) = u32x2{Tr::pack2(a, b), Tr::pack2(c, d)};
 }
 
 // Maximum / sum over the lanes that hold the same own row (lanes l, l + SBS, ...)
@@ -294,9 +373,9 @@ __device__ static inline float row_sum(float v) {
 // and V, or of Q and dO), its mask and bias block.  Entries the causal predicate rules out as a whole are left out of
 // `live`; `special` marks those whose scores need more than the scale; `apart` says that some block's slices are
 // missing or do not lie one behind the other.
-template <int SBS, int NS, int NB, bool kOwnIsQuery>
+template <int ES, int SBS, int NS, int NB, bool kOwnIsQuery>
 struct Walk {
-  using T = Tile<SBS, NS, NB>;
+  using T = Tile<ES, SBS, NS, NB>;
   int64_t b, own;          // batch entry, own block
   int end, base, seq_len;  // end of the list, first entry of the window; valid length of a causal sequence
   int other, first_a, first_b, mask, bias;  // of this lane's entry
@@ -435,20 +514,18 @@ struct Walk {
       if (p->bias) {
         const char *blk = static_cast<const char *>(p->bias) + (int64_t)s.bias[t] * T::kPiece;
 #pragma unroll
-        for (int w = 0; w < kRegs / 4; ++w) {
-          u32x2 bw{0u, 0u};
-          if (s.bias[t] >= 0) {
-            if constexpr (kOwnIsQuery) {
-              bw = *reinterpret_cast<const u32x2 *>(blk + me * (2 * SBS) + 16 * w + 8 * group);
-            } else {
-              const uint16_t *col = reinterpret_cast<const uint16_t *>(blk) + (8 * w + 4 * group) * SBS + me;
-              bw = u32x2{col[0] | (uint32_t)col[SBS] << 16, col[2 * SBS] | (uint32_t)col[3 * SBS] << 16};
-            }
-          }
+        for (int w = 0; w < kRegs / 4; ++w)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            v[4 * w + i] = v[4 * w + i] * qk_scale + Tr::widen((uint16_t)(bw[i / 2] >> (16 * (i % 2)))) * kLog2e;
-        }
+          for (int i = 0; i < 4; ++i) {
+            const int theirs = 8 * w + 4 * group + i;
+            const int at = kOwnIsQuery ? me * SBS + theirs : theirs * SBS + me;
+            float bias_value = 0.f;
+            if (s.bias[t] >= 0) {
+              if constexpr (ES == 4) bias_value = reinterpret_cast<const float *>(blk)[at];
+              else bias_value = Tr::widen(reinterpret_cast<const uint16_t *>(blk)[at]);
+            }
+            v[4 * w + i] = v[4 * w + i] * qk_scale + bias_value * kLog2e;
+          }
       }
       if (s.mask[t] >= 0) {
         const uint8_t *blk = static_cast<const uint8_t *>(p->mask) + (int64_t)s.mask[t] * (SBS * SBS);
@@ -485,7 +562,6 @@ struct Walk {
 // Whether the kernels for blocks of 16 and 32 take these arguments (up to the head slices they are built for)
 inline bool small_applies(const bsa_attn_args &a) {
   if (a.sbs != 16 && a.sbs != 32) return false;
-  if (a.dtype != BSA_BF16 && a.dtype != BSA_F16) return false;
   // the forward kernel takes the row maximum before the scale is applied
   if (!(a.scale > 0.f) || a.scale > 3.0e38f) return false;
   const int64_t most = 0x7fffffffLL;  // indices and positions are 32-bit numbers

@@ -1,4 +1,5 @@
-// Block-sparse flash attention forward for 16-bit operands in blocks of 16 and 32, on the 16-bit matrix cores.
+// Block-sparse flash attention forward for blocks of 16 and 32 and head dimensions up to 128, fp16, bf16 and fp32, on the
+// matrix cores of the operand type.
 //
 // A wave owns one query block (or a share of its key list, below) and walks the list alone: no barrier, no tile
 // shared between waves, so waves of a compute unit drift apart and fill each other's waits.  A step takes one key
@@ -17,7 +18,9 @@
 // wave at a time; matrix cores 16 % busy, 113 vector and 63 scalar instructions per step of 32 x 32 at head dimension 64.
 // Against the fp32 matrix-core kernel that ran these shapes before: 48 x 4096 queries, sbs 32, head dimension 64, fp16,
 // 33 key blocks per query block: 0.65 -> 0.075 ms (443 TFLOP/s); 32 prompts of 1032 to 2064 tokens, sbs 16, bf16, causal:
-// 0.54 -> 0.060 ms.
+// 0.54 -> 0.060 ms.  fp32, where the products take eight times as long and hide the rest: 8 x 2048 queries, half of the
+// blocks, head dimension 64: 0.089 -> 0.054 ms (80 TFLOP/s, half of the fp32 matrix-core peak; 512 lists of 32 +- 4 blocks
+// cut in four fill the chip once, so the launch waits for the longest).
 //
 // Score pipeline (log2 domain), in the reference's order (blksprs/ops/flash_attention.py:1058-1224): scale * q k^T,
 // + bias, native causal predicate, explicit mask; probabilities are rounded to the operand type before they multiply
@@ -34,27 +37,27 @@ using namespace small;
 constexpr float kRescaleStep = 8.f;  // log2 units, see attn_mfma.hip
 constexpr int kWaves = 4;
 
-template <int SBS, int NS>
+template <int ES, int SBS, int NS>
 struct FwdShape {
   // Key blocks per step.  Two blocks of 32 leave registers for three waves per SIMD instead of four (97 against 84 us,
   // 6144 rows of 33 blocks, head dimension 64); four blocks of 16 take twice the LDS, which leaves half the waves (76
   // against 60 us, 4128 rows, causal, head dimension 64).
   static constexpr int NB = SBS == 32 ? 1 : 2;
-  using T = Tile<SBS, NS, NB>;
+  using T = Tile<ES, SBS, NS, NB>;
   static constexpr int kScores = SBS == 32 ? 16 * NB : 4 * NB;  // per lane and step
   static constexpr int kRegs = SBS == 32 ? 16 : 4;              // accumulator registers per block
   // K tile, V tile; at the end the partial output of a wave that shares a query block with others
   static constexpr int kPartial = SBS * SBS * NS * 4;
   static constexpr int kLds = (2 * T::kBytes > kPartial ? 2 * T::kBytes : kPartial) + 512;
-  static constexpr int kMinWaves = SBS == 32 ? (NS <= 2 ? 4 : 2) : (NS <= 4 ? 4 : 3);
+  static constexpr int kMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS <= 2 ? 4 : 2) : (NS <= 4 ? 4 : 3);
 };
 
 // split: 1, 2 or 4 waves share one query block, each walking a contiguous part of its key list
 template <typename Tr, int SBS, int NS>
-__global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void attn_small_fwd_kernel(bsa_attn_args a, int split) {
-  using Shape = FwdShape<SBS, NS>;
+__global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWaves)) void attn_small_fwd_kernel(bsa_attn_args a, int split) {
+  using Shape = FwdShape<Tr::kElem, SBS, NS>;
   using T = typename Shape::T;
-  using W = Walk<SBS, NS, Shape::NB, true>;
+  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs, kPiece = T::kPiece;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
@@ -68,7 +71,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
   W walk;
   walk.start(a, me.b, me.own, me.there, me.part, split);
 
-  OwnRows<SBS, NS> qf;
+  OwnRows<Tr::kElem, SBS, NS> qf;
   qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, lane);
   acc_t oacc[NS];
 #pragma unroll
@@ -137,11 +140,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
       sum += sv[x];
     }
     l_i += sum;
-    u32x4 pf[kScores / 8];
-#pragma unroll
-    for (int m = 0; m < kScores / 8; ++m)
-#pragma unroll
-      for (int w = 0; w < 4; ++w) pf[m][w] = Tr::pack2(sv[8 * m + 2 * w], sv[8 * m + 2 * w + 1]);
+    const Weights<Tr, kScores> pf(sv);
 
     // ---- O^T += V^T P^T.  In flight at most: V of this step, K of the next.
     if (counted) wait_vmem<T::kCopies>();
@@ -203,19 +202,16 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<SBS, NS>::kMinWaves)) void a
     if (po < 0 || po >= p->n_o_blocks) continue;
     char *out = static_cast<char *>(p->o) + po * kPiece;
 #pragma unroll
-    for (int r = 0; r < kRegs; r += 4) {  // eight bytes of a row per lane: columns 2 r + 4 kq .. + 3
-      u32x2 w;
-      w[0] = Tr::pack2(oacc[h][r] * inv_l, oacc[h][r + 1] * inv_l);
-      w[1] = Tr::pack2(oacc[h][r + 2] * inv_l, oacc[h][r + 3] * inv_l);
-      *reinterpret_cast<u32x2 *>(out + qi * (2 * SBS) + 4 * r + 8 * kq) = w;
-    }
+    for (int r = 0; r < kRegs; r += 4)  // columns 2 r + 4 kq .. + 3 of a row per lane
+      store4<Tr>(out + (qi * SBS + 2 * r + 4 * kq) * Tr::kElem, oacc[h][r] * inv_l, oacc[h][r + 1] * inv_l,
+                 oacc[h][r + 2] * inv_l, oacc[h][r + 3] * inv_l);
   }
   if (kq == 0) p->lse[row * SBS + qi] = (l_i != 0.f) ? m_i + log2f(l_i) : -INFINITY;
 }
 
 template <typename Tr, int SBS, int NS>
 int launch(const bsa_attn_args &a, hipStream_t s) {
-  using Shape = FwdShape<SBS, NS>;
+  using Shape = FwdShape<Tr::kElem, SBS, NS>;
   const int64_t rows = a.B * a.nq;
   const int split = waves_per_row(rows);
   constexpr int lds = Shape::kLds * kWaves;
@@ -260,7 +256,7 @@ int dispatch(const bsa_attn_args &a, hipStream_t s) {
 int attn_fwd_small(const bsa_attn_args &a, hipStream_t s) {
   if (!small_applies(a)) return 1;
   if (a.B * a.nq == 0) return BSA_OK;
-  return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, s) : dispatch<SF16>(a, s);
+  return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, s) : a.dtype == BSA_F16 ? dispatch<SF16>(a, s) : dispatch<SF32>(a, s);
 }
 
 }  // namespace bsa

@@ -1,4 +1,4 @@
-"""The 16-bit attention kernels for blocks of 16 and 32 (attn_small_fwd.hip, attn_small_bwd.hip) at the edges of their
+"""The attention kernels for blocks of 16 and 32 (attn_small_fwd.hip, attn_small_bwd.hip) at the edges of their
 tiles and of their dispatch: every number of head slices they are built for and one more, different numbers for q / k
 and v, key lists of one block, of a step and one more, of more than the 64 entries of a window, launches small and
 large enough for every way of sharing a list between waves."""
@@ -11,7 +11,10 @@ from tests.test_attention_gpu import _run_case
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+DTYPES = [torch.float16, torch.bfloat16, torch.float32]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("sbs,nh,nhv", [(16, n, n) for n in range(1, 10)] + [(32, n, n) for n in range(1, 6)]
                          + [(16, 3, 5), (16, 6, 2), (32, 1, 3), (32, 4, 2)])
 def test_head_slices(device, dtype, sbs, nh, nhv):
@@ -20,18 +23,20 @@ def test_head_slices(device, dtype, sbs, nh, nhv):
               use_bias=True, sparse_heads=True, custom_o=True)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("sbs", [16, 32])
 @pytest.mark.parametrize("nk", [1, 4, 5, 63, 64, 65, 150])
-def test_list_lengths(device, sbs, nk):
-    _run_case(device, torch.bfloat16, sbs, B=1, nq=2, nk=nk, nh=2, nhv=2, density=1.0, seed=nk)
-    _run_case(device, torch.float16, sbs, B=1, nq=5, nk=nk, nh=2, nhv=2, density=0.5, seed=nk + 1, use_mask=True)
+def test_list_lengths(device, dtype, sbs, nk):
+    _run_case(device, dtype, sbs, B=1, nq=2, nk=nk, nh=2, nhv=2, density=1.0, seed=nk)
+    _run_case(device, dtype, sbs, B=1, nq=5, nk=nk, nh=2, nhv=2, density=0.5, seed=nk + 1, use_mask=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("sbs", [16, 32])
 @pytest.mark.parametrize("B,n", [(1, 70), (9, 64), (140, 60)])
 @pytest.mark.parametrize("use_causal", [False, True])
-def test_rows_of_a_launch(device, sbs, B, n, use_causal):
+def test_rows_of_a_launch(device, dtype, sbs, B, n, use_causal):
     """70, 576 and 8400 query blocks: four, two and one wave per query block (and per key block)."""
     nk = n if use_causal else 3
-    _run_case(device, torch.bfloat16, sbs, B=B, nq=n, nk=nk, nh=1, nhv=1, density=0.1 if use_causal else 0.6,
+    _run_case(device, dtype, sbs, B=B, nq=n, nk=nk, nh=1, nhv=1, density=0.1 if use_causal else 0.6,
               seed=B + n, use_causal=use_causal)
