@@ -1,12 +1,11 @@
 // Block-sparse GEMM: out[n] = sum over the contraction list of block n of x[px] @ y[py].
 //
-// One wavefront owns one TILE x TILE tile of one output block (TILE = min(sbs, 64))
-// and walks that block's list of (x block, y block) pairs in ascending k, so only
-// non-zero K-blocks are touched and the fp32 accumulation order is fixed.  Four
-// waves (four neighbouring tiles) share a workgroup but never synchronise: each
-// has a private 16 KiB LDS region.
+// sbs 32: one wavefront owns one output block (TILE = 32) and walks that block's list of (x block, y block) pairs in
+// ascending k, so only non-zero K-blocks are touched and the fp32 accumulation order is fixed.  Four waves (four
+// neighbouring blocks) share a workgroup but never synchronise: each has a private LDS region.
+// Larger blocks: matmul_quad_kernel, further down.
 //
-// Data path per K-chunk (64 k for 16-bit types, 32 k for fp32):
+// Data path per K-chunk (32 k):
 //   global --16 B per lane, consecutive lanes = consecutive bytes--> VGPRs
 //          --ds_write_b128--> LDS --> MFMA operand fragments --> v_mfma_f32_32x32x*.
 // The loads of chunk t+1 are issued before the MFMAs of chunk t.
@@ -31,7 +30,7 @@
 
 #include <type_traits>
 
-#include "common.h"
+#include "attn_mfma_common.h"
 
 namespace {
 
@@ -41,6 +40,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 // native vector (not HIP's uint4 struct): arrays of it are always promoted to registers
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef short i16x4 __attribute__((ext_vector_type(4)));
 
 struct Bf16Traits {
   static constexpr int kElem = 2;
@@ -398,6 +399,180 @@ __global__ __launch_bounds__(256, 2) void matmul_mfma_kernel(const char *__restr
   }
 }
 
+// ---- LDS chunks of the kernel whose workgroup shares a tile: 64 rows of 128 bytes (k contiguous, or 16-bit k rows), or
+// 32 k rows of 256 bytes (fp32, k strided)
+
+// chunk index XOR of a 128-byte row, by row % 8: row reads of eight consecutive rows fall on eight chunks; for 16-bit
+// elements also the four rows of a transposing read on different halves of their rows
+template <int ES>
+__device__ inline int quad_swizzle(int r) {
+  return ES == 2 ? bsa::mfma::t_swizzle(r & 7) : r & 7;
+}
+// 16 bytes of k of one row
+template <int ES>
+__device__ inline u32x4 quad_rows(const char *lds, int row, int chunk) {
+  return *reinterpret_cast<const u32x4 *>(lds + row * 128 + ((chunk ^ quad_swizzle<ES>(row)) << 4));
+}
+// the same values of k (step s: 16-bit 16 s + 8 (lane / 32) .. + 7, fp32 8 s + 4 (lane / 32) .. + 3) of column
+// col0 + lane % 32, from k rows
+template <int ES>
+__device__ inline u32x4 quad_cols(const char *lds, int col0, int s, int lane) {
+  const int kg = lane >> 5;
+  if constexpr (ES == 2) {
+    const int chunk = (col0 >> 3) + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+    u32x4 v;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = 16 * s + 8 * kg + 4 * i + ((lane & 15) >> 2);
+      const char *p = lds + r * 128 + ((chunk ^ quad_swizzle<2>(r)) << 4) + ((lane & 1) << 3);
+      const auto t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4 *)p);
+      const u32x2 w = __builtin_bit_cast(u32x2, t);
+      v[2 * i] = w[0];
+      v[2 * i + 1] = w[1];
+    }
+    return v;
+  } else {
+    const uint32_t *p = reinterpret_cast<const uint32_t *>(lds) + (8 * s + 4 * kg) * 64 + col0 + (lane & 31);
+    return u32x4{p[0], p[64], p[128], p[192]};
+  }
+}
+
+// sbs >= 64 on the tile path: fp32, and 16-bit elements at sbs 128 and above (or where neither the row nor the line kernel
+// applies).  A workgroup of four waves owns one 64 x 64 tile of an output block, each wave a 32 x 32 quadrant, and walks
+// the block's pair list in chunks of 128 bytes of k; the chunk of x and the chunk of y lie in LDS for all four waves,
+// double buffered, copied asynchronously while the chunk before is multiplied, with one barrier per chunk.
+//
+// What this split is for: lists differ in length (a few pairs, Poisson-like), and a wave that owns a whole 64 x 64 tile
+// takes the whole difference: 2080 tiles of 4 to 16 pairs on 2048 places of a wave (two per SIMD, by registers and LDS) run
+// as long as the SIMD with the two longest, and a workgroup of four such tiles holds its LDS until the longest is done.
+// Here the four waves of a workgroup are equal, five workgroups share a compute unit, and tiles are handed out as places
+// become free.  fp32, 8 x 2048^3 at 25 %: 0.126 -> 0.103
+// ms forward, 0.134 and 0.125 -> 0.099 ms for the gradients (83 TFLOP/s; a dense layout 118, rocBLAS' fp32 product 154);
+// bf16, sbs 128, 8 x 2944 x 3968 x 2048 at 25 %: 0.064 -> 0.059, 0.061 -> 0.055, 0.064 -> 0.052 ms.  What is left is the
+// chain in front of a tile's first chunk (order, offsets, pairs, operands) and the last tiles of a launch.
+template <typename Tr, bool XT, bool YT>
+__global__ __launch_bounds__(256, 5) void matmul_quad_kernel(const char *__restrict__ x, const char *__restrict__ y,
+                                                             char *__restrict__ out,
+                                                             const int32_t *__restrict__ pair_offsets,
+                                                             const int32_t *__restrict__ pairs,
+                                                             const int32_t *__restrict__ block_order, int64_t n_tiles,
+                                                             int sbs, int side_log2, int64_t nnz_x, int64_t nnz_y) {
+  constexpr int ES = Tr::kElem, KC = 128 / ES;  // k per chunk
+  constexpr int kOperand = 64 * 128, kBuffer = 2 * kOperand;
+  __shared__ __attribute__((aligned(1024))) char smem[2 * kBuffer];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wi = wave >> 1, wj = wave & 1;  // the wave's quadrant
+  // XCD c takes the c-th contiguous eighth of the ordered work list (workgroup g runs on XCD g % 8)
+  const int64_t item = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (item >= n_tiles) return;
+  const int64_t per_block = (int64_t)1 << (2 * side_log2);
+  const int64_t n = block_order ? (int64_t)__builtin_amdgcn_readfirstlane(block_order[item >> (2 * side_log2)])
+                                : item >> (2 * side_log2);
+  const int tile = (int)(item & (per_block - 1));
+  const int ti = tile >> side_log2, tj = tile & ((1 << side_log2) - 1);
+  const int64_t block_bytes = (int64_t)sbs * sbs * ES;
+  const uint32_t ld = (uint32_t)sbs * ES;
+  const int n_chunks = sbs / KC;  // per pair
+
+  const int p_begin = __builtin_amdgcn_readfirstlane(pair_offsets[n]);
+  const int p_end = __builtin_amdgcn_readfirstlane(pair_offsets[n + 1]);
+
+  // Copies: one instruction moves 1 KiB, lane l supplying the 16 bytes at position l; wave w takes KiB 2 w and 2 w + 1 of
+  // either chunk.  An operand whose k is contiguous: 64 rows of 128 bytes, eight to a KiB, chunk index swizzled by the row.
+  // Otherwise KC rows of k: 128 bytes each (16-bit, the same swizzle) or 256 (fp32, as they lie).
+  const int row8 = lane >> 3;
+  const uint32_t off128 = (uint32_t)row8 * ld + (uint32_t)(((lane & 7) ^ quad_swizzle<ES>(row8)) << 4);
+  const uint32_t off256 = (uint32_t)(lane >> 4) * ld + (uint32_t)((lane & 15) << 4);
+  auto copy_operand = [&](const char *base, bool k_strided, char *dst) {
+    const bool wide = ES == 4 && k_strided;
+    const int rows = wide ? 4 : 8;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      bsa::mfma::copy_1k_to_lds(base + (int64_t)((2 * wave + i) * rows) * ld, wide ? off256 : off128, dst + (2 * wave + i) * 1024);
+  };
+  // 64 entries of the pair list at a time, one per lane
+  int win_base = p_begin, win_x = 0, win_y = 0;
+  auto load_window = [&]() {
+    const int t = win_base + lane;
+    win_x = win_y = 0;
+    if (t < p_end) {
+      const int2 v = *reinterpret_cast<const int2 *>(pairs + 2 * (int64_t)t);
+      win_x = v.x;
+      win_y = v.y;
+    }
+  };
+  int p = p_begin, kc = 0;  // next chunk to request
+  auto request = [&](char *buf) {
+    if (p - win_base >= 64) {
+      win_base += 64;
+      load_window();
+    }
+    const int sel = p - win_base;
+    int64_t px = __builtin_amdgcn_readlane(win_x, sel), py = __builtin_amdgcn_readlane(win_y, sel);
+    // a corrupt list must not turn into a wild read
+    px = (px < 0 || px >= nnz_x) ? 0 : px;
+    py = (py < 0 || py >= nnz_y) ? 0 : py;
+    // x: rows i from 64 ti, k from kc KC; y: k likewise, columns j from 64 tj; a transposed operand is stored the other way
+    const int64_t k_along = (int64_t)kc * 128, k_down = (int64_t)kc * KC * ld;
+    const int64_t i_down = (int64_t)ti * 64 * ld, i_along = (int64_t)ti * 64 * ES;
+    const int64_t j_down = (int64_t)tj * 64 * ld, j_along = (int64_t)tj * 64 * ES;
+    copy_operand(x + px * block_bytes + (XT ? k_down + i_along : i_down + k_along), XT, buf);
+    copy_operand(y + py * block_bytes + (YT ? j_down + k_along : k_down + j_along), !YT, buf + kOperand);
+    if (++kc == n_chunks) kc = 0, ++p;
+  };
+
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  const int n_iter = (p_end - p_begin) * n_chunks;
+  const int li = lane & 31, kg = lane >> 5;
+  if (n_iter > 0) {
+    load_window();
+    request(smem);
+  }
+  for (int it = 0; it < n_iter; ++it) {
+    // the copies of this chunk have landed and, behind the barrier, those of the other waves too; nobody reads the other
+    // buffer any more
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    if (it + 1 < n_iter) request(smem + ((it + 1) & 1) * kBuffer);
+    const char *bx = smem + (it & 1) * kBuffer, *by = bx + kOperand;
+    u32x4 fx[4], fy[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      fx[s] = XT ? quad_cols<ES>(bx, 32 * wi, s, lane) : quad_rows<ES>(bx, 32 * wi + li, 2 * s + kg);
+      fy[s] = YT ? quad_rows<ES>(by, 32 * wj + li, 2 * s + kg) : quad_cols<ES>(by, 32 * wj, s, lane);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc = Tr::mfma(fy[s], fx[s], acc);
+  }
+
+  // acc[r] = O[i = 32 wi + lane % 32][j = 32 wj + 8 (r / 4) + 4 (lane / 32) + r % 4]: through LDS (the wave's own 4 KiB,
+  // when nobody reads the tiles any more) into whole rows of the quadrant, stored past the caches
+  __syncthreads();
+  constexpr int kRow = 32 * ES, kChunks = kRow / 16;
+  char *stage = smem + wave * 4096;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int at = (8 * q + 4 * kg) * ES;  // byte of the row
+    char *dst = stage + li * kRow + ((((at >> 4) ^ li) & (kChunks - 1)) << 4) + (at & 15);
+    if constexpr (ES == 2)
+      *reinterpret_cast<uint2 *>(dst) = uint2{(uint32_t)Tr::round(acc[4 * q]) | ((uint32_t)Tr::round(acc[4 * q + 1]) << 16),
+                                              (uint32_t)Tr::round(acc[4 * q + 2]) | ((uint32_t)Tr::round(acc[4 * q + 3]) << 16)};
+    else
+      *reinterpret_cast<f32x4 *>(dst) = f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  char *ob = out + n * block_bytes + (int64_t)(64 * ti + 32 * wi) * ld + (64 * tj + 32 * wj) * ES;
+#pragma unroll
+  for (int t = 0; t < 32 * kChunks / 64; ++t) {
+    const int row = (t * 64 + lane) / kChunks, chunk = lane & (kChunks - 1);
+    const u32x4 v = *reinterpret_cast<const u32x4 *>(stage + row * kRow + (((chunk ^ row) & (kChunks - 1)) << 4));
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(ob + row * ld + chunk * 16));
+  }
+}
+
 // sbs == 16: one wave per output block, fp32 FMAs; lane -> row lane/4, columns 4*(lane%4)..+3
 template <typename Tr>
 __global__ __launch_bounds__(256) void matmul_small_kernel(const typename Tr::store_t *__restrict__ x,
@@ -454,8 +629,6 @@ __global__ __launch_bounds__(256) void matmul_small_kernel(const typename Tr::st
 // per pair instead of two, which is what the kernel's time follows); both pass through 1 KiB of LDS, from which
 // an operand whose contraction index is contiguous in memory (x, or y when it is used transposed) is read as it
 // lies and the other one through the transposing read.
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
 struct Bf16Small {
@@ -599,6 +772,29 @@ int launch_mfma(const void *x, const void *y, void *out, const int32_t *pair_off
 }
 
 template <typename Tr>
+int launch_quad(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs,
+                const int32_t *block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int sbs, int trans_x,
+                int trans_y, hipStream_t s) {
+  int side_log2 = 0;
+  while ((64 << side_log2) < sbs) ++side_log2;
+  const int64_t n_tiles = nnz_o << (2 * side_log2);
+  const int64_t blocks = bsa::cdiv(n_tiles, 8) * 8;
+  if (blocks > 0x7fffffffLL) return bsa::fail(BSA_ELIMIT, "bsa_matmul: too many output tiles");
+  const char *xc = static_cast<const char *>(x);
+  const char *yc = static_cast<const char *>(y);
+  char *oc = static_cast<char *>(out);
+#define BSA_MM_LAUNCH(XT, YT)                                                                                     \
+  matmul_quad_kernel<Tr, XT, YT><<<(unsigned)blocks, 256, 0, s>>>(xc, yc, oc, pair_offsets, pairs, block_order, n_tiles, \
+                                                                  sbs, side_log2, nnz_x, nnz_y)
+  if (!trans_x && !trans_y) BSA_MM_LAUNCH(false, false);
+  else if (!trans_x && trans_y) BSA_MM_LAUNCH(false, true);
+  else if (trans_x && !trans_y) BSA_MM_LAUNCH(true, false);
+  else BSA_MM_LAUNCH(true, true);
+#undef BSA_MM_LAUNCH
+  return bsa::check_launch("matmul_quad_kernel");
+}
+
+template <typename Tr>
 int launch_any(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs,
                const int32_t *block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int sbs, int trans_x,
                int trans_y, hipStream_t s) {
@@ -633,7 +829,7 @@ int launch_any(const void *x, const void *y, void *out, const int32_t *pair_offs
   }
   if (sbs == 32)
     return launch_mfma<Tr, 32>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, sbs, trans_x, trans_y, s);
-  return launch_mfma<Tr, 64>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, sbs, trans_x, trans_y, s);
+  return launch_quad<Tr>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, sbs, trans_x, trans_y, s);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
