@@ -10,7 +10,7 @@ from torch import Tensor
 
 from .. import _capi
 from ..utils.blksprs_tensor import BlksprsTensor
-from ..utils.tools import (eager_only, finalize_layout_cache, nonzero_from_packed, pack_layout, prepare_layout_cache)
+from ..utils.tools import (build_packed_indices, eager_only, finalize_layout_cache, nonzero_from_packed, pack_layout, prepare_layout_cache)
 from ..utils.validation import (ensure_contiguous, validate_contiguous, validate_device, validate_dimensions,
                                 validate_dtype_supported, validate_sparsity, validate_sparsity_block_size,
                                 validate_sparsity_dense)
@@ -90,7 +90,7 @@ def to_sparse_build_layout_cache(layout_cache: dict | None, sparsity_layout: Ten
 def to_dense_build_layout_cache(layout_cache: dict | None, sparsity_layout: Tensor) -> dict:
     layout_cache = prepare_layout_cache(layout_cache, "to_dense", sparsity_layout)
     if "packed_indices" not in layout_cache:
-        layout_cache["packed_indices"] = pack_layout(sparsity_layout).packed
+        layout_cache["packed_indices"] = build_packed_indices(sparsity_layout)
     validate_contiguous(layout_cache["packed_indices"])
     return finalize_layout_cache(layout_cache)
 

@@ -266,14 +266,15 @@ def _normalise_causal_lengths(causal_lengths: Tensor | None, n_batches: int, q_l
         raise TypeError("causal_lengths must use an integral dtype")
     validate_device(causal_lengths, torch.empty(0, device=device))
     validate_shape(causal_lengths, (n_batches,), "causal_lengths")
-    # The range check reads the device (two waits of the host): its verdict on one tensor is remembered, per
+    # The range check reads the device (one wait of the host): its verdict on one tensor is remembered, per
     # thread, for as long as the tensor's version counter says that nothing was written to it in place (the
     # reference checks on every call, blksprs/ops/flash_attention.py:239-241; a write through .data goes unseen,
     # as for the facts kept per mask).
     seen = getattr(_LENGTHS_SEEN, "last", None)
     key = (causal_lengths._version, int(q_length)) if not torch.is_inference(causal_lengths) else None
     if seen is None or seen[0] is not causal_lengths or seen[1] != key or key is None:
-        if torch.any(causal_lengths < 0) or torch.any(causal_lengths > q_length):
+        on_host = causal_lengths.tolist()  # one read; two reductions on the device were four launches and two waits
+        if on_host and (min(on_host) < 0 or max(on_host) > q_length):
             raise ValueError(f"causal_lengths values must be between zero and {q_length}")
         _LENGTHS_SEEN.last = (causal_lengths, key, ensure_contiguous(causal_lengths.to(dtype=torch.int64)))
     return _LENGTHS_SEEN.last[2]

@@ -71,14 +71,15 @@ class PackedLayout:
         self.packed, self.count, self.row_offsets, self.max_per_row = packed, count, row_offsets, max_per_row
 
 
-def pack_layouts(*specs, then=None):
+def pack_layouts(*specs, then=None, counts=True):
     """Scans several layouts on the device, ``specs`` being ``(layout, row_len)`` pairs: reverse index, block
     count and optional CSR row offsets of each.
 
     One stream synchronisation for all of them (the counts size the caller's next allocations).  ``then``, if
     given, is called with the reverse indices before that synchronisation: it launches what depends on them
     alone and returns an int64 device tensor of its own statistics, which are read back in the same transfer;
-    the function then returns ``(infos, statistics as a list)``.
+    the function then returns ``(infos, statistics as a list)``.  ``counts`` false: nothing is read back and nothing
+    waits; ``count`` and ``max_per_row`` of the results are ``None``.
     """
     lib = _capi.load()
     results = []
@@ -100,6 +101,8 @@ def pack_layouts(*specs, then=None):
                        row_offsets.data_ptr() if row_offsets is not None else 0,
                        stats_dev[number].data_ptr(), 0, _capi.ptr(workspace), ws_bytes, _capi.stream(dev))
         results.append((packed, row_offsets))
+    if not counts:
+        return [PackedLayout(packed, None, row_offsets, None) for packed, row_offsets in results]
     if then is None:
         stats = stats_dev.tolist() if results else []
         extra = None
@@ -120,7 +123,7 @@ def pack_layout(layout: Tensor, row_len: int = 0) -> PackedLayout:
 
 def build_packed_indices(sparsity_layout: Tensor) -> Tensor:
     """int64 reverse index of a layout: position among the active blocks, ``-1`` for inactive ones."""
-    return pack_layout(sparsity_layout).packed
+    return pack_layouts((sparsity_layout, 0), counts=False)[0].packed
 
 
 def nonzero_from_packed(packed: Tensor, shape, count: int) -> Tensor:
