@@ -579,25 +579,36 @@ inline bool small_applies(const bsa_attn_args &a) {
 // with one, two, four; 6144 rows (sbs 32, 33 steps): 83 / 75 / 82.
 inline int waves_per_row(int64_t rows) { return rows <= 512 ? 4 : rows <= 8192 ? 2 : 1; }
 
-// The row of a wave.  XCD c (workgroup g runs on XCD g % 8) takes a contiguous eighth of the rows, so that the waves in
-// flight on one L2 share few batch entries' partner blocks; inside a batch entry the long rows of a causal layout (the
-// last query blocks, the first key blocks) come first.
+// The row of a wave.  Workgroup g runs on XCD g % 8, each with its own L2.  Of B batch entries an XCD takes B / 8 whole
+// ones, whose partner blocks no other XCD reads, and every eighth row of the B % 8 that are left.  It walks the rows of all
+// its entries together, eight neighbours (whose lists overlap) of one entry, then eight of the next, in the order in which
+// a causal layout's lists get shorter (the last query blocks, the first key blocks first): a launch lasts as long as its
+// longest lists, so none may start late.  Entry by entry, the long lists of an XCD's last entry start behind the short ones
+// of the others, 6144 rows (sbs 32, windows of 33 blocks, a quarter of the rows beyond the sequences): 79 / 95 us
+// (forward / dQ) against 70 / 89; 4128 rows (sbs 16, causal): 57.5 against 48.5; 8192 rows (sbs 32, causal): 172 / 212
+// against 156 / 198; two long columns among short ones in 13 entries (dK / dV, where XCDs also differed in work): 97 against
+// 67; lists of equal lengths: the same.  Rows of one entry on several XCDs where whole entries would do: 5 to 14 % slower
+// (their partner blocks pass several L2s).
 struct RowOfWave {
   int64_t b, own;
   int part;
   bool there;
   __device__ inline RowOfWave(int64_t batches, int64_t rows_per_batch, bool last_first, int wave, int waves, int split) {
-    const int64_t group = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-    const int64_t item = group * (waves / split) + wave / split;
+    const uint32_t xcd = blockIdx.x & 7, item = (blockIdx.x >> 3) * (waves / split) + wave / split;
     part = wave % split;
-    there = item < batches * rows_per_batch;
-    b = there ? item / rows_per_batch : 0;
-    own = there ? item % rows_per_batch : 0;
+    // eight rows of every entry: 8 items for each of an XCD's own entries, one for each shared one (the last of all)
+    const uint32_t own_items = (uint32_t)batches & ~7u, items = (uint32_t)batches;
+    const uint32_t eight = item / items, rest = item - eight * items;
+    b = rest < own_items ? xcd * (own_items >> 3) + (rest >> 3) : rest;
+    own = (int64_t)eight * 8 + ((rest < own_items ? rest : xcd + rest + eight) & 7);
+    there = own < rows_per_batch;
+    if (!there) b = own = 0;
     if (last_first) own = rows_per_batch - 1 - own;
   }
 };
-inline unsigned row_groups(int64_t rows, int waves, int split) {
-  return (unsigned)(cdiv(cdiv(rows, (int64_t)(waves / split)), (int64_t)8) * 8);
+inline unsigned row_groups(int64_t batches, int64_t rows_per_batch, int waves, int split) {
+  const int64_t items = cdiv(rows_per_batch, (int64_t)8) * batches;
+  return (unsigned)(cdiv(items, (int64_t)(waves / split)) * 8);
 }
 
 }  // namespace small

@@ -17,8 +17,8 @@
 // What bounds it: a wave's chain per step (copies awaited, scores, softmax, value product) and the instructions of one
 // wave at a time; matrix cores 16 % busy, 113 vector and 63 scalar instructions per step of 32 x 32 at head dimension 64.
 // Against the fp32 matrix-core kernel that ran these shapes before: 48 x 4096 queries, sbs 32, head dimension 64, fp16,
-// 33 key blocks per query block: 0.65 -> 0.075 ms (443 TFLOP/s); 32 prompts of 1032 to 2064 tokens, sbs 16, bf16, causal:
-// 0.54 -> 0.060 ms.  fp32, where the products take eight times as long and hide the rest: 8 x 2048 queries, half of the
+// 33 key blocks per query block: 0.65 -> 0.070 ms (475 TFLOP/s); 32 prompts of 1032 to 2064 tokens, sbs 16, bf16, causal:
+// 0.54 -> 0.049 ms.  fp32, where the products take eight times as long and hide the rest: 8 x 2048 queries, half of the
 // blocks, head dimension 64: 0.089 -> 0.054 ms (80 TFLOP/s, half of the fp32 matrix-core peak; 512 lists of 32 +- 4 blocks
 // cut in four fill the chip once, so the launch waits for the longest).
 //
@@ -221,7 +221,7 @@ int launch(const bsa_attn_args &a, hipStream_t s) {
         reinterpret_cast<const void *>(&attn_small_fwd_kernel<Tr, SBS, NS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     BSA_HIP(raised);
   }
-  attn_small_fwd_kernel<Tr, SBS, NS><<<row_groups(rows, kWaves, split), 64 * kWaves, lds, s>>>(a, split);
+  attn_small_fwd_kernel<Tr, SBS, NS><<<row_groups(a.B, a.nq, kWaves, split), 64 * kWaves, lds, s>>>(a, split);
   return check_launch("attn_small_fwd_kernel");
 }
 

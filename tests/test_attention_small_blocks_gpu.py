@@ -40,3 +40,11 @@ def test_rows_of_a_launch(device, dtype, sbs, B, n, use_causal):
     nk = n if use_causal else 3
     _run_case(device, dtype, sbs, B=B, nq=n, nk=nk, nh=1, nhv=1, density=0.1 if use_causal else 0.6,
               seed=B + n, use_causal=use_causal)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("B,n", [(2, 1), (7, 7), (8, 8), (8, 9), (13, 17), (16, 3), (20, 11)])
+def test_rows_over_xcds(device, dtype, B, n):
+    """Whole batch entries of an XCD, entries shared by all eight, last rows that are no multiple of eight."""
+    _run_case(device, dtype, 16, B=B, nq=n, nk=n, nh=2, nhv=2, density=0.5, seed=100 * B + n)
+    _run_case(device, dtype, 16, B=B, nq=n, nk=n, nh=1, nhv=1, density=0.5, seed=100 * B + n, use_causal=True)
