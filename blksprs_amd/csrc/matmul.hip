@@ -794,15 +794,22 @@ int launch_quad(const void *x, const void *y, void *out, const int32_t *pair_off
   return bsa::check_launch("matmul_quad_kernel");
 }
 
+// Output blocks per wave of the kernels for blocks of 16: as many as leave 32768 waves, four times what the chip holds at
+// once.  Output blocks come with one or two pairs (forward) or with ten (gradients, of which there are fewer): waves must
+// stay many rather than their runs long.  16-bit, dX and dY of 64 x 2048^3 at 5 % (52611 blocks, 6.4 pairs each), runs of 1 /
+// 2 / 4 / 8 blocks: 41 / 41 / 46 / 55 and 39 / 40 / 49 / 60 us; forward (289445 blocks, 1.2 pairs each), 2 / 4 / 8: 55 / 44 / 40 us.
+int64_t small_run(int64_t nnz_o) {
+  const int64_t run = nnz_o / (256 * 32 * 4);
+  return run < 1 ? 1 : (run > kSmallRunMax ? kSmallRunMax : run);
+}
+
 template <typename Tr>
 int launch_any(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs,
                const int32_t *block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int sbs, int trans_x,
                int trans_y, hipStream_t s) {
   if (sbs == 16 && Tr::kElem == 2) {
     using Ts = std::conditional_t<std::is_same_v<Tr, Bf16Traits>, Bf16Small, F16Small>;
-    // enough waves to fill the chip, each with a run long enough to overlap its loads
-    int64_t run = bsa::cdiv(nnz_o, 256 * 32 * 4);
-    run = run < 8 ? 8 : (run > kSmallRunMax ? kSmallRunMax : run);
+    const int64_t run = small_run(nnz_o);
     const int64_t blocks = bsa::cdiv(bsa::cdiv(bsa::cdiv(nnz_o, run), 4), 8) * 8;
     if (blocks > 0x7fffffffLL) return bsa::fail(BSA_ELIMIT, "bsa_matmul: too many output blocks");
     const char *xc = static_cast<const char *>(x);
