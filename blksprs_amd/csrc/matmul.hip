@@ -23,8 +23,7 @@
 // is rounded to the output type, staged through LDS and written with 16-byte
 // stores that cover whole rows.
 //
-// sbs == 16 has kernels of its own (16 x 16 x 16 products for 16-bit elements, FMAs
-// for fp32): at 13 flop/byte it is a gather problem, not a matrix-core problem.
+// sbs == 16 has kernels of its own: at 13 flop/byte (7 in fp32) it is a gather problem, not a matrix-core problem.
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
@@ -573,51 +572,6 @@ __global__ __launch_bounds__(256, 5) void matmul_quad_kernel(const char *__restr
   }
 }
 
-// sbs == 16: one wave per output block, fp32 FMAs; lane -> row lane/4, columns 4*(lane%4)..+3
-template <typename Tr>
-__global__ __launch_bounds__(256) void matmul_small_kernel(const typename Tr::store_t *__restrict__ x,
-                                                           const typename Tr::store_t *__restrict__ y,
-                                                           typename Tr::store_t *__restrict__ out,
-                                                           const int32_t *__restrict__ pair_offsets,
-                                                           const int32_t *__restrict__ pairs, int64_t nnz_o,
-                                                           int64_t nnz_x, int64_t nnz_y, int xt, int yt) {
-  __shared__ float sx[4][16][17];
-  __shared__ float sy[4][16][20];
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int64_t n = (int64_t)blockIdx.x * 4 + wave;
-  if (n >= nnz_o) return;
-  const int p_begin = pair_offsets[n], p_end = pair_offsets[n + 1];
-  const int i = lane >> 2, j0 = (lane & 3) * 4;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int p = p_begin; p < p_end; ++p) {
-    int64_t px = pairs[2 * (int64_t)p], py = pairs[2 * (int64_t)p + 1];
-    if (px < 0 || px >= nnz_x) px = 0;
-    if (py < 0 || py >= nnz_y) py = 0;
-    const typename Tr::store_t *xb = x + px * 256 + lane * 4;
-    const typename Tr::store_t *yb = y + py * 256 + lane * 4;
-    // each lane moves 4 consecutive elements (row lane/4, columns 4*(lane%4)..) of both blocks
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float xv = Tr::widen(xb[e]);
-      const float yv = Tr::widen(yb[e]);
-      if (xt) sx[wave][j0 + e][i] = xv; else sx[wave][i][j0 + e] = xv;
-      if (yt) sy[wave][j0 + e][i] = yv; else sy[wave][i][j0 + e] = yv;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const float a = sx[wave][i][k];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] = fmaf(a, sy[wave][k][j0 + e], acc[e]);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  }
-  typename Tr::store_t *ob = out + n * 256 + lane * 4;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) ob[e] = Tr::round(acc[e]);
-}
-
 // sbs == 16, 16-bit elements: one 16 x 16 x 16 matrix-core product per pair.  A block is 512 bytes and an output
 // block has one or two pairs, so a wave that handled a single block would be a chain of dependent loads
 // (offsets -> pairs -> operands -> store) and nothing else.  Here a wave owns a run of consecutive output blocks,
@@ -746,6 +700,90 @@ __global__ __launch_bounds__(256) void matmul_small16_kernel(const char *__restr
   flush_until(p_last);
 }
 
+// sbs == 16, fp32: the same walk.  A block is 1 KiB, 16 bytes per lane.  An operand whose contraction index is contiguous is
+// a matrix operand as it is loaded (lane: row lane % 16, values 4 (lane / 16) .. + 3, one per 16 x 16 x 4 product); the other
+// one passes through LDS, its rows placed so that the four rows of a read (r, r + 4, r + 8, r + 12) are neighbours.  The product
+// is formed transposed: a lane ends with 16 consecutive bytes of an output row, a store covers the block.
+// It is bound like the 16-bit kernel by its memory instructions and the latency of a wave's chain.  Against one wave per
+// block and FMAs from LDS: out / dX / dY of 64 x 2048^3 at 5 %: 0.238 / 0.207 / 0.203 -> 0.070 / 0.093 / 0.088 ms; 8 x 2976 x 4064 x 2080
+// at 12.5 %: 0.404 / 0.393 / 0.387 -> 0.122 / 0.123 / 0.117.
+template <bool XT, bool YT>
+__global__ __launch_bounds__(256) void matmul_small16_f32_kernel(const char *__restrict__ x, const char *__restrict__ y,
+                                                                 char *__restrict__ out,
+                                                                 const int32_t *__restrict__ pair_offsets,
+                                                                 const int32_t *__restrict__ pairs, int64_t nnz_o,
+                                                                 int64_t nnz_x, int64_t nnz_y, int run) {
+  __shared__ __attribute__((aligned(16))) char stage[4][2048];  // per wave: the x block, the y block
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t group = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int64_t n0 = (group * 4 + wave) * run;
+  if (n0 >= nnz_o) return;
+  const int count = (int)(nnz_o - n0 < run ? nnz_o - n0 : run);
+  const int li = lane & 15, kg = lane >> 4;
+  // a direct operand: row li, chunk kg; one that goes through LDS: as it lies, lane l the 16 bytes at 16 l
+  const int direct_off = li * 64 + kg * 16, linear_off = lane * 16;
+  const int x_off = XT ? linear_off : direct_off, y_off = YT ? direct_off : linear_off;
+  const int row = lane >> 2, write_off = (4 * (row & 3) + (row >> 2)) * 64 + (lane & 3) * 16;
+  const int read_off = kg * 64 + li * 4;  // + 256 j: row 4 kg + j, column li
+  char *slot = stage[wave];
+  const uint32_t nx = (uint32_t)nnz_x, ny = (uint32_t)nnz_y;
+  const __amdgpu_buffer_rsrc_t ro = small_resource(out + n0 * 1024, (uint32_t)count * 1024u);
+
+  const int off_win = pair_offsets[n0 + (lane <= count ? lane : count)];
+  const int p_first = __builtin_amdgcn_readlane(off_win, 0);
+  const int p_last = __builtin_amdgcn_readlane(off_win, count);
+  f32x4 acc{0.f, 0.f, 0.f, 0.f};
+  int done = 0;
+  int block_end = __builtin_amdgcn_readlane(off_win, 1);
+  auto flush_until = [&](int p) {
+    while (done < count && block_end <= p) {
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), ro, direct_off, done * 1024, 2);
+      acc = f32x4{0.f, 0.f, 0.f, 0.f};
+      ++done;
+      block_end = __builtin_amdgcn_readlane(off_win, done + 1 <= count ? done + 1 : count);
+    }
+  };
+  for (int base = p_first; base < p_last; base += 64) {
+    const int n = p_last - base < 64 ? p_last - base : 64;
+    u32x2 win{0u, 0u};
+    if (lane < n) win = *reinterpret_cast<const u32x2 *>(pairs + 2 * (int64_t)(base + lane));
+    auto issue = [&](int i, u32x4 &xr, u32x4 &yr) {
+      const int at = i < n ? i : n - 1;  // past the end: the last pair again, so that every step issues the same loads
+      const uint32_t px = (uint32_t)__builtin_amdgcn_readlane((int)win[0], at);
+      const uint32_t py = (uint32_t)__builtin_amdgcn_readlane((int)win[1], at);
+      // a corrupt list must not turn into a wild read: such a pair reads block 0
+      xr = *reinterpret_cast<const u32x4 *>(x + (int64_t)(px < nx ? px : 0) * 1024 + x_off);
+      yr = *reinterpret_cast<const u32x4 *>(y + (int64_t)(py < ny ? py : 0) * 1024 + y_off);
+    };
+    u32x4 xs[kSmallDepth], ys[kSmallDepth];
+#pragma unroll
+    for (int d = 0; d < kSmallDepth; ++d) issue(d, xs[d], ys[d]);
+    for (int i = 0; i < n; i += kSmallDepth) {
+#pragma unroll
+      for (int d = 0; d < kSmallDepth; ++d) {
+        if (i + d < n) {
+          flush_until(base + i + d);
+          if (XT) *reinterpret_cast<u32x4 *>(slot + write_off) = xs[d];
+          if (!YT) *reinterpret_cast<u32x4 *>(slot + 1024 + write_off) = ys[d];
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          f32x4 fx = __builtin_bit_cast(f32x4, xs[d]), fy = __builtin_bit_cast(f32x4, ys[d]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if (XT) fx[j] = *reinterpret_cast<const float *>(slot + read_off + 256 * j);
+            if (!YT) fy[j] = *reinterpret_cast<const float *>(slot + 1024 + read_off + 256 * j);
+          }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(fy[j], fx[j], acc, 0, 0, 0);
+        }
+        issue(i + d + kSmallDepth, xs[d], ys[d]);
+      }
+    }
+  }
+  flush_until(p_last);
+}
+
 template <typename Tr, int TILE>
 int launch_mfma(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs,
                 const int32_t *block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int sbs, int trans_x,
@@ -826,13 +864,21 @@ int launch_any(const void *x, const void *y, void *out, const int32_t *pair_offs
     return bsa::check_launch("matmul_small16_kernel");
   }
   if (sbs == 16) {
-    using E = typename Tr::store_t;
-    const int64_t blocks = bsa::cdiv(nnz_o, 4);
+    const int64_t run = small_run(nnz_o);
+    const int64_t blocks = bsa::cdiv(bsa::cdiv(bsa::cdiv(nnz_o, run), 4), 8) * 8;
     if (blocks > 0x7fffffffLL) return bsa::fail(BSA_ELIMIT, "bsa_matmul: too many output blocks");
-    matmul_small_kernel<Tr><<<(unsigned)blocks, 256, 0, s>>>(static_cast<const E *>(x), static_cast<const E *>(y),
-                                                             static_cast<E *>(out), pair_offsets, pairs, nnz_o,
-                                                             nnz_x, nnz_y, trans_x, trans_y);
-    return bsa::check_launch("matmul_small_kernel");
+    const char *xc = static_cast<const char *>(x);
+    const char *yc = static_cast<const char *>(y);
+    char *oc = static_cast<char *>(out);
+#define BSA_MM_SMALL(XT, YT)                                                                                          \
+  matmul_small16_f32_kernel<XT, YT><<<(unsigned)blocks, 256, 0, s>>>(xc, yc, oc, pair_offsets, pairs, nnz_o, nnz_x, nnz_y, \
+                                                                     (int)run)
+    if (!trans_x && !trans_y) BSA_MM_SMALL(false, false);
+    else if (!trans_x && trans_y) BSA_MM_SMALL(false, true);
+    else if (trans_x && !trans_y) BSA_MM_SMALL(true, false);
+    else BSA_MM_SMALL(true, true);
+#undef BSA_MM_SMALL
+    return bsa::check_launch("matmul_small16_f32_kernel");
   }
   if (sbs == 32)
     return launch_mfma<Tr, 32>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, sbs, trans_x, trans_y, s);
