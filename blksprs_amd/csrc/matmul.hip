@@ -1,29 +1,14 @@
 // Block-sparse GEMM: out[n] = sum over the contraction list of block n of x[px] @ y[py].
 //
-// sbs 32: one wavefront owns one output block (TILE = 32) and walks that block's list of (x block, y block) pairs in
-// ascending k, so only non-zero K-blocks are touched and the fp32 accumulation order is fixed.  Four waves (four
-// neighbouring blocks) share a workgroup but never synchronise: each has a private LDS region.
-// Larger blocks: matmul_quad_kernel, further down.
+// Block sizes 16 and 32: a wave owns a run of consecutive output blocks and walks their pairs (matmul_small16_kernel,
+// matmul_small16_f32_kernel, matmul_runs32_kernel); larger blocks: a workgroup owns a 64 x 64 tile (matmul_quad_kernel).  Every
+// kernel walks a block's pairs in ascending k, so only non-zero K-blocks are touched and the fp32 accumulation order is fixed.
 //
-// Data path per K-chunk (32 k):
-//   global --16 B per lane, consecutive lanes = consecutive bytes--> VGPRs
-//          --ds_write_b128--> LDS --> MFMA operand fragments --> v_mfma_f32_32x32x*.
-// The loads of chunk t+1 are issued before the MFMAs of chunk t.
+// An operand whose k index is contiguous in memory (x, or y read transposed) is read from LDS as it lies; one whose k index
+// is strided (y, or x read transposed) through the transposing LDS read for 16-bit types, and by 32-bit reads for fp32.
 //
-// An operand whose k index is contiguous in memory (x, or y read transposed) is
-// kept row-major in LDS with the 16-byte chunks of a row XOR-swizzled, and a
-// fragment is one ds_read_b128.  An operand whose k index is strided (y, or x read
-// transposed) cannot be fed to the matrix core as stored, because a lane needs 8
-// consecutive k of one column: for 16-bit types two k rows are interleaved in
-// registers (v_perm_b32) before the LDS write, so LDS holds (k, k+1) pairs per
-// column and a fragment is four conflict-free ds_read_b32; fp32 needs no packing.
-//
-// The product is formed transposed (y fragments as the A operand, x fragments as
-// B), which leaves 4 consecutive output columns of one row in each lane; the tile
-// is rounded to the output type, staged through LDS and written with 16-byte
-// stores that cover whole rows.
-//
-// sbs == 16 has kernels of its own: at 13 flop/byte (7 in fp32) it is a gather problem, not a matrix-core problem.
+// The product is formed transposed (y fragments as the A operand, x fragments as B), which leaves 4 consecutive output
+// columns of one row in each lane.
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
@@ -82,319 +67,197 @@ struct F32Traits {
   __device__ static float widen(float v) { return v; }
 };
 
-// Geometry of one operand chunk in LDS (TILE rows of the non-contracted index, KC values of k).
-template <typename Tr, int TILE>
-struct Geom {
+// ---- blocks of 32 x 32 in LDS: rows of 64 bytes (16-bit) or 128 (fp32), the 16-byte chunks of row r exchanged by an XOR
+template <typename Tr>
+struct Block32 {
   static constexpr int ES = Tr::kElem;
-  static constexpr int KC = (ES == 2) ? TILE : 32;       // k per chunk
-  static constexpr int STEPS = (ES == 2) ? KC / 16 : KC / 8;  // fragments along k per chunk
-  static constexpr int NB = TILE / 32;                    // 32-wide MFMA blocks per side
-  static constexpr int REGION = TILE * KC * ES;           // bytes of one operand chunk
-  // k-contiguous staging
-  static constexpr int CPR = KC * ES / 16;                // 16-byte chunks per row
-  static constexpr int RPL = (CPR >= 8) ? 1 : 8 / CPR;    // rows per 128-byte LDS line
-  static constexpr int KCONT_LOADS = TILE * CPR / 64;     // uint4 per lane
-  // k-strided staging
-  static constexpr int KSTR_LOADS = (ES == 2) ? (KC / 2) * (TILE / 8) * 2 / 64 : KC * (TILE / 4) / 64;
-  static constexpr int LOADS = KCONT_LOADS > KSTR_LOADS ? KCONT_LOADS : KSTR_LOADS;
-  // output staging
-  static constexpr int OCPR = TILE * ES / 16;
-  static constexpr int OUT_STORES = TILE * OCPR / 64;
-  static constexpr int OUT_BYTES = TILE * TILE * ES;
-  static constexpr int WAVE_LDS = (2 * REGION > OUT_BYTES) ? 2 * REGION : OUT_BYTES;
+  static constexpr int kRow = 32 * ES, kBytes = 32 * kRow, kChunks = kRow / 16;
+  static constexpr int kCopies = kBytes / 1024;  // asynchronous copies per block
+  // along the contraction; fragment s: values 16 s + 8 (lane / 32) .. + 7 (fp32: 8 s + 4 (lane / 32) .. + 3)
+  static constexpr int kFrags = ES == 2 ? 2 : 4;
+
+  // eight consecutive rows read at one chunk fall on different chunks of 128 bytes; 16-bit rows r and r + 2 also put the 32
+  // bytes of a transposing read into different halves
+  __device__ static int swizzle(int r) { return ES == 4 ? r & 7 : ((((r >> 1) ^ (r >> 3)) & 1) << 1) | ((r >> 2) & 1); }
+
+  // lane l supplies the 16 bytes at position 16 l of every KiB (the swizzle is the same for all of them)
+  __device__ static uint32_t source_offset(int lane) {
+    const int r = lane / kChunks;
+    return (uint32_t)(r * kRow + (((lane % kChunks) ^ swizzle(r)) << 4));
+  }
+  __device__ static void request(const char *base, uint32_t off, char *dst) {
+#pragma unroll
+    for (int i = 0; i < kBytes; i += 2048) bsa::mfma::copy_2k_to_lds(base + i, off, dst + i);
+  }
+
+  // fragments of an operand whose contraction runs along the rows (row lane % 32), or down the columns (column lane % 32)
+  template <bool kDown>
+  struct Reader {
+    static constexpr int kBases = !kDown ? 1 : ES == 2 ? 2 : 4;
+    uint32_t at[kBases];
+    __device__ explicit Reader(int lane) {
+      const int li = lane & 31, kg = lane >> 5;
+      if constexpr (!kDown) {
+        at[0] = li * kRow + ((kg ^ swizzle(li)) << 4);
+      } else if constexpr (ES == 2) {
+        // lane s of a group of 16 points at row s / 4 of four, values 4 (s % 4) .. + 3 of the group's 16 columns
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int r = 8 * kg + 4 * i + ((lane & 15) >> 2), c = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+          at[i] = r * kRow + ((c ^ swizzle(r)) << 4) + ((lane & 1) << 3);
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) at[t] = (4 * kg + t) * kRow + (((li >> 2) ^ swizzle(4 * kg + t)) << 4) + ((li & 3) << 2);
+      }
+    }
+    __device__ u32x4 frag(const char *lds, int s) const {
+      u32x4 v;
+      if constexpr (!kDown) {
+        v = *reinterpret_cast<const u32x4 *>(lds + (at[0] ^ (32 * s)));
+      } else if constexpr (ES == 2) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const auto t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4 *)(lds + at[i] + 1024 * s));
+          const u32x2 w = __builtin_bit_cast(u32x2, t);
+          v[2 * i] = w[0], v[2 * i + 1] = w[1];
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[t] = *reinterpret_cast<const uint32_t *>(lds + at[t] + 1024 * s);
+      }
+      return v;
+    }
+  };
 };
 
-template <int CPR, int RPL>
-__device__ inline int swizzle(int row, int chunk) {
-  return chunk ^ ((row / RPL) & (CPR - 1));
-}
 
-// Dword offset of column c inside pair row kp of the (k, k+1)-packed layout of a k-strided operand.
-// Columns are kept in quads (one ds_write_b128 each).  Quad q = 2a + h is placed so that (i) the eight
-// lanes that write the even (or the odd) quads of consecutive column octets hit eight different quad
-// banks and (ii) the 32 lanes that read 32 consecutive columns of one pair row do too.
-template <int TILE>
-__device__ inline int pair_col_offset(int kp, int c) {
-  const int q = c >> 2, a = q >> 1, h = q & 1;
-  int pos;
-  if constexpr (TILE == 64)
-    pos = ((a + 4 * h) & 7) + 8 * h;
-  else
-    pos = a + 4 * (h ^ (kp & 1));
-  return 4 * pos + (c & 3);
-}
 
-// ---- global -> registers -------------------------------------------------
-
-// k contiguous: element (row, k) at base[row * ld + k]
-template <typename G>
-__device__ inline void load_kcont(u32x4 (&r)[G::LOADS], const char *base, uint32_t ld_bytes, int lane) {
-#pragma unroll
-  for (int i = 0; i < G::KCONT_LOADS; ++i) {
-    const int q = i * 64 + lane;
-    const int row = q / G::CPR, c = q % G::CPR;
-    r[i] = *reinterpret_cast<const u32x4 *>(base + (uint32_t)(row * ld_bytes + c * 16));
-  }
-}
-
-// k strided: element (row, k) at base[k * ld + row]
-template <typename G, int TILE>
-__device__ inline void load_kstr(u32x4 (&r)[G::LOADS], const char *base, uint32_t ld_bytes, int lane) {
-  if constexpr (G::ES == 2) {
-#pragma unroll
-    for (int i = 0; i < G::KSTR_LOADS / 2; ++i) {
-      const int q = i * 64 + lane;
-      const int ro = q % (TILE / 8), kp = q / (TILE / 8);
-      r[2 * i] = *reinterpret_cast<const u32x4 *>(base + (uint32_t)((2 * kp) * ld_bytes + ro * 16));
-      r[2 * i + 1] = *reinterpret_cast<const u32x4 *>(base + (uint32_t)((2 * kp + 1) * ld_bytes + ro * 16));
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < G::KSTR_LOADS; ++i) {
-      const int q = i * 64 + lane;
-      const int rc = q % (TILE / 4), k = q / (TILE / 4);
-      r[i] = *reinterpret_cast<const u32x4 *>(base + (uint32_t)(k * ld_bytes + rc * 16));
-    }
-  }
-}
-
-// ---- registers -> LDS ----------------------------------------------------
-
-template <typename G>
-__device__ inline void stage_kcont(const u32x4 (&r)[G::LOADS], char *lds, int lane) {
-#pragma unroll
-  for (int i = 0; i < G::KCONT_LOADS; ++i) {
-    const int q = i * 64 + lane;
-    const int row = q / G::CPR, c = q % G::CPR;
-    *reinterpret_cast<u32x4 *>(lds + row * (G::CPR * 16) + swizzle<G::CPR, G::RPL>(row, c) * 16) = r[i];
-  }
-}
-
-template <typename G, int TILE>
-__device__ inline void stage_kstr(const u32x4 (&r)[G::LOADS], char *lds, int lane) {
-  if constexpr (G::ES == 2) {
-#pragma unroll
-    for (int i = 0; i < G::KSTR_LOADS / 2; ++i) {
-      const int q = i * 64 + lane;
-      const int ro = q % (TILE / 8), kp = q / (TILE / 8);
-      const u32x4 e = r[2 * i], o = r[2 * i + 1];  // rows 2kp and 2kp+1, 8 columns each
-      // dword for column c = (even-row value, odd-row value)
-      u32x4 lo, hi;
-      lo.x = __builtin_amdgcn_perm(o.x, e.x, 0x05040100u);
-      lo.y = __builtin_amdgcn_perm(o.x, e.x, 0x07060302u);
-      lo.z = __builtin_amdgcn_perm(o.y, e.y, 0x05040100u);
-      lo.w = __builtin_amdgcn_perm(o.y, e.y, 0x07060302u);
-      hi.x = __builtin_amdgcn_perm(o.z, e.z, 0x05040100u);
-      hi.y = __builtin_amdgcn_perm(o.z, e.z, 0x07060302u);
-      hi.z = __builtin_amdgcn_perm(o.w, e.w, 0x05040100u);
-      hi.w = __builtin_amdgcn_perm(o.w, e.w, 0x07060302u);
-      uint32_t *row = reinterpret_cast<uint32_t *>(lds) + kp * TILE;
-      *reinterpret_cast<u32x4 *>(row + pair_col_offset<TILE>(kp, ro * 8)) = lo;
-      *reinterpret_cast<u32x4 *>(row + pair_col_offset<TILE>(kp, ro * 8 + 4)) = hi;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < G::KSTR_LOADS; ++i) {
-      const int q = i * 64 + lane;
-      const int rc = q % (TILE / 4), k = q / (TILE / 4);
-      *reinterpret_cast<u32x4 *>(reinterpret_cast<uint32_t *>(lds) + k * TILE + rc * 4) = r[i];
-    }
-  }
-}
-
-// ---- LDS -> MFMA fragment ------------------------------------------------
-// fragment (block mb, step s) of lane (row = 32 mb + lane % 32, kg = lane / 32)
-
-template <typename G>
-__device__ inline u32x4 frag_kcont(const char *lds, int mb, int s, int lane) {
-  const int row = 32 * mb + (lane & 31), kg = lane >> 5;
-  return *reinterpret_cast<const u32x4 *>(lds + row * (G::CPR * 16) + swizzle<G::CPR, G::RPL>(row, 2 * s + kg) * 16);
-}
-
-template <typename G, int TILE>
-__device__ inline u32x4 frag_kstr(const char *lds, int mb, int s, int lane) {
-  const int row = 32 * mb + (lane & 31), kg = lane >> 5;
-  // 16-bit: (k,k+1) pair rows 8s + 4kg + t; fp32: k rows 8s + 4kg + t
-  const uint32_t *p = reinterpret_cast<const uint32_t *>(lds) + (8 * s + 4 * kg) * TILE;
-  u32x4 v;
-  if constexpr (G::ES == 2) {
-    v[0] = p[pair_col_offset<TILE>(0, row)];
-    v[1] = p[TILE + pair_col_offset<TILE>(1, row)];
-    v[2] = p[2 * TILE + pair_col_offset<TILE>(0, row)];
-    v[3] = p[3 * TILE + pair_col_offset<TILE>(1, row)];
-  } else {
-    v[0] = p[row];
-    v[1] = p[TILE + row];
-    v[2] = p[2 * TILE + row];
-    v[3] = p[3 * TILE + row];
-  }
-  return v;
-}
-
-template <typename Tr, int TILE, bool XT, bool YT>
-__global__ __launch_bounds__(256, 2) void matmul_mfma_kernel(const char *__restrict__ x, const char *__restrict__ y,
-                                                             char *__restrict__ out,
-                                                             const int32_t *__restrict__ pair_offsets,
-                                                             const int32_t *__restrict__ pairs,
-                                                             const int32_t *__restrict__ block_order,
-                                                             int64_t n_tiles, int sbs, int side_log2, int64_t nnz_x,
-                                                             int64_t nnz_y) {
-  using G = Geom<Tr, TILE>;
-  constexpr int ES = G::ES;
-  __shared__ __attribute__((aligned(16))) char smem[4 * G::WAVE_LDS];
-
+// sbs 32.  A wave owns a run of consecutive output blocks, whose pairs are one contiguous range of the pair list, and walks
+// the pairs with the operand blocks of the next ones on their way into its own LDS (asynchronous copies, no barriers): a
+// pair is copied over as soon as its fragments are in registers, so one pair in LDS (fp32, where a pair's products last
+// longer than its copies) or two (16-bit) keep the loads going, and 20 waves share a compute unit.  A finished block is
+// rounded and stored in between.  The products of a block are added in list order.
+//
+// What bounds it for 16-bit operands: the operand bytes behind the L2 (4 KiB per pair of 65 kFLOP; 480 to 610 MB per launch
+// of 8 x 2976 x 4064 x 2080 at 25 %, whatever the order of the blocks), then the instructions of a pair's control; fp32:
+// the matrix cores, half busy.  Against a kernel that staged operands through registers and gave a wave one block: that
+// size, bf16, out / dX / dY: 0.096 / 0.100 / 0.107 -> 0.094 / 0.093 / 0.098 ms, 16 x 4096^3 0.553 / 0.684 / 0.591 -> 0.490 / 0.545 /
+// 0.566; fp32 0.366 / 0.324 / 0.308 -> 0.276 / 0.298 / 0.277 ms.  Two pairs in LDS for fp32 leave 10 waves: 0.316 / 0.328 / 0.323.
+template <typename Tr, bool XT, bool YT>
+__global__ __launch_bounds__(256, 5) void matmul_runs32_kernel(
+    const char *__restrict__ x, const char *__restrict__ y, char *__restrict__ out, const int32_t *__restrict__ pair_offsets,
+    const int32_t *__restrict__ pairs, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int run) {
+  using B = Block32<Tr>;
+  constexpr int ES = B::ES, kPair = 2 * B::kBytes, kStores = B::kBytes / 1024, kWaves = 4;
+  constexpr int kDepth = ES == 2 ? 2 : 1;  // pairs in LDS or on their way
+  __shared__ __attribute__((aligned(1024))) char smem[kWaves * kDepth * kPair];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Give XCD c the c-th contiguous
-  // eighth of the (ordered) work list, so that the tiles in flight on one L2 are neighbours in the list.
-  const int64_t per_xcd = gridDim.x >> 3;
-  const int64_t group = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  const int64_t item = group * 4 + wave;
-  if (item >= n_tiles) return;
-  int64_t tile = item;
-  if (block_order) {
-    const int64_t per_block = (int64_t)1 << (2 * side_log2);
-    tile = (int64_t)__builtin_amdgcn_readfirstlane(block_order[item >> (2 * side_log2)]) * per_block +
-           (item & (per_block - 1));
-  }
-  char *lds_x = smem + wave * G::WAVE_LDS;
-  char *lds_y = lds_x + G::REGION;
+  // every XCD takes a contiguous eighth of the runs (workgroup g runs on XCD g % 8)
+  const int64_t group = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int64_t n0 = (group * kWaves + wave) * run;
+  if (n0 >= nnz_o) return;
+  const int count = (int)(nnz_o - n0 < run ? nnz_o - n0 : run);
+  const int off_win = pair_offsets[n0 + (lane <= count ? lane : count)];
+  const int p_first = __builtin_amdgcn_readlane(off_win, 0), p_last = __builtin_amdgcn_readlane(off_win, count);
+  char *const ring = smem + wave * kDepth * kPair;
+  const uint32_t source = B::source_offset(lane);
+  const typename B::template Reader<XT> rx(lane);
+  const typename B::template Reader<!YT> ry(lane);
 
-  const int side_mask = (1 << side_log2) - 1;
-  const int64_t n = tile >> (2 * side_log2);
-  const int ti = (int)(tile >> side_log2) & side_mask;
-  const int tj = (int)tile & side_mask;
-  const int64_t block_bytes = (int64_t)sbs * sbs * ES;
-  const uint32_t ld_bytes = (uint32_t)sbs * ES;
-  const int n_chunks = sbs / G::KC;  // K-chunks per pair
+  // 64 entries of the pair list at a time, one per lane; a corrupt list must not turn into a wild read
+  int next = p_first, base = p_first - 64;  // the next pair to request
+  uint32_t win_x = 0, win_y = 0;
+  auto request = [&](char *slot) {
+    if (next - base >= 64) {
+      base += 64;
+      u32x2 v{0u, 0u};
+      if (base + lane < p_last) v = *reinterpret_cast<const u32x2 *>(pairs + 2 * (int64_t)(base + lane));
+      win_x = v[0] < (uint32_t)nnz_x ? v[0] : 0u;
+      win_y = v[1] < (uint32_t)nnz_y ? v[1] : 0u;
+    }
+    const uint32_t px = __builtin_amdgcn_readlane((int)win_x, next - base), py = __builtin_amdgcn_readlane((int)win_y, next - base);
+    B::request(x + (uint64_t)px * B::kBytes, source, slot);
+    B::request(y + (uint64_t)py * B::kBytes, source, slot + B::kBytes);
+    ++next;
+  };
 
-  const int p_begin = __builtin_amdgcn_readfirstlane(pair_offsets[n]);
-  const int p_end = __builtin_amdgcn_readfirstlane(pair_offsets[n + 1]);
-  const int n_iter = (p_end - p_begin) * n_chunks;
-
-  f32x16 acc[G::NB][G::NB];  // [block along j][block along i]
+  f32x16 acc;
 #pragma unroll
-  for (int a = 0; a < G::NB; ++a)
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  int done = 0, block_end = __builtin_amdgcn_readlane(off_win, 1);  // the block in work, the end of its pairs
+  const int li = lane & 31, kg = lane >> 5;
+  // acc[r] = O[lane % 32][8 (r / 4) + 4 (lane / 32) + r % 4]: through LDS into whole rows, stored past the caches
+  auto flush = [&](char *stage) {
 #pragma unroll
-    for (int b = 0; b < G::NB; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-
-  u32x4 rx[G::LOADS], ry[G::LOADS];
-
-  // 64 entries of this block's pair list at a time, one per lane (a dependent index load per K-chunk would
-  // put a full memory latency on the critical path of every iteration)
-  int win_base = p_begin, win_px = 0, win_py = 0;
-#define BSA_LOAD_WINDOW()                                                            \
-  do {                                                                               \
-    const int t_ = win_base + lane;                                                  \
-    win_px = win_py = 0;                                                             \
-    if (t_ < p_end) {                                                                \
-      const int2 v_ = *reinterpret_cast<const int2 *>(pairs + 2 * (int64_t)t_);      \
-      win_px = v_.x;                                                                 \
-      win_py = v_.y;                                                                 \
-    }                                                                                \
-  } while (0)
-  BSA_LOAD_WINDOW();
-
-  // Issues the global loads of iteration `it` (pair it / n_chunks, K-chunk it % n_chunks) into rx / ry.
-#define BSA_FETCH(it_)                                                                                           \
-  do {                                                                                                           \
-    const int p_ = p_begin + (it_) / n_chunks;                                                                   \
-    const int kc_ = (it_) % n_chunks;                                                                            \
-    /* the pair indices come from a 64-entry register window, not from memory: no load latency here */          \
-    if (p_ - win_base >= 64) {                                                                                   \
-      win_base += 64;                                                                                            \
-      BSA_LOAD_WINDOW();                                                                                         \
-    }                                                                                                            \
-    const int sel_ = __builtin_amdgcn_readfirstlane(p_ - win_base);                                              \
-    int64_t px_ = __builtin_amdgcn_readlane(win_px, sel_);                                                       \
-    int64_t py_ = __builtin_amdgcn_readlane(win_py, sel_);                                                       \
-    /* a corrupt list must not turn into a wild read */                                                         \
-    px_ = (px_ < 0 || px_ >= nnz_x) ? 0 : px_;                                                                   \
-    py_ = (py_ < 0 || py_ >= nnz_y) ? 0 : py_;                                                                   \
-    const char *xb_ = x + px_ * block_bytes;                                                                     \
-    const char *yb_ = y + py_ * block_bytes;                                                                     \
-    /* x tile: rows i = ti*TILE.., k = kc*KC..;  y tile: k rows, columns j = tj*TILE.. */                        \
-    if constexpr (!XT)                                                                                           \
-      load_kcont<G>(rx, xb_ + (int64_t)ti * TILE * (int64_t)ld_bytes + (int64_t)kc_ * G::KC * ES, ld_bytes, lane);        \
-    else /* block holds x^T: element (i, k) at blk[k][i] */                                                      \
-      load_kstr<G, TILE>(rx, xb_ + (int64_t)kc_ * G::KC * (int64_t)ld_bytes + (int64_t)ti * TILE * ES, ld_bytes, lane);   \
-    if constexpr (!YT)                                                                                           \
-      load_kstr<G, TILE>(ry, yb_ + (int64_t)kc_ * G::KC * (int64_t)ld_bytes + (int64_t)tj * TILE * ES, ld_bytes, lane);   \
-    else /* block holds y^T: element (k, j) at blk[j][k] */                                                      \
-      load_kcont<G>(ry, yb_ + (int64_t)tj * TILE * (int64_t)ld_bytes + (int64_t)kc_ * G::KC * ES, ld_bytes, lane);        \
-  } while (0)
-
-  if (n_iter > 0) BSA_FETCH(0);
-  for (int it = 0; it < n_iter; ++it) {
-    if constexpr (!XT) stage_kcont<G>(rx, lds_x, lane); else stage_kstr<G, TILE>(rx, lds_x, lane);
-    if constexpr (!YT) stage_kstr<G, TILE>(ry, lds_y, lane); else stage_kcont<G>(ry, lds_y, lane);
-    // prefetch the next chunk while this one is multiplied; the last iteration re-reads itself (cache hit)
-    // so that the loads stay unconditional and the staging registers never leave the register file
-    const int nxt = (it + 1 < n_iter) ? it + 1 : it;
-    BSA_FETCH(nxt);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-    for (int s = 0; s < G::STEPS; ++s) {
-      u32x4 fx[G::NB], fy[G::NB];
-#pragma unroll
-      for (int b = 0; b < G::NB; ++b) {
-        if constexpr (!XT) fx[b] = frag_kcont<G>(lds_x, b, s, lane); else fx[b] = frag_kstr<G, TILE>(lds_x, b, s, lane);
-        if constexpr (!YT) fy[b] = frag_kstr<G, TILE>(lds_y, b, s, lane); else fy[b] = frag_kcont<G>(lds_y, b, s, lane);
-      }
-#pragma unroll
-      for (int bj = 0; bj < G::NB; ++bj)
-#pragma unroll
-        for (int bi = 0; bi < G::NB; ++bi) acc[bj][bi] = Tr::mfma(fy[bj], fx[bi], acc[bj][bi]);
+    for (int q = 0; q < 4; ++q) {
+      const int at = (8 * q + 4 * kg) * ES;  // byte of the row
+      char *dst = stage + li * B::kRow + ((((at >> 4) ^ li) & (B::kChunks - 1)) << 4) + (at & 15);
+      if constexpr (ES == 2)
+        *reinterpret_cast<uint2 *>(dst) = uint2{(uint32_t)Tr::round(acc[4 * q]) | ((uint32_t)Tr::round(acc[4 * q + 1]) << 16),
+                                                (uint32_t)Tr::round(acc[4 * q + 2]) | ((uint32_t)Tr::round(acc[4 * q + 3]) << 16)};
+      else
+        *reinterpret_cast<f32x4 *>(dst) = f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  }
-#undef BSA_FETCH
-#undef BSA_LOAD_WINDOW
-
-  // epilogue: acc[bj][bi][r] = O[i = 32 bi + lane%32][j = 32 bj + 8 (r/4) + 4 (lane/32) + r%4]
-  char *stage = lds_x;
-  const int li = lane & 31, lh = lane >> 5;
+    char *ob = out + (n0 + done) * B::kBytes + lane * 16;
 #pragma unroll
-  for (int bj = 0; bj < G::NB; ++bj)
-#pragma unroll
-    for (int bi = 0; bi < G::NB; ++bi)
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        const int i = 32 * bi + li;
-        const int j = 32 * bj + 8 * rq + 4 * lh;
-        const int chunk = (j * ES) / 16, within = (j * ES) % 16;
-        char *dst = stage + i * (G::OCPR * 16) + ((chunk ^ (i & (G::OCPR - 1) & 7)) * 16) + within;
-        // 16-bit: rows i and i + OCPR share a chunk position; put their 8-byte pieces in opposite halves
-        if constexpr (ES == 2) dst = stage + i * (G::OCPR * 16) + ((chunk ^ (i & (G::OCPR - 1) & 7)) * 16) +
-                                     (within ^ (((i / G::OCPR) & 1) * 8));
-        if constexpr (ES == 2) {
-          uint2 v;
-          v.x = (uint32_t)Tr::round(acc[bj][bi][4 * rq]) | ((uint32_t)Tr::round(acc[bj][bi][4 * rq + 1]) << 16);
-          v.y = (uint32_t)Tr::round(acc[bj][bi][4 * rq + 2]) | ((uint32_t)Tr::round(acc[bj][bi][4 * rq + 3]) << 16);
-          *reinterpret_cast<uint2 *>(dst) = v;
-        } else {
-          float4 v;
-          v.x = acc[bj][bi][4 * rq];
-          v.y = acc[bj][bi][4 * rq + 1];
-          v.z = acc[bj][bi][4 * rq + 2];
-          v.w = acc[bj][bi][4 * rq + 3];
-          *reinterpret_cast<float4 *>(dst) = v;
-        }
-      }
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  char *ob = out + n * block_bytes + (int64_t)ti * TILE * (int64_t)ld_bytes + (int64_t)tj * TILE * ES;
-#pragma unroll
-  for (int t = 0; t < G::OUT_STORES; ++t) {
-    const int q = t * 64 + lane;
-    const int row = q / G::OCPR, chunk = q % G::OCPR;
-    u32x4 v =
-        *reinterpret_cast<const u32x4 *>(stage + row * (G::OCPR * 16) + ((chunk ^ (row & (G::OCPR - 1) & 7)) * 16));
-    if constexpr (ES == 2) {
-      if ((row / G::OCPR) & 1) v = u32x4{v[2], v[3], v[0], v[1]};
+    for (int t = 0; t < kStores; ++t) {
+      const int row = (t * 64 + lane) / B::kChunks, chunk = lane & (B::kChunks - 1);
+      const u32x4 v = *reinterpret_cast<const u32x4 *>(stage + row * B::kRow + (((chunk ^ row) & (B::kChunks - 1)) << 4));
+      __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(ob + t * 1024));
     }
-    *reinterpret_cast<u32x4 *>(ob + row * ld_bytes + chunk * 16) = v;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  };
+  auto advance = [&]() {
+    ++done;
+    block_end = __builtin_amdgcn_readlane(off_win, done + 1 <= count ? done + 1 : count);
+  };
+  // blocks without a pair in front of pair p
+  auto zeros_until = [&](int p) {
+    while (done < count && block_end <= p) {
+      char *ob = out + (n0 + done) * B::kBytes + lane * 16;
+#pragma unroll
+      for (int t = 0; t < kStores; ++t) __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u}, reinterpret_cast<u32x4 *>(ob + t * 1024));
+      advance();
+    }
+  };
+
+  if (p_first < p_last) request(ring);
+  if (kDepth > 1 && p_first + 1 < p_last) request(ring + kPair);
+  zeros_until(p_first);
+  int place = 0;
+  bool stored = false;  // exactly kStores stores were issued between the requests of the next two pairs
+  for (int p = p_first; p < p_last; ++p) {
+    // this pair's copies have landed; what may be on its way is what was issued behind them
+    if (kDepth == 1 || p + 1 >= p_last) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (stored) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * B::kCopies + kStores) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * B::kCopies) : "memory");
+    stored = false;
+    char *const slot = ring + place;
+    if (kDepth > 1) place ^= kPair;
+    u32x4 fx[B::kFrags], fy[B::kFrags];
+#pragma unroll
+    for (int s = 0; s < B::kFrags; ++s) fx[s] = rx.frag(slot, s), fy[s] = ry.frag(slot + B::kBytes, s);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next blocks are copied over them
+    if (p + 1 < block_end && next < p_last) {
+      request(slot);
+#pragma unroll
+      for (int s = 0; s < B::kFrags; ++s) acc = Tr::mfma(fy[s], fx[s], acc);
+    } else {
+#pragma unroll
+      for (int s = 0; s < B::kFrags; ++s) acc = Tr::mfma(fy[s], fx[s], acc);
+      if (p + 1 >= block_end) {
+        flush(slot);
+        advance();
+        stored = done == count || block_end > p + 1;
+        zeros_until(p + 1);
+      }
+      if (next < p_last) request(slot);
+    }
   }
 }
 
@@ -784,29 +647,30 @@ __global__ __launch_bounds__(256) void matmul_small16_f32_kernel(const char *__r
   flush_until(p_last);
 }
 
-template <typename Tr, int TILE>
-int launch_mfma(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs,
-                const int32_t *block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int sbs, int trans_x,
-                int trans_y, hipStream_t s) {
-  const int side = sbs / TILE;
-  int side_log2 = 0;
-  while ((1 << side_log2) < side) ++side_log2;
-  const int64_t n_tiles = nnz_o * side * side;
-  // a multiple of 8 workgroups so that every XCD owns the same number of list positions
-  const int64_t blocks = bsa::cdiv(bsa::cdiv(n_tiles, 4), 8) * 8;
-  if (blocks > 0x7fffffffLL) return bsa::fail(BSA_ELIMIT, "bsa_matmul: too many output tiles");
+template <typename Tr>
+int launch_runs32(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs, int64_t nnz_o,
+                  int64_t nnz_x, int64_t nnz_y, int trans_x, int trans_y, hipStream_t s) {
+  constexpr int kWaves = 4;
+  // The forward product's lists are short and its output dense: a run of up to three blocks spreads a wave's first loads
+  // (offsets, pairs, operands: three latencies) over more pairs, as long as there are enough waves (bf16, 16 x 4096^3, run
+  // 1 / 2 / 3 / 4: 521 / 487 / 490 / 488 us; 36259 blocks of 1.2 pairs: 28.9 / 26.6 / 24.9 / 25.2).  The gradients' lists are long, and longer
+  // runs only scatter what is in flight on an L2 (dX of the first: 545 / 764 / 875 / 927).
+  int64_t run = trans_x || trans_y ? 1 : nnz_o / 12288;
+  run = run < 1 ? 1 : (run > 3 ? 3 : run);
+  const int64_t blocks = bsa::cdiv(bsa::cdiv(bsa::cdiv(nnz_o, run), (int64_t)kWaves), (int64_t)8) * 8;
+  if (blocks > 0x7fffffffLL) return bsa::fail(BSA_ELIMIT, "bsa_matmul: too many output blocks");
   const char *xc = static_cast<const char *>(x);
   const char *yc = static_cast<const char *>(y);
   char *oc = static_cast<char *>(out);
-#define BSA_MM_LAUNCH(XT, YT)                                                                                      \
-  matmul_mfma_kernel<Tr, TILE, XT, YT><<<(unsigned)blocks, 256, 0, s>>>(xc, yc, oc, pair_offsets, pairs, block_order, \
-                                                                        n_tiles, sbs, side_log2, nnz_x, nnz_y)
+#define BSA_MM_LAUNCH(XT, YT)                                                                                        \
+  matmul_runs32_kernel<Tr, XT, YT><<<(unsigned)blocks, 64 * kWaves, 0, s>>>(xc, yc, oc, pair_offsets, pairs, nnz_o, \
+                                                                                    nnz_x, nnz_y, (int)run)
   if (!trans_x && !trans_y) BSA_MM_LAUNCH(false, false);
   else if (!trans_x && trans_y) BSA_MM_LAUNCH(false, true);
   else if (trans_x && !trans_y) BSA_MM_LAUNCH(true, false);
   else BSA_MM_LAUNCH(true, true);
 #undef BSA_MM_LAUNCH
-  return bsa::check_launch("matmul_mfma_kernel");
+  return bsa::check_launch("matmul_runs32_kernel");
 }
 
 template <typename Tr>
@@ -881,7 +745,7 @@ int launch_any(const void *x, const void *y, void *out, const int32_t *pair_offs
     return bsa::check_launch("matmul_small16_f32_kernel");
   }
   if (sbs == 32)
-    return launch_mfma<Tr, 32>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, sbs, trans_x, trans_y, s);
+    return launch_runs32<Tr>(x, y, out, pair_offsets, pairs, nnz_o, nnz_x, nnz_y, trans_x, trans_y, s);
   return launch_quad<Tr>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, sbs, trans_x, trans_y, s);
 }
 

@@ -1,4 +1,5 @@
-"""The matmul kernels for blocks of 16 and 32 (csrc/matmul.hip) where they can go wrong: output blocks without a pair in front of, between and behind others, lists
+"""The matmul kernels for blocks of 16 and 32 (csrc/matmul.hip: matmul_runs32_kernel, matmul_small16_kernel,
+matmul_small16_f32_kernel) where they can go wrong: output blocks without a pair in front of, between and behind others, lists
 longer than the 64 entries of a window, launches of one, two and more output blocks per wave."""
 
 import pytest
