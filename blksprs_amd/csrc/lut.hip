@@ -1,9 +1,13 @@
 // Layout -> lookup-table kernels (integer only, bit-exact).
 //
 // Everything derives from one primitive, an exclusive prefix sum over the
-// flattened layout done in three launches (per-tile counts, a scan of the tile
-// counts, a per-tile scan that writes results).  Tiles are 2048 entries; a
-// layout of a million entries is 512 tiles.
+// flattened layout in tiles of 2048 entries (a layout of a million entries is 512
+// tiles).  What a tile's workgroup needs to know is the sum of all entries in front
+// of its tile.  These kernels are a few microseconds of latency each, so the rule
+// is to launch few: small layouts are counted again from the front by every
+// workgroup (one launch), larger ones have their tiles counted first and every
+// workgroup adds up the counts in front of its own (two), and only beyond 1024 tiles
+// a launch of its own scans the counts (three).
 #include "common.h"
 
 #include <mutex>
@@ -80,12 +84,63 @@ __global__ __launch_bounds__(kScanThreads) void scan_tiles_kernel(const int32_t 
   }
 }
 
+// Where a tile's workgroup finds the sum of the entries in front of its tile.
+//   kFromOffsets: scan_tiles_kernel has left it (and the totals).
+//   kFromCounts: it adds up the counts of the tiles in front of its own; at most kMaxCountedTiles of them.
+//   kFromLayout: it counts the layout bytes in front of its tile, 16 at a time; at most kMaxRecounted of them, from a
+//   16-byte aligned layout.
+// In the last two the workgroup of the last tile writes the totals.  65536 entries: one launch of 5.1 us instead of 4.7 +
+// 3.9 + 4.5 us and the two gaps between them; a conversion to sparse and back of 16 x 4096 x 4096 (two scans): 293 -> 287 us; a
+//   first attention call on a new layout (eight scans): 382 -> 325 us.
+// Each limit is where the reads repeated by all workgroups, half of the tiles each on average, reach 4 to 8 MB in
+// all, which is still less than the launch it saves: 2^17 bytes in 64 tiles, or 1024 counts in 1024 tiles.
+enum Prefix { kFromOffsets, kFromCounts, kFromLayout };
+constexpr int64_t kMaxCountedTiles = 1024;
+constexpr int64_t kMaxRecounted = (int64_t)1 << 17;
+
+template <Prefix kPrefix>
+__device__ inline int64_t sum_in_front(const int64_t *tile_offsets, const int32_t *tile_counts, const uint8_t *layout) {
+  if constexpr (kPrefix == kFromOffsets) return tile_offsets[blockIdx.x];
+  // below 2^31: at most 1024 tiles of 2048 entries
+  int s = 0;
+  if constexpr (kPrefix == kFromCounts) {
+    for (int64_t i = threadIdx.x; i < blockIdx.x; i += kScanThreads) s += tile_counts[i];
+  } else {
+    const uint4 *chunks = reinterpret_cast<const uint4 *>(layout);
+    auto count = [](uint32_t v) { return __popc((((v & 0x7f7f7f7fu) + 0x7f7f7f7fu) | v) & 0x80808080u); };
+    const int end = (int)blockIdx.x * (kScanTile / 16);
+    // eight loads in flight per thread: one by one, the 16 rounds of the last tiles of 65536 entries took 5 us
+    for (int i = threadIdx.x; i < end; i += 8 * kScanThreads) {
+      uint4 v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = i + j * kScanThreads < end ? chunks[i + j * kScanThreads] : uint4{0, 0, 0, 0};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += count(v[j].x) + count(v[j].y) + count(v[j].z) + count(v[j].w);
+    }
+  }
+  int total;
+  block_exclusive_scan(s, total);
+  return total;
+}
+
+// what scan_tiles_kernel writes besides the offsets
+__device__ inline void write_totals(int64_t total, int64_t *stats, int32_t *last_i32) {
+  if (blockIdx.x != gridDim.x - 1 || threadIdx.x != 0) return;
+  stats[0] = total;
+  stats[1] = 0;
+  if (last_i32) *last_i32 = (int32_t)total;
+}
+
 // Per tile: writes the reverse index and, when row_len > 0, the CSR offset of
 // every row that starts inside the tile.
+template <Prefix kPrefix>
 __global__ __launch_bounds__(kScanThreads) void write_packed_kernel(const uint8_t *__restrict__ layout, int64_t n,
                                                                     const int64_t *__restrict__ tile_offsets,
+                                                                    const int32_t *__restrict__ tile_counts,
                                                                     int64_t row_len, int64_t *__restrict__ packed,
-                                                                    int32_t *__restrict__ row_offsets) {
+                                                                    int32_t *__restrict__ row_offsets,
+                                                                    int64_t *__restrict__ stats,
+                                                                    int32_t *__restrict__ last_i32) {
   const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
   int flags[kScanItems];
   int s = 0;
@@ -96,7 +151,9 @@ __global__ __launch_bounds__(kScanThreads) void write_packed_kernel(const uint8_
     s += flags[i];
   }
   int total;
-  int64_t prefix = tile_offsets[blockIdx.x] + block_exclusive_scan(s, total);
+  const int64_t front = sum_in_front<kPrefix>(tile_offsets, tile_counts, layout);
+  int64_t prefix = front + block_exclusive_scan(s, total);
+  if constexpr (kPrefix != kFromOffsets) write_totals(front + total, stats, last_i32);
 #pragma unroll
   for (int i = 0; i < kScanItems; ++i) {
     int64_t p = base + i;
@@ -332,10 +389,22 @@ int lut_packed_launch(const char *who, const uint8_t *layout, int64_t n, int64_t
   BSA_REQUIRE(tile_counts && tile_offsets, "%s: no workspace", who);
   const int64_t tiles = bsa::cdiv(n, kScanTile);
   const int64_t n_rows = row_len > 0 ? n / row_len : 0;
-  tile_counts_kernel<uint8_t><<<(unsigned)tiles, kScanThreads, 0, s>>>(layout, n, tile_counts);
-  scan_tiles_kernel<<<1, kScanThreads, 0, s>>>(tile_counts, tiles, tile_offsets, stats_dev,
-                                               row_len > 0 ? row_offsets + n_rows : nullptr);
-  write_packed_kernel<<<(unsigned)tiles, kScanThreads, 0, s>>>(layout, n, tile_offsets, row_len, packed, row_offsets);
+  int32_t *last = row_len > 0 ? row_offsets + n_rows : nullptr;
+#define BSA_WRITE_PACKED(PREFIX)                                                                                       \
+  write_packed_kernel<PREFIX><<<(unsigned)tiles, kScanThreads, 0, s>>>(layout, n, tile_offsets, tile_counts, row_len, \
+                                                                       packed, row_offsets, stats_dev, last)
+  if (n <= kMaxRecounted && (reinterpret_cast<uintptr_t>(layout) & 15) == 0) {
+    BSA_WRITE_PACKED(kFromLayout);
+  } else {
+    tile_counts_kernel<uint8_t><<<(unsigned)tiles, kScanThreads, 0, s>>>(layout, n, tile_counts);
+    if (tiles <= kMaxCountedTiles) {
+      BSA_WRITE_PACKED(kFromCounts);
+    } else {
+      scan_tiles_kernel<<<1, kScanThreads, 0, s>>>(tile_counts, tiles, tile_offsets, stats_dev, last);
+      BSA_WRITE_PACKED(kFromOffsets);
+    }
+  }
+#undef BSA_WRITE_PACKED
   if (row_len > 0) row_max_kernel<<<grid_for(n_rows, 256), 256, 0, s>>>(row_offsets, n_rows, stats_dev);
   if (int rc = bsa::check_launch(who)) return rc;
   return fetch_stats(stats_dev, stats_host, s);
