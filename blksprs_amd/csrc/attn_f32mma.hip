@@ -1,7 +1,8 @@
-// Block-sparse flash attention forward on the fp32 matrix-core instruction (v_mfma_f32_16x16x4_f32): fp32
-// operands of every block size, and 16-bit operands of the block sizes the 16-bit matrix-core kernel does not
-// take (they are widened to fp32 while they are staged, probabilities are rounded to the operand type before
-// they multiply V, as the reference does, blksprs/ops/flash_attention.py:1193).
+// Block-sparse flash attention forward on the fp32 matrix-core instruction (v_mfma_f32_16x16x4_f32): what the kernels
+// of attn_mfma.hip (16-bit, 64 x 64) and attn_small_fwd.hip (blocks of 16 and 32) leave: fp32 blocks of 64, longer
+// head dimensions, scales that are not positive, tensors that do not start on 16 bytes.  16-bit operands are widened
+// to fp32 while they are staged, probabilities are rounded to the operand type before they multiply V, as the
+// reference does (blksprs/ops/flash_attention.py:1193).
 //
 // One workgroup owns one (batch entry, query block).  Its waves form G groups of sbs / 16 waves: the groups
 // share the key list (group g takes the entries g, g + G, ...), each with its own LDS tile and its own running

@@ -1,6 +1,5 @@
 // Block-sparse flash attention backward on the fp32 matrix-core instruction (v_mfma_f32_16x16x4_f32), for the
-// configurations attn_f32mma.hip computes forward: fp32 operands of every block size, 16-bit operands of the
-// block sizes and head slice counts the 16-bit matrix-core kernels do not take (widened to fp32 while staged; P
+// configurations attn_f32mma.hip computes forward (16-bit operands are widened to fp32 while staged; P
 // and dS are rounded to the operand type before they enter a product, as the reference does,
 // blksprs/ops/flash_attention.py:1452, :1468, :1692).
 //

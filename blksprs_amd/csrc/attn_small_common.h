@@ -568,6 +568,14 @@ inline bool small_applies(const bsa_attn_args &a) {
   if (a.n_q_blocks > most || a.n_k_blocks > most || a.n_v_blocks > most || a.n_o_blocks > most ||
       a.n_mask_blocks > most || a.n_bias_blocks > most || a.nq * a.sbs > most || a.nk * a.sbs > most)
     return false;
+  // slices are copied into LDS and stored 16 bytes at a time, mask rows are read 4 bytes at a time: a tensor that starts in
+  // the middle of such a piece (a view into a larger buffer) takes the kernels that load through registers
+  const uintptr_t starts = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
+                           reinterpret_cast<uintptr_t>(a.v) | reinterpret_cast<uintptr_t>(a.o) |
+                           reinterpret_cast<uintptr_t>(a.d_o) | reinterpret_cast<uintptr_t>(a.dq) |
+                           reinterpret_cast<uintptr_t>(a.dk) | reinterpret_cast<uintptr_t>(a.dv) |
+                           reinterpret_cast<uintptr_t>(a.dbias);
+  if ((starts & 15) != 0 || (reinterpret_cast<uintptr_t>(a.mask) & 3) != 0) return false;
   const int64_t slices = a.nh > a.nhv ? a.nh : a.nhv;
   return slices >= 1 && slices <= 128 / a.sbs;
 }

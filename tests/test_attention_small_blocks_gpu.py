@@ -6,7 +6,9 @@ large enough for every way of sharing a list between waves."""
 import pytest
 import torch
 
-from tests.test_attention_gpu import _run_case
+import blksprs_amd as bs
+from oracle import blksprs_oracle as orc
+from tests.test_attention_gpu import TOL, _run_case, assert_close, rand_blocks
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +50,35 @@ def test_rows_over_xcds(device, dtype, B, n):
     """Whole batch entries of an XCD, entries shared by all eight, last rows that are no multiple of eight."""
     _run_case(device, dtype, 16, B=B, nq=n, nk=n, nh=2, nhv=2, density=0.5, seed=100 * B + n)
     _run_case(device, dtype, 16, B=B, nq=n, nk=n, nh=1, nhv=1, density=0.5, seed=100 * B + n, use_causal=True)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("sbs", [16, 32])
+def test_tensors_that_start_inside_a_16_byte_piece(device, dtype, sbs):
+    """Operands, output gradient and mask as contiguous views one element into a larger buffer: the kernels that move
+    16 bytes at a time leave them to the ones that load through registers, forward and backward, one by one."""
+    def inside(t):
+        buffer = torch.empty(t.numel() + 1, dtype=t.dtype, device=device)
+        view = buffer[1:].view(t.shape).copy_(t)
+        assert view.is_contiguous() and view.data_ptr() % 16 == t.element_size()
+        return view
+
+    g = torch.Generator().manual_seed(sbs)
+    B, n, nh = 2, 5, 2
+    la = orc.random_layout((B, n, n), 0.6, g, ensure_rows=True)
+    full = torch.ones((B, n, nh), dtype=torch.bool)
+    q, k, v, go = (rand_blocks(B * n * nh, sbs, dtype, sbs + i) for i in range(4))
+    mask = torch.rand((int(la.sum()), sbs, sbs), generator=g) < 0.3
+    r64 = [t.double().requires_grad_(True) for t in (q, k, v)]
+    ref = orc.flash_attention(r64[0], full.numpy(), r64[1], full.numpy(), r64[2], full.numpy(), la.numpy(), sbs, mask=mask,
+                              layout_mask=la.numpy(), acc_dtype=torch.float64)
+    ref.backward(go.double())
+    fd, ld = full.to(device), la.to(device)
+    for which in ("q", "k", "v", "go", "mask", "all"):
+        place = lambda name, t: inside(t) if which in (name, "all") else t.to(device)
+        ops = [place(name, t).detach().requires_grad_(True) for name, t in zip("qkv", (q, k, v))]
+        out = bs.ops.flash_attention(ops[0], fd, ops[1], fd, ops[2], fd, ld, sbs, attention_mask=place("mask", mask),
+                                     sparsity_layout_mask=ld)
+        out.backward(place("go", go))
+        for name, got, want in zip(("O", "dQ", "dK", "dV"), (out, *(t.grad for t in ops)), (ref, *(t.grad for t in r64))):
+            assert_close(got, want, TOL[dtype], f"{name}, {which} inside a piece")
