@@ -13,7 +13,7 @@ from torch import Tensor
 
 from .. import _capi
 from ..utils.blksprs_tensor import BlksprsTensor
-from ..utils.tools import (build_packed_indices, ceil_pow2, eager_only, finalize_layout_cache, nonzero_from_packed, pack_layout,
+from ..utils.tools import (ceil_pow2, eager_only, finalize_layout_cache, nonzero_from_packed, pack_layout,
                            prepare_layout_cache, sorted_rows_from_offsets)
 from ..utils.validation import (ensure_contiguous, validate_contiguous, validate_device, validate_dimensions,
                                 validate_dtype_float_32, validate_sparsity, validate_sparsity_block_size)
@@ -80,7 +80,7 @@ def softmax_build_layout_cache(layout_cache: dict | None, sparsity_layout: Tenso
     if "packed_indices_rws" not in layout_cache:
         offsets = layout_cache["row_offsets"]
         rows_active = (offsets[1:] != offsets[:-1])
-        layout_cache["packed_indices_rws"] = build_packed_indices(rows_active)
+        layout_cache["packed_indices_rws"] = pack_layout(rows_active).packed
     validate_contiguous(sparsity_layout, layout_cache["layout_indices"], layout_cache["packed_indices_rws"])
     return finalize_layout_cache(layout_cache)
 

@@ -123,7 +123,7 @@ def pack_layout(layout: Tensor, row_len: int = 0) -> PackedLayout:
 
 def build_packed_indices(sparsity_layout: Tensor) -> Tensor:
     """int64 reverse index of a layout: position among the active blocks, ``-1`` for inactive ones."""
-    return pack_layouts((sparsity_layout, 0), counts=False)[0].packed
+    return pack_layout(sparsity_layout).packed
 
 
 def nonzero_from_packed(packed: Tensor, shape, count: int) -> Tensor:
