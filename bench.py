@@ -62,7 +62,7 @@ def traffic_bytes(config):
 
 # file stem of the summary of a configuration under profiles/: the kernel(s) and the workload
 PROFILE_STEMS = {
-    "c1": "matmul_mfma_kernel_c1_fp32_matmul",
+    "c1": "matmul_runs32_kernel_c1_fp32_matmul",
     "c2": "matmul_rows_kernel_c2_bf16_matmul",
     "c2bwd": "matmul_lines_kernel_c2bwd_bf16_matmul_backward",
     "c3": "softmax_fwd_kernel_c3_fp32_softmax",
@@ -71,11 +71,11 @@ PROFILE_STEMS = {
     "c4cl": "attn_fwd_mfma_kernel_c4cl_bf16_attention_forward_causal_lengths",
     "c4bwd": "attn_kernels_c4_bf16_attention_forward_backward",
     "c5": "matmul_small16_kernel_c5_fp16_sbs16",
-    "a1": "attn_f32mma_kernels_a1_fp32_reference_benchmark",
-    "a1bwd": "attn_f32mma_kernels_a1bwd_fp32_reference_benchmark_backward",
-    "m32": "matmul_mfma_kernel_m32_bf16_sbs32",
-    "m128": "matmul_mfma_kernel_m128_bf16_sbs128",
-    "mf32": "matmul_mfma_kernel_mf32_fp32_sbs64",
+    "a1": "attn_small_kernels_a1_fp32_reference_benchmark",
+    "a1bwd": "attn_small_kernels_a1bwd_fp32_reference_benchmark_backward",
+    "m32": "matmul_runs32_kernel_m32_bf16_sbs32",
+    "m128": "matmul_quad_kernel_m128_bf16_sbs128",
+    "mf32": "matmul_quad_kernel_mf32_fp32_sbs64",
     "v1": "to_sparse_kernel_v1_bf16_to_sparse",
     "v2": "to_dense_kernel_v2_bf16_to_dense",
     "t1": "transpose_blocks16_kernel_t1_bf16_transpose",
@@ -399,14 +399,14 @@ def matmul_workload(name, B, n, sbs, dtype, density, ensure_rows, value_scale, d
                           f"torch matmul + to_sparse, {dt * reps:.1f} s"}
 
     dt_name = {torch.bfloat16: "bf16", torch.float16: "f16", torch.float32: "f32"}[dtype]
+    tile_kernel = ("matmul_quad_kernel" if sbs >= 64 else "matmul_runs32_kernel" if sbs == 32 else
+                   "matmul_small16_kernel" if dtype != torch.float32 else "matmul_small16_f32_kernel")
     if backward:
         kernel = ("matmul_lines_kernel (two launches: dX by rows of dO, dY by its columns)"
                   if sbs == 64 and dtype != torch.float32 else
-                  "matmul_mfma_kernel (two launches: dX with y read transposed, dY with x read transposed)")
-    elif sbs > 16:
-        kernel = "matmul_rows_kernel" if sbs == 64 and dtype != torch.float32 else "matmul_mfma_kernel"
+                  f"{tile_kernel} (two launches: dX with y read transposed, dY with x read transposed)")
     else:
-        kernel = "matmul_small16_kernel" if dtype != torch.float32 else "matmul_small_kernel"
+        kernel = "matmul_rows_kernel" if sbs == 64 and dtype != torch.float32 else tile_kernel
     # 172 FLOP per byte at sbs 64 and 25 % density: below the balance of the 16-bit matrix cores (312 FLOP/B), above
     # that of the fp32 ones (20 FLOP/B): fp32 products of large problems are bound by the fp32 matrix-core peak
     bound = "mfma" if dtype == torch.float32 and sbs >= 32 and B * n * sbs >= 16 * 4096 else "hbm"
@@ -844,7 +844,7 @@ def reference_attention_benchmark(dev, m=2048, backward=False):
                 "sample": f"1 of {bh} heads x {reps} passes, dense masked fp32 torch attention, {dt * reps:.1f} s"}
 
     return dict(step=step, flops=flops, alg_bytes=alg_bytes, dtype="f32", bound="mfma", cpu_baseline=cpu_baseline,
-                check=check, kernel="attn_fwd_f32mma_kernel" + (" + attn_f32mma_delta / dkdv / dq kernels" if backward else ""),
+                check=check, kernel="attn_small_fwd_kernel" + (" + attn_small_dq / dkv kernels" if backward else ""),
                 config={"workload": "a1_flash_attention_fp32_reference_benchmark" + ("_fwd_bwd" if backward else ""),
                         "batch_heads": bh, "seq": m,
                         "head_dim": hd, "sparsity_block_size": sbs, "layout_blocks": nnz,
@@ -861,7 +861,7 @@ def make_workload(name, dev):
         return matmul_workload("c2_matmul_bf16_backward", 16, 64, 64, torch.bfloat16, 0.25, False, 1.0 / 64.0, dev,
                                16, backward=True, check_batch=3)
     # the C2 problem (4096^3, 25 % density, product layout) off the one shape the row kernel takes: other block
-    # sizes and fp32 run on the tile kernel (blksprs/ops/matmul.py:148-253 serves every dtype and block size)
+    # sizes and fp32 run on the kernels of matmul.hip (blksprs/ops/matmul.py:148-253 serves every dtype and block size)
     if name == "m32":
         return matmul_workload("c2_problem_bf16_sbs32", 16, 128, 32, torch.bfloat16, 0.25, False, 1.0 / 64.0, dev, 4,
                                check_batch=3)
