@@ -34,7 +34,6 @@ namespace {
 
 using namespace small;
 
-constexpr float kRescaleStep = 8.f;  // log2 units, see attn_mfma.hip
 constexpr int kWaves = 4;
 
 template <int ES, int SBS, int NS>
@@ -116,15 +115,17 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWav
       for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
     if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, qi, kq);
 
-    // ---- online softmax of the row, the reference maximum following lazily (attn_mfma.hip)
+    // ---- online softmax of the row.  The reference is the exact running maximum: the largest probabilities then lie at
+    // and just below 1, where rounding to 16 bits costs least.  A maximum that follows in steps of up to 2^8 (as in
+    // attn_mfma.hip) saves most of the rescaling and lets them fall anywhere between two powers of two: errors of the output
+    // against 64 bits of 2.27e-3 instead of 2.09e-3 (bf16, 1024 keys, half of the blocks).
     float m_blk = sv[0];
 #pragma unroll
     for (int x = 1; x < kScores; ++x) m_blk = fmaxf(m_blk, sv[x]);
     m_blk = row_max<SBS>(m_blk) * cc;
     const float m_cand = fmaxf(m_i, m_blk);
-    if (__any((m_cand - m_i) > kRescaleStep)) {
-      const bool both_ninf = (m_i == -INFINITY) && (m_cand == -INFINITY);
-      const float alpha = both_ninf ? 1.f : __builtin_amdgcn_exp2f(m_i - m_cand);
+    if (__any(m_cand > m_i)) {
+      const float alpha = m_cand > m_i ? __builtin_amdgcn_exp2f(m_i - m_cand) : 1.f;
       m_i = m_cand;
       l_i *= alpha;
 #pragma unroll
