@@ -173,11 +173,12 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWa
 #pragma unroll
       for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
     if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, qi, kq);
+    apply_factor<Tr, kScores>(sv, cc);
 
     // ---- dS = P (dP - delta)
 #pragma unroll
     for (int x = 0; x < kScores; ++x)
-      sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], cc, neg_lse)) * (dp[x / kRegs][x % kRegs] - delta);
+      sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), neg_lse)) * (dp[x / kRegs][x % kRegs] - delta);
     if (now.special) {
       const late_args_t p = late_args();
       if (p->dbias) {  // every pair is visited once: plain stores
@@ -299,6 +300,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinW
 #pragma unroll
       for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
     if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, kj, kq);
+    apply_factor<Tr, kScores>(sv, cc);
 #pragma unroll
     for (int x = 0; x < kScores; x += 4) {
       const f32x4 l4 = *reinterpret_cast<const f32x4 *>(lse + (x / kRegs) * SBS + 2 * (x % kRegs) + 4 * kq);
@@ -315,7 +317,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinW
         if (ls[x] == -INFINITY) ls[x] = INFINITY;
     }
 #pragma unroll
-    for (int x = 0; x < kScores; ++x) sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], cc, -ls[x]));
+    for (int x = 0; x < kScores; ++x) sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), -ls[x]));
     const Weights<Tr, kScores> pw(sv);
 
     // ---- dS = P (dP - delta)

@@ -339,6 +339,25 @@ __device__ static inline void product_cols(Acc (&out)[NS], const typename Tile<T
   }
 }
 
+// The factor cc of the scores, inside the exponential.  16-bit: fused with the subtraction of the maximum or lse.  fp32: a
+// multiplication of its own in front, since the maximum and lse come from products that were rounded: the score they come
+// from must differ from them by exactly zero (a probability of exactly 1: the output of a query that sees one key is that
+// key's value), where a fused product leaves the rounding of the first (dV of short causal rows 6 % further from 64 bits).
+template <typename Tr, int kScores>
+__device__ static inline void apply_factor(float *sv, float cc) {
+  if constexpr (Tr::kElem == 4) {
+#pragma unroll
+    for (int x = 0; x < kScores; ++x) {
+      sv[x] *= cc;
+      asm("" : "+v"(sv[x]));  // not to be fused after all
+    }
+  }
+}
+template <typename Tr>
+__device__ static inline float late_factor(float cc) {
+  return Tr::kElem == 4 ? 1.f : cc;
+}
+
 // four consecutive values of an output row
 template <typename Tr>
 __device__ static inline void store4(char *p, float a, float b, float c, float d) {

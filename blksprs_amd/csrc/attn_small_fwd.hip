@@ -107,13 +107,14 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWav
     counted = false;
     if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
 
-    // ---- scores: sv holds them up to the positive factor cc, applied inside the exponential
+    // ---- scores: sv holds them up to the positive factor cc, applied inside the exponential (16-bit)
     float sv[kScores];
 #pragma unroll
     for (int t = 0; t < NB; ++t)
 #pragma unroll
       for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
     if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, qi, kq);
+    apply_factor<Tr, kScores>(sv, cc);
 
     // ---- online softmax of the row.  The reference is the exact running maximum: the largest probabilities then lie at
     // and just below 1, where rounding to 16 bits costs least.  A maximum that follows in steps of up to 2^8 (as in
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWav
     float m_blk = sv[0];
 #pragma unroll
     for (int x = 1; x < kScores; ++x) m_blk = fmaxf(m_blk, sv[x]);
-    m_blk = row_max<SBS>(m_blk) * cc;
+    m_blk = row_max<SBS>(m_blk) * late_factor<Tr>(cc);
     const float m_cand = fmaxf(m_i, m_blk);
     if (__any(m_cand > m_i)) {
       const float alpha = m_cand > m_i ? __builtin_amdgcn_exp2f(m_i - m_cand) : 1.f;
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWav
     float sum = 0.f;
 #pragma unroll
     for (int x = 0; x < kScores; ++x) {
-      sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], cc, -m_sub));
+      sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), -m_sub));
       sum += sv[x];
     }
     l_i += sum;

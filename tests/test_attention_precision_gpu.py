@@ -1,5 +1,5 @@
 """Rounding of the attention kernels for blocks of 16 and 32: probabilities are rounded against the exact running maximum
-of their row."""
+of their row, and the score a maximum or lse comes from differs from it by exactly zero."""
 
 import math
 
@@ -48,3 +48,21 @@ def test_probabilities_are_rounded_against_the_exact_maximum(device, dtype, sbs,
         norm += float(want.square().sum())
     assert math.sqrt(exact_error / norm) <= 1.03 * math.sqrt(dense_error / norm), (
         math.sqrt(exact_error / norm), math.sqrt(dense_error / norm))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("sbs", [16, 32])
+def test_a_query_that_sees_one_key_returns_its_value(device, dtype, sbs):
+    """Its probability is exactly one, forward and backward: O is V of that key, and its dO arrives in dV as it is."""
+    n, slices = 3, 64 // sbs
+    lay = torch.ones((1, n, slices), dtype=torch.bool, device=device)
+    la = torch.eye(n, dtype=torch.bool, device=device)[None].contiguous()
+    q, k, v, go = (rand_blocks(n * slices, sbs, dtype, seed, 3.0).to(device) for seed in range(4))
+    # key i alone is left of each block for query i
+    mask = ~torch.eye(sbs, dtype=torch.bool, device=device).expand(n, sbs, sbs).contiguous()
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    out = bs.ops.flash_attention(q, lay, k, lay, v, lay, la, sbs, scale=0.37, attention_mask=mask, sparsity_layout_mask=la)
+    dv, = torch.autograd.grad(out, v, go)
+    assert torch.equal(out.detach(), v.detach())
+    assert torch.equal(dv, go)
