@@ -394,12 +394,12 @@ int launch(const bsa_attn_args &a, hipStream_t s) {
     if (int rc = check_launch("small_zero_kernel")) return rc;
   }
   if (const int64_t rows = a.B * a.nq) {
-    const int split = waves_per_row(rows);
+    const int split = waves_per_row<Tr>(rows);
     attn_small_dq_kernel<Tr, SBS, NS><<<row_groups(a.B, a.nq, kWaves, split), 64 * kWaves, q_lds, s>>>(a, split);
     if (int rc = check_launch("attn_small_dq_kernel")) return rc;
   }
   if (const int64_t rows = a.B * a.nk) {
-    const int split = waves_per_row(rows);
+    const int split = waves_per_row<Tr>(rows);
     attn_small_dkv_kernel<Tr, SBS, NS><<<row_groups(a.B, a.nk, kWaves, split), 64 * kWaves, kv_lds, s>>>(a, split);
     if (int rc = check_launch("attn_small_dkv_kernel")) return rc;
   }

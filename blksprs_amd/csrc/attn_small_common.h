@@ -396,7 +396,8 @@ template <int ES, int SBS, int NS, int NB, bool kOwnIsQuery>
 struct Walk {
   using T = Tile<ES, SBS, NS, NB>;
   int64_t b, own;          // batch entry, own block
-  int end, base, seq_len;  // end of the list, first entry of the window; valid length of a causal sequence
+  int first, step;         // the wave's entries of the list: first, first + step, ...
+  int end, base, seq_len;  // their number, the first one of the window; valid length of a causal sequence
   int other, first_a, first_b, mask, bias;  // of this lane's entry
   uint64_t live, special;
   bool apart;
@@ -408,7 +409,9 @@ struct Walk {
     bool special, apart;
   };
 
-  // part of parts: the contiguous share of the list that this wave walks
+  // part of parts: this wave walks every parts-th entry of the list.  The sums of the parts then have about the same size: with
+  // contiguous parts the first query rows of a causal layout, whose probabilities are the largest, all go into one of them,
+  // and dV of fp32 is 3 to 10 % further from 64 bits.
   __device__ inline void start(const bsa_attn_args &a, int64_t b_, int64_t own_, bool there, int part, int parts) {
     b = b_, own = own_;
     seq_len = 0x7fffffff;
@@ -417,15 +420,12 @@ struct Walk {
       seq_len = len < 0 ? 0 : (len > 0x7fffffffLL ? 0x7fffffff : (int)len);
     }
     const int32_t *offsets = (kOwnIsQuery ? a.key_offsets : a.query_offsets) + b * (kOwnIsQuery ? a.nq : a.nk) + own;
-    int begin = first_lane(offsets[0]);
-    end = first_lane(offsets[1]);
-    if (parts > 1) {
-      const int64_t n = end - begin;
-      end = begin + (int)(n * (part + 1) / parts);
-      begin += (int)(n * part / parts);
-    }
-    if (!there || (int)own * SBS >= seq_len) end = begin;
-    base = begin - 64;
+    first = first_lane(offsets[0]) + part;
+    step = parts;
+    const int left = first_lane(offsets[1]) - first;
+    end = left > 0 ? (int)(((unsigned)left + parts - 1) / parts) : 0;
+    if (!there || (int)own * SBS >= seq_len) end = 0;
+    base = -64;
     other = first_a = first_b = 0;
     mask = bias = -1;
     live = special = 0;
@@ -435,9 +435,8 @@ struct Walk {
   __device__ inline void refill(int lane) {
     const late_args_t p = late_args();
     base += 64;
-    const int e = base + lane;
-    bool in = e < end;
-    other = in ? (kOwnIsQuery ? p->key_indices : p->query_indices)[e] : 0;
+    bool in = base + lane < end;
+    other = in ? (kOwnIsQuery ? p->key_indices : p->query_indices)[first + step * (base + lane)] : 0;
     const bool causal = p->causal_lengths != nullptr;
     in = in && !(causal && ((kOwnIsQuery ? other > (int)own : other < (int)own) || other * SBS >= seq_len));
     const int64_t place = b * (kOwnIsQuery ? p->nk : p->nq) + other;
@@ -599,12 +598,15 @@ inline bool small_applies(const bsa_attn_args &a) {
   return slices >= 1 && slices <= 128 / a.sbs;
 }
 
-// Waves that share one row of a launch of `rows` rows, each walking a contiguous part of its list.  A launch lasts as
-// long as the serial walk of its longest lists, and the last round of a launch of few rounds is mostly empty: shorter
+// Waves that share one row of a launch of `rows` rows, each walking every second or fourth entry of its list.  A launch lasts
+// as long as the serial walk of its longest lists, and the last round of a launch of few rounds is mostly empty: shorter
 // shares help until their prologue (four dependent loads) costs more than the walk.  Forward, 64 rows (8 key blocks
 // each, sbs 32): 9.6 us with two waves per row, 8.1 with four; 4128 rows (sbs 16, causal, up to 65 steps): 80 / 60 / 61 us
-// with one, two, four; 6144 rows (sbs 32, 33 steps): 83 / 75 / 82.
-inline int waves_per_row(int64_t rows) { return rows <= 512 ? 4 : rows <= 8192 ? 2 : 1; }
+// with one, two, four; 6144 rows (sbs 32, 33 steps): 83 / 75 / 82.  Nothing was measured between 64 and 4128 rows, nor beyond
+// 6144.  fp32: always four, for four partial sums: with two and one, O is 14 and 38 % further from 64 bits, dK and dV of a
+// causal layout 26 and 50 % (1024 keys, sbs 16).
+template <typename Tr>
+inline int waves_per_row(int64_t rows) { return Tr::kElem == 4 || rows <= 512 ? 4 : rows <= 8192 ? 2 : 1; }
 
 // The row of a wave.  Workgroup g runs on XCD g % 8, each with its own L2.  Of B batch entries an XCD takes B / 8 whole
 // ones, whose partner blocks no other XCD reads, and every eighth row of the B % 8 that are left.  It walks the rows of all

@@ -51,7 +51,7 @@ struct FwdShape {
   static constexpr int kMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS <= 2 ? 4 : 2) : (NS <= 4 ? 4 : 3);
 };
 
-// split: 1, 2 or 4 waves share one query block, each walking a contiguous part of its key list
+// split: 1, 2 or 4 waves share one query block, each walking every split-th entry of its key list
 template <typename Tr, int SBS, int NS>
 __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWaves)) void attn_small_fwd_kernel(bsa_attn_args a, int split) {
   using Shape = FwdShape<Tr::kElem, SBS, NS>;
@@ -215,7 +215,7 @@ template <typename Tr, int SBS, int NS>
 int launch(const bsa_attn_args &a, hipStream_t s) {
   using Shape = FwdShape<Tr::kElem, SBS, NS>;
   const int64_t rows = a.B * a.nq;
-  const int split = waves_per_row(rows);
+  const int split = waves_per_row<Tr>(rows);
   constexpr int lds = Shape::kLds * kWaves;
   static_assert(lds <= 160 * 1024, "LDS");
   if (lds > 64 * 1024) {

@@ -66,3 +66,29 @@ def test_a_query_that_sees_one_key_returns_its_value(device, dtype, sbs):
     dv, = torch.autograd.grad(out, v, go)
     assert torch.equal(out.detach(), v.detach())
     assert torch.equal(dv, go)
+
+
+@pytest.mark.parametrize("sbs", [16, 32])
+@pytest.mark.parametrize("causal", [False, True])
+def test_fp32_sums_do_not_depend_on_the_number_of_rows(device, sbs, causal):
+    """fp32 sums of a row are formed in four parts whatever the launch: a batch entry's output and gradients are the
+    same bits alone (few rows) and among 140 or 300 others (thousands of rows)."""
+    n, slices = 32, 64 // sbs
+    la = torch.ones((1, n, n), dtype=torch.bool, device=device)
+    if causal:
+        la = la.tril().contiguous()
+    lay = torch.ones((1, n, slices), dtype=torch.bool, device=device)
+    alone = [rand_blocks(n * slices, sbs, torch.float32, seed).to(device) for seed in range(4)]
+
+    def step(batches):
+        q, k, v, go = (t.repeat(batches, 1, 1) for t in alone)
+        for t in (q, k, v):
+            t.requires_grad_(True)
+        full, layout = (t.expand(batches, -1, -1).contiguous() for t in (lay, la))
+        out = bs.ops.flash_attention(q, full, k, full, v, full, layout, sbs)
+        return (out.detach(), *torch.autograd.grad(out, (q, k, v), go))
+
+    first = step(1)
+    for batches in (140, 300):
+        for name, got, want in zip(("O", "dQ", "dK", "dV"), step(batches), first):
+            assert torch.equal(got, want.repeat(batches, 1, 1)), (name, batches)
