@@ -30,7 +30,8 @@ class AttnArgs(ctypes.Structure):
         + [(n, c_int64) for n in ("B", "nq", "nk", "nh", "nhv", "n_q_blocks", "n_k_blocks", "n_v_blocks",
                                   "n_o_blocks", "n_mask_blocks", "n_bias_blocks")]
         + [("sbs", ctypes.c_int32), ("dtype", ctypes.c_int32), ("mask_kind", ctypes.c_int32), ("scale", c_float)]
-        + [("group_offsets", c_void_p), ("group_records", c_void_p), ("group_size", ctypes.c_int32)]
+        + [("group_offsets", c_void_p), ("group_records", c_void_p), ("group_size", ctypes.c_int32),
+           ("o_rows_whole", ctypes.c_int32)]
         + [("bwd_scratch", c_void_p), ("n_layout_blocks", c_int64), ("bwd_scratch_ready", c_int64),
            ("bwd_scratch_bytes", c_int64), ("bwd_ds", c_void_p), ("bwd_ds_bytes", c_int64)]
     )

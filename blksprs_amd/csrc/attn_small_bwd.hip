@@ -100,11 +100,11 @@ __device__ inline void store_gradient(const Acc (&acc)[NS], float scale, void *o
   }
 }
 
-template <typename Tr, int SBS, int NS>
+template <typename Tr, int SBS, int NS, bool kSome>
 __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWaves)) void attn_small_dq_kernel(bsa_attn_args a, int split) {
   using Shape = BwdShape<Tr::kElem, SBS, NS>;
   using T = typename Shape::T;
-  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true>;
+  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true, kSome>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWa
     if (counted) wait_vmem<T::kCopies>();
     else wait_vmem<0>();
     acc_t dp[NB], sacc[NB];
-    product_rows<Tr, SBS, NS, NB>(dp, v_rows, gf);
+    W::template multiply_rows<Tr, true>(dp, now, v_rows, gf, lane);
     wait_lds();
     walk.take(next, lane);
     counted = false;
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWa
     // ---- S^T = K Q^T.  In flight at most: K of this step, V of the next.
     if (counted) wait_vmem<T::kCopies>();
     else wait_vmem<0>();
-    product_rows<Tr, SBS, NS, NB>(sacc, k_rows, qf);
+    W::template multiply_rows<Tr, false>(sacc, now, k_rows, qf, lane);
     float sv[kScores];
 #pragma unroll
     for (int t = 0; t < NB; ++t)
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWa
       }
     }
     // ---- dQ^T += K^T dS^T
-    product_cols<Tr, SBS, NS, NB>(dq, k_cols, Weights<Tr, kScores>(sv));
+    W::template multiply_cols<Tr, false, kScores>(dq, now, k_cols, Weights<Tr, kScores>(sv));
     wait_lds();
     counted = false;
     if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
@@ -213,11 +213,11 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWa
   store_gradient<Tr, SBS, NS>(dq, p->scale, p->dq, p->pidx_q + row * p->nh, (int)p->nh, p->n_q_blocks, qi, kq);
 }
 
-template <typename Tr, int SBS, int NS>
+template <typename Tr, int SBS, int NS, bool kSome>
 __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinWaves)) void attn_small_dkv_kernel(bsa_attn_args a, int split) {
   using Shape = BwdShape<Tr::kElem, SBS, NS>;
   using T = typename Shape::T;
-  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, false>;
+  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, false, kSome>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs, kBufs = Shape::kBufs;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinW
     }
     copy_words_to_lds(stats + (int64_t)other * SBS, dst);
   };
-  auto copy_all = [&](const typename W::Step &s, char *buf) {
+  auto copy_all = [&](typename W::Step &s, char *buf) {
     const bool q_whole = walk.template copy<false>(s, tensor_q, buf, source, lane);
     const bool g_whole = walk.template copy<true>(s, tensor_g, buf + T::kBytes, source, lane);
     copy_stats(s, buf + 2 * T::kBytes);
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinW
 
     // ---- S = Q K^T, P = exp2(S - lse)
     acc_t sacc[NB], dp[NB];
-    product_rows<Tr, SBS, NS, NB>(sacc, q_rows, kf);
+    W::template multiply_rows<Tr, false>(sacc, now, q_rows, kf, lane);
     float sv[kScores], ls[kScores];
 #pragma unroll
     for (int t = 0; t < NB; ++t)
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinW
 #pragma unroll
       for (int i = 0; i < 4; ++i) ls[x + i] = l4[i];
     }
-    product_rows<Tr, SBS, NS, NB>(dp, g_rows, vf);
+    W::template multiply_rows<Tr, true>(dp, now, g_rows, vf, lane);
     float lowest = ls[0];
 #pragma unroll
     for (int x = 1; x < kScores; ++x) lowest = fminf(lowest, ls[x]);
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinW
       for (int i = 0; i < 4; ++i) sv[x + i] *= dp[x / kRegs][x % kRegs + i] - d4[i];
     }
     // ---- dV^T += dO^T P
-    product_cols<Tr, SBS, NS, NB>(dv, g_cols, pw);
+    W::template multiply_cols<Tr, true, kScores>(dv, now, g_cols, pw);
     if constexpr (kBufs == 1) {
       wait_lds();
       walk.take(next, lane);
@@ -338,7 +338,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinW
       }
     }
     // ---- dK^T += Q^T dS
-    product_cols<Tr, SBS, NS, NB>(dk, q_cols, Weights<Tr, kScores>(sv));
+    W::template multiply_cols<Tr, false, kScores>(dk, now, q_cols, Weights<Tr, kScores>(sv));
     if constexpr (kBufs == 1) {
       wait_lds();
       if (next.count) walk.template copy<false>(next, tensor_q, lds, source, lane);
@@ -378,14 +378,14 @@ int raise_lds(K kernel, int bytes) {
   return BSA_OK;
 }
 
-template <typename Tr, int SBS, int NS>
-int launch(const bsa_attn_args &a, hipStream_t s) {
+template <typename Tr, int SBS, int NS, bool kSome>
+int launch_kind(const bsa_attn_args &a, hipStream_t s) {
   using Shape = BwdShape<Tr::kElem, SBS, NS>;
   constexpr int q_lds = Shape::kQLds * kWaves, kv_lds = Shape::kKvLds * kWaves;
   static_assert(q_lds <= 160 * 1024 && kv_lds <= 160 * 1024, "LDS");
   static const int raised = [] {
-    const int rc = raise_lds(&attn_small_dq_kernel<Tr, SBS, NS>, q_lds);
-    return rc ? rc : raise_lds(&attn_small_dkv_kernel<Tr, SBS, NS>, kv_lds);
+    const int rc = raise_lds(&attn_small_dq_kernel<Tr, SBS, NS, kSome>, q_lds);
+    return rc ? rc : raise_lds(&attn_small_dkv_kernel<Tr, SBS, NS, kSome>, kv_lds);
   }();
   if (raised) return raised;
   if (a.dbias && a.n_bias_blocks > 0) {
@@ -395,15 +395,20 @@ int launch(const bsa_attn_args &a, hipStream_t s) {
   }
   if (const int64_t rows = a.B * a.nq) {
     const int split = waves_per_row<Tr>(rows);
-    attn_small_dq_kernel<Tr, SBS, NS><<<row_groups(a.B, a.nq, kWaves, split), 64 * kWaves, q_lds, s>>>(a, split);
+    attn_small_dq_kernel<Tr, SBS, NS, kSome><<<row_groups(a.B, a.nq, kWaves, split), 64 * kWaves, q_lds, s>>>(a, split);
     if (int rc = check_launch("attn_small_dq_kernel")) return rc;
   }
   if (const int64_t rows = a.B * a.nk) {
     const int split = waves_per_row<Tr>(rows);
-    attn_small_dkv_kernel<Tr, SBS, NS><<<row_groups(a.B, a.nk, kWaves, split), 64 * kWaves, kv_lds, s>>>(a, split);
+    attn_small_dkv_kernel<Tr, SBS, NS, kSome><<<row_groups(a.B, a.nk, kWaves, split), 64 * kWaves, kv_lds, s>>>(a, split);
     if (int rc = check_launch("attn_small_dkv_kernel")) return rc;
   }
   return BSA_OK;
+}
+
+template <typename Tr, int SBS, int NS>
+int launch(const bsa_attn_args &a, hipStream_t s) {
+  return all_slices(a, true) ? launch_kind<Tr, SBS, NS, false>(a, s) : launch_kind<Tr, SBS, NS, true>(a, s);
 }
 
 template <typename Tr>

@@ -150,22 +150,18 @@ struct Tile {
     }
   }
 
-  // The same for a block whose slices are missing (zeros) or lie apart: synchronous, slice by slice.  pidx: the packed
-  // indices of the block's n_slices slices (wave uniform).
-  __device__ static inline void gather_block(const char *tensor, const int64_t *pidx, int n_slices, int64_t n_blocks,
-                                             char *dst, uint32_t offset, int lane) {
-    for (int h = 0; h < NS; ++h) {
-      const int64_t idx = h < n_slices ? pidx[h] : -1;
-      const bool on = idx >= 0 && idx < n_blocks;
+  // The same for one slice of a block, packed index idx
+  __device__ static inline void copy_piece(const char *tensor, int idx, char *dst, uint32_t offset, int lane) {
+    const char *src = tensor + (uint64_t)(uint32_t)idx * kPiece;
+    if constexpr (kPiece >= 1024) copy_kib_to_lds<kPiece / 1024>(src, offset, dst);
+    else if (lane < 32) copy_kib_to_lds<1>(src, offset, dst);
+  }
+
+  // zeros for a whole block, written by the wave itself
+  __device__ static inline void clear_block(char *dst, int lane) {
 #pragma unroll
-      for (int i = 0; i < kPiece; i += 1024) {
-        u32x4 v{0u, 0u, 0u, 0u};
-        if (kPiece >= 1024 || lane < 32) {
-          if (on) v = *reinterpret_cast<const u32x4 *>(tensor + idx * kPiece + i + offset);
-          *reinterpret_cast<u32x4 *>(dst + h * kPiece + i + lane * 16) = v;
-        }
-      }
-    }
+    for (int i = 0; i < kBlock; i += 1024)
+      if (kBlock - i >= 1024 || lane < 32) *reinterpret_cast<u32x4 *>(dst + i + lane * 16) = u32x4{0u, 0u, 0u, 0u};
   }
 
   // ---- row fragments (contraction over the head dimension): 16 bytes of a row per lane
@@ -259,10 +255,13 @@ template <int ES, int SBS, int NS>
 struct OwnRows {
   using T = Tile<ES, SBS, NS, 2>;
   u32x4 fr[T::kFrags];
+  uint32_t there;  // bit h: the block has slice h (wave uniform)
 
   // pidx: packed indices of the block's slices, n_slices of them are there
   __device__ inline void load(const void *tensor, const int64_t *pidx, int n_slices, int64_t n_blocks, int lane) {
     const int r = lane % SBS, g = lane / SBS;
+    const int64_t mine = lane < n_slices ? pidx[lane] : -1;
+    there = (uint32_t)__ballot(mine >= 0 && mine < n_blocks);
 #pragma unroll
     for (int f = 0; f < T::kFrags; ++f) {
       int h, chunk;
@@ -297,6 +296,30 @@ __device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<T
   for (int f = 0; f < Tile<Tr::kElem, SBS, NS, NB>::kFrags; ++f)
 #pragma unroll
     for (int t = 0; t < NB; ++t) Tr::rows(acc[t], rows.frag(t, f), own.fr[f]);
+}
+
+// The same over the slices in have[t] only: a slice that one of the two blocks does not have adds nothing, where its zeros
+// would turn an infinite or NaN value of the other into NaN
+template <typename Tr, int SBS, int NS, int NB, typename Acc>
+__device__ static inline void product_some_rows(Acc (&acc)[NB], const typename Tile<Tr::kElem, SBS, NS, NB>::RowReader &rows,
+                                                const OwnRows<Tr::kElem, SBS, NS> &own, const uint32_t (&have)[NB], int lane) {
+  using T = Tile<Tr::kElem, SBS, NS, NB>;
+#pragma unroll
+  for (int t = 0; t < NB; ++t)
+#pragma unroll
+    for (int r = 0; r < (SBS == 32 ? 16 : 4); ++r) acc[t][r] = 0.f;
+#pragma unroll
+  for (int t = 0; t < NB; ++t)
+#pragma unroll
+    for (int f = 0; f < T::kFrags; ++f) {
+      if constexpr (Tr::kElem == 2 && SBS == 16) {  // lanes below 32 hold slice 2 f, the others 2 f + 1
+        const bool on = (have[t] >> (2 * f + (lane >> 5))) & 1;
+        const u32x4 none{0u, 0u, 0u, 0u}, theirs = rows.frag(t, f);
+        Tr::rows(acc[t], on ? theirs : none, on ? own.fr[f] : none);
+      } else {
+        if ((have[t] >> (f / T::kSliceFrags)) & 1) Tr::rows(acc[t], rows.frag(t, f), own.fr[f]);
+      }
+    }
 }
 
 // Probabilities (or dS) of a step, as the accumulators of its NB blocks hold them one after the other, made the second
@@ -336,6 +359,39 @@ __device__ static inline void product_cols(Acc (&out)[NS], const typename Tile<T
 #pragma unroll
       for (int m = 0; m < kScores / 8; ++m)
         Tr::rows(out[h], SBS == 32 ? cols.frag(m >> 1, m & 1, h) : cols.frag(0, m, h), w.w[m]);
+  }
+}
+
+// the same over the slices in have[t]
+template <typename Tr, int SBS, int NS, int NB, int kScores, typename Acc>
+__device__ static inline void product_some_cols(Acc (&out)[NS], const typename Tile<Tr::kElem, SBS, NS, NB>::ColReader &cols,
+                                                const Weights<Tr, kScores> &w, const uint32_t (&have)[NB]) {
+  if constexpr (Tr::kElem == 4) {
+    constexpr int kRegs = kScores / NB;
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+      for (int h = 0; h < NS; ++h)
+        if ((have[t] >> h) & 1) {
+#pragma unroll
+          for (int r = 0; r < kRegs; ++r) out[h] = Tr::one(cols.value(t, h, r), w.w[kRegs * t + r], out[h]);
+        }
+  } else if constexpr (SBS == 32) {
+#pragma unroll
+    for (int h = 0; h < NS; ++h)
+      if ((have[0] >> h) & 1) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m) Tr::rows(out[h], cols.frag(0, m, h), w.w[m]);
+      }
+  } else {  // one product of two blocks: registers 0 and 1 of either operand the first, 2 and 3 the second
+#pragma unroll
+    for (int h = 0; h < NS; ++h) {
+      const bool on0 = (have[0] >> h) & 1, on1 = (have[NB - 1] >> h) & 1;
+      if (!on0 && !on1) continue;
+      const u32x4 f = cols.frag(0, 0, h), v = w.w[0];
+      Tr::rows(out[h], u32x4{on0 ? f[0] : 0u, on0 ? f[1] : 0u, on1 ? f[2] : 0u, on1 ? f[3] : 0u},
+               u32x4{on0 ? v[0] : 0u, on0 ? v[1] : 0u, on1 ? v[2] : 0u, on1 ? v[3] : 0u});
+    }
   }
 }
 
@@ -390,23 +446,30 @@ __device__ static inline float row_sum(float v) {
 //
 // The list is read 64 entries at a time, one per lane: the partner block, the packed indices of its first slices (of K
 // and V, or of Q and dO), its mask and bias block.  Entries the causal predicate rules out as a whole are left out of
-// `live`; `special` marks those whose scores need more than the scale; `apart` says that some block's slices are
-// missing or do not lie one behind the other.
-template <int ES, int SBS, int NS, int NB, bool kOwnIsQuery>
+// `live`; `special` marks those whose scores need more than the scale.
+//
+// kSome: head slices may be missing on either side, or q / k and v / o have different numbers of them (NS is the larger
+// one); only slices that are there are copied, and only those that both blocks of a pair have are multiplied.  `apart` marks
+// entries of whose slices some are missing or do not lie one behind the other.  The two are kernels of their own: with
+// both kinds of products in one loop the compiler needs 5 to 30 registers more, which costs a wave per SIMD or spills.
+// 16 x 2048 queries, a quarter of the blocks, head dimension 64, 9 of 10 slices there, forward / forward and backward: bf16,
+// sbs 16: 45 / 165 us (61 / 189 with every block of a window of 64 gathered as soon as one had a gap), fp32: 96 / 352
+// (131 / 453); full layouts 27 / 164 and 67 / 256.
+template <int ES, int SBS, int NS, int NB, bool kOwnIsQuery, bool kSome>
 struct Walk {
   using T = Tile<ES, SBS, NS, NB>;
   int64_t b, own;          // batch entry, own block
   int first, step;         // the wave's entries of the list: first, first + step, ...
   int end, base, seq_len;  // their number, the first one of the window; valid length of a causal sequence
   int other, first_a, first_b, mask, bias;  // of this lane's entry
-  uint64_t live, special;
-  bool apart;
+  uint64_t live, special, apart;
 
   // a step: how many entries it takes and their places in the window, and, if special, their facts (the window may be
   // another one by the time the scores are formed)
   struct Step {
     int count, slot[NB], other[NB], mask[NB], bias[NB];
-    bool special, apart;
+    bool special;
+    uint32_t have[NB];  // kSome: slices of each block that are there, bits 0 .. 7 of the first tensor, 8 .. 15 of the second; set by copy()
   };
 
   // part of parts: this wave walks every parts-th entry of the list.  The sums of the parts then have about the same size: with
@@ -428,8 +491,15 @@ struct Walk {
     base = -64;
     other = first_a = first_b = 0;
     mask = bias = -1;
-    live = special = 0;
-    apart = false;
+    live = special = apart = 0;
+  }
+
+  // the first of n packed indices; far if they are not one behind the other or do not all exist
+  __device__ static inline int in_a_row(const int64_t *pidx, int n, int64_t n_blocks, bool &far) {
+    const int64_t first = n > 0 ? pidx[0] : 0;
+    far = far || first < 0 || first + n > n_blocks;
+    for (int h = 1; h < n; ++h) far = far || pidx[h] != first + h;
+    return (int)first;
   }
 
   __device__ inline void refill(int lane) {
@@ -440,19 +510,21 @@ struct Walk {
     const bool causal = p->causal_lengths != nullptr;
     in = in && !(causal && ((kOwnIsQuery ? other > (int)own : other < (int)own) || other * SBS >= seq_len));
     const int64_t place = b * (kOwnIsQuery ? p->nk : p->nq) + other;
-    bool far = p->nh != NS || p->nhv != NS;
-    if (in && !far) {
-      const int64_t *pa = (kOwnIsQuery ? p->pidx_k : p->pidx_q) + place * NS;
-      const int64_t *pb = (kOwnIsQuery ? p->pidx_v : p->pidx_o) + place * NS;
-      const int64_t a0 = pa[0], b0 = pb[0];
-      far = a0 < 0 || b0 < 0 || a0 + NS > (kOwnIsQuery ? p->n_k_blocks : p->n_q_blocks) ||
-            b0 + NS > (kOwnIsQuery ? p->n_v_blocks : p->n_o_blocks);
-#pragma unroll
-      for (int h = 1; h < NS; ++h) far = far || pa[h] != a0 + h || pb[h] != b0 + h;
+    const int64_t *pa = kOwnIsQuery ? p->pidx_k : p->pidx_q, *pb = kOwnIsQuery ? p->pidx_v : p->pidx_o;
+    const int64_t end_a = kOwnIsQuery ? p->n_k_blocks : p->n_q_blocks, end_b = kOwnIsQuery ? p->n_v_blocks : p->n_o_blocks;
+    if constexpr (kSome) {
+      bool far = false;
+      if (in) {
+        first_a = in_a_row(pa + place * p->nh, (int)p->nh, end_a, far);
+        first_b = in_a_row(pb + place * p->nhv, (int)p->nhv, end_b, far);
+      }
+      apart = __ballot(in && far);
+    } else if (in) {  // every slice of every partner block is there: the others follow the first
+      const int64_t a0 = pa[place * NS], b0 = pb[place * NS];
       first_a = (int)a0;
       first_b = (int)b0;
+      in = a0 >= 0 && b0 >= 0 && a0 + NS <= end_a && b0 + NS <= end_b;  // a wrong index must not turn into a wild read
     }
-    apart = __any(in && far);
     bool extra = causal && (other == (int)own || ((int)own + 1) * SBS > seq_len || (other + 1) * SBS > seq_len);
     const int64_t pair = kOwnIsQuery ? (b * p->nq + own) * p->nk + other : (b * p->nq + other) * p->nk + own;
     if (p->mask) {
@@ -477,11 +549,11 @@ struct Walk {
     for (int t = 0; t < NB; ++t) {
       const uint64_t lowest = live & -live;
       s.slot[t] = lowest ? __builtin_ctzll(lowest) : 0;
+      if constexpr (kSome) s.have[t] = 0;
       s.count += lowest ? 1 : 0;
       live ^= lowest;
       taken |= lowest;
     }
-    s.apart = apart;
     s.special = (taken & special) != 0 || (NB > 1 && s.count < NB);
     if (s.special) {
 #pragma unroll
@@ -494,28 +566,74 @@ struct Walk {
   }
 
   // Requests the step's blocks of the first (K or Q) or second (V or dO) tensor; returns whether exactly T::kCopies
-  // asynchronous copies are on their way.  To be called before the next take().  Blocks that are not there (the last
-  // step of a list) become zeros.
+  // asynchronous copies are on their way.  To be called before the next take().
   template <bool kSecond>
-  __device__ inline bool copy(const Step &s, const char *tensor, char *dst, uint32_t offset, int lane) const {
-    if (!s.apart) {
-#pragma unroll
-      for (int t = 0; t < NB; ++t)
-        if (NB == 1 || t < s.count)
-          T::copy_block(tensor, __builtin_amdgcn_readlane(kSecond ? first_b : first_a, s.slot[t]), dst + t * T::kBlock, offset, lane);
-      if (NB == 1 || s.count == NB) return true;
+  __device__ inline bool copy(Step &s, const char *tensor, char *dst, uint32_t offset, int lane) const {
+    if constexpr (kSome) {
+      copy_some<kSecond>(s, tensor, dst, offset, lane);
+      return false;
     }
-    const late_args_t p = late_args();
 #pragma unroll
     for (int t = 0; t < NB; ++t) {
-      if (!s.apart && t < s.count) continue;
-      const int n = t < s.count ? (int)(kSecond ? p->nhv : p->nh) : 0;
-      const int64_t place = b * (kOwnIsQuery ? p->nk : p->nq) + __builtin_amdgcn_readlane(other, s.slot[t]);
-      const int64_t *pidx = kSecond ? (kOwnIsQuery ? p->pidx_v : p->pidx_o) : (kOwnIsQuery ? p->pidx_k : p->pidx_q);
-      const int64_t count = kSecond ? (kOwnIsQuery ? p->n_v_blocks : p->n_o_blocks) : (kOwnIsQuery ? p->n_k_blocks : p->n_q_blocks);
-      T::gather_block(tensor, pidx + place * n, n, count, dst + t * T::kBlock, offset, lane);
+      char *const to = dst + t * T::kBlock;
+      if (NB == 1 || t < s.count)
+        T::copy_block(tensor, __builtin_amdgcn_readlane(kSecond ? first_b : first_a, s.slot[t]), to, offset, lane);
+      else T::clear_block(to, lane);  // the last step of a list
     }
-    return false;
+    return NB == 1 || s.count == NB;
+  }
+  template <bool kSecond>
+  __device__ inline void copy_some(Step &s, const char *tensor, char *dst, uint32_t offset, int lane) const {
+    const late_args_t p = late_args();
+    const int n = kSecond ? (int)p->nhv : (int)p->nh;
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      uint32_t on = 0;
+      if (t < s.count) {
+        int mine = __builtin_amdgcn_readlane(kSecond ? first_b : first_a, s.slot[t]) + lane;  // lane h: packed index of slice h
+        on = (1u << n) - 1;
+        if ((apart >> s.slot[t]) & 1) {
+          const int64_t place = b * (kOwnIsQuery ? p->nk : p->nq) + __builtin_amdgcn_readlane(other, s.slot[t]);
+          const int64_t *pidx = kSecond ? (kOwnIsQuery ? p->pidx_v : p->pidx_o) : (kOwnIsQuery ? p->pidx_k : p->pidx_q);
+          const int64_t count = kSecond ? (kOwnIsQuery ? p->n_v_blocks : p->n_o_blocks) : (kOwnIsQuery ? p->n_k_blocks : p->n_q_blocks);
+          const int64_t at = lane < n ? pidx[place * n + lane] : -1;
+          on = (uint32_t)__ballot(at >= 0 && at < count);
+          mine = (int)at;
+        }
+        for (uint32_t left = on; left != 0; left &= left - 1) {
+          const int h = __builtin_ctz(left);
+          T::copy_piece(tensor, __builtin_amdgcn_readlane(mine, h), dst + t * T::kBlock + h * T::kPiece, offset, lane);
+        }
+      }
+      if constexpr (kSecond) s.have[t] = (s.have[t] & 0xffu) | on << 8;
+      else s.have[t] = (s.have[t] & 0xff00u) | on;
+    }
+  }
+
+  // acc = rows of the step's blocks of the first (second) tensor x own rows, and out += their columns^T x weights
+  template <typename Tr, bool kSecond, typename Acc>
+  __device__ static inline void multiply_rows(Acc (&acc)[NB], const Step &s, const typename T::RowReader &rows,
+                                              const OwnRows<ES, SBS, NS> &own, int lane) {
+    if constexpr (kSome) {
+      uint32_t have[NB];
+#pragma unroll
+      for (int t = 0; t < NB; ++t) have[t] = (kSecond ? s.have[t] >> 8 : s.have[t]) & own.there;
+      product_some_rows<Tr, SBS, NS, NB>(acc, rows, own, have, lane);
+    } else {
+      product_rows<Tr, SBS, NS, NB>(acc, rows, own);
+    }
+  }
+  template <typename Tr, bool kSecond, int kScores, typename Acc>
+  __device__ static inline void multiply_cols(Acc (&out)[NS], const Step &s, const typename T::ColReader &cols,
+                                              const Weights<Tr, kScores> &w) {
+    if constexpr (kSome) {
+      uint32_t have[NB];
+#pragma unroll
+      for (int t = 0; t < NB; ++t) have[t] = kSecond ? s.have[t] >> 8 : s.have[t];
+      product_some_cols<Tr, SBS, NS, NB>(out, cols, w, have);
+    } else {
+      product_cols<Tr, SBS, NS, NB>(out, cols, w);
+    }
   }
 
   // Bias, mask, causal predicate and missing blocks of a special step, in this order (blksprs/ops/flash_attention.py
@@ -596,6 +714,14 @@ inline bool small_applies(const bsa_attn_args &a) {
   if ((starts & 15) != 0 || (reinterpret_cast<uintptr_t>(a.mask) & 3) != 0) return false;
   const int64_t slices = a.nh > a.nhv ? a.nh : a.nhv;
   return slices >= 1 && slices <= 128 / a.sbs;
+}
+
+// Whether all blocks of all rows have all their head slices, as many of q / k as of v / o: the block counts say so.  Of the output
+// only the backward kernels read, and query blocks that attend to nothing may go without.
+inline bool all_slices(const bsa_attn_args &a, bool backward) {
+  if (a.nh != a.nhv || a.n_q_blocks != a.B * a.nq * a.nh || a.n_k_blocks != a.B * a.nk * a.nh || a.n_v_blocks != a.B * a.nk * a.nhv)
+    return false;
+  return !backward || a.n_o_blocks == a.B * a.nq * a.nhv || a.o_rows_whole != 0;
 }
 
 // Waves that share one row of a launch of `rows` rows, each walking every second or fourth entry of its list.  A launch lasts

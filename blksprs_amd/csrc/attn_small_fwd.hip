@@ -52,11 +52,11 @@ struct FwdShape {
 };
 
 // split: 1, 2 or 4 waves share one query block, each walking every split-th entry of its key list
-template <typename Tr, int SBS, int NS>
+template <typename Tr, int SBS, int NS, bool kSome>
 __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWaves)) void attn_small_fwd_kernel(bsa_attn_args a, int split) {
   using Shape = FwdShape<Tr::kElem, SBS, NS>;
   using T = typename Shape::T;
-  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true>;
+  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true, kSome>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs, kPiece = T::kPiece;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWav
     if (counted) wait_vmem<T::kCopies>();
     else wait_vmem<0>();
     acc_t sacc[NB];
-    product_rows<Tr, SBS, NS, NB>(sacc, k_rows, qf);
+    W::template multiply_rows<Tr, false>(sacc, now, k_rows, qf, lane);
 
     // ---- K of the next step
     wait_lds();
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWav
     // ---- O^T += V^T P^T.  In flight at most: V of this step, K of the next.
     if (counted) wait_vmem<T::kCopies>();
     else wait_vmem<0>();
-    product_cols<Tr, SBS, NS, NB>(oacc, v_cols, pf);
+    W::template multiply_cols<Tr, true, kScores>(oacc, now, v_cols, pf);
     wait_lds();
     counted = false;
     if (next.count) counted = walk.template copy<true>(next, tensor_v, lds_v, source, lane);
@@ -211,8 +211,8 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWav
   if (kq == 0) p->lse[row * SBS + qi] = (l_i != 0.f) ? m_i + log2f(l_i) : -INFINITY;
 }
 
-template <typename Tr, int SBS, int NS>
-int launch(const bsa_attn_args &a, hipStream_t s) {
+template <typename Tr, int SBS, int NS, bool kSome>
+int launch_kind(const bsa_attn_args &a, hipStream_t s) {
   using Shape = FwdShape<Tr::kElem, SBS, NS>;
   const int64_t rows = a.B * a.nq;
   const int split = waves_per_row<Tr>(rows);
@@ -220,11 +220,16 @@ int launch(const bsa_attn_args &a, hipStream_t s) {
   static_assert(lds <= 160 * 1024, "LDS");
   if (lds > 64 * 1024) {
     static const hipError_t raised = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(&attn_small_fwd_kernel<Tr, SBS, NS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        reinterpret_cast<const void *>(&attn_small_fwd_kernel<Tr, SBS, NS, kSome>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     BSA_HIP(raised);
   }
-  attn_small_fwd_kernel<Tr, SBS, NS><<<row_groups(a.B, a.nq, kWaves, split), 64 * kWaves, lds, s>>>(a, split);
+  attn_small_fwd_kernel<Tr, SBS, NS, kSome><<<row_groups(a.B, a.nq, kWaves, split), 64 * kWaves, lds, s>>>(a, split);
   return check_launch("attn_small_fwd_kernel");
+}
+
+template <typename Tr, int SBS, int NS>
+int launch(const bsa_attn_args &a, hipStream_t s) {
+  return all_slices(a, false) ? launch_kind<Tr, SBS, NS, false>(a, s) : launch_kind<Tr, SBS, NS, true>(a, s);
 }
 
 template <typename Tr>

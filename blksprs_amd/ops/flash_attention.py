@@ -409,7 +409,7 @@ def _mask_facts(layout_cache: dict, attention_layout: Tensor, mask: Tensor | Non
 class _Meta:
     """Everything the kernels need besides the differentiable tensors."""
 
-    __slots__ = ("tables", "dims", "sbs", "scale", "has_bias", "facts")
+    __slots__ = ("tables", "dims", "sbs", "scale", "has_bias", "facts", "o_rows_whole")
 
 
 def _fill_args(meta: "_Meta", q, k, v, bias, mask, causal_lengths) -> _capi.AttnArgs:
@@ -448,6 +448,7 @@ def _fill_args(meta: "_Meta", q, k, v, bias, mask, causal_lengths) -> _capi.Attn
     a.sbs = meta.sbs
     a.dtype = _capi.DTYPE_CODES[q.dtype]
     a.scale = meta.scale
+    a.o_rows_whole = meta.o_rows_whole
     return a
 
 
@@ -688,6 +689,8 @@ def flash_attention(q: BlksprsTensor, sparsity_layout_q: Tensor,
     meta.sbs = sparsity_block_size
     meta.scale = scale
     meta.has_bias = has_bias
+    # the default output layout: rows of a full V layout are there as a whole where a query block has a key block
+    meta.o_rows_whole = 1 if sparsity_layout_o is None else 0
     meta.facts = _mask_facts(layout_cache, attention_layout, attention_mask, mask_bytes, lengths, meta.dims,
                              sparsity_block_size)
 

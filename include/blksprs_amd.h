@@ -383,7 +383,8 @@ int bsa_layout_from_dense(const void *dense, uint8_t *layout, int64_t B, int64_t
  * Arguments of the block-sparse flash-attention kernels.  Layout shapes:
  * q/o (B, nq, nh) resp. (B, nq, nhv); k (B, nk, nh); v (B, nk, nhv); the
  * attention layout, mask and bias layouts (B, nq, nk).  pidx_* are int64
- * reverse indices of those layouts (-1 = inactive); NULL mask/bias = absent;
+ * reverse indices of those layouts (-1 = inactive, active blocks numbered in
+ * row-major order); NULL mask/bias = absent;
  * NULL causal_lengths = no native causal predicate.  lse and delta are fp32
  * (B, nq, sbs); lse is in the log2 domain.
  */
@@ -414,6 +415,10 @@ typedef struct bsa_attn_args {
    * of a pair.  No counterpart in the reference. */
   const int32_t *group_offsets, *group_records;
   int32_t group_size;
+  /* Backward only.  Non-zero: a query block has all of its nhv output slices, or none, and none only if it has no key
+   * block (as in the product of the attention layout and a full layout of v).  0: not known.  The kernels for blocks of 16
+   * and 32 then leave output slices that are missing out of their products one by one. */
+  int32_t o_rows_whole;
   /* Backward only.  Scratch of bsa_attn_bwd_scratch_bytes(...) bytes in which bsa_attn_bwd first writes, per query
    * block and per key block, one record for every pair that some score survives (a pair whose mask block masks
    * everything, or that the causal predicate rules out as a whole, adds nothing to any gradient and is then
