@@ -388,19 +388,20 @@ int launch_kind(const bsa_attn_args &a, hipStream_t s) {
     return rc ? rc : raise_lds(&attn_small_dkv_kernel<Tr, SBS, NS, kSome>, kv_lds);
   }();
   if (raised) return raised;
+  const int q_split = waves_per_row<Tr>(a.B * a.nq, a.nk, Shape::NB), kv_split = waves_per_row<Tr>(a.B * a.nk, a.nq, Shape::NB);
+  const int64_t q_groups = row_groups(a.B, a.nq, kWaves, q_split), kv_groups = row_groups(a.B, a.nk, kWaves, kv_split);
+  if (!fits_launch(q_groups, kWaves) || !fits_launch(kv_groups, kWaves)) return 1;
   if (a.dbias && a.n_bias_blocks > 0) {
     const int64_t n = a.n_bias_blocks * SBS * SBS / 4, blocks = cdiv(n, (int64_t)256);
     small_zero_kernel<<<(unsigned)(blocks < 65536 ? blocks : 65536), 256, 0, s>>>(reinterpret_cast<f32x4 *>(a.dbias), n);
     if (int rc = check_launch("small_zero_kernel")) return rc;
   }
-  if (const int64_t rows = a.B * a.nq) {
-    const int split = waves_per_row<Tr>(rows);
-    attn_small_dq_kernel<Tr, SBS, NS, kSome><<<row_groups(a.B, a.nq, kWaves, split), 64 * kWaves, q_lds, s>>>(a, split);
+  if (a.B * a.nq) {
+    attn_small_dq_kernel<Tr, SBS, NS, kSome><<<(unsigned)q_groups, 64 * kWaves, q_lds, s>>>(a, q_split);
     if (int rc = check_launch("attn_small_dq_kernel")) return rc;
   }
-  if (const int64_t rows = a.B * a.nk) {
-    const int split = waves_per_row<Tr>(rows);
-    attn_small_dkv_kernel<Tr, SBS, NS, kSome><<<row_groups(a.B, a.nk, kWaves, split), 64 * kWaves, kv_lds, s>>>(a, split);
+  if (a.B * a.nk) {
+    attn_small_dkv_kernel<Tr, SBS, NS, kSome><<<(unsigned)kv_groups, 64 * kWaves, kv_lds, s>>>(a, kv_split);
     if (int rc = check_launch("attn_small_dkv_kernel")) return rc;
   }
   return BSA_OK;

@@ -730,20 +730,28 @@ inline bool all_slices(const bsa_attn_args &a, bool backward) {
 // each, sbs 32): 9.6 us with two waves per row, 8.1 with four; 4128 rows (sbs 16, causal, up to 65 steps): 80 / 60 / 61 us
 // with one, two, four; 6144 rows (sbs 32, 33 steps): 83 / 75 / 82.  Nothing was measured between 64 and 4128 rows, nor beyond
 // 6144.  fp32: always four, for four partial sums: with two and one, O is 14 and 38 % further from 64 bits, dK and dV of a
-// causal layout 26 and 50 % (1024 keys, sbs 16).
+// causal layout 26 and 50 % (1024 keys, sbs 16).  Never more waves than a list of all partners has steps.
 template <typename Tr>
-inline int waves_per_row(int64_t rows) { return Tr::kElem == 4 || rows <= 512 ? 4 : rows <= 8192 ? 2 : 1; }
+inline int waves_per_row(int64_t rows, int64_t partners, int blocks_per_step) {
+  const int64_t steps = cdiv(partners, (int64_t)blocks_per_step);
+  const int most = steps >= 3 ? 4 : steps == 2 ? 2 : 1;
+  const int wanted = Tr::kElem == 4 || rows <= 512 ? 4 : rows <= 8192 ? 2 : 1;
+  return wanted < most ? wanted : most;
+}
 
 // The row of a wave.  Workgroup g runs on XCD g % 8, each with its own L2.  Of B batch entries an XCD takes B / 8 whole
 // ones, whose partner blocks no other XCD reads, and every eighth row of the B % 8 that are left.  It walks the rows of all
 // its entries together, eight neighbours (whose lists overlap) of one entry, then eight of the next, in the order in which
 // a causal layout's lists get shorter (the last query blocks, the first key blocks first): a launch lasts as long as its
-// longest lists, so none may start late.  Entry by entry, the long lists of an XCD's last entry start behind the short ones
+// longest lists, and there none starts late.  Entry by entry, the long lists of an XCD's last entry start behind the short ones
 // of the others, 6144 rows (sbs 32, windows of 33 blocks, a quarter of the rows beyond the sequences): 79 / 95 us
 // (forward / dQ) against 70 / 89; 4128 rows (sbs 16, causal): 57.5 against 48.5; 8192 rows (sbs 32, causal): 172 / 212
 // against 156 / 198; two long columns among short ones in 13 entries (dK / dV, where XCDs also differed in work): 97 against
 // 67; lists of equal lengths: the same.  Rows of one entry on several XCDs where whole entries would do: 5 to 14 % slower
-// (their partner blocks pass several L2s).
+// (their partner blocks pass several L2s).  List lengths are not looked at: where the first query blocks have the longest lists
+// (global rows of a BigBird layout) these start last.
+// Entries of fewer than eight rows are taken as they are: with eight places each, most of them empty, an entry of one row
+// (64 key blocks, 4096 entries, head dimension 64, sbs 32, fp32, forward) took 3.17 ms, now 0.77; bf16 0.72, now 0.38.
 struct RowOfWave {
   int64_t b, own;
   int part;
@@ -751,20 +759,29 @@ struct RowOfWave {
   __device__ inline RowOfWave(int64_t batches, int64_t rows_per_batch, bool last_first, int wave, int waves, int split) {
     const uint32_t xcd = blockIdx.x & 7, item = (blockIdx.x >> 3) * (waves / split) + wave / split;
     part = wave % split;
-    // eight rows of every entry: 8 items for each of an XCD's own entries, one for each shared one (the last of all)
-    const uint32_t own_items = (uint32_t)batches & ~7u, items = (uint32_t)batches;
+    // up to eight rows of every entry: as many items for each of an XCD's own entries, one for each shared one (the last of all)
+    const uint32_t near = rows_per_batch < 8 ? (uint32_t)rows_per_batch : 8, entries = (uint32_t)(batches >> 3);
+    const uint32_t own_items = entries * near, items = own_items + ((uint32_t)batches & 7);
     const uint32_t eight = item / items, rest = item - eight * items;
-    b = rest < own_items ? xcd * (own_items >> 3) + (rest >> 3) : rest;
-    own = (int64_t)eight * 8 + ((rest < own_items ? rest : xcd + rest + eight) & 7);
+    if (rest < own_items) {
+      const uint32_t entry = near == 8 ? rest >> 3 : rest / near;
+      b = (int64_t)xcd * entries + entry;
+      own = (int64_t)eight * 8 + (rest - entry * near);
+    } else {
+      b = (int64_t)entries * 8 + (rest - own_items);
+      own = (int64_t)eight * 8 + ((xcd + rest + eight) & 7);
+    }
     there = own < rows_per_batch;
     if (!there) b = own = 0;
     if (last_first) own = rows_per_batch - 1 - own;
   }
 };
-inline unsigned row_groups(int64_t batches, int64_t rows_per_batch, int waves, int split) {
-  const int64_t items = cdiv(rows_per_batch, (int64_t)8) * batches;
-  return (unsigned)(cdiv(items, (int64_t)(waves / split)) * 8);
+inline int64_t row_groups(int64_t batches, int64_t rows_per_batch, int waves, int split) {
+  const int64_t items = cdiv(rows_per_batch, (int64_t)8) * ((batches >> 3) * (rows_per_batch < 8 ? rows_per_batch : 8) + (batches & 7));
+  return cdiv(items, (int64_t)(waves / split)) * 8;
 }
+// a launch has fewer than 2^32 threads; what is more goes to the kernels that give a workgroup a row
+inline bool fits_launch(int64_t groups, int waves) { return groups * waves * 64 < ((int64_t)1 << 32); }
 
 }  // namespace small
 }  // namespace bsa

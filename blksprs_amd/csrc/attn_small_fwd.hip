@@ -215,7 +215,9 @@ template <typename Tr, int SBS, int NS, bool kSome>
 int launch_kind(const bsa_attn_args &a, hipStream_t s) {
   using Shape = FwdShape<Tr::kElem, SBS, NS>;
   const int64_t rows = a.B * a.nq;
-  const int split = waves_per_row<Tr>(rows);
+  const int split = waves_per_row<Tr>(rows, a.nk, Shape::NB);
+  const int64_t groups = row_groups(a.B, a.nq, kWaves, split);
+  if (!fits_launch(groups, kWaves)) return 1;
   constexpr int lds = Shape::kLds * kWaves;
   static_assert(lds <= 160 * 1024, "LDS");
   if (lds > 64 * 1024) {
@@ -223,7 +225,7 @@ int launch_kind(const bsa_attn_args &a, hipStream_t s) {
         reinterpret_cast<const void *>(&attn_small_fwd_kernel<Tr, SBS, NS, kSome>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     BSA_HIP(raised);
   }
-  attn_small_fwd_kernel<Tr, SBS, NS, kSome><<<row_groups(a.B, a.nq, kWaves, split), 64 * kWaves, lds, s>>>(a, split);
+  attn_small_fwd_kernel<Tr, SBS, NS, kSome><<<(unsigned)groups, 64 * kWaves, lds, s>>>(a, split);
   return check_launch("attn_small_fwd_kernel");
 }
 

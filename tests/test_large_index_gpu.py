@@ -179,3 +179,22 @@ def test_bf16_matmul_and_its_gradients_across_the_limit_with_64_blocks(device):
         rows = slice(bi * n_rows, (bi + 1) * n_rows)
         want = torch.einsum("nrk,nrc->kc", x.detach()[rows].float(), go[rows].float())
         assert torch.allclose(dy[bi].float(), want, rtol=2e-2, atol=2e-2), bi
+
+
+def test_flash_attention_of_more_than_2_23_sequences_of_one_block(device):
+    """2^23 + 40 batch entries of one query and one key block of 16: a launch of the kernels for small blocks has a wave
+    per row, not eight places per batch entry (2^24 workgroups are more threads than a launch may have).  Sampled
+    entries against softmax(q k^T / 4) v in fp32, gradients of sampled entries likewise."""
+    _require_free(64)
+    sbs, b = 16, 2 ** 23 + 40
+    g = torch.Generator(device=device).manual_seed(0)
+    q, k, v = (torch.randn((b, sbs, sbs), device=device, dtype=torch.float16, generator=g).requires_grad_(True) for _ in range(3))
+    one = torch.ones((b, 1, 1), dtype=torch.bool, device=device)
+    out = bs.ops.flash_attention(q, one, k, one, v, one, one, sbs)
+    go = torch.ones_like(out)
+    dq, dk, dv = torch.autograd.grad(out, (q, k, v), go)
+    picks = torch.tensor(_samples(b) + [8, 63, 2 ** 20 + 1, 2 ** 23, b - 9], device=device)
+    qs, ks, vs = (t.detach()[picks].float().requires_grad_(True) for t in (q, k, v))
+    want = torch.softmax(qs @ ks.transpose(1, 2).contiguous() / 4, dim=-1) @ vs
+    for got, ref in zip((out.detach(), dq, dk, dv), (want.detach(), *torch.autograd.grad(want, (qs, ks, vs), torch.ones_like(want)))):
+        assert torch.allclose(got[picks].float(), ref, rtol=2e-2, atol=2e-2)
