@@ -26,7 +26,6 @@
 //
 // The two waves that share a half of the stationary block hold partial sums over the two halves of the streamed
 // blocks; they are added through LDS once, at the end.  No atomics, fixed summation order.
-#include <atomic>
 #include <type_traits>
 
 #include "attn_mfma_common.h"
@@ -1480,24 +1479,12 @@ __global__ void fill_zero_f32_kernel(float *p, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = 0.f;
 }
 
-// The kernels that ask for more than 64 KiB of LDS say so once per process and device: the attribute belongs to
-// the loaded code object of a device, so the calls are made the first time a launch runs on it.
-constexpr int kMaxDevices = 64;
 template <typename Tr, int NH, int NHV>
 int set_lds_attributes(int lds_q, int lds_walk, int lds_dq) {
-  static std::atomic<bool> done[kMaxDevices];
-  int dev = 0;
-  BSA_HIP(hipGetDevice(&dev));
-  const bool tracked = dev >= 0 && dev < kMaxDevices;
-  if (tracked && done[dev].load(std::memory_order_acquire)) return BSA_OK;
-  BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_bwd_q_kernel<Tr, NH, NHV>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_q));
-  BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_bwd_kv8_walk_kernel<Tr, NH, NHV>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_walk));
-  BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_bwd_dq_kernel<Tr, NH>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_dq));
-  if (tracked) done[dev].store(true, std::memory_order_release);
-  return BSA_OK;
+  static LdsLimit limit_q, limit_walk, limit_dq;
+  if (int rc = allow_lds(limit_q, &attn_bwd_q_kernel<Tr, NH, NHV>, lds_q)) return rc;
+  if (int rc = allow_lds(limit_walk, &attn_bwd_kv8_walk_kernel<Tr, NH, NHV>, lds_walk)) return rc;
+  return allow_lds(limit_dq, &attn_bwd_dq_kernel<Tr, NH>, lds_dq);
 }
 
 __global__ void fill_zero_u32x4_kernel(u32x4 *p, int64_t n) {

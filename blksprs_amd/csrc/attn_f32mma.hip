@@ -299,12 +299,8 @@ __global__ __launch_bounds__(F32mmaShape<SBS>::kThreads) void attn_fwd_f32mma_ke
 template <typename Tr, int SBS, int NHV>
 int launch_f32mma(const bsa_attn_args &a, hipStream_t s) {
   const size_t lds = F32mmaShape<SBS>::lds_floats(a.nh, NHV) * sizeof(float);
-  static size_t configured = 0;  // the dynamic LDS limit of this instantiation, raised on demand
-  if (lds > configured) {
-    BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_fwd_f32mma_kernel<Tr, SBS, NHV>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    configured = lds;
-  }
+  static LdsLimit limit;
+  if (int rc = allow_lds(limit, &attn_fwd_f32mma_kernel<Tr, SBS, NHV>, lds)) return rc;
   attn_fwd_f32mma_kernel<Tr, SBS, NHV><<<(unsigned)(a.B * a.nq), F32mmaShape<SBS>::kThreads, lds, s>>>(a);
   return check_launch("attn_fwd_f32mma_kernel");
 }

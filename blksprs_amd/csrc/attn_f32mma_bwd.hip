@@ -459,14 +459,9 @@ int bwd_f32mma(const bsa_attn_args &a, hipStream_t s) {
     if (int rc = check_launch("attn_f32mma_delta_kernel")) return rc;
   }
   const size_t lds = S::lds_floats(a.nh + a.nhv) * sizeof(float);
-  static size_t configured = 0;  // the dynamic LDS limit of these instantiations, raised on demand
-  if (lds > configured) {
-    BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_f32mma_dkdv_kernel<Tr, SBS>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_f32mma_dq_kernel<Tr, SBS>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    configured = lds;
-  }
+  static LdsLimit limit_dkdv, limit_dq;
+  if (int rc = allow_lds(limit_dkdv, &attn_f32mma_dkdv_kernel<Tr, SBS>, lds)) return rc;
+  if (int rc = allow_lds(limit_dq, &attn_f32mma_dq_kernel<Tr, SBS>, lds)) return rc;
   const int64_t slices = a.nh > a.nhv ? a.nh : a.nhv;
   if (krows > 0 && (slices > 0 || a.dbias)) {
     dim3 grid((unsigned)krows, (unsigned)(slices > 0 ? slices : 1));

@@ -371,23 +371,14 @@ __global__ void small_zero_kernel(f32x4 *out, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) out[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
-template <typename K>
-int raise_lds(K kernel, int bytes) {
-  if (bytes > 64 * 1024)
-    BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-  return BSA_OK;
-}
-
 template <typename Tr, int SBS, int NS, bool kSome>
 int launch_kind(const bsa_attn_args &a, hipStream_t s) {
   using Shape = BwdShape<Tr::kElem, SBS, NS>;
   constexpr int q_lds = Shape::kQLds * kWaves, kv_lds = Shape::kKvLds * kWaves;
   static_assert(q_lds <= 160 * 1024 && kv_lds <= 160 * 1024, "LDS");
-  static const int raised = [] {
-    const int rc = raise_lds(&attn_small_dq_kernel<Tr, SBS, NS, kSome>, q_lds);
-    return rc ? rc : raise_lds(&attn_small_dkv_kernel<Tr, SBS, NS, kSome>, kv_lds);
-  }();
-  if (raised) return raised;
+  static LdsLimit limit_q, limit_kv;
+  if (int rc = allow_lds(limit_q, &attn_small_dq_kernel<Tr, SBS, NS, kSome>, q_lds)) return rc;
+  if (int rc = allow_lds(limit_kv, &attn_small_dkv_kernel<Tr, SBS, NS, kSome>, kv_lds)) return rc;
   const int q_split = waves_per_row<Tr>(a.B * a.nq, a.nk, Shape::NB), kv_split = waves_per_row<Tr>(a.B * a.nk, a.nq, Shape::NB);
   const int64_t q_groups = row_groups(a.B, a.nq, kWaves, q_split), kv_groups = row_groups(a.B, a.nk, kWaves, kv_split);
   if (!fits_launch(q_groups, kWaves) || !fits_launch(kv_groups, kWaves)) return 1;

@@ -220,11 +220,8 @@ int launch_kind(const bsa_attn_args &a, hipStream_t s) {
   if (!fits_launch(groups, kWaves)) return 1;
   constexpr int lds = Shape::kLds * kWaves;
   static_assert(lds <= 160 * 1024, "LDS");
-  if (lds > 64 * 1024) {
-    static const hipError_t raised = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(&attn_small_fwd_kernel<Tr, SBS, NS, kSome>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    BSA_HIP(raised);
-  }
+  static LdsLimit limit;
+  if (int rc = allow_lds(limit, &attn_small_fwd_kernel<Tr, SBS, NS, kSome>, lds)) return rc;
   attn_small_fwd_kernel<Tr, SBS, NS, kSome><<<(unsigned)groups, 64 * kWaves, lds, s>>>(a, split);
   return check_launch("attn_small_fwd_kernel");
 }

@@ -8,6 +8,7 @@
 #include <cstdio>
 
 #include "../../include/blksprs_amd.h"
+#include "lds_limit.h"
 
 namespace bsa {
 
@@ -39,3 +40,18 @@ inline bool is_pow2(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
     hipError_t e_ = (call);                                                                   \
     if (e_ != hipSuccess) return ::bsa::fail(BSA_ELAUNCH, "%s: %s", #call, hipGetErrorString(e_)); \
   } while (0)
+
+namespace bsa {
+
+// Lets launches of `kernel` on the current device have `bytes` of dynamic LDS.  limit: an object of this kernel's own.
+template <typename Kernel>
+int allow_lds(LdsLimit &limit, Kernel *kernel, size_t bytes) {
+  int device = 0;
+  BSA_HIP(hipGetDevice(&device));
+  return limit.raise(device, (int)bytes, [&]() -> int {
+    BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    return BSA_OK;
+  });
+}
+
+}  // namespace bsa

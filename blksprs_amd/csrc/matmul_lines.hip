@@ -459,14 +459,9 @@ __global__ __launch_bounds__(kWaves * 64, 1) void matmul_lines_kernel(LinesArgs 
 
 template <typename Tr>
 int launch_lines(const LinesArgs &a, int64_t max_parts, int contract_rows, hipStream_t s) {
-  static bool configured = false;  // raising the dynamic LDS limit is per function, once per process
-  if (!configured) {
-    BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&matmul_lines_kernel<Tr, false>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kLinesLds));
-    BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&matmul_lines_kernel<Tr, true>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kLinesLds));
-    configured = true;
-  }
+  static bsa::LdsLimit limit_down, limit_along;
+  if (int rc = bsa::allow_lds(limit_along, &matmul_lines_kernel<Tr, false>, kLinesLds)) return rc;
+  if (int rc = bsa::allow_lds(limit_down, &matmul_lines_kernel<Tr, true>, kLinesLds)) return rc;
   const unsigned grid = (unsigned)(bsa::cdiv(max_parts, 8) * 8);
   if (contract_rows) matmul_lines_kernel<Tr, true><<<grid, kWaves * 64, kLinesLds, s>>>(a);
   else matmul_lines_kernel<Tr, false><<<grid, kWaves * 64, kLinesLds, s>>>(a);

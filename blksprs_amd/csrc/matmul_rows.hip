@@ -542,12 +542,8 @@ template <typename Tr>
 int launch_rows(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs,
                 const int32_t *records, int64_t n_items, int items_per_wg, int64_t nnz_o, int64_t nnz_x,
                 int64_t nnz_y, hipStream_t s) {
-  static bool configured = false;  // raising the dynamic LDS limit is per function, once per process
-  if (!configured) {
-    BSA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&matmul_rows_kernel<Tr>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kRowsLds));
-    configured = true;
-  }
+  static bsa::LdsLimit limit;
+  if (int rc = bsa::allow_lds(limit, &matmul_rows_kernel<Tr>, kRowsLds)) return rc;
   // groups of 8 * items_per_wg records, one workgroup per XCD and group
   const int64_t groups = bsa::cdiv(n_items, (int64_t)8 * items_per_wg);
   matmul_rows_kernel<Tr><<<(unsigned)(groups * 8), kWaves * 64, kRowsLds, s>>>(
