@@ -252,6 +252,19 @@ def flash_attention_build_layout_cache(attention_layout: Tensor,
 _LENGTHS_SEEN = threading.local()
 
 
+# Up to this many values all of them are read and compared on the host; beyond, the device reduces them first.
+_COMPARED_ON_HOST = 1024
+
+
+def _smallest_and_largest(values: Tensor) -> tuple[int, int]:
+    """Of an int64 tensor, (0, 0) of an empty one; one wait of the host."""
+    if values.numel() <= _COMPARED_ON_HOST:
+        on_host = values.tolist()
+        return min(on_host, default=0), max(on_host, default=0)
+    smallest, largest = torch.stack(torch.aminmax(values)).tolist()
+    return smallest, largest
+
+
 def _normalise_causal_lengths(causal_lengths: Tensor | None, n_batches: int, q_length: int, k_length: int,
                               device: torch.device) -> Tensor | None:
     if causal_lengths is None:
@@ -273,10 +286,11 @@ def _normalise_causal_lengths(causal_lengths: Tensor | None, n_batches: int, q_l
     seen = getattr(_LENGTHS_SEEN, "last", None)
     key = (causal_lengths._version, int(q_length)) if not torch.is_inference(causal_lengths) else None
     if seen is None or seen[0] is not causal_lengths or seen[1] != key or key is None:
-        on_host = causal_lengths.tolist()  # one read; two reductions on the device were four launches and two waits
-        if on_host and (min(on_host) < 0 or max(on_host) > q_length):
+        lengths = ensure_contiguous(causal_lengths.to(dtype=torch.int64))
+        smallest, largest = _smallest_and_largest(lengths)
+        if smallest < 0 or largest > q_length:
             raise ValueError(f"causal_lengths values must be between zero and {q_length}")
-        _LENGTHS_SEEN.last = (causal_lengths, key, ensure_contiguous(causal_lengths.to(dtype=torch.int64)))
+        _LENGTHS_SEEN.last = (causal_lengths, key, lengths)
     return _LENGTHS_SEEN.last[2]
 
 

@@ -1,6 +1,8 @@
 """Causal layout and mask builders (pure torch, run on the CPU): the known answers the reference's own tests
 hold (test/cases/test_causal_layout.py:12-55), and brute force against the token-level oracle."""
 
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -8,6 +10,7 @@ import torch
 from blksprs_amd.layouting import (build_causal_self_attention_layout, build_causal_self_attention_mask,
                                    build_causal_window_self_attention_layout,
                                    build_causal_window_self_attention_mask)
+from blksprs_amd.utils import validation
 from oracle import blksprs_oracle as orc
 
 
@@ -104,3 +107,27 @@ def test_layout_and_mask_against_the_token_level_oracle(lengths, window):
                     assert unrefined or not want.any()
                 else:
                     assert want.all()           # a dropped block holds no score that counts
+
+
+@pytest.mark.parametrize("dtype", [torch.int16, torch.int64])
+@pytest.mark.parametrize("n", [0, 1, 1024, 1025, 30000])
+def test_range_check_of_causal_lengths_reads_few_values_back(dtype, n, monkeypatch):
+    """Values at the ends of the range pass, one beyond either end anywhere raises, and however many sequences there are
+    at most 1024 numbers come to the host (a list of 10^6 took 13.6 ms per call)."""
+    check = sys.modules["blksprs_amd.ops.flash_attention"]._normalise_causal_lengths
+    monkeypatch.setattr(validation, "_validation_enabled", lambda: False)  # it wants tensors on a GPU
+    read = []
+    to_list = torch.Tensor.tolist
+    monkeypatch.setattr(torch.Tensor, "tolist", lambda t: (read.append(t.numel()), to_list(t))[1])
+    lengths = (torch.arange(n) % 97).to(dtype)
+    if n:
+        lengths[n // 2] = 96
+    got = check(lengths, n, 96, 96, lengths.device)
+    assert got.dtype == torch.int64 and torch.equal(got, lengths.long())
+    assert sum(read) <= 1024
+    for place in {0, n // 3, n - 1} if n else ():
+        for value in (-1, 97):
+            bad = lengths.clone()
+            bad[place] = value
+            with pytest.raises(ValueError, match="between zero and 96"):
+                check(bad, n, 96, 96, bad.device)
