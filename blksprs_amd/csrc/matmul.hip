@@ -317,17 +317,18 @@ __global__ __launch_bounds__(256, 5) void matmul_quad_kernel(const char *__restr
                                                              char *__restrict__ out,
                                                              const int32_t *__restrict__ pair_offsets,
                                                              const int32_t *__restrict__ pairs,
-                                                             const int32_t *__restrict__ block_order, int64_t n_tiles,
-                                                             int sbs, int side_log2, int64_t nnz_x, int64_t nnz_y) {
+                                                             const int32_t *__restrict__ block_order, int64_t first,
+                                                             int64_t end, int sbs, int side_log2, int64_t nnz_x,
+                                                             int64_t nnz_y) {
   constexpr int ES = Tr::kElem, KC = 128 / ES;  // k per chunk
   constexpr int kOperand = 64 * 128, kBuffer = 2 * kOperand;
   __shared__ __attribute__((aligned(1024))) char smem[2 * kBuffer];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wi = wave >> 1, wj = wave & 1;  // the wave's quadrant
-  // XCD c takes the c-th contiguous eighth of the ordered work list (workgroup g runs on XCD g % 8)
-  const int64_t item = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  if (item >= n_tiles) return;
+  // XCD c takes the c-th contiguous eighth of the launch's part of the ordered work list (workgroup g runs on XCD g % 8)
+  const int64_t item = first + (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (item >= end) return;
   const int64_t per_block = (int64_t)1 << (2 * side_log2);
   const int64_t n = block_order ? (int64_t)__builtin_amdgcn_readfirstlane(block_order[item >> (2 * side_log2)])
                                 : item >> (2 * side_log2);
@@ -647,6 +648,10 @@ __global__ __launch_bounds__(256) void matmul_small16_f32_kernel(const char *__r
   flush_until(p_last);
 }
 
+// Workgroups of 256 in one launch.  A launch has fewer than 2^32 threads; one that asks for more is not refused, the
+// workgroups beyond are missing from it.
+constexpr int64_t kMostWorkgroups = (int64_t)1 << 23;
+
 template <typename Tr>
 int launch_runs32(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs, int64_t nnz_o,
                   int64_t nnz_x, int64_t nnz_y, int trans_x, int trans_y, hipStream_t s) {
@@ -657,8 +662,11 @@ int launch_runs32(const void *x, const void *y, void *out, const int32_t *pair_o
   // runs only scatter what is in flight on an L2 (dX of the first: 545 / 764 / 875 / 927).
   int64_t run = trans_x || trans_y ? 1 : nnz_o / 12288;
   run = run < 1 ? 1 : (run > 3 ? 3 : run);
+  // a launch has fewer than 2^32 threads: longer runs where these would be more workgroups
+  const int64_t least = bsa::cdiv(nnz_o, kWaves * kMostWorkgroups);
+  run = run < least ? least : run;
+  if (run > kSmallRunMax) return bsa::fail(BSA_ELIMIT, "bsa_matmul: too many output blocks");
   const int64_t blocks = bsa::cdiv(bsa::cdiv(bsa::cdiv(nnz_o, run), (int64_t)kWaves), (int64_t)8) * 8;
-  if (blocks > 0x7fffffffLL) return bsa::fail(BSA_ELIMIT, "bsa_matmul: too many output blocks");
   const char *xc = static_cast<const char *>(x);
   const char *yc = static_cast<const char *>(y);
   char *oc = static_cast<char *>(out);
@@ -680,20 +688,22 @@ int launch_quad(const void *x, const void *y, void *out, const int32_t *pair_off
   int side_log2 = 0;
   while ((64 << side_log2) < sbs) ++side_log2;
   const int64_t n_tiles = nnz_o << (2 * side_log2);
-  const int64_t blocks = bsa::cdiv(n_tiles, 8) * 8;
-  if (blocks > 0x7fffffffLL) return bsa::fail(BSA_ELIMIT, "bsa_matmul: too many output tiles");
   const char *xc = static_cast<const char *>(x);
   const char *yc = static_cast<const char *>(y);
   char *oc = static_cast<char *>(out);
-#define BSA_MM_LAUNCH(XT, YT)                                                                                     \
-  matmul_quad_kernel<Tr, XT, YT><<<(unsigned)blocks, 256, 0, s>>>(xc, yc, oc, pair_offsets, pairs, block_order, n_tiles, \
-                                                                  sbs, side_log2, nnz_x, nnz_y)
-  if (!trans_x && !trans_y) BSA_MM_LAUNCH(false, false);
-  else if (!trans_x && trans_y) BSA_MM_LAUNCH(false, true);
-  else if (trans_x && !trans_y) BSA_MM_LAUNCH(true, false);
-  else BSA_MM_LAUNCH(true, true);
+#define BSA_MM_LAUNCH(XT, YT)                                                                                        \
+  matmul_quad_kernel<Tr, XT, YT><<<(unsigned)(bsa::cdiv(tiles, 8) * 8), 256, 0, s>>>(                                \
+      xc, yc, oc, pair_offsets, pairs, block_order, first, first + tiles, sbs, side_log2, nnz_x, nnz_y)
+  for (int64_t first = 0; first < n_tiles; first += kMostWorkgroups) {
+    const int64_t tiles = n_tiles - first < kMostWorkgroups ? n_tiles - first : kMostWorkgroups;
+    if (!trans_x && !trans_y) BSA_MM_LAUNCH(false, false);
+    else if (!trans_x && trans_y) BSA_MM_LAUNCH(false, true);
+    else if (trans_x && !trans_y) BSA_MM_LAUNCH(true, false);
+    else BSA_MM_LAUNCH(true, true);
+    if (int rc = bsa::check_launch("matmul_quad_kernel")) return rc;
+  }
 #undef BSA_MM_LAUNCH
-  return bsa::check_launch("matmul_quad_kernel");
+  return BSA_OK;
 }
 
 // Output blocks per wave of the kernels for blocks of 16: as many as leave 32768 waves, four times what the chip holds at

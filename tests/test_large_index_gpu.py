@@ -198,3 +198,22 @@ def test_flash_attention_of_more_than_2_23_sequences_of_one_block(device):
     want = torch.softmax(qs @ ks.transpose(1, 2).contiguous() / 4, dim=-1) @ vs
     for got, ref in zip((out.detach(), dq, dk, dv), (want.detach(), *torch.autograd.grad(want, (qs, ks, vs), torch.ones_like(want)))):
         assert torch.allclose(got[picks].float(), ref, rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("sbs,n_rows,n_cols", [(128, 2048, 2056), (32, 8192, 8200)])
+def test_matmul_of_more_output_than_workgroups_of_a_launch(device, sbs, n_rows, n_cols):
+    """Output blocks of 128 in bf16 with 2^24 + 2^16 tiles of 64 x 64, and 2^26 + 2^16 output blocks of 32: 2^32 threads and
+    more if every tile (every four blocks) had a workgroup in one launch, which then starts a part of them only and
+    reports nothing.  Sampled blocks against torch, among them those around the limit and around the cuts between
+    launches."""
+    _require_free(160)
+    g = torch.Generator(device=device).manual_seed(0)
+    x, y = (torch.randn((n, sbs, sbs), device=device, dtype=torch.bfloat16, generator=g) for n in (n_rows, n_cols))
+    lx, ly, lo = (torch.ones(shape, dtype=torch.bool, device=device) for shape in ((1, n_rows, 1), (1, 1, n_cols), (1, n_rows, n_cols)))
+    out = bs.ops.matmul(x, lx, y, ly, lo, sbs)
+    total = n_rows * n_cols
+    picks = torch.tensor(sorted({*_samples(total), *(n for k in range(1, 5) for n in range(k * 2 ** 20 - 3, k * 2 ** 20 + 4)),
+                                 *(n for k in (22, 25, 26) for n in range(2 ** k - 3, 2 ** k + 4) if n < total),
+                                 *range(17, total, total // 200)}), device=device)
+    want = (x[picks // n_cols].float() @ y[picks % n_cols].float())
+    assert torch.allclose(out[picks].float(), want, rtol=1e-2, atol=0.02 * sbs ** 0.5)
