@@ -139,15 +139,20 @@ struct Block32 {
 // longer than its copies) or two (16-bit) keep the loads going, and 20 waves share a compute unit.  A finished block is
 // rounded and stored in between.  The products of a block are added in list order.
 //
-// What bounds it for 16-bit operands: the operand bytes behind the L2 (4 KiB per pair of 65 kFLOP; 480 to 610 MB per launch
-// of 8 x 2976 x 4064 x 2080 at 25 %, whatever the order of the blocks), then the instructions of a pair's control; fp32:
-// the matrix cores, half busy.  Against a kernel that staged operands through registers and gave a wave one block: that
+// With a block order (the caller has one for long lists) a wave owns a single block, and the blocks in flight on an L2 lie
+// in one super-tile of the output, whose operands it then holds: bf16, 4 x 4096^3, 128 / 32 / 16 pairs per block, storage
+// order in runs 2184 / 566 / 258 us, in the order 1312 / 365 / 190.
+//
+// What bounds it for 16-bit operands: the operand bytes behind the L2 (4 KiB per pair of 65 kFLOP; in storage order nearly
+// all of them pass it, 3.0 GB for 16 x 4096^3 at 25 %), then the instructions of a pair's control; fp32: the matrix cores,
+// half busy.  Against a kernel that staged operands through registers and gave a wave one block: that
 // size, bf16, out / dX / dY: 0.096 / 0.100 / 0.107 -> 0.094 / 0.093 / 0.098 ms, 16 x 4096^3 0.553 / 0.684 / 0.591 -> 0.490 / 0.545 /
 // 0.566; fp32 0.366 / 0.324 / 0.308 -> 0.276 / 0.298 / 0.277 ms.  Two pairs in LDS for fp32 leave 10 waves: 0.316 / 0.328 / 0.323.
 template <typename Tr, bool XT, bool YT>
 __global__ __launch_bounds__(256, 5) void matmul_runs32_kernel(
     const char *__restrict__ x, const char *__restrict__ y, char *__restrict__ out, const int32_t *__restrict__ pair_offsets,
-    const int32_t *__restrict__ pairs, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int run) {
+    const int32_t *__restrict__ pairs, const int32_t *__restrict__ block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y,
+    int run) {
   using B = Block32<Tr>;
   constexpr int ES = B::ES, kPair = 2 * B::kBytes, kStores = B::kBytes / 1024, kWaves = 4;
   constexpr int kDepth = ES == 2 ? 2 : 1;  // pairs in LDS or on their way
@@ -156,9 +161,10 @@ __global__ __launch_bounds__(256, 5) void matmul_runs32_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // every XCD takes a contiguous eighth of the runs (workgroup g runs on XCD g % 8)
   const int64_t group = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const int64_t n0 = (group * kWaves + wave) * run;
+  int64_t n0 = (group * kWaves + wave) * run;
   if (n0 >= nnz_o) return;
   const int count = (int)(nnz_o - n0 < run ? nnz_o - n0 : run);
+  if (block_order) n0 = __builtin_amdgcn_readfirstlane(block_order[n0]);  // with an order, runs are single blocks
   const int off_win = pair_offsets[n0 + (lane <= count ? lane : count)];
   const int p_first = __builtin_amdgcn_readlane(off_win, 0), p_last = __builtin_amdgcn_readlane(off_win, count);
   char *const ring = smem + wave * kDepth * kPair;
@@ -653,26 +659,28 @@ __global__ __launch_bounds__(256) void matmul_small16_f32_kernel(const char *__r
 constexpr int64_t kMostWorkgroups = (int64_t)1 << 23;
 
 template <typename Tr>
-int launch_runs32(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs, int64_t nnz_o,
-                  int64_t nnz_x, int64_t nnz_y, int trans_x, int trans_y, hipStream_t s) {
+int launch_runs32(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs,
+                  const int32_t *block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int trans_x, int trans_y,
+                  hipStream_t s) {
   constexpr int kWaves = 4;
-  // The forward product's lists are short and its output dense: a run of up to three blocks spreads a wave's first loads
+  // Where a forward product's lists are short and its output dense, a run of up to three blocks spreads a wave's first loads
   // (offsets, pairs, operands: three latencies) over more pairs, as long as there are enough waves (bf16, 16 x 4096^3, run
-  // 1 / 2 / 3 / 4: 521 / 487 / 490 / 488 us; 36259 blocks of 1.2 pairs: 28.9 / 26.6 / 24.9 / 25.2).  The gradients' lists are long, and longer
-  // runs only scatter what is in flight on an L2 (dX of the first: 545 / 764 / 875 / 927).
-  int64_t run = trans_x || trans_y ? 1 : nnz_o / 12288;
+  // 1 / 2 / 3 / 4: 521 / 487 / 490 / 488 us; 36259 blocks of 1.2 pairs: 28.9 / 26.6 / 24.9 / 25.2).  The gradients' lists are
+  // long, and longer runs only scatter what is in flight on an L2 (dX of the first: 545 / 764 / 875 / 927).
+  int64_t run = trans_x || trans_y || block_order ? 1 : nnz_o / 12288;
   run = run < 1 ? 1 : (run > 3 ? 3 : run);
   // a launch has fewer than 2^32 threads: longer runs where these would be more workgroups
   const int64_t least = bsa::cdiv(nnz_o, kWaves * kMostWorkgroups);
   run = run < least ? least : run;
+  const int32_t *const order = run == 1 ? block_order : nullptr;  // longer runs lie in storage order
   if (run > kSmallRunMax) return bsa::fail(BSA_ELIMIT, "bsa_matmul: too many output blocks");
   const int64_t blocks = bsa::cdiv(bsa::cdiv(bsa::cdiv(nnz_o, run), (int64_t)kWaves), (int64_t)8) * 8;
   const char *xc = static_cast<const char *>(x);
   const char *yc = static_cast<const char *>(y);
   char *oc = static_cast<char *>(out);
 #define BSA_MM_LAUNCH(XT, YT)                                                                                        \
-  matmul_runs32_kernel<Tr, XT, YT><<<(unsigned)blocks, 64 * kWaves, 0, s>>>(xc, yc, oc, pair_offsets, pairs, nnz_o, \
-                                                                                    nnz_x, nnz_y, (int)run)
+  matmul_runs32_kernel<Tr, XT, YT><<<(unsigned)blocks, 64 * kWaves, 0, s>>>(xc, yc, oc, pair_offsets, pairs, order, \
+                                                                            nnz_o, nnz_x, nnz_y, (int)run)
   if (!trans_x && !trans_y) BSA_MM_LAUNCH(false, false);
   else if (!trans_x && trans_y) BSA_MM_LAUNCH(false, true);
   else if (trans_x && !trans_y) BSA_MM_LAUNCH(true, false);
@@ -755,7 +763,7 @@ int launch_any(const void *x, const void *y, void *out, const int32_t *pair_offs
     return bsa::check_launch("matmul_small16_f32_kernel");
   }
   if (sbs == 32)
-    return launch_runs32<Tr>(x, y, out, pair_offsets, pairs, nnz_o, nnz_x, nnz_y, trans_x, trans_y, s);
+    return launch_runs32<Tr>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, trans_x, trans_y, s);
   return launch_quad<Tr>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, sbs, trans_x, trans_y, s);
 }
 

@@ -287,12 +287,24 @@ def _publish_backward_lists(layout_cache: dict, plan: _Plan) -> None:
         finalize_layout_cache(layout_cache)
 
 
+def _follows_order(n_pairs: int, n_out: int, sbs: int) -> bool:
+    """Whether a forward product of this many block pairs takes its output blocks in the work order of ``_block_order``.
+
+    Blocks of 16 never do, blocks of 64 and more always.  Blocks of 32 from 12 pairs per output block: the order, block by
+    block, keeps operands in the L2s, storage order in runs of up to three blocks spreads what a wave waits for over more
+    pairs.  bf16, order against runs: 4 x 4096^3, 128 / 32 / 16 / 8 / 4 / 2 pairs per block 1312 / 365 / 190 / 112 / 76 / 45
+    against 2184 / 566 / 258 / 126 / 67 / 37 us; 16 x 2048^3, 64 / 16 / 8 / 4: 652 / 193 / 113 / 69 against 761 / 204 / 105 / 62;
+    16 x 4096^3, 8: 489 against 487.  fp32, 8 x 2976 x 4064 x 2080, 32 / 16 / 8 / 4: 956 / 468 / 265 / 154 against
+    1220 / 574 / 272 / 149."""
+    return sbs > 32 or (sbs == 32 and n_pairs >= 12 * n_out)
+
+
 def _forward(x: Tensor, y: Tensor, plan: _Plan, sparsity_block_size: int) -> Tensor:
     if (sparsity_block_size == 64 and x.dtype in (torch.float16, torch.bfloat16)
             and plan.row_records is not None):
         return _launch_rows(x, y, plan, sparsity_block_size)
-    return _launch(x, y, plan.pair_offsets, plan.pairs, plan.block_order, plan.n_out, sparsity_block_size,
-                   False, False)
+    order = plan.block_order if _follows_order(plan.pairs.numel() // 2, plan.n_out, sparsity_block_size) else None
+    return _launch(x, y, plan.pair_offsets, plan.pairs, order, plan.n_out, sparsity_block_size, False, False)
 
 
 class _Matmul(torch.autograd.Function):

@@ -235,6 +235,8 @@ int bsa_softmax_bwd(const float *grad_out, const float *y, float *grad_in,
  * such operands with transpose() first (blksprs/ops/matmul.py:135-143).
  * block_order (int32 [nnz_o], a permutation, or NULL for identity) is the order in
  * which output blocks are worked on; it only affects cache behaviour, never results.
+ * Block size 16 does not read it; at 32 it pays for long pair lists (12 pairs per
+ * output block and more), below which NULL lets a wave take up to three neighbours.
  */
 int bsa_matmul(const void *x, const void *y, void *out, const int32_t *pair_offsets,
                const int32_t *pairs, const int32_t *block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int sbs, int dtype,

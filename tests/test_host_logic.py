@@ -288,3 +288,26 @@ def test_line_kernel_is_chosen_within_its_limits_only():
     assert not ok(1, 513, 8, 8) and not ok(1, 8, 513, 8) and not ok(1, 8, 8, 513)
     assert ok((1 << 25) // 512 - 1, 512, 8, 8) and not ok((1 << 25) // 512, 512, 8, 8)
     assert not ok((1 << 25) // 512, 8, 8, 512)
+
+
+def test_long_lists_of_blocks_of_32_follow_the_work_order():
+    """A large product of long lists took its output blocks in storage order at block size 32, which re-read its operands
+    behind the L2s; short lists keep to runs of neighbours, blocks of 16 never read an order."""
+    import importlib
+    mm = importlib.import_module("blksprs_amd.ops.matmul")
+
+    class Plan:
+        pair_offsets, block_order, row_records, n_out = "offsets", "order", None, 100
+
+        def __init__(self, n_pairs):
+            self.pairs = torch.empty((n_pairs, 2), dtype=torch.int32)
+
+    seen = []
+    launch = mm._launch
+    mm._launch = lambda x, y, offsets, pairs, order, *rest: seen.append(order)
+    try:
+        for sbs, n_pairs in ((32, 1200), (32, 1199), (16, 12800), (64, 0), (128, 100)):
+            mm._forward(torch.empty(0), torch.empty(0), Plan(n_pairs), sbs)
+    finally:
+        mm._launch = launch
+    assert seen == ["order", None, None, "order", "order"]

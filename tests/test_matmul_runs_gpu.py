@@ -2,10 +2,14 @@
 matmul_small16_f32_kernel) where they can go wrong: output blocks without a pair in front of, between and behind others, lists
 longer than the 64 entries of a window, launches of one, two and more output blocks per wave."""
 
+import importlib
+
 import pytest
 import torch
 
 import blksprs_amd as bs
+
+mm = importlib.import_module("blksprs_amd.ops.matmul")
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +69,24 @@ def test_runs(device, dtype, sbs, B, n):
     lx, ly = torch.rand((B, n, 3), generator=g) < 0.5, torch.rand((B, 3, n), generator=g) < 0.5
     lx[0, 0, 0] = ly[0, 0, 0] = True
     _run(device, dtype, sbs, lx.to(device), ly.to(device), torch.ones((B, n, n), dtype=torch.bool, device=device), seed=n)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,R,K,C,density", [(1, 1, 12, 1, 1.0), (2, 17, 40, 33, 0.6), (1, 5, 70, 19, 1.0), (3, 16, 24, 16, 0.75)])
+def test_order_of_blocks(device, dtype, B, R, K, C, density):
+    """Products of 12 and more pairs per output block follow the work order (super-tiles that are not whole, counts that
+    are no multiple of a workgroup's four blocks); any order, or none, gives the same bits."""
+    sbs, g = 32, torch.Generator().manual_seed(R * K * C)
+    lx, ly = torch.rand((B, R, K), generator=g) < density, torch.rand((B, K, C), generator=g) < density
+    lo = torch.ones((B, R, C), dtype=torch.bool)
+    lx, ly, lo = lx.to(device), ly.to(device), lo.to(device)
+    _run(device, dtype, sbs, lx, ly, lo, seed=C)
+    cache = {}
+    gd = torch.Generator(device=device).manual_seed(C)
+    x, y = (torch.randn((int(layout.sum()), sbs, sbs), generator=gd, device=device).to(dtype) for layout in (lx, ly))
+    out = bs.ops.matmul(x, lx, y, ly, lo, sbs, layout_cache=cache)
+    plan = cache["plan"]
+    assert mm._follows_order(plan.pairs.numel() // 2, plan.n_out, sbs)
+    for order in (None, torch.randperm(plan.n_out, generator=gd, device=device).to(torch.int32)):
+        other = mm._launch(x, y, plan.pair_offsets, plan.pairs, order, plan.n_out, sbs, False, False)
+        assert torch.equal(other, out)
