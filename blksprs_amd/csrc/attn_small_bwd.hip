@@ -16,11 +16,10 @@
 //     dV^T += dO^T P, dK^T += Q^T dS columns of dO, Q from LDS
 //
 // What bounds it: the chain of a step (tiles awaited, products, exponentials, products) with two to four waves per SIMD
-// to overlap it; matrix cores 21 % busy in the second kernel.  Against the fp32 matrix-core kernels that ran these shapes
-// before (48 x 4096 queries, sbs 32, head dimension 64, fp16, 33 key blocks per query block): delta + zero fill
-// 0.071 -> 0, dK / dV 1.89 -> 0.125 ms, dQ 1.24 -> 0.096 ms (delta included); bf16, sbs 16, 32 causal sequences of 1032 to
-// 2064: dK / dV 0.067, dQ 0.065 ms; fp32, 8 x 2048 queries, sbs 32, half of the blocks, head dimension 64: dK / dV 0.238 -> 0.096,
-// dQ 0.198 -> 0.077 ms (89 and 84 TFLOP/s).
+// to overlap it.  Against the fp32 matrix-core kernels that ran these shapes before (48 x 4096 queries, sbs 32, head
+// dimension 64, fp16, 33 key blocks per query block): delta + zero fill 0.071 -> 0, dK / dV 1.89 -> 0.125 ms (530 TFLOP/s),
+// dQ 1.24 -> 0.090 ms (delta included); fp32, 8 x 2048 queries, sbs 32, half of the blocks, head dimension 64: dK / dV 0.238
+// -> 0.096, dQ 0.198 -> 0.076 ms (89 and 85 TFLOP/s).
 //
 // Scores as in the forward kernel; p = exp2(s - lse), 0 where lse = -inf; P and dS are rounded to the operand type
 // before they enter a product (blksprs/ops/flash_attention.py:1452, :1468, :1692).

@@ -724,12 +724,19 @@ inline bool all_slices(const bsa_attn_args &a, bool backward) {
   return !backward || a.n_o_blocks == a.B * a.nq * a.nhv || a.o_rows_whole != 0;
 }
 
-// Waves that share one row of a launch of `rows` rows, each walking every second or fourth entry of its list.  A launch lasts
-// as long as the serial walk of its longest lists, and the last round of a launch of few rounds is mostly empty: shorter
-// shares help until their prologue (four dependent loads) costs more than the walk.  Forward, 64 rows (8 key blocks
-// each, sbs 32): 9.6 us with two waves per row, 8.1 with four; 4128 rows (sbs 16, causal, up to 65 steps): 80 / 60 / 61 us
-// with one, two, four; 6144 rows (sbs 32, 33 steps): 83 / 75 / 82.  Nothing was measured between 64 and 4128 rows, nor beyond
-// 6144.  fp32: always four, for four partial sums: with two and one, O is 14 and 38 % further from 64 bits, dK and dV of a
+// Waves that share one row of a launch of `rows` rows, each walking every second or fourth entry of its list.  A launch
+// lasts as long as the serial walk of its longest lists, and the last round of a launch of few rounds is mostly empty:
+// shorter shares help until their prologue (four dependent loads) costs more than the walk.  bf16 forward, one / two /
+// four waves, us (sbs 32, head dimension 64; every block of a half, causal, windows of 9 blocks, BigBird):
+//     512 rows of 32 blocks:   18.3 / 12.2 / 10.1   31.2 / 18.6 / 12.4   13.1 / 9.5 / 8.6      34.8 / 20.5 / 14.5
+//    1024 rows of 32 blocks:   19.6 / 14.8 / 14.6   32.4 / 19.9 / 13.8   13.7 / 10.6 / 10.7    35.8 / 23.5 / 19.2
+//    4096 rows of 64 blocks:   66.1 / 64.1 / 69.1   67.3 / 45.8 / 51.4   26.1 / 26.8 / 35.3    96.3 / 73.6 / 72.9
+//    8192 rows of 64 blocks:    138 / 129 / 139     81.8 / 86.7 / 98.6   42.6 / 47.3 / 65.4     131 / 117 / 127
+//   16384 rows of 64 blocks:    333 / 261 / 280      152 / 166 / 195     76.5 / 89.8 / 126      233 / 249 / 251
+// Up to 512 rows four are best throughout; at 1024 they are for half of the layouts, and at head dimension 128 two are (22.9
+// against 27.7 for every block of a half).  From 8192 rows it depends on the layout, which the rule does not look at:
+// short and causal lists want one wave, long lists of about equal length two.
+// fp32: always four, for four partial sums: with two and one, O is 14 and 38 % further from 64 bits, dK and dV of a
 // causal layout 26 and 50 % (1024 keys, sbs 16).  Never more waves than a list of all partners has steps.
 template <typename Tr>
 inline int waves_per_row(int64_t rows, int64_t partners, int blocks_per_step) {

@@ -15,12 +15,12 @@
 // handed out with v_readlane.  Entries the causal predicate rules out as a whole are taken out of the list there.
 //
 // What bounds it: a wave's chain per step (copies awaited, scores, softmax, value product) and the instructions of one
-// wave at a time; matrix cores 16 % busy, 113 vector and 63 scalar instructions per step of 32 x 32 at head dimension 64.
-// Against the fp32 matrix-core kernel that ran these shapes before: 48 x 4096 queries, sbs 32, head dimension 64, fp16,
-// 33 key blocks per query block: 0.65 -> 0.070 ms (475 TFLOP/s); 32 prompts of 1032 to 2064 tokens, sbs 16, bf16, causal:
-// 0.54 -> 0.049 ms.  fp32, where the products take eight times as long and hide the rest: 8 x 2048 queries, half of the
-// blocks, head dimension 64: 0.089 -> 0.054 ms (80 TFLOP/s, half of the fp32 matrix-core peak; 512 lists of 32 +- 4 blocks
-// cut in four fill the chip once, so the launch waits for the longest).
+// wave at a time.  Against the fp32 matrix-core kernel that ran these shapes before: 48 x 4096 queries, sbs 32, head
+// dimension 64, fp16, 33 key blocks per query block: 0.65 -> 0.072 ms (460 TFLOP/s, 18 % of the matrix cores' peak); 32
+// prompts of 1032 to 2064 tokens, sbs 16, bf16, causal: 0.54 -> 0.044 ms.  fp32, where the products take eight times as
+// long and hide the rest: 8 x 2048 queries, half of the blocks, head dimension 64: 0.089 -> 0.054 ms (80 TFLOP/s, half
+// of the fp32 matrix-core peak; 512 lists of 32 +- 4 blocks cut in four fill the chip once, so the launch waits for the
+// longest).
 //
 // Score pipeline (log2 domain), in the reference's order (blksprs/ops/flash_attention.py:1058-1224): scale * q k^T,
 // + bias, native causal predicate, explicit mask; probabilities are rounded to the operand type before they multiply

@@ -90,10 +90,10 @@ __global__ __launch_bounds__(kScanThreads) void scan_tiles_kernel(const int32_t 
 //   kFromLayout: it counts the layout bytes in front of its tile, 16 at a time; at most kMaxRecounted of them, from a
 //   16-byte aligned layout.
 // In the last two the workgroup of the last tile writes the totals.  65536 entries: one launch of 5.1 us instead of 4.7 +
-// 3.9 + 4.5 us and the two gaps between them; a conversion to sparse and back of 16 x 4096 x 4096 (two scans): 293 -> 287 us; a
-//   first attention call on a new layout (eight scans): 382 -> 325 us.
-// Each limit is where the reads repeated by all workgroups, half of the tiles each on average, reach 4 to 8 MB in
-// all, which is still less than the launch it saves: 2^17 bytes in 64 tiles, or 1024 counts in 1024 tiles.
+// 3.9 + 4.5 us and the two gaps between them; a conversion to sparse and back of 16 x 4096 x 4096 (two scans): 293 -> 287
+// us; a first attention call on a new layout (eight scans): 382 -> 325 us.
+// The reads repeated by all workgroups, half of the tiles each on average, are 4 MiB in all at the limit of the layout (64
+// workgroups x 32 tiles of 2 KiB) and 2 MiB at the limit of the counts (1024 workgroups x 512 counts of 4 bytes).
 enum Prefix { kFromOffsets, kFromCounts, kFromLayout };
 constexpr int64_t kMaxCountedTiles = 1024;
 constexpr int64_t kMaxRecounted = (int64_t)1 << 17;

@@ -1,10 +1,10 @@
-// Work orders of the matmul kernels, built on the device (integer only): the order in which the tile kernel takes
-// the output blocks, and the table by which the row kernel hands parts of block rows to workgroups.  Both are a
-// stable sort of small integers by a 64-bit key that a kernel computes from tables already on the device, so no
-// count is read back and the host never waits.  The sort is rocPRIM's radix sort (through hipCUB); its scratch
-// comes from the caller like every other scratch of this library.  Neither order has a counterpart in the
-// reference, whose kernels take output blocks in launch order (blksprs/ops/matmul.py:88-128); they only change
-// which blocks are in flight together, never a result.
+// Work orders of the matmul kernels, built on the device (integer only): the order in which the kernels of
+// bsa_matmul for blocks of 32 and more take the output blocks, and the table by which the row kernel hands
+// parts of block rows to workgroups.  Both are a stable sort of small integers by a 64-bit key that a kernel
+// computes from tables already on the device, so no count is read back and the host never waits.  The sort is
+// rocPRIM's radix sort (through hipCUB); its scratch comes from the caller like every other scratch of this
+// library.  Neither order has a counterpart in the reference, whose kernels take output blocks in launch order
+// (blksprs/ops/matmul.py:88-128); they only change which blocks are in flight together, never a result.
 #include "common.h"
 
 #include <hipcub/device/device_radix_sort.hpp>
@@ -62,7 +62,7 @@ int sort_pairs(const SortScratch &s, int64_t n, hipStream_t stream) {
   return BSA_OK;
 }
 
-// ---- order of the output blocks for the tile kernel: super-tiles of tile x tile blocks of the block grid, the
+// ---- order of the output blocks for bsa_matmul: super-tiles of tile x tile blocks of the block grid, the
 // super-tiles of a batch entry row by row, the blocks of a super-tile row by row
 __global__ __launch_bounds__(kThreads) void block_order_keys_kernel(const int64_t *__restrict__ coords, int64_t n,
                                                                     int64_t n_i, int64_t n_j, int tile,

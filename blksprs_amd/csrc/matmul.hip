@@ -18,14 +18,14 @@
 
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-// native vector (not HIP's uint4 struct): arrays of it are always promoted to registers
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-typedef short i16x4 __attribute__((ext_vector_type(4)));
+// native vectors (not HIP's uint4 struct): arrays of them are always promoted to registers
+using bsa::mfma::bf16x8;
+using bsa::mfma::f16x8;
+using bsa::mfma::f32x16;
+using bsa::mfma::f32x4;
+using bsa::mfma::i16x4;
+using bsa::mfma::u32x2;
+using bsa::mfma::u32x4;
 
 struct Bf16Traits {
   static constexpr int kElem = 2;
@@ -143,11 +143,12 @@ struct Block32 {
 // in one super-tile of the output, whose operands it then holds: bf16, 4 x 4096^3, 128 / 32 / 16 pairs per block, storage
 // order in runs 2184 / 566 / 258 us, in the order 1312 / 365 / 190.
 //
-// What bounds it for 16-bit operands: the operand bytes behind the L2 (4 KiB per pair of 65 kFLOP; in storage order nearly
-// all of them pass it, 3.0 GB for 16 x 4096^3 at 25 %), then the instructions of a pair's control; fp32: the matrix cores,
-// half busy.  Against a kernel that staged operands through registers and gave a wave one block: that
-// size, bf16, out / dX / dY: 0.096 / 0.100 / 0.107 -> 0.094 / 0.093 / 0.098 ms, 16 x 4096^3 0.553 / 0.684 / 0.591 -> 0.490 / 0.545 /
-// 0.566; fp32 0.366 / 0.324 / 0.308 -> 0.276 / 0.298 / 0.277 ms.  Two pairs in LDS for fp32 leave 10 waves: 0.316 / 0.328 / 0.323.
+// What bounds it for 16-bit operands: the operand bytes behind the L2 (4 KiB per pair of 65 kFLOP; of the 8.6 GB of 16
+// x 4096^3 at 25 % 3.0 pass it in storage order), then the instructions of a pair's control; fp32: the matrix cores,
+// half busy.  Against a kernel that staged operands through registers and gave a wave one block: that size, bf16, out /
+// dX / dY: 0.096 / 0.100 / 0.107 -> 0.094 / 0.093 / 0.098 ms, 16 x 4096^3 0.553 / 0.684 / 0.591 -> 0.490 / 0.545 /
+// 0.566; fp32 0.366 / 0.324 / 0.308 -> 0.276 / 0.298 / 0.277 ms.  Two pairs in LDS for fp32 leave 10 waves: 0.316 /
+// 0.328 / 0.323.
 template <typename Tr, bool XT, bool YT>
 __global__ __launch_bounds__(256, 5) void matmul_runs32_kernel(
     const char *__restrict__ x, const char *__restrict__ y, char *__restrict__ out, const int32_t *__restrict__ pair_offsets,

@@ -159,7 +159,8 @@ def to_dense(x: BlksprsTensor, sparsity_layout: Tensor,
 
     if layout_cache is None:
         # a reverse index of this call alone is read on this call's stream only, so the host does not wait for the
-        # scan (one wait less: 328 -> 291 us for layout + to_sparse + to_dense of a 537 MB tensor); in a cache it may be read on another stream next, and the scan is waited for
+        # scan (one wait less: 328 -> 291 us for layout + to_sparse + to_dense of a 537 MB tensor); in a cache it may be
+        # read on another stream next, and the scan is waited for
         packed_indices = pack_layouts((sparsity_layout, 0), counts=False)[0].packed
     else:
         packed_indices = to_dense_build_layout_cache(layout_cache, sparsity_layout)["packed_indices"]

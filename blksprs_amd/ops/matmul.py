@@ -253,7 +253,7 @@ class _Plan:
                                           cache["n_sparse_blocks_y"])
         self.packed_x, self.packed_y, self.packed_o = (cache["packed_indices_x"], cache["packed_indices_y"],
                                                        cache["packed_indices_o"])
-        self.grad_lists = None  # contraction lists of the two backward products (tile kernel)
+        self.grad_lists = None  # contraction lists of the two backward products (bsa_matmul)
         self.grad_lines = self.lines_error = None  # part offsets of the two backward products (line kernel)
 
 

@@ -252,7 +252,7 @@ int bsa_matmul(const void *x, const void *y, void *out, const int32_t *pair_offs
  * bsa_lut_block_order: order (int32 [n], a permutation) lists the n active blocks of a layout, given by their
  * coordinates layout_indices (int64 [n, 3]: batch, row, column, as bsa_lut_nonzero writes them), by super-tiles of
  * tile x tile blocks of the n_rows x n_cols block grid: the super-tiles of a batch entry row by row, the blocks of
- * a super-tile row by row.  It is the block_order argument of bsa_matmul.
+ * a super-tile row by row.  It is the block_order argument of bsa_matmul (block sizes of 32 and more).
  *
  * bsa_lut_row_work_table: the work_table argument of bsa_matmul_rows_records (see there for the entries' format
  * and for why the order is what it is): table_len = 8 * ceil(n_rows / 8) << parts_log2 entries; every XCD's

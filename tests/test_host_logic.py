@@ -279,7 +279,7 @@ def test_measurement_knobs_are_clamped_and_malformed_values_ignored(monkeypatch)
 def test_line_kernel_is_chosen_within_its_limits_only():
     """The backward products take the line kernel for 16-bit operands at sbs 64 when no line of either layout has
     more than 512 blocks and there are fewer than 2^25 lines (the part table holds the line in 25 bits and
-    bsa_matmul_lines_parts refuses more); everything else takes the tile kernel."""
+    bsa_matmul_lines_parts refuses more); everything else takes the kernels of bsa_matmul."""
     import importlib
     mm = importlib.import_module("blksprs_amd.ops.matmul")
     ok = lambda B, R, K, C, sbs=64, dt=torch.bfloat16: mm._lines_apply(None, ((B, R, K), (B, K, C)), sbs, dt)
