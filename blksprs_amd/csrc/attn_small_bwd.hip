@@ -34,10 +34,10 @@ using namespace small;
 
 constexpr int kWaves = 4;
 
-template <int ES, int SBS, int NS>
+template <int ES, int SBS, int NS, int kHalves>
 struct BwdShape {
   static constexpr int NB = SBS == 32 ? 1 : 2;  // partner blocks per step
-  using T = Tile<ES, SBS, NS, NB>;
+  using T = Tile<ES, SBS, NS, NB, kHalves>;
   static constexpr int kRegs = SBS == 32 ? 16 : 4;
   static constexpr int kScores = kRegs * NB;
   static constexpr int kPartial = SBS * SBS * NS * 4;
@@ -83,27 +83,28 @@ __device__ inline void add_partial(Acc (&acc)[NS], const float *other, int lane)
 }
 
 // gradient blocks of the own row, columns 2 r + 4 group .. + 3 of a row per lane
-template <typename Tr, int SBS, int NS, typename Acc>
+template <typename Tr, int SBS, int NS, int kHalves, typename Acc>
 __device__ inline void store_gradient(const Acc (&acc)[NS], float scale, void *out, const int64_t *pidx, int n_slices,
-                                      int64_t n_blocks, int me, int group) {
+                                      int64_t n_blocks, int own, int me, int group) {
   constexpr int kRegs = SBS == 32 ? 16 : 4;
 #pragma unroll
   for (int h = 0; h < NS; ++h) {
-    if (h >= n_slices) break;
-    const int64_t p = pidx[h];
+    if (h / kHalves >= n_slices) break;
+    const int64_t p = pidx[h / kHalves];
     if (p < 0 || p >= n_blocks) continue;
-    char *blk = static_cast<char *>(out) + (p * SBS * SBS + me * SBS + 4 * group) * Tr::kElem;
+    char *blk = static_cast<char *>(out) + Place<Tr::kElem, SBS, kHalves>::row(p, own, me, h) + 4 * group * Tr::kElem;
 #pragma unroll
     for (int r = 0; r < kRegs; r += 4)
       store4<Tr>(blk + 2 * r * Tr::kElem, acc[h][r] * scale, acc[h][r + 1] * scale, acc[h][r + 2] * scale, acc[h][r + 3] * scale);
   }
 }
 
-template <typename Tr, int SBS, int NS, bool kSome>
-__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWaves)) void attn_small_dq_kernel(bsa_attn_args a, int split) {
-  using Shape = BwdShape<Tr::kElem, SBS, NS>;
+// kHalves 2: blocks of 64, whose halves are the blocks of 32 spoken of here (Place)
+template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
+__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>::kQMinWaves)) void attn_small_dq_kernel(bsa_attn_args a, int split) {
+  using Shape = BwdShape<Tr::kElem, SBS, NS, kHalves>;
   using T = typename Shape::T;
-  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true, kSome>;
+  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true, kSome, kHalves>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
@@ -111,24 +112,25 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWa
   const int wave = first_lane(threadIdx.x >> 6);
   char *lds_k = small_smem + wave * Shape::kQLds, *lds_v = lds_k + T::kBytes;
 
-  const RowOfWave me(a.B, a.nq, true, wave, kWaves, split);
-  const int64_t row = me.b * a.nq + me.own;
+  const RowOfWave me(a.B, kHalves * a.nq, true, wave, kWaves, split);
+  const int64_t row = me.b * a.nq + me.own / kHalves;  // of the layout
+  const int64_t stats = (row * kHalves + me.own % kHalves) * SBS;  // of lse and delta
   const int qi = lane % SBS, kq = lane / SBS;
   W walk;
   walk.start(a, me.b, me.own, me.there, me.part, split);
 
-  OwnRows<Tr::kElem, SBS, NS> qf, gf;
-  qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, lane);
-  gf.load(a.d_o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, lane);
-  float delta = 0.f, neg_lse = -a.lse[row * SBS + qi];
+  OwnRows<Tr::kElem, SBS, NS, kHalves> qf, gf;
+  qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, (int)me.own, lane);
+  gf.load(a.d_o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, (int)me.own, lane);
+  float delta = 0.f, neg_lse = -a.lse[stats + qi];
   if (neg_lse == INFINITY) neg_lse = -INFINITY;  // a query that sees nothing: p = 0
   {
-    OwnRows<Tr::kElem, SBS, NS> of;
-    of.load(a.o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, lane);
+    OwnRows<Tr::kElem, SBS, NS, kHalves> of;
+    of.load(a.o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, (int)me.own, lane);
 #pragma unroll
     for (int f = 0; f < T::kFrags; ++f) delta = Tr::dot(of.fr[f], gf.fr[f], delta);
     delta = row_sum<SBS>(delta);
-    if (me.there && me.part == 0 && kq == 0) a.delta[row * SBS + qi] = delta;
+    if (me.there && me.part == 0 && kq == 0) a.delta[stats + qi] = delta;
   }
   acc_t dq[NS];
 #pragma unroll
@@ -184,7 +186,9 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWa
 #pragma unroll
         for (int t = 0; t < NB; ++t)
           if (now.bias[t] >= 0) {
-            float *out = p->dbias + ((int64_t)now.bias[t] * SBS + qi) * SBS + 4 * kq;
+            constexpr int kSide = kHalves * SBS;
+            float *out = p->dbias + ((int64_t)now.bias[t] * kSide + (int)me.own % kHalves * SBS + qi) * kSide +
+                         now.other[t] % kHalves * SBS + 4 * kq;
 #pragma unroll
             for (int r = 0; r < kRegs; r += 4) {
               const float *v = sv + kRegs * t + r;
@@ -209,14 +213,14 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kQMinWa
   }
   if (!me.there) return;
   const late_args_t p = late_args();
-  store_gradient<Tr, SBS, NS>(dq, p->scale, p->dq, p->pidx_q + row * p->nh, (int)p->nh, p->n_q_blocks, qi, kq);
+  store_gradient<Tr, SBS, NS, kHalves>(dq, p->scale, p->dq, p->pidx_q + row * p->nh, (int)p->nh, p->n_q_blocks, (int)me.own, qi, kq);
 }
 
-template <typename Tr, int SBS, int NS, bool kSome>
-__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinWaves)) void attn_small_dkv_kernel(bsa_attn_args a, int split) {
-  using Shape = BwdShape<Tr::kElem, SBS, NS>;
+template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
+__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>::kKvMinWaves)) void attn_small_dkv_kernel(bsa_attn_args a, int split) {
+  using Shape = BwdShape<Tr::kElem, SBS, NS, kHalves>;
   using T = typename Shape::T;
-  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, false, kSome>;
+  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, false, kSome, kHalves>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs, kBufs = Shape::kBufs;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
@@ -224,15 +228,15 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinW
   const int wave = first_lane(threadIdx.x >> 6);
   char *lds = small_smem + wave * Shape::kKvLds;  // per buffer: Q tile, dO tile, lse and delta
 
-  const RowOfWave me(a.B, a.nk, false, wave, kWaves, split);
-  const int64_t row = me.b * a.nk + me.own;
+  const RowOfWave me(a.B, kHalves * a.nk, false, wave, kWaves, split);
+  const int64_t row = me.b * a.nk + me.own / kHalves;  // of the layout
   const int kj = lane % SBS, kq = lane / SBS;  // key row; which queries of a block this lane's registers hold
   W walk;
   walk.start(a, me.b, me.own, me.there, me.part, split);
 
-  OwnRows<Tr::kElem, SBS, NS> kf, vf;
-  kf.load(a.k, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, lane);
-  vf.load(a.v, a.pidx_v + row * a.nhv, (int)a.nhv, a.n_v_blocks, lane);
+  OwnRows<Tr::kElem, SBS, NS, kHalves> kf, vf;
+  kf.load(a.k, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, (int)me.own, lane);
+  vf.load(a.v, a.pidx_v + row * a.nhv, (int)a.nhv, a.n_v_blocks, (int)me.own, lane);
   acc_t dk[NS], dv[NS];
 #pragma unroll
   for (int h = 0; h < NS; ++h)
@@ -244,7 +248,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinW
   const uint32_t source = T::source_offset(lane);
   const char *const tensor_q = static_cast<const char *>(a.q), *const tensor_g = static_cast<const char *>(a.d_o);
   // this lane's share of the statistics copy: lanes 0 .. 31 lse, 32 .. 63 delta of the step's 32 queries
-  const float *const stats = (lane < 32 ? a.lse : a.delta) + me.b * a.nq * SBS + lane % SBS;
+  const float *const stats = (lane < 32 ? a.lse : a.delta) + me.b * a.nq * (kHalves * SBS) + lane % SBS;
   const int stats_block = SBS == 16 ? (lane >> 4) & 1 : 0;
   auto copy_stats = [&](const typename W::Step &s, char *dst) {
     int other = __builtin_amdgcn_readlane(walk.other, s.slot[0]);
@@ -360,8 +364,8 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS>::kKvMinW
   }
   if (!me.there) return;
   const late_args_t p = late_args();
-  store_gradient<Tr, SBS, NS>(dk, p->scale, p->dk, p->pidx_k + row * p->nh, (int)p->nh, p->n_k_blocks, kj, kq);
-  store_gradient<Tr, SBS, NS>(dv, 1.f, p->dv, p->pidx_v + row * p->nhv, (int)p->nhv, p->n_v_blocks, kj, kq);
+  store_gradient<Tr, SBS, NS, kHalves>(dk, p->scale, p->dk, p->pidx_k + row * p->nh, (int)p->nh, p->n_k_blocks, (int)me.own, kj, kq);
+  store_gradient<Tr, SBS, NS, kHalves>(dv, 1.f, p->dv, p->pidx_v + row * p->nhv, (int)p->nhv, p->n_v_blocks, (int)me.own, kj, kq);
 }
 
 // bias blocks outside the attention layout, and pairs the causal predicate rules out, have no wave that writes them
@@ -370,28 +374,29 @@ __global__ void small_zero_kernel(f32x4 *out, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) out[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
-template <typename Tr, int SBS, int NS, bool kSome>
+template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
 int launch_kind(const bsa_attn_args &a, hipStream_t s) {
-  using Shape = BwdShape<Tr::kElem, SBS, NS>;
+  using Shape = BwdShape<Tr::kElem, SBS, NS, kHalves>;
   constexpr int q_lds = Shape::kQLds * kWaves, kv_lds = Shape::kKvLds * kWaves;
   static_assert(q_lds <= 160 * 1024 && kv_lds <= 160 * 1024, "LDS");
   static LdsLimit limit_q, limit_kv;
-  if (int rc = allow_lds(limit_q, &attn_small_dq_kernel<Tr, SBS, NS, kSome>, q_lds)) return rc;
-  if (int rc = allow_lds(limit_kv, &attn_small_dkv_kernel<Tr, SBS, NS, kSome>, kv_lds)) return rc;
-  const int q_split = waves_per_row<Tr>(a.B * a.nq, a.nk, Shape::NB), kv_split = waves_per_row<Tr>(a.B * a.nk, a.nq, Shape::NB);
-  const int64_t q_groups = row_groups(a.B, a.nq, kWaves, q_split), kv_groups = row_groups(a.B, a.nk, kWaves, kv_split);
+  if (int rc = allow_lds(limit_q, &attn_small_dq_kernel<Tr, SBS, NS, kSome, kHalves>, q_lds)) return rc;
+  if (int rc = allow_lds(limit_kv, &attn_small_dkv_kernel<Tr, SBS, NS, kSome, kHalves>, kv_lds)) return rc;
+  const int64_t q_rows = kHalves * a.nq, k_rows = kHalves * a.nk;  // of a batch entry
+  const int q_split = waves_per_row<Tr>(a.B * q_rows, k_rows, Shape::NB), kv_split = waves_per_row<Tr>(a.B * k_rows, q_rows, Shape::NB);
+  const int64_t q_groups = row_groups(a.B, q_rows, kWaves, q_split), kv_groups = row_groups(a.B, k_rows, kWaves, kv_split);
   if (!fits_launch(q_groups, kWaves) || !fits_launch(kv_groups, kWaves)) return 1;
   if (a.dbias && a.n_bias_blocks > 0) {
-    const int64_t n = a.n_bias_blocks * SBS * SBS / 4, blocks = cdiv(n, (int64_t)256);
+    const int64_t n = a.n_bias_blocks * a.sbs * a.sbs / 4, blocks = cdiv(n, (int64_t)256);
     small_zero_kernel<<<(unsigned)(blocks < 65536 ? blocks : 65536), 256, 0, s>>>(reinterpret_cast<f32x4 *>(a.dbias), n);
     if (int rc = check_launch("small_zero_kernel")) return rc;
   }
   if (a.B * a.nq) {
-    attn_small_dq_kernel<Tr, SBS, NS, kSome><<<(unsigned)q_groups, 64 * kWaves, q_lds, s>>>(a, q_split);
+    attn_small_dq_kernel<Tr, SBS, NS, kSome, kHalves><<<(unsigned)q_groups, 64 * kWaves, q_lds, s>>>(a, q_split);
     if (int rc = check_launch("attn_small_dq_kernel")) return rc;
   }
   if (a.B * a.nk) {
-    attn_small_dkv_kernel<Tr, SBS, NS, kSome><<<(unsigned)kv_groups, 64 * kWaves, kv_lds, s>>>(a, kv_split);
+    attn_small_dkv_kernel<Tr, SBS, NS, kSome, kHalves><<<(unsigned)kv_groups, 64 * kWaves, kv_lds, s>>>(a, kv_split);
     if (int rc = check_launch("attn_small_dkv_kernel")) return rc;
   }
   return BSA_OK;
@@ -399,12 +404,15 @@ int launch_kind(const bsa_attn_args &a, hipStream_t s) {
 
 template <typename Tr, int SBS, int NS>
 int launch(const bsa_attn_args &a, hipStream_t s) {
-  return all_slices(a, true) ? launch_kind<Tr, SBS, NS, false>(a, s) : launch_kind<Tr, SBS, NS, true>(a, s);
+  return all_slices(a, true) ? launch_kind<Tr, SBS, NS, false, 1>(a, s) : launch_kind<Tr, SBS, NS, true, 1>(a, s);
 }
 
 template <typename Tr>
 int dispatch(const bsa_attn_args &a, hipStream_t s) {
   const int64_t slices = a.nh > a.nhv ? a.nh : a.nhv;
+  if constexpr (Tr::kElem == 4) {
+    if (a.sbs == 64) return slices == 1 ? launch_kind<Tr, 32, 2, false, 2>(a, s) : launch_kind<Tr, 32, 4, false, 2>(a, s);
+  }
   if (a.sbs == 32) {
     switch (slices) {
       case 1: return launch<Tr, 32, 1>(a, s);
@@ -431,7 +439,7 @@ int dispatch(const bsa_attn_args &a, hipStream_t s) {
 
 // 1: not covered
 int attn_bwd_small(const bsa_attn_args &a, hipStream_t s) {
-  if (!small_applies(a)) return 1;
+  if (!small_applies(a, true)) return 1;
   return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, s) : a.dtype == BSA_F16 ? dispatch<SF16>(a, s) : dispatch<SF32>(a, s);
 }
 

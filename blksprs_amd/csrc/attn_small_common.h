@@ -117,8 +117,36 @@ __device__ static inline void copy_kib_to_lds(const char *base, uint32_t off, ch
                  : : "v"(off), "s"(base), "s"(lds_addr) : "memory");
 }
 
+// N KiB of LDS (2 or 4) from every second KiB of memory: half of the columns of blocks twice as wide.  The offset field
+// moves both addresses, the other KiB comes from the lane's offset.
+template <int N>
+__device__ static inline void copy_every_second_kib_to_lds(const char *base, uint32_t off, char *dst) {
+  const uint32_t lds_addr = (uint32_t)(uintptr_t)(lds_ptr_t)dst;
+  static_assert(N == 2 || N == 4, "KiB of a slice");
+  if constexpr (N == 2)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %3, %1 offset:1024"
+                 : : "v"(off), "s"(base), "s"(lds_addr), "v"(off + 1024) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %3, %1 offset:1024\n\t"
+                 "global_load_lds_dwordx4 %4, %1 offset:2048\n\tglobal_load_lds_dwordx4 %5, %1 offset:3072"
+                 : : "v"(off), "s"(base), "s"(lds_addr), "v"(off + 1024), "v"(off + 2048), "v"(off + 3072) : "memory");
+}
+
+// Where the blocks of the kernels lie in memory.  kHalves 1: a block is a block of the layout.  kHalves 2: a block of the
+// layout (64 x 64) is four of theirs, its head slice two of theirs: block i of a row is half i % 2 of the rows of the layout's
+// block i / 2, slice h the columns from SBS (h % 2) of the layout's slice h / 2.
+template <int ES, int SBS, int kHalves>
+struct Place {
+  static constexpr int kPitch = kHalves * SBS * ES;             // bytes from row to row
+  static constexpr int64_t kBlockBytes = (int64_t)kHalves * SBS * kPitch;  // of a slice of a block of the layout
+  // byte offset of (row r, slice h) of block `own`, whose slice h / kHalves has packed index idx
+  __device__ static inline int64_t row(int64_t idx, int own, int r, int h) {
+    return idx * kBlockBytes + (int64_t)(own % kHalves * SBS + r) * kPitch + h % kHalves * (SBS * ES);
+  }
+};
+
 // Geometry of one wave's tile: NB partner blocks of NS head slices each, slice h of block t at piece t * NS + h.
-template <int ES, int SBS, int NS, int NB>
+template <int ES, int SBS, int NS, int NB, int kHalves = 1>
 struct Tile {
   static constexpr int kPiece = SBS * SBS * ES;
   static constexpr int kRowBytes = SBS * ES;
@@ -133,12 +161,20 @@ struct Tile {
     constexpr int kChunks = kRowBytes / 16;
     const int place = lane / kChunks % SBS;  // row_place is its own inverse
     const int r = row_place<ES, SBS>(place);
-    return (uint32_t)((lane * 16 / kPiece) * kPiece + r * kRowBytes + (((lane % kChunks) ^ chunk_swizzle<ES, SBS>(r)) << 4));
+    return (uint32_t)((lane * 16 / kPiece) * kPiece + r * (kHalves * kRowBytes) + (((lane % kChunks) ^ chunk_swizzle<ES, SBS>(r)) << 4));
   }
 
-  // Requests block t of the tile, all of whose slices are there and lie one behind the other from packed index idx:
-  // kBlockCopies asynchronous copies.
+  // Requests block t of the tile, all of whose slices are there and lie one behind the other from packed index idx (kHalves
+  // times the packed index, plus the half): kBlockCopies asynchronous copies.
   __device__ static inline void copy_block(const char *tensor, int idx, char *dst, uint32_t offset, int lane) {
+    if constexpr (kHalves == 2) {
+      static_assert(SBS == 32 && NS % 2 == 0, "halves of blocks of 64");
+      const char *src = tensor + (uint64_t)(uint32_t)idx * (2 * kPiece);
+#pragma unroll
+      for (int h = 0; h < NS; ++h)
+        copy_every_second_kib_to_lds<kPiece / 1024>(src + h / 2 * (4 * kPiece) + h % 2 * kRowBytes, offset, dst + h * kPiece);
+      return;
+    }
     const char *src = tensor + (uint64_t)(uint32_t)idx * kPiece;
     constexpr int kKib = kBlock / 1024;
 #pragma unroll
@@ -251,14 +287,14 @@ struct Tile {
 
 // One block's own rows as the other operand of the score products, in registers for the whole walk (the same values
 // per lane as RowReader's fragments).
-template <int ES, int SBS, int NS>
+template <int ES, int SBS, int NS, int kHalves>
 struct OwnRows {
-  using T = Tile<ES, SBS, NS, 2>;
+  using T = Tile<ES, SBS, NS, 2, kHalves>;
   u32x4 fr[T::kFrags];
-  uint32_t there;  // bit h: the block has slice h (wave uniform)
+  uint32_t there;  // bit h: the block has slice h of the layout (wave uniform)
 
-  // pidx: packed indices of the block's slices, n_slices of them are there
-  __device__ inline void load(const void *tensor, const int64_t *pidx, int n_slices, int64_t n_blocks, int lane) {
+  // pidx: packed indices of the slices of block `own` in the layout, n_slices of them are there
+  __device__ inline void load(const void *tensor, const int64_t *pidx, int n_slices, int64_t n_blocks, int own, int lane) {
     const int r = lane % SBS, g = lane / SBS;
     const int64_t mine = lane < n_slices ? pidx[lane] : -1;
     there = (uint32_t)__ballot(mine >= 0 && mine < n_blocks);
@@ -267,27 +303,28 @@ struct OwnRows {
       int h, chunk;
       if constexpr (ES == 2 && SBS == 16) h = 2 * f + (g >> 1), chunk = g & 1;
       else h = f / T::kSliceFrags, chunk = 64 / SBS * (f % T::kSliceFrags) + g;
-      const int64_t idx = h < n_slices ? pidx[h] : -1;
+      const int64_t idx = h / kHalves < n_slices ? pidx[h / kHalves] : -1;
       fr[f] = u32x4{0u, 0u, 0u, 0u};
       if (idx >= 0 && idx < n_blocks)
-        fr[f] = *reinterpret_cast<const u32x4 *>(static_cast<const char *>(tensor) + idx * T::kPiece + r * T::kRowBytes + chunk * 16);
+        fr[f] = *reinterpret_cast<const u32x4 *>(static_cast<const char *>(tensor) + Place<ES, SBS, kHalves>::row(idx, own, r, h) +
+                                                 chunk * 16);
     }
   }
 };
 
 // Makes the compiler wait for the loads of the own rows here: left to their first use, the wait sits inside the loop and
 // is for every load in flight, each time round.
-template <int ES, int SBS, int NS>
-__device__ static inline void settle(OwnRows<ES, SBS, NS> &own) {
+template <int ES, int SBS, int NS, int kHalves>
+__device__ static inline void settle(OwnRows<ES, SBS, NS, kHalves> &own) {
 #pragma unroll
-  for (int f = 0; f < OwnRows<ES, SBS, NS>::T::kFrags; ++f) asm volatile("" : "+v"(own.fr[f]));
+  for (int f = 0; f < OwnRows<ES, SBS, NS, kHalves>::T::kFrags; ++f) asm volatile("" : "+v"(own.fr[f]));
 }
 
 // acc (per partner block t) = partner rows x own rows over all head slices: acc[t] belongs to this lane's own row
 // (lane % SBS) and partner rows 8 (r / 4) + 4 (lane / 32) + r % 4 (SBS 32) or 4 (lane / 16) + r (SBS 16).
-template <typename Tr, int SBS, int NS, int NB, typename Acc>
-__device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<Tr::kElem, SBS, NS, NB>::RowReader &rows,
-                                           const OwnRows<Tr::kElem, SBS, NS> &own) {
+template <typename Tr, int SBS, int NS, int NB, int kHalves, typename Acc>
+__device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<Tr::kElem, SBS, NS, NB, kHalves>::RowReader &rows,
+                                           const OwnRows<Tr::kElem, SBS, NS, kHalves> &own) {
 #pragma unroll
   for (int t = 0; t < NB; ++t)
 #pragma unroll
@@ -302,7 +339,7 @@ __device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<T
 // would turn an infinite or NaN value of the other into NaN
 template <typename Tr, int SBS, int NS, int NB, typename Acc>
 __device__ static inline void product_some_rows(Acc (&acc)[NB], const typename Tile<Tr::kElem, SBS, NS, NB>::RowReader &rows,
-                                                const OwnRows<Tr::kElem, SBS, NS> &own, const uint32_t (&have)[NB], int lane) {
+                                                const OwnRows<Tr::kElem, SBS, NS, 1> &own, const uint32_t (&have)[NB], int lane) {
   using T = Tile<Tr::kElem, SBS, NS, NB>;
 #pragma unroll
   for (int t = 0; t < NB; ++t)
@@ -344,8 +381,8 @@ struct Weights<SF32, kScores> {
 };
 
 // out[h] += partner columns^T x weights
-template <typename Tr, int SBS, int NS, int NB, int kScores, typename Acc>
-__device__ static inline void product_cols(Acc (&out)[NS], const typename Tile<Tr::kElem, SBS, NS, NB>::ColReader &cols,
+template <typename Tr, int SBS, int NS, int NB, int kHalves, int kScores, typename Acc>
+__device__ static inline void product_cols(Acc (&out)[NS], const typename Tile<Tr::kElem, SBS, NS, NB, kHalves>::ColReader &cols,
                                            const Weights<Tr, kScores> &w) {
   if constexpr (Tr::kElem == 4) {
     constexpr int kRegs = kScores / NB;
@@ -455,11 +492,13 @@ __device__ static inline float row_sum(float v) {
 // 16 x 2048 queries, a quarter of the blocks, head dimension 64, 9 of 10 slices there, forward / forward and backward: bf16,
 // sbs 16: 45 / 165 us (61 / 189 with every block of a window of 64 gathered as soon as one had a gap), fp32: 96 / 352
 // (131 / 453); full layouts 27 / 164 and 67 / 256.
-template <int ES, int SBS, int NS, int NB, bool kOwnIsQuery, bool kSome>
+// kHalves 2 (blocks of 64): blocks, slices and places are those of the kernels (Place), so an entry of the list is two.
+template <int ES, int SBS, int NS, int NB, bool kOwnIsQuery, bool kSome, int kHalves>
 struct Walk {
-  using T = Tile<ES, SBS, NS, NB>;
+  static_assert(kHalves == 1 || !kSome, "missing slices of blocks of 64 take another kernel");
+  using T = Tile<ES, SBS, NS, NB, kHalves>;
   int64_t b, own;          // batch entry, own block
-  int first, step;         // the wave's entries of the list: first, first + step, ...
+  int list, first, step;   // start of the list; the wave's places in it: first, first + step, ...
   int end, base, seq_len;  // their number, the first one of the window; valid length of a causal sequence
   int other, first_a, first_b, mask, bias;  // of this lane's entry
   uint64_t live, special, apart;
@@ -482,10 +521,11 @@ struct Walk {
       const int64_t len = a.causal_lengths[b];
       seq_len = len < 0 ? 0 : (len > 0x7fffffffLL ? 0x7fffffff : (int)len);
     }
-    const int32_t *offsets = (kOwnIsQuery ? a.key_offsets : a.query_offsets) + b * (kOwnIsQuery ? a.nq : a.nk) + own;
-    first = first_lane(offsets[0]) + part;
+    const int32_t *offsets = (kOwnIsQuery ? a.key_offsets : a.query_offsets) + b * (kOwnIsQuery ? a.nq : a.nk) + own / kHalves;
+    list = first_lane(offsets[0]);
+    first = part;
     step = parts;
-    const int left = first_lane(offsets[1]) - first;
+    const int left = kHalves * (first_lane(offsets[1]) - list) - part;
     end = left > 0 ? (int)(((unsigned)left + parts - 1) / parts) : 0;
     if (!there || (int)own * SBS >= seq_len) end = 0;
     base = -64;
@@ -506,10 +546,11 @@ struct Walk {
     const late_args_t p = late_args();
     base += 64;
     bool in = base + lane < end;
-    other = in ? (kOwnIsQuery ? p->key_indices : p->query_indices)[first + step * (base + lane)] : 0;
+    const int at = first + step * (base + lane);
+    other = in ? kHalves * (kOwnIsQuery ? p->key_indices : p->query_indices)[list + at / kHalves] + at % kHalves : 0;
     const bool causal = p->causal_lengths != nullptr;
     in = in && !(causal && ((kOwnIsQuery ? other > (int)own : other < (int)own) || other * SBS >= seq_len));
-    const int64_t place = b * (kOwnIsQuery ? p->nk : p->nq) + other;
+    const int64_t place = b * (kOwnIsQuery ? p->nk : p->nq) + other / kHalves;
     const int64_t *pa = kOwnIsQuery ? p->pidx_k : p->pidx_q, *pb = kOwnIsQuery ? p->pidx_v : p->pidx_o;
     const int64_t end_a = kOwnIsQuery ? p->n_k_blocks : p->n_q_blocks, end_b = kOwnIsQuery ? p->n_v_blocks : p->n_o_blocks;
     if constexpr (kSome) {
@@ -520,13 +561,16 @@ struct Walk {
       }
       apart = __ballot(in && far);
     } else if (in) {  // every slice of every partner block is there: the others follow the first
-      const int64_t a0 = pa[place * NS], b0 = pb[place * NS];
-      first_a = (int)a0;
-      first_b = (int)b0;
-      in = a0 >= 0 && b0 >= 0 && a0 + NS <= end_a && b0 + NS <= end_b;  // a wrong index must not turn into a wild read
+      constexpr int kSlices = NS / kHalves;  // of the layout
+      const int64_t a0 = pa[place * kSlices], b0 = pb[place * kSlices];
+      first_a = kHalves * (int)a0 + other % kHalves;
+      first_b = kHalves * (int)b0 + other % kHalves;
+      // a wrong index must not turn into a wild read
+      in = a0 >= 0 && b0 >= 0 && a0 + kSlices <= end_a && b0 + kSlices <= end_b;
     }
     bool extra = causal && (other == (int)own || ((int)own + 1) * SBS > seq_len || (other + 1) * SBS > seq_len);
-    const int64_t pair = kOwnIsQuery ? (b * p->nq + own) * p->nk + other : (b * p->nq + other) * p->nk + own;
+    const int64_t mine = own / kHalves, theirs = other / kHalves;
+    const int64_t pair = kOwnIsQuery ? (b * p->nq + mine) * p->nk + theirs : (b * p->nq + theirs) * p->nk + mine;
     if (p->mask) {
       const int64_t m = in ? p->pidx_mask[pair] : -1;
       mask = m < p->n_mask_blocks ? (int)m : -1;
@@ -613,14 +657,14 @@ struct Walk {
   // acc = rows of the step's blocks of the first (second) tensor x own rows, and out += their columns^T x weights
   template <typename Tr, bool kSecond, typename Acc>
   __device__ static inline void multiply_rows(Acc (&acc)[NB], const Step &s, const typename T::RowReader &rows,
-                                              const OwnRows<ES, SBS, NS> &own, int lane) {
+                                              const OwnRows<ES, SBS, NS, kHalves> &own, int lane) {
     if constexpr (kSome) {
       uint32_t have[NB];
 #pragma unroll
       for (int t = 0; t < NB; ++t) have[t] = (kSecond ? s.have[t] >> 8 : s.have[t]) & own.there;
       product_some_rows<Tr, SBS, NS, NB>(acc, rows, own, have, lane);
     } else {
-      product_rows<Tr, SBS, NS, NB>(acc, rows, own);
+      product_rows<Tr, SBS, NS, NB, kHalves>(acc, rows, own);
     }
   }
   template <typename Tr, bool kSecond, int kScores, typename Acc>
@@ -632,7 +676,7 @@ struct Walk {
       for (int t = 0; t < NB; ++t) have[t] = kSecond ? s.have[t] >> 8 : s.have[t];
       product_some_cols<Tr, SBS, NS, NB>(out, cols, w, have);
     } else {
-      product_cols<Tr, SBS, NS, NB>(out, cols, w);
+      product_cols<Tr, SBS, NS, NB, kHalves>(out, cols, w);
     }
   }
 
@@ -642,19 +686,23 @@ struct Walk {
   template <typename Tr>
   __device__ inline void finish_scores(const Step &s, float *sv, float qk_scale, int me, int group) const {
     constexpr int kRegs = SBS == 32 ? 16 : 4;
+    constexpr int kSide = kHalves * SBS;  // of a block of the layout, for mask and bias
     const late_args_t p = late_args();
 #pragma unroll
     for (int t = 0; t < NB; ++t) {
       float *v = sv + kRegs * t;
+      // first row and column of this block's part of the layout's mask and bias blocks
+      const int mine0 = (int)own % kHalves * SBS, theirs0 = s.other[t] % kHalves * SBS;
+      const int corner = kOwnIsQuery ? mine0 * kSide + theirs0 : theirs0 * kSide + mine0;
       // registers 4 w .. 4 w + 3 belong to partner rows 8 w + 4 group .. + 3
       if (p->bias) {
-        const char *blk = static_cast<const char *>(p->bias) + (int64_t)s.bias[t] * T::kPiece;
+        const char *blk = static_cast<const char *>(p->bias) + ((int64_t)s.bias[t] * (kSide * kSide) + corner) * ES;
 #pragma unroll
         for (int w = 0; w < kRegs / 4; ++w)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int theirs = 8 * w + 4 * group + i;
-            const int at = kOwnIsQuery ? me * SBS + theirs : theirs * SBS + me;
+            const int at = kOwnIsQuery ? me * kSide + theirs : theirs * kSide + me;
             float bias_value = 0.f;
             if (s.bias[t] >= 0) {
               if constexpr (ES == 4) bias_value = reinterpret_cast<const float *>(blk)[at];
@@ -664,15 +712,15 @@ struct Walk {
           }
       }
       if (s.mask[t] >= 0) {
-        const uint8_t *blk = static_cast<const uint8_t *>(p->mask) + (int64_t)s.mask[t] * (SBS * SBS);
+        const uint8_t *blk = static_cast<const uint8_t *>(p->mask) + (int64_t)s.mask[t] * (kSide * kSide) + corner;
         uint32_t mw[kRegs / 4];
 #pragma unroll
         for (int w = 0; w < kRegs / 4; ++w) {
           if constexpr (kOwnIsQuery) {
-            mw[w] = *reinterpret_cast<const uint32_t *>(blk + me * SBS + 8 * w + 4 * group);
+            mw[w] = *reinterpret_cast<const uint32_t *>(blk + me * kSide + 8 * w + 4 * group);
           } else {
-            const uint8_t *col = blk + (8 * w + 4 * group) * SBS + me;
-            mw[w] = col[0] | (uint32_t)col[SBS] << 8 | (uint32_t)col[2 * SBS] << 16 | (uint32_t)col[3 * SBS] << 24;
+            const uint8_t *col = blk + (8 * w + 4 * group) * kSide + me;
+            mw[w] = col[0] | (uint32_t)col[kSide] << 8 | (uint32_t)col[2 * kSide] << 16 | (uint32_t)col[3 * kSide] << 24;
           }
         }
 #pragma unroll
@@ -695,12 +743,21 @@ struct Walk {
   }
 };
 
-// Whether the kernels for blocks of 16 and 32 take these arguments (up to the head slices they are built for)
-inline bool small_applies(const bsa_attn_args &a) {
-  if (a.sbs != 16 && a.sbs != 32) return false;
+// Whether all blocks of all rows have all their head slices, as many of q / k as of v / o: the block counts say so.  Of the output
+// only the backward kernels read, and query blocks that attend to nothing may go without.
+inline bool all_slices(const bsa_attn_args &a, bool backward) {
+  if (a.nh != a.nhv || a.n_q_blocks != a.B * a.nq * a.nh || a.n_k_blocks != a.B * a.nk * a.nh || a.n_v_blocks != a.B * a.nk * a.nhv)
+    return false;
+  return !backward || a.n_o_blocks == a.B * a.nq * a.nhv || a.o_rows_whole != 0;
+}
+
+// Whether the kernels for blocks of 16 and 32 take these arguments (up to the head slices they are built for).  Blocks of 64
+// are for them only in fp32 (16-bit operands: attn_mfma.hip, attn_bwd_mfma.hip) and with all slices there.
+inline bool small_applies(const bsa_attn_args &a, bool backward) {
+  if (a.sbs != 16 && a.sbs != 32 && !(a.sbs == 64 && a.dtype == BSA_F32 && all_slices(a, backward))) return false;
   // the forward kernel takes the row maximum before the scale is applied
   if (!(a.scale > 0.f) || a.scale > 3.0e38f) return false;
-  const int64_t most = 0x7fffffffLL;  // indices and positions are 32-bit numbers
+  const int64_t most = a.sbs == 64 ? 0x3fffffffLL : 0x7fffffffLL;  // indices (of halves) and positions are 32-bit numbers
   if (a.n_q_blocks > most || a.n_k_blocks > most || a.n_v_blocks > most || a.n_o_blocks > most ||
       a.n_mask_blocks > most || a.n_bias_blocks > most || a.nq * a.sbs > most || a.nk * a.sbs > most)
     return false;
@@ -714,14 +771,6 @@ inline bool small_applies(const bsa_attn_args &a) {
   if ((starts & 15) != 0 || (reinterpret_cast<uintptr_t>(a.mask) & 3) != 0) return false;
   const int64_t slices = a.nh > a.nhv ? a.nh : a.nhv;
   return slices >= 1 && slices <= 128 / a.sbs;
-}
-
-// Whether all blocks of all rows have all their head slices, as many of q / k as of v / o: the block counts say so.  Of the output
-// only the backward kernels read, and query blocks that attend to nothing may go without.
-inline bool all_slices(const bsa_attn_args &a, bool backward) {
-  if (a.nh != a.nhv || a.n_q_blocks != a.B * a.nq * a.nh || a.n_k_blocks != a.B * a.nk * a.nh || a.n_v_blocks != a.B * a.nk * a.nhv)
-    return false;
-  return !backward || a.n_o_blocks == a.B * a.nq * a.nhv || a.o_rows_whole != 0;
 }
 
 // Waves that share one row of a launch of `rows` rows, each walking every second or fourth entry of its list.  A launch

@@ -36,13 +36,13 @@ using namespace small;
 
 constexpr int kWaves = 4;
 
-template <int ES, int SBS, int NS>
+template <int ES, int SBS, int NS, int kHalves>
 struct FwdShape {
   // Key blocks per step.  Two blocks of 32 leave registers for three waves per SIMD instead of four (97 against 84 us,
   // 6144 rows of 33 blocks, head dimension 64); four blocks of 16 take twice the LDS, which leaves half the waves (76
   // against 60 us, 4128 rows, causal, head dimension 64).
   static constexpr int NB = SBS == 32 ? 1 : 2;
-  using T = Tile<ES, SBS, NS, NB>;
+  using T = Tile<ES, SBS, NS, NB, kHalves>;
   static constexpr int kScores = SBS == 32 ? 16 * NB : 4 * NB;  // per lane and step
   static constexpr int kRegs = SBS == 32 ? 16 : 4;              // accumulator registers per block
   // K tile, V tile; at the end the partial output of a wave that shares a query block with others
@@ -52,26 +52,28 @@ struct FwdShape {
 };
 
 // split: 1, 2 or 4 waves share one query block, each walking every split-th entry of its key list
-template <typename Tr, int SBS, int NS, bool kSome>
-__global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWaves)) void attn_small_fwd_kernel(bsa_attn_args a, int split) {
-  using Shape = FwdShape<Tr::kElem, SBS, NS>;
+// kHalves 2: blocks of 64, whose halves are the blocks of 32 spoken of here (Place)
+template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
+__global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>::kMinWaves)) void attn_small_fwd_kernel(bsa_attn_args a, int split) {
+  using Shape = FwdShape<Tr::kElem, SBS, NS, kHalves>;
   using T = typename Shape::T;
-  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true, kSome>;
-  constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs, kPiece = T::kPiece;
+  using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true, kSome, kHalves>;
+  using P = Place<Tr::kElem, SBS, kHalves>;
+  constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
   const int lane = threadIdx.x & 63;
   const int wave = first_lane(threadIdx.x >> 6);
   char *lds_k = small_smem + wave * Shape::kLds, *lds_v = lds_k + T::kBytes;
 
-  const RowOfWave me(a.B, a.nq, true, wave, kWaves, split);
-  const int64_t row = me.b * a.nq + me.own;
+  const RowOfWave me(a.B, kHalves * a.nq, true, wave, kWaves, split);
+  const int64_t row = me.b * a.nq + me.own / kHalves;  // of the layout
   const int qi = lane % SBS, kq = lane / SBS;  // query row; which keys of a block this lane's registers hold
   W walk;
   walk.start(a, me.b, me.own, me.there, me.part, split);
 
-  OwnRows<Tr::kElem, SBS, NS> qf;
-  qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, lane);
+  OwnRows<Tr::kElem, SBS, NS, kHalves> qf;
+  qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, (int)me.own, lane);
   acc_t oacc[NS];
 #pragma unroll
   for (int h = 0; h < NS; ++h)
@@ -199,41 +201,44 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS>::kMinWav
   const float inv_l = (l_i != 0.f) ? 1.f / l_i : 0.f;
 #pragma unroll
   for (int h = 0; h < NS; ++h) {
-    if (h >= nhv) break;
-    const int64_t po = p->pidx_o[row * nhv + h];
+    if (h / kHalves >= nhv) break;
+    const int64_t po = p->pidx_o[row * nhv + h / kHalves];
     if (po < 0 || po >= p->n_o_blocks) continue;
-    char *out = static_cast<char *>(p->o) + po * kPiece;
+    char *out = static_cast<char *>(p->o) + P::row(po, (int)me.own, qi, h);
 #pragma unroll
     for (int r = 0; r < kRegs; r += 4)  // columns 2 r + 4 kq .. + 3 of a row per lane
-      store4<Tr>(out + (qi * SBS + 2 * r + 4 * kq) * Tr::kElem, oacc[h][r] * inv_l, oacc[h][r + 1] * inv_l,
+      store4<Tr>(out + (2 * r + 4 * kq) * Tr::kElem, oacc[h][r] * inv_l, oacc[h][r + 1] * inv_l,
                  oacc[h][r + 2] * inv_l, oacc[h][r + 3] * inv_l);
   }
-  if (kq == 0) p->lse[row * SBS + qi] = (l_i != 0.f) ? m_i + log2f(l_i) : -INFINITY;
+  if (kq == 0) p->lse[(row * kHalves + me.own % kHalves) * SBS + qi] = (l_i != 0.f) ? m_i + log2f(l_i) : -INFINITY;
 }
 
-template <typename Tr, int SBS, int NS, bool kSome>
+template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
 int launch_kind(const bsa_attn_args &a, hipStream_t s) {
-  using Shape = FwdShape<Tr::kElem, SBS, NS>;
-  const int64_t rows = a.B * a.nq;
-  const int split = waves_per_row<Tr>(rows, a.nk, Shape::NB);
-  const int64_t groups = row_groups(a.B, a.nq, kWaves, split);
+  using Shape = FwdShape<Tr::kElem, SBS, NS, kHalves>;
+  const int64_t rows = kHalves * a.nq;  // of a batch entry
+  const int split = waves_per_row<Tr>(a.B * rows, kHalves * a.nk, Shape::NB);
+  const int64_t groups = row_groups(a.B, rows, kWaves, split);
   if (!fits_launch(groups, kWaves)) return 1;
   constexpr int lds = Shape::kLds * kWaves;
   static_assert(lds <= 160 * 1024, "LDS");
   static LdsLimit limit;
-  if (int rc = allow_lds(limit, &attn_small_fwd_kernel<Tr, SBS, NS, kSome>, lds)) return rc;
-  attn_small_fwd_kernel<Tr, SBS, NS, kSome><<<(unsigned)groups, 64 * kWaves, lds, s>>>(a, split);
+  if (int rc = allow_lds(limit, &attn_small_fwd_kernel<Tr, SBS, NS, kSome, kHalves>, lds)) return rc;
+  attn_small_fwd_kernel<Tr, SBS, NS, kSome, kHalves><<<(unsigned)groups, 64 * kWaves, lds, s>>>(a, split);
   return check_launch("attn_small_fwd_kernel");
 }
 
 template <typename Tr, int SBS, int NS>
 int launch(const bsa_attn_args &a, hipStream_t s) {
-  return all_slices(a, false) ? launch_kind<Tr, SBS, NS, false>(a, s) : launch_kind<Tr, SBS, NS, true>(a, s);
+  return all_slices(a, false) ? launch_kind<Tr, SBS, NS, false, 1>(a, s) : launch_kind<Tr, SBS, NS, true, 1>(a, s);
 }
 
 template <typename Tr>
 int dispatch(const bsa_attn_args &a, hipStream_t s) {
   const int64_t slices = a.nh > a.nhv ? a.nh : a.nhv;
+  if constexpr (Tr::kElem == 4) {
+    if (a.sbs == 64) return slices == 1 ? launch_kind<Tr, 32, 2, false, 2>(a, s) : launch_kind<Tr, 32, 4, false, 2>(a, s);
+  }
   if (a.sbs == 32) {
     switch (slices) {
       case 1: return launch<Tr, 32, 1>(a, s);
@@ -260,7 +265,7 @@ int dispatch(const bsa_attn_args &a, hipStream_t s) {
 
 // 1: not covered
 int attn_fwd_small(const bsa_attn_args &a, hipStream_t s) {
-  if (!small_applies(a)) return 1;
+  if (!small_applies(a, false)) return 1;
   if (a.B * a.nq == 0) return BSA_OK;
   return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, s) : a.dtype == BSA_F16 ? dispatch<SF16>(a, s) : dispatch<SF32>(a, s);
 }
