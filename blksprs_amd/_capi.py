@@ -37,6 +37,13 @@ class AttnArgs(ctypes.Structure):
     )
 
 
+class AttnShares(ctypes.Structure):
+    """Mirror of ``struct bsa_attn_shares``."""
+
+    _fields_ = [("groups", c_void_p), ("merges", c_void_p), ("n_groups", c_int64), ("n_merges", c_int64),
+                ("n_slots", c_int64), ("scratch", c_void_p), ("scratch_bytes", c_int64)]
+
+
 class LinesArgs(ctypes.Structure):
     """Mirror of ``struct bsa_lines_args``."""
 
@@ -51,6 +58,7 @@ class LinesArgs(ctypes.Structure):
 
 
 ATTN_RECORD_INTS = 16  # BSA_ATTN_RECORD_INTS
+SHARE_INTS = 12  # BSA_SHARE_INTS
 ROWS_RECORD_INTS = 128  # BSA_ROWS_RECORD_INTS
 
 # name -> (restype, argtypes); must list every symbol of include/blksprs_amd.h
@@ -102,6 +110,14 @@ SIGNATURES = {
     "bsa_attn_mask_dead": (c_int, [c_void_p, c_int64, ctypes.c_int32, c_void_p, c_void_p]),
     "bsa_attn_bwd_scratch_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int64, c_int64]),
     "bsa_attn_bwd_ds_bytes": (c_size_t, [c_int64, ctypes.c_int32]),
+    "bsa_attn_shares_piece": (c_int, [ctypes.POINTER(AttnArgs), c_int, c_int64, c_int64, ctypes.POINTER(c_int64),
+                                      ctypes.POINTER(c_int64), ctypes.POINTER(c_int64)]),
+    "bsa_attn_shares_build": (c_int, [ctypes.POINTER(AttnArgs), c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p,
+                                      c_void_p, c_void_p]),
+    "bsa_attn_shares_scratch_bytes": (c_size_t, [ctypes.POINTER(AttnArgs), c_int, c_int64]),
+    "bsa_attn_fwd_shares": (c_int, [ctypes.POINTER(AttnArgs), ctypes.POINTER(AttnShares), c_void_p]),
+    "bsa_attn_bwd_shares": (c_int, [ctypes.POINTER(AttnArgs), ctypes.POINTER(AttnShares), ctypes.POINTER(AttnShares),
+                                    c_void_p]),
     "bsa_attn_fwd": (c_int, [ctypes.POINTER(AttnArgs), c_void_p]),
     "bsa_attn_bwd": (c_int, [ctypes.POINTER(AttnArgs), c_void_p]),
 }

@@ -1,7 +1,7 @@
 // C ABI of block-sparse flash attention: argument checks and the choice of kernels: 16-bit operands in 64 x 64 blocks
-// with at most two head slices (attn_mfma.hip, attn_bwd_mfma.hip), blocks of 16 and 32 with head dimensions up to 128
-// (attn_small_fwd.hip, attn_small_bwd.hip), the rest on the fp32 matrix-core instruction (attn_f32mma.hip: fp32 blocks
-// of 64, longer head dimensions, scales that are not positive, tensors that do not start on 16 bytes), and the generic
+// with at most two head slices (attn_mfma.hip, attn_bwd_mfma.hip), blocks of 16 and 32 and fp32 blocks of 64 with head
+// dimensions up to 128 (attn_small_fwd.hip, attn_small_bwd.hip), the rest on the fp32 matrix-core instruction
+// (attn_f32mma.hip: fp32 blocks of 64 with missing slices, longer head dimensions, scales that are not positive, tensors that do not start on 16 bytes), and the generic
 // kernels for more head slices than fit LDS.
 #include "attn_common.h"
 
@@ -43,14 +43,62 @@ int check_args(const char *who, const bsa_attn_args *a, bool backward) {
   return BSA_OK;
 }
 
+int check_shares(const char *who, const bsa_attn_shares *s) {
+  if (s == nullptr) return BSA_OK;
+  BSA_REQUIRE(s->n_groups >= 0 && s->n_merges >= 0 && s->n_slots >= 0 && s->scratch_bytes >= 0, "%s: negative number in the shares", who);
+  BSA_REQUIRE(s->n_groups < 0x7fffffffLL && s->n_merges < 0x3fffffffLL && s->n_slots < 0x3fffffffLL, "%s: too many shares", who);
+  BSA_REQUIRE(s->groups != nullptr && s->n_groups > 0 && s->n_groups % 8 == 0, "%s: shares without groups, or not as many for each XCD", who);
+  BSA_REQUIRE(s->n_merges == 0 || (s->merges != nullptr && s->scratch != nullptr), "%s: shares without merges or scratch", who);
+  BSA_REQUIRE((reinterpret_cast<uintptr_t>(s->scratch) & 15) == 0, "%s: scratch of the shares must be 16-byte aligned", who);
+  return BSA_OK;
+}
+
+int check_plan(const char *who, const bsa_attn_args *a, int key_rows) {
+  BSA_REQUIRE(a != nullptr, "%s: NULL argument block", who);
+  BSA_REQUIRE(key_rows == 0 || key_rows == 1, "%s: key_rows must be 0 or 1 (got %d)", who, key_rows);
+  BSA_REQUIRE(a->B >= 0 && a->nq >= 0 && a->nk >= 0 && a->nh >= 0 && a->nhv >= 0, "%s: negative layout size", who);
+  BSA_REQUIRE(a->B * a->nq < 0x7fffffffLL && a->B * a->nk < 0x7fffffffLL, "%s: too many sequence blocks", who);
+  return BSA_OK;
+}
+
 }  // namespace
 
-extern "C" int bsa_attn_fwd(const bsa_attn_args *args, bsa_stream_t stream) {
+extern "C" int bsa_attn_fwd(const bsa_attn_args *args, bsa_stream_t stream) { return bsa_attn_fwd_shares(args, nullptr, stream); }
+
+extern "C" int bsa_attn_shares_piece(const bsa_attn_args *a, int key_rows, int64_t n_entries, int64_t longest, int64_t *piece,
+                                     int64_t *max_groups, int64_t *max_merges) {
+  const char *who = "bsa_attn_shares_piece";
+  if (int rc = check_plan(who, a, key_rows)) return rc;
+  BSA_REQUIRE(piece && max_groups && max_merges, "%s: NULL argument", who);
+  *piece = bsa::attn_shares_piece(*a, key_rows != 0, n_entries, longest);
+  *max_groups = *max_merges = 0;
+  if (*piece > 0) bsa::attn_shares_limits(*a, key_rows != 0, n_entries, *piece, max_groups, max_merges);
+  return BSA_OK;
+}
+
+extern "C" int bsa_attn_shares_build(const bsa_attn_args *a, int key_rows, int64_t piece, int64_t max_groups, int64_t max_merges,
+                                     int32_t *groups, int32_t *merges, int64_t *stats, bsa_stream_t stream) {
+  const char *who = "bsa_attn_shares_build";
+  if (int rc = check_plan(who, a, key_rows)) return rc;
+  BSA_REQUIRE(piece > 0, "%s: piece must be positive", who);
+  BSA_REQUIRE(max_groups > 0 && max_groups % 8 == 0 && max_merges > 0, "%s: bad limits", who);
+  BSA_REQUIRE((key_rows ? a->query_offsets : a->key_offsets) != nullptr && groups && merges && stats, "%s: NULL argument", who);
+  BSA_REQUIRE(a->B > 0 && (key_rows ? a->nk : a->nq) > 0 && a->B * (key_rows ? a->nk : a->nq) <= 65536, "%s: 1 to 65536 rows", who);
+  return bsa::attn_shares_build(*a, key_rows != 0, piece, max_groups, max_merges, groups, merges, stats, bsa::as_stream(stream));
+}
+
+extern "C" size_t bsa_attn_shares_scratch_bytes(const bsa_attn_args *a, int what, int64_t n_slots) {
+  if (a == nullptr || what < 0 || what > 2 || n_slots <= 0) return 0;
+  return (size_t)(n_slots * bsa::attn_shares_slot_bytes(*a, what));
+}
+
+extern "C" int bsa_attn_fwd_shares(const bsa_attn_args *args, const bsa_attn_shares *shares, bsa_stream_t stream) {
   if (int rc = check_args("bsa_attn_fwd", args, false)) return rc;
+  if (int rc = check_shares("bsa_attn_fwd_shares", shares)) return rc;
   hipStream_t s = bsa::as_stream(stream);
   int rc = bsa::attn_fwd_mfma(*args, s);          // 16-bit operands, 64 x 64 blocks
-  if (rc == 1) rc = bsa::attn_fwd_small(*args, s);   // blocks of 16 and 32
-  if (rc == 1) rc = bsa::attn_fwd_f32mma(*args, s);  // everything else, on the fp32 matrix-core instruction
+  if (rc == 1) rc = bsa::attn_fwd_small(*args, shares, s);  // blocks of 16 and 32, fp32 blocks of 64
+  if (rc == 1) rc = bsa::attn_fwd_f32mma(*args, s);         // everything else, on the fp32 matrix-core instruction
   if (rc == 1) rc = bsa::attn_fwd_generic(*args, s);
   return rc;
 }
@@ -95,7 +143,14 @@ extern "C" size_t bsa_attn_bwd_ds_bytes(int64_t n_layout_blocks, int32_t sbs) {
 }
 
 extern "C" int bsa_attn_bwd(const bsa_attn_args *args, bsa_stream_t stream) {
+  return bsa_attn_bwd_shares(args, nullptr, nullptr, stream);
+}
+
+extern "C" int bsa_attn_bwd_shares(const bsa_attn_args *args, const bsa_attn_shares *query_shares, const bsa_attn_shares *key_shares,
+                                   bsa_stream_t stream) {
   if (int rc = check_args("bsa_attn_bwd", args, true)) return rc;
+  if (int rc = check_shares("bsa_attn_bwd_shares", query_shares)) return rc;
+  if (int rc = check_shares("bsa_attn_bwd_shares", key_shares)) return rc;
   BSA_REQUIRE(args->bwd_scratch == nullptr || args->n_layout_blocks >= 0, "bsa_attn_bwd: negative n_layout_blocks");
   BSA_REQUIRE(args->bwd_scratch_bytes >= 0, "bsa_attn_bwd: negative bwd_scratch_bytes");
   BSA_REQUIRE((reinterpret_cast<uintptr_t>(args->bwd_scratch) & 15) == 0, "bsa_attn_bwd: bwd_scratch must be 16-byte aligned");
@@ -108,7 +163,7 @@ extern "C" int bsa_attn_bwd(const bsa_attn_args *args, bsa_stream_t stream) {
   }
   hipStream_t s = bsa::as_stream(stream);
   int rc = bsa::attn_bwd_mfma(*args, s);
-  if (rc == 1) rc = bsa::attn_bwd_small(*args, s);
+  if (rc == 1) rc = bsa::attn_bwd_small(*args, query_shares, key_shares, s);
   if (rc == 1) rc = bsa::attn_bwd_f32mma(*args, s);
   if (rc == 1) rc = bsa::attn_bwd_generic(*args, s);
   return rc;

@@ -49,9 +49,14 @@ int attn_fwd_records(const bsa_attn_args &a, const int32_t *entries, int32_t *re
 int attn_bwd_generic(const bsa_attn_args &a, hipStream_t s);
 // MFMA paths; return 1 if the configuration is not covered (caller falls back to the generic kernels)
 int attn_fwd_mfma(const bsa_attn_args &a, hipStream_t s);
-int attn_fwd_small(const bsa_attn_args &a, hipStream_t s);
+int attn_fwd_small(const bsa_attn_args &a, const bsa_attn_shares *shares, hipStream_t s);
+int64_t attn_shares_piece(const bsa_attn_args &a, bool key_rows, int64_t n_entries, int64_t longest);
+void attn_shares_limits(const bsa_attn_args &a, bool key_rows, int64_t n_entries, int64_t piece, int64_t *max_groups, int64_t *max_merges);
+int attn_shares_build(const bsa_attn_args &a, bool key_rows, int64_t piece, int64_t max_groups, int64_t max_merges, int32_t *groups,
+                      int32_t *merges, int64_t *stats, hipStream_t s);
+int64_t attn_shares_slot_bytes(const bsa_attn_args &a, int what);
 int attn_fwd_f32mma(const bsa_attn_args &a, hipStream_t s);
-int attn_bwd_small(const bsa_attn_args &a, hipStream_t s);
+int attn_bwd_small(const bsa_attn_args &a, const bsa_attn_shares *query_shares, const bsa_attn_shares *key_shares, hipStream_t s);
 int attn_bwd_f32mma(const bsa_attn_args &a, hipStream_t s);
 int attn_bwd_mfma(const bsa_attn_args &a, hipStream_t s);
 int attn_mask_dead(const void *mask, int64_t n_mask_blocks, uint8_t *dead, hipStream_t s);

@@ -1,5 +1,6 @@
 // Block-sparse flash attention forward on the fp32 matrix-core instruction (v_mfma_f32_16x16x4_f32): what the kernels
-// of attn_mfma.hip (16-bit, 64 x 64) and attn_small_fwd.hip (blocks of 16 and 32) leave: fp32 blocks of 64, longer
+// of attn_mfma.hip (16-bit, 64 x 64) and attn_small_fwd.hip (blocks of 16 and 32) leave: fp32 blocks of 64
+// with missing slices, longer
 // head dimensions, scales that are not positive, tensors that do not start on 16 bytes.  16-bit operands are widened
 // to fp32 while they are staged, probabilities are rounded to the operand type before they multiply V, as the
 // reference does (blksprs/ops/flash_attention.py:1193).

@@ -19,7 +19,9 @@
 // to overlap it.  Against the fp32 matrix-core kernels that ran these shapes before (48 x 4096 queries, sbs 32, head
 // dimension 64, fp16, 33 key blocks per query block): delta + zero fill 0.071 -> 0, dK / dV 1.89 -> 0.125 ms (530 TFLOP/s),
 // dQ 1.24 -> 0.090 ms (delta included); fp32, 8 x 2048 queries, sbs 32, half of the blocks, head dimension 64: dK / dV 0.238
-// -> 0.096, dQ 0.198 -> 0.076 ms (89 and 85 TFLOP/s).
+// -> 0.096, dQ 0.198 -> 0.076 ms (89 and 85 TFLOP/s).  fp32 blocks of 64, whose halves walk alone like blocks of 32: 34
+// sequences of 480 to 960, head dimension 64, causal: delta + zero fill 0.023 -> 0, dK / dV 0.222 -> 0.076, dQ 0.132 ->
+// 0.059 ms.
 //
 // Scores as in the forward kernel; p = exp2(s - lse), 0 where lse = -inf; P and dS are rounded to the operand type
 // before they enter a product (blksprs/ops/flash_attention.py:1452, :1468, :1692).
@@ -41,6 +43,7 @@ struct BwdShape {
   static constexpr int kRegs = SBS == 32 ? 16 : 4;
   static constexpr int kScores = kRegs * NB;
   static constexpr int kPartial = SBS * SBS * NS * 4;
+  static constexpr int kSlot = SBS * SBS * NS;  // floats of a slot of the scratch, twice for dK and dV
   static constexpr int kStats = 256;  // lse and delta of the 32 queries of a step
   // dK / dV kernel: Q and dO of two steps where registers allow two waves per SIMD anyway (sbs 32: 133 against 137 us);
   // at sbs 16 one step's tiles and twice the waves are faster (67 against 92 us)
@@ -58,28 +61,6 @@ struct BwdShape {
 __device__ inline void copy_words_to_lds(const float *addr, char *dst) {
   const uint32_t lds_addr = (uint32_t)(uintptr_t)(lds_ptr_t)dst;
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(addr), "s"(lds_addr) : "memory");
-}
-
-// the partial sums of the waves that share a row, added up in order into those of the first
-template <int NS, int kRegs, typename Acc>
-__device__ inline void leave_partial(const Acc (&acc)[NS], float *mine, int lane) {
-#pragma unroll
-  for (int h = 0; h < NS; ++h)
-#pragma unroll
-    for (int r = 0; r < kRegs; r += 4)
-      *reinterpret_cast<f32x4 *>(mine + ((h * kRegs + r) / 4 * 64 + lane) * 4) =
-          f32x4{acc[h][r], acc[h][r + 1], acc[h][r + 2], acc[h][r + 3]};
-}
-template <int NS, int kRegs, typename Acc>
-__device__ inline void add_partial(Acc (&acc)[NS], const float *other, int lane) {
-#pragma unroll
-  for (int h = 0; h < NS; ++h)
-#pragma unroll
-    for (int r = 0; r < kRegs; r += 4) {
-      const f32x4 v = *reinterpret_cast<const f32x4 *>(other + ((h * kRegs + r) / 4 * 64 + lane) * 4);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[h][r + i] += v[i];
-    }
 }
 
 // gradient blocks of the own row, columns 2 r + 4 group .. + 3 of a row per lane
@@ -101,7 +82,7 @@ __device__ inline void store_gradient(const Acc (&acc)[NS], float scale, void *o
 
 // kHalves 2: blocks of 64, whose halves are the blocks of 32 spoken of here (Place)
 template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
-__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>::kQMinWaves)) void attn_small_dq_kernel(bsa_attn_args a, int split) {
+__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>::kQMinWaves)) void attn_small_dq_kernel(bsa_attn_args a, int split, Shares shares) {
   using Shape = BwdShape<Tr::kElem, SBS, NS, kHalves>;
   using T = typename Shape::T;
   using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true, kSome, kHalves>;
@@ -112,12 +93,12 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
   const int wave = first_lane(threadIdx.x >> 6);
   char *lds_k = small_smem + wave * Shape::kQLds, *lds_v = lds_k + T::kBytes;
 
-  const RowOfWave me(a.B, kHalves * a.nq, true, wave, kWaves, split);
+  const RowOfWave me(shares, kHalves, a.B, kHalves * a.nq, true, wave, kWaves, split);
   const int64_t row = me.b * a.nq + me.own / kHalves;  // of the layout
   const int64_t stats = (row * kHalves + me.own % kHalves) * SBS;  // of lse and delta
   const int qi = lane % SBS, kq = lane / SBS;
   W walk;
-  walk.start(a, me.b, me.own, me.there, me.part, split);
+  walk.start(a, me.b, me.own, me.there, me.part, me.parts);
 
   OwnRows<Tr::kElem, SBS, NS, kHalves> qf, gf;
   qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, (int)me.own, lane);
@@ -204,20 +185,24 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
     if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
     now = next;
   }
-  if (split > 1) {
+  if (me.waves > 1) {
     float *mine = reinterpret_cast<float *>(lds_k);
-    if (me.part != 0) leave_partial<NS, kRegs>(dq, mine, lane);
+    if (me.place != 0) leave_partial<NS, kRegs>(dq, mine, lane);
     __syncthreads();
-    if (me.part != 0) return;
-    for (int p = 1; p < split; ++p) add_partial<NS, kRegs>(dq, mine + p * (Shape::kQLds / 4), lane);
+    if (me.place != 0) return;
+    for (int p = 1; p < me.waves; ++p) add_partial<NS, kRegs>(dq, mine + p * (Shape::kQLds / 4), lane);
   }
   if (!me.there) return;
+  if (me.slot >= 0) {  // other workgroups have the rest of the row: attn_small_bwd_merge_kernel adds them up
+    leave_partial<NS, kRegs>(dq, shares.partials + (int64_t)me.slot * Shape::kSlot, lane);
+    return;
+  }
   const late_args_t p = late_args();
   store_gradient<Tr, SBS, NS, kHalves>(dq, p->scale, p->dq, p->pidx_q + row * p->nh, (int)p->nh, p->n_q_blocks, (int)me.own, qi, kq);
 }
 
 template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
-__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>::kKvMinWaves)) void attn_small_dkv_kernel(bsa_attn_args a, int split) {
+__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>::kKvMinWaves)) void attn_small_dkv_kernel(bsa_attn_args a, int split, Shares shares) {
   using Shape = BwdShape<Tr::kElem, SBS, NS, kHalves>;
   using T = typename Shape::T;
   using W = Walk<Tr::kElem, SBS, NS, Shape::NB, false, kSome, kHalves>;
@@ -228,11 +213,11 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
   const int wave = first_lane(threadIdx.x >> 6);
   char *lds = small_smem + wave * Shape::kKvLds;  // per buffer: Q tile, dO tile, lse and delta
 
-  const RowOfWave me(a.B, kHalves * a.nk, false, wave, kWaves, split);
+  const RowOfWave me(shares, kHalves, a.B, kHalves * a.nk, false, wave, kWaves, split);
   const int64_t row = me.b * a.nk + me.own / kHalves;  // of the layout
   const int kj = lane % SBS, kq = lane / SBS;  // key row; which queries of a block this lane's registers hold
   W walk;
-  walk.start(a, me.b, me.own, me.there, me.part, split);
+  walk.start(a, me.b, me.own, me.there, me.part, me.parts);
 
   OwnRows<Tr::kElem, SBS, NS, kHalves> kf, vf;
   kf.load(a.k, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, (int)me.own, lane);
@@ -349,23 +334,58 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
     now = next;
     buf ^= 1;
   }
-  if (split > 1) {
+  if (me.waves > 1) {
     float *mine = reinterpret_cast<float *>(lds);
-    if (me.part != 0) {
+    if (me.place != 0) {
       leave_partial<NS, kRegs>(dk, mine, lane);
       leave_partial<NS, kRegs>(dv, mine + Shape::kPartial / 4, lane);
     }
     __syncthreads();
-    if (me.part != 0) return;
-    for (int p = 1; p < split; ++p) {
+    if (me.place != 0) return;
+    for (int p = 1; p < me.waves; ++p) {
       add_partial<NS, kRegs>(dk, mine + p * (Shape::kKvLds / 4), lane);
       add_partial<NS, kRegs>(dv, mine + p * (Shape::kKvLds / 4) + Shape::kPartial / 4, lane);
     }
   }
   if (!me.there) return;
+  if (me.slot >= 0) {
+    float *out = shares.partials + (int64_t)me.slot * (2 * Shape::kSlot);
+    leave_partial<NS, kRegs>(dk, out, lane);
+    leave_partial<NS, kRegs>(dv, out + Shape::kSlot, lane);
+    return;
+  }
   const late_args_t p = late_args();
   store_gradient<Tr, SBS, NS, kHalves>(dk, p->scale, p->dk, p->pidx_k + row * p->nh, (int)p->nh, p->n_k_blocks, (int)me.own, kj, kq);
   store_gradient<Tr, SBS, NS, kHalves>(dv, 1.f, p->dv, p->pidx_v + row * p->nhv, (int)p->nhv, p->n_v_blocks, (int)me.own, kj, kq);
+}
+
+// The gradients of rows that several workgroups share, one wave each: dQ of the first n_q merges (times the halves), then dK
+// and dV of the others.  A merge is (batch entry, row of the layout, first slot, slots).
+template <typename Tr, int SBS, int NS, int kHalves>
+__global__ __launch_bounds__(64) void attn_small_bwd_merge_kernel(bsa_attn_args a, const int32_t *merges_q, const float *partials_q,
+                                                                  int64_t n_q, const int32_t *merges_kv, const float *partials_kv) {
+  using Shape = BwdShape<Tr::kElem, SBS, NS, kHalves>;
+  constexpr int kRegs = Shape::kRegs;
+  using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
+  const int lane = threadIdx.x, me = lane % SBS, group = lane / SBS, half = blockIdx.x % kHalves;
+  const int64_t m = blockIdx.x / kHalves;
+  const bool is_q = m < n_q;
+  const int32_t *merge = is_q ? merges_q + m * 4 : merges_kv + (m - n_q) * 4;
+  const int64_t row = (int64_t)merge[0] * (is_q ? a.nq : a.nk) + merge[1];
+  const int own = merge[1] * kHalves + half;
+  const int kStep = is_q ? Shape::kSlot : 2 * Shape::kSlot;
+  for (int what = 0; what < (is_q ? 1 : 2); ++what) {  // dQ, or dK and dV
+    const float *part = (is_q ? partials_q : partials_kv) + ((int64_t)merge[2] * kHalves + half) * kStep + what * Shape::kSlot;
+    acc_t acc[NS];
+#pragma unroll
+    for (int h = 0; h < NS; ++h)
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) acc[h][r] = 0.f;
+    for (int s = 0; s < merge[3]; ++s) add_partial<NS, kRegs>(acc, part + (int64_t)s * kHalves * kStep, lane);
+    if (what == 1) store_gradient<Tr, SBS, NS, kHalves>(acc, 1.f, a.dv, a.pidx_v + row * a.nhv, (int)a.nhv, a.n_v_blocks, own, me, group);
+    else if (is_q) store_gradient<Tr, SBS, NS, kHalves>(acc, a.scale, a.dq, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, own, me, group);
+    else store_gradient<Tr, SBS, NS, kHalves>(acc, a.scale, a.dk, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, own, me, group);
+  }
 }
 
 // bias blocks outside the attention layout, and pairs the causal predicate rules out, have no wave that writes them
@@ -375,7 +395,7 @@ __global__ void small_zero_kernel(f32x4 *out, int64_t n) {
 }
 
 template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
-int launch_kind(const bsa_attn_args &a, hipStream_t s) {
+int launch_kind(const bsa_attn_args &a, const bsa_attn_shares *sh_q, const bsa_attn_shares *sh_kv, hipStream_t s) {
   using Shape = BwdShape<Tr::kElem, SBS, NS, kHalves>;
   constexpr int q_lds = Shape::kQLds * kWaves, kv_lds = Shape::kKvLds * kWaves;
   static_assert(q_lds <= 160 * 1024 && kv_lds <= 160 * 1024, "LDS");
@@ -383,54 +403,70 @@ int launch_kind(const bsa_attn_args &a, hipStream_t s) {
   if (int rc = allow_lds(limit_q, &attn_small_dq_kernel<Tr, SBS, NS, kSome, kHalves>, q_lds)) return rc;
   if (int rc = allow_lds(limit_kv, &attn_small_dkv_kernel<Tr, SBS, NS, kSome, kHalves>, kv_lds)) return rc;
   const int64_t q_rows = kHalves * a.nq, k_rows = kHalves * a.nk;  // of a batch entry
-  const int q_split = waves_per_row<Tr>(a.B * q_rows, k_rows, Shape::NB), kv_split = waves_per_row<Tr>(a.B * k_rows, q_rows, Shape::NB);
-  const int64_t q_groups = row_groups(a.B, q_rows, kWaves, q_split), kv_groups = row_groups(a.B, k_rows, kWaves, kv_split);
+  const int q_split = waves_per_row<Tr::kElem>(a.B * q_rows, k_rows, Shape::NB);
+  const int kv_split = waves_per_row<Tr::kElem>(a.B * k_rows, q_rows, Shape::NB);
+  const int64_t q_groups = sh_q ? kHalves * sh_q->n_groups : row_groups(a.B, q_rows, kWaves, q_split);
+  const int64_t kv_groups = sh_kv ? kHalves * sh_kv->n_groups : row_groups(a.B, k_rows, kWaves, kv_split);
   if (!fits_launch(q_groups, kWaves) || !fits_launch(kv_groups, kWaves)) return 1;
+  Shares shares_q{nullptr, nullptr}, shares_kv{nullptr, nullptr};
+  for (const bsa_attn_shares *sh : {sh_q, sh_kv}) {
+    if (!sh) continue;
+    const int64_t need = sh->n_slots * kHalves * Shape::kSlot * 4 * (sh == sh_kv ? 2 : 1);
+    BSA_REQUIRE(need <= sh->scratch_bytes, "bsa_attn_bwd_shares: scratch holds %lld bytes, %lld are needed",
+                (long long)sh->scratch_bytes, (long long)need);
+    (sh == sh_q ? shares_q : shares_kv) = Shares{sh->groups, static_cast<float *>(sh->scratch)};
+  }
   if (a.dbias && a.n_bias_blocks > 0) {
     const int64_t n = a.n_bias_blocks * a.sbs * a.sbs / 4, blocks = cdiv(n, (int64_t)256);
     small_zero_kernel<<<(unsigned)(blocks < 65536 ? blocks : 65536), 256, 0, s>>>(reinterpret_cast<f32x4 *>(a.dbias), n);
     if (int rc = check_launch("small_zero_kernel")) return rc;
   }
   if (a.B * a.nq) {
-    attn_small_dq_kernel<Tr, SBS, NS, kSome, kHalves><<<(unsigned)q_groups, 64 * kWaves, q_lds, s>>>(a, q_split);
+    attn_small_dq_kernel<Tr, SBS, NS, kSome, kHalves><<<(unsigned)q_groups, 64 * kWaves, q_lds, s>>>(a, q_split, shares_q);
     if (int rc = check_launch("attn_small_dq_kernel")) return rc;
   }
   if (a.B * a.nk) {
-    attn_small_dkv_kernel<Tr, SBS, NS, kSome, kHalves><<<(unsigned)kv_groups, 64 * kWaves, kv_lds, s>>>(a, kv_split);
+    attn_small_dkv_kernel<Tr, SBS, NS, kSome, kHalves><<<(unsigned)kv_groups, 64 * kWaves, kv_lds, s>>>(a, kv_split, shares_kv);
     if (int rc = check_launch("attn_small_dkv_kernel")) return rc;
+  }
+  const int64_t q_merges = sh_q ? sh_q->n_merges : 0, kv_merges = sh_kv ? sh_kv->n_merges : 0;
+  if (q_merges + kv_merges > 0) {
+    attn_small_bwd_merge_kernel<Tr, SBS, NS, kHalves><<<(unsigned)((q_merges + kv_merges) * kHalves), 64, 0, s>>>(
+        a, sh_q ? sh_q->merges : nullptr, shares_q.partials, q_merges, sh_kv ? sh_kv->merges : nullptr, shares_kv.partials);
+    if (int rc = check_launch("attn_small_bwd_merge_kernel")) return rc;
   }
   return BSA_OK;
 }
 
 template <typename Tr, int SBS, int NS>
-int launch(const bsa_attn_args &a, hipStream_t s) {
-  return all_slices(a, true) ? launch_kind<Tr, SBS, NS, false, 1>(a, s) : launch_kind<Tr, SBS, NS, true, 1>(a, s);
+int launch(const bsa_attn_args &a, const bsa_attn_shares *sh_q, const bsa_attn_shares *sh_kv, hipStream_t s) {
+  return all_slices(a, true) ? launch_kind<Tr, SBS, NS, false, 1>(a, sh_q, sh_kv, s) : launch_kind<Tr, SBS, NS, true, 1>(a, sh_q, sh_kv, s);
 }
 
 template <typename Tr>
-int dispatch(const bsa_attn_args &a, hipStream_t s) {
+int dispatch(const bsa_attn_args &a, const bsa_attn_shares *sh_q, const bsa_attn_shares *sh_kv, hipStream_t s) {
   const int64_t slices = a.nh > a.nhv ? a.nh : a.nhv;
   if constexpr (Tr::kElem == 4) {
-    if (a.sbs == 64) return slices == 1 ? launch_kind<Tr, 32, 2, false, 2>(a, s) : launch_kind<Tr, 32, 4, false, 2>(a, s);
+    if (a.sbs == 64) return slices == 1 ? launch_kind<Tr, 32, 2, false, 2>(a, sh_q, sh_kv, s) : launch_kind<Tr, 32, 4, false, 2>(a, sh_q, sh_kv, s);
   }
   if (a.sbs == 32) {
     switch (slices) {
-      case 1: return launch<Tr, 32, 1>(a, s);
-      case 2: return launch<Tr, 32, 2>(a, s);
-      case 3: return launch<Tr, 32, 3>(a, s);
-      case 4: return launch<Tr, 32, 4>(a, s);
+      case 1: return launch<Tr, 32, 1>(a, sh_q, sh_kv, s);
+      case 2: return launch<Tr, 32, 2>(a, sh_q, sh_kv, s);
+      case 3: return launch<Tr, 32, 3>(a, sh_q, sh_kv, s);
+      case 4: return launch<Tr, 32, 4>(a, sh_q, sh_kv, s);
     }
     return 1;
   }
   switch (slices) {
-    case 1: return launch<Tr, 16, 1>(a, s);
-    case 2: return launch<Tr, 16, 2>(a, s);
-    case 3: return launch<Tr, 16, 3>(a, s);
-    case 4: return launch<Tr, 16, 4>(a, s);
-    case 5: return launch<Tr, 16, 5>(a, s);
-    case 6: return launch<Tr, 16, 6>(a, s);
-    case 7: return launch<Tr, 16, 7>(a, s);
-    case 8: return launch<Tr, 16, 8>(a, s);
+    case 1: return launch<Tr, 16, 1>(a, sh_q, sh_kv, s);
+    case 2: return launch<Tr, 16, 2>(a, sh_q, sh_kv, s);
+    case 3: return launch<Tr, 16, 3>(a, sh_q, sh_kv, s);
+    case 4: return launch<Tr, 16, 4>(a, sh_q, sh_kv, s);
+    case 5: return launch<Tr, 16, 5>(a, sh_q, sh_kv, s);
+    case 6: return launch<Tr, 16, 6>(a, sh_q, sh_kv, s);
+    case 7: return launch<Tr, 16, 7>(a, sh_q, sh_kv, s);
+    case 8: return launch<Tr, 16, 8>(a, sh_q, sh_kv, s);
   }
   return 1;
 }
@@ -438,9 +474,9 @@ int dispatch(const bsa_attn_args &a, hipStream_t s) {
 }  // namespace
 
 // 1: not covered
-int attn_bwd_small(const bsa_attn_args &a, hipStream_t s) {
+int attn_bwd_small(const bsa_attn_args &a, const bsa_attn_shares *sh_q, const bsa_attn_shares *sh_kv, hipStream_t s) {
   if (!small_applies(a, true)) return 1;
-  return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, s) : a.dtype == BSA_F16 ? dispatch<SF16>(a, s) : dispatch<SF32>(a, s);
+  return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, sh_q, sh_kv, s) : a.dtype == BSA_F16 ? dispatch<SF16>(a, sh_q, sh_kv, s) : dispatch<SF32>(a, sh_q, sh_kv, s);
 }
 
 }  // namespace bsa

@@ -1,5 +1,6 @@
-// Pieces shared by the attention kernels for blocks of 16 and 32 (attn_small_fwd.hip, attn_small_bwd.hip): LDS layout of
-// a block slice, operand fragments, asynchronous copies of block slices, waits, the walk over a list of partner blocks.
+// Pieces shared by the attention kernels for blocks of 16 and 32, and for fp32 blocks of 64 as halves of 32
+// (attn_small_fwd.hip, attn_small_bwd.hip, attn_shares.hip): LDS layout of a block slice, operand fragments, asynchronous
+// copies of block slices, waits, the walk over a list of partner blocks, the order of the rows.
 //
 // A block slice (SBS x SBS elements, 512 bytes to 4 KiB, contiguous in memory) lies row-major in LDS, the 16-byte chunks
 // of a row exchanged by a function of the row.  It is read both ways: rows as they lie (contraction over the head
@@ -134,7 +135,8 @@ __device__ static inline void copy_every_second_kib_to_lds(const char *base, uin
 
 // Where the blocks of the kernels lie in memory.  kHalves 1: a block is a block of the layout.  kHalves 2: a block of the
 // layout (64 x 64) is four of theirs, its head slice two of theirs: block i of a row is half i % 2 of the rows of the layout's
-// block i / 2, slice h the columns from SBS (h % 2) of the layout's slice h / 2.
+// block i / 2, slice h the columns from SBS (h % 2) of the layout's slice h / 2.  A wave has the
+// accumulators that it has for blocks of 32, and a layout twice as many rows to spread over the chip.
 template <int ES, int SBS, int kHalves>
 struct Place {
   static constexpr int kPitch = kHalves * SBS * ES;             // bytes from row to row
@@ -784,14 +786,14 @@ inline bool small_applies(const bsa_attn_args &a, bool backward) {
 //   16384 rows of 64 blocks:    333 / 261 / 280      152 / 166 / 195     76.5 / 89.8 / 126      233 / 249 / 251
 // Up to 512 rows four are best throughout; at 1024 they are for half of the layouts, and at head dimension 128 two are (22.9
 // against 27.7 for every block of a half).  From 8192 rows it depends on the layout, which the rule does not look at:
-// short and causal lists want one wave, long lists of about equal length two.
+// short and causal lists want one wave, long lists of about equal length two.  Uneven lists: attn_shares.hip.
 // fp32: always four, for four partial sums: with two and one, O is 14 and 38 % further from 64 bits, dK and dV of a
 // causal layout 26 and 50 % (1024 keys, sbs 16).  Never more waves than a list of all partners has steps.
-template <typename Tr>
+template <int ES>
 inline int waves_per_row(int64_t rows, int64_t partners, int blocks_per_step) {
   const int64_t steps = cdiv(partners, (int64_t)blocks_per_step);
   const int most = steps >= 3 ? 4 : steps == 2 ? 2 : 1;
-  const int wanted = Tr::kElem == 4 || rows <= 512 ? 4 : rows <= 8192 ? 2 : 1;
+  const int wanted = ES == 4 || rows <= 512 ? 4 : rows <= 8192 ? 2 : 1;
   return wanted < most ? wanted : most;
 }
 
@@ -805,36 +807,98 @@ inline int waves_per_row(int64_t rows, int64_t partners, int blocks_per_step) {
 // against 156 / 198; two long columns among short ones in 13 entries (dK / dV, where XCDs also differed in work): 97 against
 // 67; lists of equal lengths: the same.  Rows of one entry on several XCDs where whole entries would do: 5 to 14 % slower
 // (their partner blocks pass several L2s).  List lengths are not looked at: where the first query blocks have the longest lists
-// (global rows of a BigBird layout) these start last.
+// (global rows of a BigBird layout) these start last, unless the launch has shares (attn_shares.hip).
 // Entries of fewer than eight rows are taken as they are: with eight places each, most of them empty, an entry of one row
 // (64 key blocks, 4096 entries, head dimension 64, sbs 32, fp32, forward) took 3.17 ms, now 0.77; bf16 0.72, now 0.38.
+// Item `item` of XCD `xcd` in that order; whether the row is there.
+__host__ __device__ inline bool row_of_item(uint32_t xcd, uint32_t item, int64_t batches, int64_t rows_per_batch, bool last_first,
+                                            int64_t &b, int64_t &own) {
+  // up to eight rows of every entry: as many items for each of an XCD's own entries, one for each shared one (the last of all)
+  const uint32_t near = rows_per_batch < 8 ? (uint32_t)rows_per_batch : 8, entries = (uint32_t)(batches >> 3);
+  const uint32_t own_items = entries * near, items = own_items + ((uint32_t)batches & 7);
+  const uint32_t eight = item / items, rest = item - eight * items;
+  if (rest < own_items) {
+    const uint32_t entry = near == 8 ? rest >> 3 : rest / near;
+    b = (int64_t)xcd * entries + entry;
+    own = (int64_t)eight * 8 + (rest - entry * near);
+  } else {
+    b = (int64_t)entries * 8 + (rest - own_items);
+    own = (int64_t)eight * 8 + ((xcd + rest + eight) & 7);
+  }
+  const bool there = own < rows_per_batch;
+  if (!there) b = own = 0;
+  if (last_first) own = rows_per_batch - 1 - own;
+  return there;
+}
+
+// Items of each XCD
+inline int64_t row_items(int64_t batches, int64_t rows_per_batch) {
+  return cdiv(rows_per_batch, (int64_t)8) * ((batches >> 3) * (rows_per_batch < 8 ? rows_per_batch : 8) + (batches & 7));
+}
+
+// What a launch knows of the shares of its rows (bsa_attn_shares); groups NULL: `split` waves for every row
+struct Shares {
+  const int32_t *groups;
+  float *partials;  // one per slot (and half, where blocks are halves of the layout's)
+};
+
 struct RowOfWave {
   int64_t b, own;
-  int part;
+  int part, parts;   // this wave walks every parts-th entry of the row's list, from entry `part` on
+  int place, waves;  // among the waves of this workgroup that share the row
+  int slot;          // the workgroup's sum is one of several: where it goes; -1: it is the row's
   bool there;
-  __device__ inline RowOfWave(int64_t batches, int64_t rows_per_batch, bool last_first, int wave, int waves, int split) {
-    const uint32_t xcd = blockIdx.x & 7, item = (blockIdx.x >> 3) * (waves / split) + wave / split;
-    part = wave % split;
-    // up to eight rows of every entry: as many items for each of an XCD's own entries, one for each shared one (the last of all)
-    const uint32_t near = rows_per_batch < 8 ? (uint32_t)rows_per_batch : 8, entries = (uint32_t)(batches >> 3);
-    const uint32_t own_items = entries * near, items = own_items + ((uint32_t)batches & 7);
-    const uint32_t eight = item / items, rest = item - eight * items;
-    if (rest < own_items) {
-      const uint32_t entry = near == 8 ? rest >> 3 : rest / near;
-      b = (int64_t)xcd * entries + entry;
-      own = (int64_t)eight * 8 + (rest - entry * near);
+  __device__ inline RowOfWave(const Shares &shares, int halves, int64_t batches, int64_t rows_per_batch, bool last_first, int wave,
+                              int waves_of_group, int split) {
+    if (shares.groups) {
+      // groups of an XCD are BSA_SHARE_XCDS apart, also with two halves each
+      const uint32_t xcd = blockIdx.x & 7, turn = blockIdx.x >> 3;
+      const int32_t *g = shares.groups + (int64_t)((turn / halves) * 8 + xcd) * BSA_SHARE_INTS;
+      own = first_lane(g[wave]);
+      b = first_lane(g[4 + wave]);
+      there = own >= 0 && own < rows_per_batch / halves && b >= 0 && b < batches;
+      if (!there) b = own = 0;
+      own = own * halves + turn % halves;
+      parts = first_lane(g[9]);
+      waves = parts < waves_of_group ? parts : waves_of_group;
+      place = wave % waves;
+      part = first_lane(g[8]) + place;
+      const int s = first_lane(g[10]);
+      slot = s < 0 ? -1 : s * halves + (int)(turn % halves);
     } else {
-      b = (int64_t)entries * 8 + (rest - own_items);
-      own = (int64_t)eight * 8 + ((xcd + rest + eight) & 7);
+      part = place = wave % split;
+      parts = waves = split;
+      slot = -1;
+      there = row_of_item(blockIdx.x & 7, (blockIdx.x >> 3) * (waves_of_group / split) + wave / split, batches, rows_per_batch,
+                          last_first, b, own);
     }
-    there = own < rows_per_batch;
-    if (!there) b = own = 0;
-    if (last_first) own = rows_per_batch - 1 - own;
   }
 };
+
+// Sums of a row that several workgroups share: accumulators as they lie, 16 bytes per lane
+template <int NS, int kRegs, typename Acc, typename Float>
+__device__ static inline void leave_partial(const Acc (&acc)[NS], Float *mine, int lane) {
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
+#pragma unroll
+    for (int r = 0; r < kRegs; r += 4)
+      *reinterpret_cast<f32x4 *>(mine + ((h * kRegs + r) / 4 * 64 + lane) * 4) =
+          f32x4{acc[h][r], acc[h][r + 1], acc[h][r + 2], acc[h][r + 3]};
+}
+template <int NS, int kRegs, typename Acc>
+__device__ static inline void add_partial(Acc (&acc)[NS], const float *other, int lane) {
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
+#pragma unroll
+    for (int r = 0; r < kRegs; r += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4 *>(other + ((h * kRegs + r) / 4 * 64 + lane) * 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[h][r + i] += v[i];
+    }
+}
+
 inline int64_t row_groups(int64_t batches, int64_t rows_per_batch, int waves, int split) {
-  const int64_t items = cdiv(rows_per_batch, (int64_t)8) * ((batches >> 3) * (rows_per_batch < 8 ? rows_per_batch : 8) + (batches & 7));
-  return cdiv(items, (int64_t)(waves / split)) * 8;
+  return cdiv(row_items(batches, rows_per_batch), (int64_t)(waves / split)) * 8;
 }
 // a launch has fewer than 2^32 threads; what is more goes to the kernels that give a workgroup a row
 inline bool fits_launch(int64_t groups, int waves) { return groups * waves * 64 < ((int64_t)1 << 32); }

@@ -20,7 +20,8 @@
 // prompts of 1032 to 2064 tokens, sbs 16, bf16, causal: 0.54 -> 0.044 ms.  fp32, where the products take eight times as
 // long and hide the rest: 8 x 2048 queries, half of the blocks, head dimension 64: 0.089 -> 0.054 ms (80 TFLOP/s, half
 // of the fp32 matrix-core peak; 512 lists of 32 +- 4 blocks cut in four fill the chip once, so the launch waits for the
-// longest).
+// longest).  fp32 blocks of 64, whose halves walk alone like blocks of 32: 34 sequences of 480 to 960, head dimension 64,
+// causal: 0.100 -> 0.041 ms.
 //
 // Score pipeline (log2 domain), in the reference's order (blksprs/ops/flash_attention.py:1058-1224): scale * q k^T,
 // + bias, native causal predicate, explicit mask; probabilities are rounded to the operand type before they multiply
@@ -47,18 +48,59 @@ struct FwdShape {
   static constexpr int kRegs = SBS == 32 ? 16 : 4;              // accumulator registers per block
   // K tile, V tile; at the end the partial output of a wave that shares a query block with others
   static constexpr int kPartial = SBS * SBS * NS * 4;
+  static constexpr int kSlot = SBS * SBS * NS + 2 * SBS;  // floats of a slot of the scratch: O, then (m, l) of every query
   static constexpr int kLds = (2 * T::kBytes > kPartial ? 2 * T::kBytes : kPartial) + 512;
   static constexpr int kMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS <= 2 ? 4 : 2) : (NS <= 4 ? 4 : 3);
 };
 
-// split: 1, 2 or 4 waves share one query block, each walking every split-th entry of its key list
+// (m_i, l_i, oacc) of a row and those of another part of its list, scaled to the common maximum and added up
+template <int NS, int kRegs, typename Acc>
+__device__ inline void merge_partial(Acc (&oacc)[NS], float &m_i, float &l_i, const float *other, float m_o, float l_o, int lane) {
+  const float m_new = fmaxf(m_i, m_o);
+  const bool nothing = m_new == -INFINITY;
+  const float s_i = nothing ? 1.f : __builtin_amdgcn_exp2f(m_i - m_new);
+  const float s_o = nothing ? 1.f : __builtin_amdgcn_exp2f(m_o - m_new);
+  l_i = l_i * s_i + l_o * s_o;
+  m_i = m_new;
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
+#pragma unroll
+    for (int r = 0; r < kRegs; r += 4) {
+      const f32x4 o4 = *reinterpret_cast<const f32x4 *>(other + ((h * kRegs + r) / 4 * 64 + lane) * 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) oacc[h][r + i] = oacc[h][r + i] * s_i + o4[i] * s_o;
+    }
+}
+
+// output blocks and lse of query block `own`, which belongs to `row` of the layout
+template <typename Tr, int SBS, int NS, int kHalves, typename Acc>
+__device__ inline void store_output(const Acc (&oacc)[NS], float m_i, float l_i, int64_t row, int own, int qi, int kq) {
+  constexpr int kRegs = SBS == 32 ? 16 : 4;
+  const late_args_t p = late_args();
+  const int nhv = (int)p->nhv;
+  const float inv_l = (l_i != 0.f) ? 1.f / l_i : 0.f;
+#pragma unroll
+  for (int h = 0; h < NS; ++h) {
+    if (h / kHalves >= nhv) break;
+    const int64_t po = p->pidx_o[row * nhv + h / kHalves];
+    if (po < 0 || po >= p->n_o_blocks) continue;
+    char *out = static_cast<char *>(p->o) + Place<Tr::kElem, SBS, kHalves>::row(po, own, qi, h);
+#pragma unroll
+    for (int r = 0; r < kRegs; r += 4)  // columns 2 r + 4 kq .. + 3 of a row per lane
+      store4<Tr>(out + (2 * r + 4 * kq) * Tr::kElem, oacc[h][r] * inv_l, oacc[h][r + 1] * inv_l, oacc[h][r + 2] * inv_l,
+                 oacc[h][r + 3] * inv_l);
+  }
+  if (kq == 0) p->lse[(row * kHalves + own % kHalves) * SBS + qi] = (l_i != 0.f) ? m_i + log2f(l_i) : -INFINITY;
+}
+
+// split: 1, 2 or 4 waves share one query block, each walking every split-th entry of its key list, unless `shares` says how
+// many do, of how many workgroups
 // kHalves 2: blocks of 64, whose halves are the blocks of 32 spoken of here (Place)
 template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
-__global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>::kMinWaves)) void attn_small_fwd_kernel(bsa_attn_args a, int split) {
+__global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>::kMinWaves)) void attn_small_fwd_kernel(bsa_attn_args a, int split, Shares shares) {
   using Shape = FwdShape<Tr::kElem, SBS, NS, kHalves>;
   using T = typename Shape::T;
   using W = Walk<Tr::kElem, SBS, NS, Shape::NB, true, kSome, kHalves>;
-  using P = Place<Tr::kElem, SBS, kHalves>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
@@ -66,11 +108,11 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
   const int wave = first_lane(threadIdx.x >> 6);
   char *lds_k = small_smem + wave * Shape::kLds, *lds_v = lds_k + T::kBytes;
 
-  const RowOfWave me(a.B, kHalves * a.nq, true, wave, kWaves, split);
+  const RowOfWave me(shares, kHalves, a.B, kHalves * a.nq, true, wave, kWaves, split);
   const int64_t row = me.b * a.nq + me.own / kHalves;  // of the layout
   const int qi = lane % SBS, kq = lane / SBS;  // query row; which keys of a block this lane's registers hold
   W walk;
-  walk.start(a, me.b, me.own, me.there, me.part, split);
+  walk.start(a, me.b, me.own, me.there, me.part, me.parts);
 
   OwnRows<Tr::kElem, SBS, NS, kHalves> qf;
   qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, (int)me.own, lane);
@@ -158,105 +200,109 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
 
   // ---- epilogue
   l_i = row_sum<SBS>(l_i);
-  if (split > 1) {
+  if (me.waves > 1) {
     // every wave leaves (m, l, O) of its part; the first wave of a query block scales them to the common maximum and
     // adds them up, in order
     float *mine = reinterpret_cast<float *>(lds_k);
-    if (me.part != 0) {
-#pragma unroll
-      for (int h = 0; h < NS; ++h)
-#pragma unroll
-        for (int r = 0; r < kRegs; r += 4)
-          *reinterpret_cast<f32x4 *>(mine + ((h * kRegs + r) / 4 * 64 + lane) * 4) =
-              f32x4{oacc[h][r], oacc[h][r + 1], oacc[h][r + 2], oacc[h][r + 3]};
-      if (kq == 0) {
-        mine[Shape::kLds / 4 - 128 + 2 * qi] = m_i;
-        mine[Shape::kLds / 4 - 128 + 2 * qi + 1] = l_i;
-      }
+    constexpr int kStats = Shape::kLds / 4 - 128;
+    if (me.place != 0) {
+      leave_partial<NS, kRegs>(oacc, mine, lane);
+      if (kq == 0) mine[kStats + 2 * qi] = m_i, mine[kStats + 2 * qi + 1] = l_i;
     }
     __syncthreads();
-    if (me.part != 0) return;
-    for (int p = 1; p < split; ++p) {
+    if (me.place != 0) return;
+    for (int p = 1; p < me.waves; ++p) {
       const float *other = mine + p * (Shape::kLds / 4);
-      const float m_o = other[Shape::kLds / 4 - 128 + 2 * qi], l_o = other[Shape::kLds / 4 - 128 + 2 * qi + 1];
-      const float m_new = fmaxf(m_i, m_o);
-      const bool nothing = m_new == -INFINITY;
-      const float s_i = nothing ? 1.f : __builtin_amdgcn_exp2f(m_i - m_new);
-      const float s_o = nothing ? 1.f : __builtin_amdgcn_exp2f(m_o - m_new);
-      l_i = l_i * s_i + l_o * s_o;
-      m_i = m_new;
-#pragma unroll
-      for (int h = 0; h < NS; ++h)
-#pragma unroll
-        for (int r = 0; r < kRegs; r += 4) {
-          const f32x4 o4 = *reinterpret_cast<const f32x4 *>(other + ((h * kRegs + r) / 4 * 64 + lane) * 4);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) oacc[h][r + i] = oacc[h][r + i] * s_i + o4[i] * s_o;
-        }
+      merge_partial<NS, kRegs>(oacc, m_i, l_i, other, other[kStats + 2 * qi], other[kStats + 2 * qi + 1], lane);
     }
   }
   if (!me.there) return;
-  const late_args_t p = late_args();
-  const int nhv = (int)p->nhv;
-  const float inv_l = (l_i != 0.f) ? 1.f / l_i : 0.f;
-#pragma unroll
-  for (int h = 0; h < NS; ++h) {
-    if (h / kHalves >= nhv) break;
-    const int64_t po = p->pidx_o[row * nhv + h / kHalves];
-    if (po < 0 || po >= p->n_o_blocks) continue;
-    char *out = static_cast<char *>(p->o) + P::row(po, (int)me.own, qi, h);
-#pragma unroll
-    for (int r = 0; r < kRegs; r += 4)  // columns 2 r + 4 kq .. + 3 of a row per lane
-      store4<Tr>(out + (2 * r + 4 * kq) * Tr::kElem, oacc[h][r] * inv_l, oacc[h][r + 1] * inv_l,
-                 oacc[h][r + 2] * inv_l, oacc[h][r + 3] * inv_l);
+  if (me.slot >= 0) {  // other workgroups have the rest of the row: attn_small_fwd_merge_kernel adds them up
+    float *out = shares.partials + (int64_t)me.slot * Shape::kSlot;
+    leave_partial<NS, kRegs>(oacc, out, lane);
+    if (kq == 0) out[Shape::kSlot - 2 * SBS + 2 * qi] = m_i, out[Shape::kSlot - 2 * SBS + 2 * qi + 1] = l_i;
+    return;
   }
-  if (kq == 0) p->lse[(row * kHalves + me.own % kHalves) * SBS + qi] = (l_i != 0.f) ? m_i + log2f(l_i) : -INFINITY;
+  store_output<Tr, SBS, NS, kHalves>(oacc, m_i, l_i, row, (int)me.own, qi, kq);
+}
+
+// The sums of query blocks that several workgroups share, one wave each: merges[m] is (batch entry, query block of the layout,
+// first slot, slots).
+template <typename Tr, int SBS, int NS, int kHalves>
+__global__ __launch_bounds__(64) void attn_small_fwd_merge_kernel(bsa_attn_args a, const int32_t *merges, const float *partials) {
+  using Shape = FwdShape<Tr::kElem, SBS, NS, kHalves>;
+  constexpr int kRegs = Shape::kRegs;
+  using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
+  const int lane = threadIdx.x, qi = lane % SBS, kq = lane / SBS, half = blockIdx.x % kHalves;
+  const int32_t *merge = merges + (int64_t)(blockIdx.x / kHalves) * 4;
+  const int64_t row = (int64_t)merge[0] * a.nq + merge[1];
+  const float *part = partials + ((int64_t)merge[2] * kHalves + half) * Shape::kSlot;
+  acc_t oacc[NS];
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
+#pragma unroll
+    for (int r = 0; r < kRegs; ++r) oacc[h][r] = 0.f;
+  float m_i = -INFINITY, l_i = 0.f;
+  for (int s = 0; s < merge[3]; ++s, part += kHalves * Shape::kSlot)
+    merge_partial<NS, kRegs>(oacc, m_i, l_i, part, part[Shape::kSlot - 2 * SBS + 2 * qi], part[Shape::kSlot - 2 * SBS + 2 * qi + 1],
+                             lane);
+  store_output<Tr, SBS, NS, kHalves>(oacc, m_i, l_i, row, merge[1] * kHalves + half, qi, kq);
 }
 
 template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
-int launch_kind(const bsa_attn_args &a, hipStream_t s) {
+int launch_kind(const bsa_attn_args &a, const bsa_attn_shares *sh, hipStream_t s) {
   using Shape = FwdShape<Tr::kElem, SBS, NS, kHalves>;
   const int64_t rows = kHalves * a.nq;  // of a batch entry
-  const int split = waves_per_row<Tr>(a.B * rows, kHalves * a.nk, Shape::NB);
-  const int64_t groups = row_groups(a.B, rows, kWaves, split);
+  const int split = waves_per_row<Tr::kElem>(a.B * rows, kHalves * a.nk, Shape::NB);
+  const int64_t groups = sh ? kHalves * sh->n_groups : row_groups(a.B, rows, kWaves, split);
   if (!fits_launch(groups, kWaves)) return 1;
   constexpr int lds = Shape::kLds * kWaves;
   static_assert(lds <= 160 * 1024, "LDS");
   static LdsLimit limit;
   if (int rc = allow_lds(limit, &attn_small_fwd_kernel<Tr, SBS, NS, kSome, kHalves>, lds)) return rc;
-  attn_small_fwd_kernel<Tr, SBS, NS, kSome, kHalves><<<(unsigned)groups, 64 * kWaves, lds, s>>>(a, split);
-  return check_launch("attn_small_fwd_kernel");
+  Shares shares{nullptr, nullptr};
+  if (sh) {
+    const int64_t need = sh->n_slots * kHalves * Shape::kSlot * 4;
+    BSA_REQUIRE(need <= sh->scratch_bytes, "bsa_attn_fwd_shares: scratch holds %lld bytes, %lld are needed",
+                (long long)sh->scratch_bytes, (long long)need);
+    shares = Shares{sh->groups, static_cast<float *>(sh->scratch)};
+  }
+  attn_small_fwd_kernel<Tr, SBS, NS, kSome, kHalves><<<(unsigned)groups, 64 * kWaves, lds, s>>>(a, split, shares);
+  if (int rc = check_launch("attn_small_fwd_kernel")) return rc;
+  if (!sh || sh->n_merges == 0) return BSA_OK;
+  attn_small_fwd_merge_kernel<Tr, SBS, NS, kHalves><<<(unsigned)(sh->n_merges * kHalves), 64, 0, s>>>(a, sh->merges, shares.partials);
+  return check_launch("attn_small_fwd_merge_kernel");
 }
 
 template <typename Tr, int SBS, int NS>
-int launch(const bsa_attn_args &a, hipStream_t s) {
-  return all_slices(a, false) ? launch_kind<Tr, SBS, NS, false, 1>(a, s) : launch_kind<Tr, SBS, NS, true, 1>(a, s);
+int launch(const bsa_attn_args &a, const bsa_attn_shares *sh, hipStream_t s) {
+  return all_slices(a, false) ? launch_kind<Tr, SBS, NS, false, 1>(a, sh, s) : launch_kind<Tr, SBS, NS, true, 1>(a, sh, s);
 }
 
 template <typename Tr>
-int dispatch(const bsa_attn_args &a, hipStream_t s) {
+int dispatch(const bsa_attn_args &a, const bsa_attn_shares *sh, hipStream_t s) {
   const int64_t slices = a.nh > a.nhv ? a.nh : a.nhv;
   if constexpr (Tr::kElem == 4) {
-    if (a.sbs == 64) return slices == 1 ? launch_kind<Tr, 32, 2, false, 2>(a, s) : launch_kind<Tr, 32, 4, false, 2>(a, s);
+    if (a.sbs == 64) return slices == 1 ? launch_kind<Tr, 32, 2, false, 2>(a, sh, s) : launch_kind<Tr, 32, 4, false, 2>(a, sh, s);
   }
   if (a.sbs == 32) {
     switch (slices) {
-      case 1: return launch<Tr, 32, 1>(a, s);
-      case 2: return launch<Tr, 32, 2>(a, s);
-      case 3: return launch<Tr, 32, 3>(a, s);
-      case 4: return launch<Tr, 32, 4>(a, s);
+      case 1: return launch<Tr, 32, 1>(a, sh, s);
+      case 2: return launch<Tr, 32, 2>(a, sh, s);
+      case 3: return launch<Tr, 32, 3>(a, sh, s);
+      case 4: return launch<Tr, 32, 4>(a, sh, s);
     }
     return 1;
   }
   switch (slices) {
-    case 1: return launch<Tr, 16, 1>(a, s);
-    case 2: return launch<Tr, 16, 2>(a, s);
-    case 3: return launch<Tr, 16, 3>(a, s);
-    case 4: return launch<Tr, 16, 4>(a, s);
-    case 5: return launch<Tr, 16, 5>(a, s);
-    case 6: return launch<Tr, 16, 6>(a, s);
-    case 7: return launch<Tr, 16, 7>(a, s);
-    case 8: return launch<Tr, 16, 8>(a, s);
+    case 1: return launch<Tr, 16, 1>(a, sh, s);
+    case 2: return launch<Tr, 16, 2>(a, sh, s);
+    case 3: return launch<Tr, 16, 3>(a, sh, s);
+    case 4: return launch<Tr, 16, 4>(a, sh, s);
+    case 5: return launch<Tr, 16, 5>(a, sh, s);
+    case 6: return launch<Tr, 16, 6>(a, sh, s);
+    case 7: return launch<Tr, 16, 7>(a, sh, s);
+    case 8: return launch<Tr, 16, 8>(a, sh, s);
   }
   return 1;
 }
@@ -264,10 +310,10 @@ int dispatch(const bsa_attn_args &a, hipStream_t s) {
 }  // namespace
 
 // 1: not covered
-int attn_fwd_small(const bsa_attn_args &a, hipStream_t s) {
+int attn_fwd_small(const bsa_attn_args &a, const bsa_attn_shares *sh, hipStream_t s) {
   if (!small_applies(a, false)) return 1;
   if (a.B * a.nq == 0) return BSA_OK;
-  return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, s) : a.dtype == BSA_F16 ? dispatch<SF16>(a, s) : dispatch<SF32>(a, s);
+  return a.dtype == BSA_BF16 ? dispatch<SBf16>(a, sh, s) : a.dtype == BSA_F16 ? dispatch<SF16>(a, sh, s) : dispatch<SF32>(a, sh, s);
 }
 
 }  // namespace bsa

@@ -333,12 +333,78 @@ class _Tables:
 
     _NAMES = ("n_sparse_blocks_o", "packed_indices_q", "packed_indices_k", "packed_indices_v", "packed_indices_o",
               "packed_indices_mask", "packed_indices_bias", "key_offsets_i32", "key_indices_i32",
-              "query_offsets_i32", "query_indices_i32", "group_offsets", "group_records", "group_size")
-    __slots__ = _NAMES
+              "query_offsets_i32", "query_indices_i32", "group_offsets", "group_records", "group_size",
+              "max_keys_per_query", "max_queries_per_key")
+    __slots__ = (*_NAMES, "shares")
 
     def __init__(self, cache: dict):
         for name in self._NAMES:
             setattr(self, name, cache.get(name))
+        self.shares = {}  # (block size, dtype, backward) -> shares of the query rows, of the key rows, added on demand
+
+
+class _Shares:
+    """Which waves share the rows of an uneven attention layout (``bsa_attn_shares``); depends on the layout, the block
+    size and the dtype only.  The scratch is a call's own."""
+
+    __slots__ = ("groups", "merges", "n_groups", "n_merges", "n_slots", "scratch_bytes", "argument")
+
+    def __init__(self, groups, merges, n_groups, n_merges, n_slots, scratch_bytes):
+        self.groups, self.merges = groups, merges
+        self.n_groups, self.n_merges, self.n_slots = n_groups, n_merges, n_slots
+        self.scratch_bytes = scratch_bytes  # of a forward pass, of dQ, of dK and dV
+        self.argument = _capi.AttnShares(groups.data_ptr(), merges.data_ptr(), n_groups, n_merges, n_slots, 0, 0)
+
+    def struct(self, what: int, device):
+        """``(argument, scratch tensor)`` for one call; the tensor has to live until the call is enqueued."""
+        size = self.scratch_bytes[what]
+        if size == 0:
+            return self.argument, None  # without slots nothing in it differs between calls
+        scratch = torch.empty(size, dtype=torch.uint8, device=device)
+        return _capi.AttnShares(self.argument.groups, self.argument.merges, self.n_groups, self.n_merges, self.n_slots,
+                                scratch.data_ptr(), size), scratch
+
+
+def _row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool) -> tuple["_Shares | None", "_Shares | None"]:
+    """Shares of the query rows and, for a backward pass, of the key rows; ``None`` where the layout is even enough."""
+    shares = meta.tables.shares.get((meta.sbs, dtype, backward))
+    return _build_row_shares(meta, dtype, device, backward) if shares is None else shares
+
+
+def _build_row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool):
+    """Builds the shares at the first call that needs them, with one wait of the host for their sizes: they are complete
+    when that call returns, whatever stream reads them next.  A call under graph capture may not wait: it goes without."""
+    tables, lib = meta.tables, _capi.load()
+    a = _capi.AttnArgs()
+    a.B, a.nq, a.nk, a.nh, a.nhv = meta.dims
+    a.sbs, a.dtype = meta.sbs, _capi.DTYPE_CODES[dtype]
+    a.key_offsets, a.query_offsets = tables.key_offsets_i32.data_ptr(), tables.query_offsets_i32.data_ptr()
+    piece, max_groups, max_merges = _capi.c_int64(), _capi.c_int64(), _capi.c_int64()
+    shares, wanted = [None, None], []
+    for key_rows in (0, 1) if backward else (0,):
+        longest = tables.max_queries_per_key if key_rows else tables.max_keys_per_query
+        _capi.check(lib.bsa_attn_shares_piece(ctypes.byref(a), key_rows, tables.key_indices_i32.numel(), int(longest),
+                                              ctypes.byref(piece), ctypes.byref(max_groups), ctypes.byref(max_merges)),
+                    "bsa_attn_shares_piece")
+        if piece.value:
+            wanted.append((key_rows, piece.value, max_groups.value, max_merges.value))
+    if wanted:
+        if torch.cuda.is_current_stream_capturing():
+            return None, None
+        stats = torch.zeros((len(wanted), 3), dtype=torch.int64, device=device)
+        built = []
+        with _capi.on_device(device):
+            for number, (key_rows, size, most_groups, most_merges) in enumerate(wanted):
+                groups = torch.empty((most_groups, _capi.SHARE_INTS), dtype=torch.int32, device=device)
+                merges = torch.empty((most_merges, 4), dtype=torch.int32, device=device)
+                _capi.call("bsa_attn_shares_build", ctypes.byref(a), key_rows, size, most_groups, most_merges,
+                           groups.data_ptr(), merges.data_ptr(), stats[number].data_ptr(), _capi.stream(device))
+                built.append((groups, merges))
+        for (key_rows, *_), (groups, merges), (per_xcd, n_merges, n_slots) in zip(wanted, built, stats.tolist()):
+            scratch = [lib.bsa_attn_shares_scratch_bytes(ctypes.byref(a), what, n_slots) for what in range(3)]
+            shares[key_rows] = _Shares(groups, merges, 8 * per_xcd, n_merges, n_slots, scratch)
+    tables.shares[(meta.sbs, dtype, backward)] = tuple(shares)
+    return tuple(shares)
 
 
 _PRUNE_AT_ONCE_BLOCKS = 32768  # active blocks of the attention layout from which dead pairs are listed at once
@@ -423,7 +489,7 @@ def _mask_facts(layout_cache: dict, attention_layout: Tensor, mask: Tensor | Non
 class _Meta:
     """Everything the kernels need besides the differentiable tensors."""
 
-    __slots__ = ("tables", "dims", "sbs", "scale", "has_bias", "facts", "o_rows_whole")
+    __slots__ = ("tables", "dims", "sbs", "scale", "has_bias", "facts", "o_rows_whole", "shares")
 
 
 def _fill_args(meta: "_Meta", q, k, v, bias, mask, causal_lengths) -> _capi.AttnArgs:
@@ -475,7 +541,11 @@ def _forward_launch(q, k, v, bias, mask, causal_lengths, meta: "_Meta"):
     args = _fill_args(meta, q, k, v, bias, mask, causal_lengths)
     args.o, args.lse = _capi.ptr(out), _capi.ptr(lse)
     with _capi.on_device(q.device):
-        _capi.call("bsa_attn_fwd", ctypes.byref(args), _capi.stream(q.device))
+        if meta.shares[0] is None:
+            _capi.call("bsa_attn_fwd", ctypes.byref(args), _capi.stream(q.device))
+        else:
+            shares, scratch = meta.shares[0].struct(0, q.device)
+            _capi.call("bsa_attn_fwd_shares", ctypes.byref(args), ctypes.byref(shares), _capi.stream(q.device))
     return out, lse
 
 
@@ -538,6 +608,12 @@ class _FlashAttention(torch.autograd.Function):
                 _capi.call("bsa_attn_bwd", ctypes.byref(args), stream)
             if facts is not None and not args.bwd_scratch_ready and not torch.cuda.is_current_stream_capturing():
                 facts.bwd_scratch, facts.bwd_stream = scratch, stream
+        elif meta.shares[0] is not None or meta.shares[1] is not None:
+            structs = [(None, None) if shares is None else shares.struct(what, q.device)
+                       for what, shares in zip((1, 2), meta.shares)]
+            with _capi.on_device(q.device):
+                _capi.call("bsa_attn_bwd_shares", ctypes.byref(args),
+                           *(None if struct is None else ctypes.byref(struct) for struct, _ in structs), stream)
         else:
             with _capi.on_device(q.device):
                 _capi.call("bsa_attn_bwd", ctypes.byref(args), stream)
@@ -710,6 +786,7 @@ def flash_attention(q: BlksprsTensor, sparsity_layout_q: Tensor,
 
     needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad
                                               or (attention_bias is not None and attention_bias.requires_grad))
+    meta.shares = _row_shares(meta, q.dtype, q.device, needs_grad)
     if not needs_grad:
         # nothing to differentiate: the launch itself, without the autograd machinery around it
         return BlksprsTensor.wrap(_forward_launch(q, k, v, attention_bias, mask_bytes, lengths, meta)[0])

@@ -485,12 +485,50 @@ size_t bsa_attn_bwd_scratch_bytes(int64_t B, int64_t nq, int64_t nk, int64_t n_l
 size_t bsa_attn_bwd_ds_bytes(int64_t n_layout_blocks, int32_t sbs);
 
 /*
+ * Optional shares of the rows of an uneven attention layout, for blocks of 16 and 32 and fp32 blocks of 64 (head dimensions up
+ * to 128; the other kernels ignore them): which rows each workgroup takes, and how many waves share a row, by the length of
+ * its list.  Without them every row gets as many waves and the launch waits for its longest list.  No counterpart in the
+ * reference, whose programs walk a row each (blksprs/ops/flash_attention.py:1058-1175).
+ */
+typedef struct bsa_attn_shares {
+  const int32_t *groups; /* n_groups * BSA_SHARE_INTS: row of each of four waves (-1: none), its batch entry, first part,
+                          * parts of the row, slot of the sum (-1: the row's own output), 0 */
+  const int32_t *merges; /* n_merges * 4: batch entry, row, first slot, number of slots */
+  int64_t n_groups, n_merges, n_slots;
+  void *scratch; /* bsa_attn_shares_scratch_bytes(...) bytes, 16-byte aligned; carries nothing from one call to the next */
+  int64_t scratch_bytes;
+} bsa_attn_shares;
+
+#define BSA_SHARE_INTS 12
+
+/*
+ * Whether shares pay for the query rows (key_rows 0: forward and dQ) or key rows (1: dK and dV) of a layout with n_entries active
+ * blocks, at most `longest` in one row: *piece is 0 if not, else the number that bsa_attn_shares_build takes, and *max_groups and
+ * *max_merges the sizes of its tables.  Reads B, nq, nk, nh, nhv, sbs and dtype of args.  Host only.
+ */
+int bsa_attn_shares_piece(const bsa_attn_args *args, int key_rows, int64_t n_entries, int64_t longest, int64_t *piece,
+                          int64_t *max_groups, int64_t *max_merges);
+/*
+ * Builds the tables on the device from key_offsets (query_offsets for key rows).  stats: three int64 on the device, zeros before the
+ * call; afterwards the groups of an XCD (n_groups is eight times that), n_merges and n_slots, to be read by the caller.  At most 65536 rows.
+ */
+int bsa_attn_shares_build(const bsa_attn_args *args, int key_rows, int64_t piece, int64_t max_groups, int64_t max_merges,
+                          int32_t *groups, int32_t *merges, int64_t *stats, bsa_stream_t stream);
+/* Size in bytes of bsa_attn_shares.scratch for n_slots slots; what: 0 forward, 1 dQ (both of query rows), 2 dK and dV. */
+size_t bsa_attn_shares_scratch_bytes(const bsa_attn_args *args, int what, int64_t n_slots);
+/* bsa_attn_fwd with shares of the query rows (NULL: none) */
+int bsa_attn_fwd_shares(const bsa_attn_args *args, const bsa_attn_shares *shares, bsa_stream_t stream);
+
+/*
  * dq, dk, dv (and dbias) from the saved lse.  Replaces
  * _FlashAttentionAutograd.backward and its three kernels
  * (blksprs/ops/flash_attention.py:505-787, :1228-1735).  Every block of dq, dk,
  * dv (and dbias) is written, zeros where nothing contributes.
  */
 int bsa_attn_bwd(const bsa_attn_args *args, bsa_stream_t stream);
+/* bsa_attn_bwd with shares of the query rows and of the key rows (NULL: none), each with a scratch of its own */
+int bsa_attn_bwd_shares(const bsa_attn_args *args, const bsa_attn_shares *query_shares, const bsa_attn_shares *key_shares,
+                        bsa_stream_t stream);
 
 #ifdef __cplusplus
 }
