@@ -63,17 +63,18 @@ __device__ inline void copy_words_to_lds(const float *addr, char *dst) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(addr), "s"(lds_addr) : "memory");
 }
 
-// gradient blocks of the own row, columns 2 r + 4 group .. + 3 of a row per lane
+// NS gradient blocks of the own row, from slice `first` on, columns 2 r + 4 group .. + 3 of a row per lane
 template <typename Tr, int SBS, int NS, int kHalves, typename Acc>
 __device__ inline void store_gradient(const Acc (&acc)[NS], float scale, void *out, const int64_t *pidx, int n_slices,
-                                      int64_t n_blocks, int own, int me, int group) {
+                                      int64_t n_blocks, int own, int first, int me, int group) {
   constexpr int kRegs = SBS == 32 ? 16 : 4;
 #pragma unroll
   for (int h = 0; h < NS; ++h) {
-    if (h / kHalves >= n_slices) break;
-    const int64_t p = pidx[h / kHalves];
+    const int slice = first + h;
+    if (slice / kHalves >= n_slices) break;
+    const int64_t p = pidx[slice / kHalves];
     if (p < 0 || p >= n_blocks) continue;
-    char *blk = static_cast<char *>(out) + Place<Tr::kElem, SBS, kHalves>::row(p, own, me, h) + 4 * group * Tr::kElem;
+    char *blk = static_cast<char *>(out) + Place<Tr::kElem, SBS, kHalves>::row(p, own, me, slice) + 4 * group * Tr::kElem;
 #pragma unroll
     for (int r = 0; r < kRegs; r += 4)
       store4<Tr>(blk + 2 * r * Tr::kElem, acc[h][r] * scale, acc[h][r + 1] * scale, acc[h][r + 2] * scale, acc[h][r + 3] * scale);
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
     return;
   }
   const late_args_t p = late_args();
-  store_gradient<Tr, SBS, NS, kHalves>(dq, p->scale, p->dq, p->pidx_q + row * p->nh, (int)p->nh, p->n_q_blocks, (int)me.own, qi, kq);
+  store_gradient<Tr, SBS, NS, kHalves>(dq, p->scale, p->dq, p->pidx_q + row * p->nh, (int)p->nh, p->n_q_blocks, (int)me.own, 0, qi, kq);
 }
 
 template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
@@ -355,37 +356,36 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
     return;
   }
   const late_args_t p = late_args();
-  store_gradient<Tr, SBS, NS, kHalves>(dk, p->scale, p->dk, p->pidx_k + row * p->nh, (int)p->nh, p->n_k_blocks, (int)me.own, kj, kq);
-  store_gradient<Tr, SBS, NS, kHalves>(dv, 1.f, p->dv, p->pidx_v + row * p->nhv, (int)p->nhv, p->n_v_blocks, (int)me.own, kj, kq);
+  store_gradient<Tr, SBS, NS, kHalves>(dk, p->scale, p->dk, p->pidx_k + row * p->nh, (int)p->nh, p->n_k_blocks, (int)me.own, 0, kj, kq);
+  store_gradient<Tr, SBS, NS, kHalves>(dv, 1.f, p->dv, p->pidx_v + row * p->nhv, (int)p->nhv, p->n_v_blocks, (int)me.own, 0, kj, kq);
 }
 
-// The gradients of rows that several workgroups share, one wave each: dQ of the first n_q merges (times the halves), then dK
-// and dV of the others.  A merge is (batch entry, row of the layout, first slot, slots).
+// The gradients of rows that several workgroups share, a wave for each head slice (blockIdx.y): dQ of the first n_q merges
+// (times the halves), then dK and dV (blockIdx.z) of the others.  A merge is (batch entry, row of the layout, first slot, slots).
 template <typename Tr, int SBS, int NS, int kHalves>
 __global__ __launch_bounds__(64) void attn_small_bwd_merge_kernel(bsa_attn_args a, const int32_t *merges_q, const float *partials_q,
                                                                   int64_t n_q, const int32_t *merges_kv, const float *partials_kv) {
   using Shape = BwdShape<Tr::kElem, SBS, NS, kHalves>;
   constexpr int kRegs = Shape::kRegs;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
-  const int lane = threadIdx.x, me = lane % SBS, group = lane / SBS, half = blockIdx.x % kHalves;
+  const int lane = threadIdx.x, me = lane % SBS, group = lane / SBS, half = blockIdx.x % kHalves, h = blockIdx.y;
   const int64_t m = blockIdx.x / kHalves;
-  const bool is_q = m < n_q;
+  const bool is_q = m < n_q, is_v = blockIdx.z == 1;
+  if (is_q && is_v) return;
   const int32_t *merge = is_q ? merges_q + m * 4 : merges_kv + (m - n_q) * 4;
   const int64_t row = (int64_t)merge[0] * (is_q ? a.nq : a.nk) + merge[1];
-  const int own = merge[1] * kHalves + half;
-  const int kStep = is_q ? Shape::kSlot : 2 * Shape::kSlot;
-  for (int what = 0; what < (is_q ? 1 : 2); ++what) {  // dQ, or dK and dV
-    const float *part = (is_q ? partials_q : partials_kv) + ((int64_t)merge[2] * kHalves + half) * kStep + what * Shape::kSlot;
-    acc_t acc[NS];
+  const int own = merge[1] * kHalves + half, n = merge[3];
+  const int64_t slot = is_q ? Shape::kSlot : 2 * Shape::kSlot, step = kHalves * slot;
+  const float *part = (is_q ? partials_q : partials_kv) + ((int64_t)merge[2] * kHalves + half) * slot + (is_v ? Shape::kSlot : 0) +
+                      h * kRegs * 64;
+  acc_t acc[1];
 #pragma unroll
-    for (int h = 0; h < NS; ++h)
-#pragma unroll
-      for (int r = 0; r < kRegs; ++r) acc[h][r] = 0.f;
-    for (int s = 0; s < merge[3]; ++s) add_partial<NS, kRegs>(acc, part + (int64_t)s * kHalves * kStep, lane);
-    if (what == 1) store_gradient<Tr, SBS, NS, kHalves>(acc, 1.f, a.dv, a.pidx_v + row * a.nhv, (int)a.nhv, a.n_v_blocks, own, me, group);
-    else if (is_q) store_gradient<Tr, SBS, NS, kHalves>(acc, a.scale, a.dq, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, own, me, group);
-    else store_gradient<Tr, SBS, NS, kHalves>(acc, a.scale, a.dk, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, own, me, group);
-  }
+  for (int r = 0; r < kRegs; ++r) acc[0][r] = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < n; ++s) add_partial<1, kRegs>(acc, part + s * step, lane);
+  if (is_v) store_gradient<Tr, SBS, 1, kHalves>(acc, 1.f, a.dv, a.pidx_v + row * a.nhv, (int)a.nhv, a.n_v_blocks, own, h, me, group);
+  else if (is_q) store_gradient<Tr, SBS, 1, kHalves>(acc, a.scale, a.dq, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, own, h, me, group);
+  else store_gradient<Tr, SBS, 1, kHalves>(acc, a.scale, a.dk, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, own, h, me, group);
 }
 
 // bias blocks outside the attention layout, and pairs the causal predicate rules out, have no wave that writes them
@@ -431,7 +431,7 @@ int launch_kind(const bsa_attn_args &a, const bsa_attn_shares *sh_q, const bsa_a
   }
   const int64_t q_merges = sh_q ? sh_q->n_merges : 0, kv_merges = sh_kv ? sh_kv->n_merges : 0;
   if (q_merges + kv_merges > 0) {
-    attn_small_bwd_merge_kernel<Tr, SBS, NS, kHalves><<<(unsigned)((q_merges + kv_merges) * kHalves), 64, 0, s>>>(
+    attn_small_bwd_merge_kernel<Tr, SBS, NS, kHalves><<<dim3((unsigned)((q_merges + kv_merges) * kHalves), NS, kv_merges ? 2 : 1), 64, 0, s>>>(
         a, sh_q ? sh_q->merges : nullptr, shares_q.partials, q_merges, sh_kv ? sh_kv->merges : nullptr, shares_kv.partials);
     if (int rc = check_launch("attn_small_bwd_merge_kernel")) return rc;
   }

@@ -72,25 +72,26 @@ __device__ inline void merge_partial(Acc (&oacc)[NS], float &m_i, float &l_i, co
     }
 }
 
-// output blocks and lse of query block `own`, which belongs to `row` of the layout
+// NS slices of the output, from slice `first` on, and lse of query block `own`, which belongs to `row` of the layout
 template <typename Tr, int SBS, int NS, int kHalves, typename Acc>
-__device__ inline void store_output(const Acc (&oacc)[NS], float m_i, float l_i, int64_t row, int own, int qi, int kq) {
+__device__ inline void store_output(const Acc (&oacc)[NS], float m_i, float l_i, int64_t row, int own, int first, int qi, int kq) {
   constexpr int kRegs = SBS == 32 ? 16 : 4;
   const late_args_t p = late_args();
   const int nhv = (int)p->nhv;
   const float inv_l = (l_i != 0.f) ? 1.f / l_i : 0.f;
 #pragma unroll
   for (int h = 0; h < NS; ++h) {
-    if (h / kHalves >= nhv) break;
-    const int64_t po = p->pidx_o[row * nhv + h / kHalves];
+    const int slice = first + h;
+    if (slice / kHalves >= nhv) break;
+    const int64_t po = p->pidx_o[row * nhv + slice / kHalves];
     if (po < 0 || po >= p->n_o_blocks) continue;
-    char *out = static_cast<char *>(p->o) + Place<Tr::kElem, SBS, kHalves>::row(po, own, qi, h);
+    char *out = static_cast<char *>(p->o) + Place<Tr::kElem, SBS, kHalves>::row(po, own, qi, slice);
 #pragma unroll
     for (int r = 0; r < kRegs; r += 4)  // columns 2 r + 4 kq .. + 3 of a row per lane
       store4<Tr>(out + (2 * r + 4 * kq) * Tr::kElem, oacc[h][r] * inv_l, oacc[h][r + 1] * inv_l, oacc[h][r + 2] * inv_l,
                  oacc[h][r + 3] * inv_l);
   }
-  if (kq == 0) p->lse[(row * kHalves + own % kHalves) * SBS + qi] = (l_i != 0.f) ? m_i + log2f(l_i) : -INFINITY;
+  if (kq == 0 && first == 0) p->lse[(row * kHalves + own % kHalves) * SBS + qi] = (l_i != 0.f) ? m_i + log2f(l_i) : -INFINITY;
 }
 
 // split: 1, 2 or 4 waves share one query block, each walking every split-th entry of its key list, unless `shares` says how
@@ -223,30 +224,44 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
     if (kq == 0) out[Shape::kSlot - 2 * SBS + 2 * qi] = m_i, out[Shape::kSlot - 2 * SBS + 2 * qi + 1] = l_i;
     return;
   }
-  store_output<Tr, SBS, NS, kHalves>(oacc, m_i, l_i, row, (int)me.own, qi, kq);
+  store_output<Tr, SBS, NS, kHalves>(oacc, m_i, l_i, row, (int)me.own, 0, qi, kq);
 }
 
-// The sums of query blocks that several workgroups share, one wave each: merges[m] is (batch entry, query block of the layout,
-// first slot, slots).
+// The sums of query blocks that several workgroups share, a wave for each head slice (blockIdx.y): merges[m] is (batch entry,
+// query block of the layout, first slot, slots).  All slots' sums are read independently of one another: with one wave per
+// query block that scaled slot by slot, 8 blocks of 128 entries at head dimension 128 took 29 us, now 4.5.
 template <typename Tr, int SBS, int NS, int kHalves>
 __global__ __launch_bounds__(64) void attn_small_fwd_merge_kernel(bsa_attn_args a, const int32_t *merges, const float *partials) {
   using Shape = FwdShape<Tr::kElem, SBS, NS, kHalves>;
   constexpr int kRegs = Shape::kRegs;
+  constexpr int64_t kStep = kHalves * Shape::kSlot;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
-  const int lane = threadIdx.x, qi = lane % SBS, kq = lane / SBS, half = blockIdx.x % kHalves;
+  const int lane = threadIdx.x, qi = lane % SBS, kq = lane / SBS, half = blockIdx.x % kHalves, h = blockIdx.y;
   const int32_t *merge = merges + (int64_t)(blockIdx.x / kHalves) * 4;
   const int64_t row = (int64_t)merge[0] * a.nq + merge[1];
   const float *part = partials + ((int64_t)merge[2] * kHalves + half) * Shape::kSlot;
-  acc_t oacc[NS];
-#pragma unroll
-  for (int h = 0; h < NS; ++h)
-#pragma unroll
-    for (int r = 0; r < kRegs; ++r) oacc[h][r] = 0.f;
+  const float *stats = part + (Shape::kSlot - 2 * SBS) + 2 * qi;
+  const int n = merge[3];
   float m_i = -INFINITY, l_i = 0.f;
-  for (int s = 0; s < merge[3]; ++s, part += kHalves * Shape::kSlot)
-    merge_partial<NS, kRegs>(oacc, m_i, l_i, part, part[Shape::kSlot - 2 * SBS + 2 * qi], part[Shape::kSlot - 2 * SBS + 2 * qi + 1],
-                             lane);
-  store_output<Tr, SBS, NS, kHalves>(oacc, m_i, l_i, row, merge[1] * kHalves + half, qi, kq);
+#pragma unroll 4
+  for (int s = 0; s < n; ++s) m_i = fmaxf(m_i, stats[s * kStep]);
+  const float m_sub = m_i == -INFINITY ? 0.f : m_i;
+  acc_t oacc[1];
+#pragma unroll
+  for (int r = 0; r < kRegs; ++r) oacc[0][r] = 0.f;
+  part += h * kRegs * 64;
+#pragma unroll 4
+  for (int s = 0; s < n; ++s) {
+    const float scale = __builtin_amdgcn_exp2f(stats[s * kStep] - m_sub);
+    l_i = fmaf(stats[s * kStep + 1], scale, l_i);
+#pragma unroll
+    for (int r = 0; r < kRegs; r += 4) {
+      const f32x4 o4 = *reinterpret_cast<const f32x4 *>(part + s * kStep + (r / 4 * 64 + lane) * 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) oacc[0][r + i] = fmaf(o4[i], scale, oacc[0][r + i]);
+    }
+  }
+  store_output<Tr, SBS, 1, kHalves>(oacc, m_i, l_i, row, merge[1] * kHalves + half, h, qi, kq);
 }
 
 template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
@@ -270,7 +285,7 @@ int launch_kind(const bsa_attn_args &a, const bsa_attn_shares *sh, hipStream_t s
   attn_small_fwd_kernel<Tr, SBS, NS, kSome, kHalves><<<(unsigned)groups, 64 * kWaves, lds, s>>>(a, split, shares);
   if (int rc = check_launch("attn_small_fwd_kernel")) return rc;
   if (!sh || sh->n_merges == 0) return BSA_OK;
-  attn_small_fwd_merge_kernel<Tr, SBS, NS, kHalves><<<(unsigned)(sh->n_merges * kHalves), 64, 0, s>>>(a, sh->merges, shares.partials);
+  attn_small_fwd_merge_kernel<Tr, SBS, NS, kHalves><<<dim3((unsigned)(sh->n_merges * kHalves), NS), 64, 0, s>>>(a, sh->merges, shares.partials);
   return check_launch("attn_small_fwd_merge_kernel");
 }
 
