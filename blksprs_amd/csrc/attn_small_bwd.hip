@@ -18,10 +18,10 @@
 // What bounds it: the chain of a step (tiles awaited, products, exponentials, products) with two to four waves per SIMD
 // to overlap it.  Against the fp32 matrix-core kernels that ran these shapes before (48 x 4096 queries, sbs 32, head
 // dimension 64, fp16, 33 key blocks per query block): delta + zero fill 0.071 -> 0, dK / dV 1.89 -> 0.125 ms (530 TFLOP/s),
-// dQ 1.24 -> 0.090 ms (delta included); fp32, 8 x 2048 queries, sbs 32, half of the blocks, head dimension 64: dK / dV 0.238
-// -> 0.096, dQ 0.198 -> 0.076 ms (89 and 85 TFLOP/s).  fp32 blocks of 64, whose halves walk alone like blocks of 32: 34
-// sequences of 480 to 960, head dimension 64, causal: delta + zero fill 0.023 -> 0, dK / dV 0.222 -> 0.076, dQ 0.132 ->
-// 0.059 ms.
+// dQ 1.24 -> 0.090 ms (delta included); fp32, sbs 32, products from bf16 parts (split_f32.h), 8 x 2048 queries, half of the
+// blocks, head dimension 64: dK / dV 94.5 -> 73.0, dQ 74.8 -> 57.7 us (118 and 112 TFLOP/s) against the fp32 instruction.  fp32
+// blocks of 64, whose halves walk alone like blocks of 32: 20 x 960, causal, head dimension 64: delta + zero fill 19 -> 0, dK /
+// dV 129 (eight waves to a tile) -> 44, dQ 128 -> 37 us.
 //
 // Scores as in the forward kernel; p = exp2(s - lse), 0 where lse = -inf; P and dS are rounded to the operand type
 // before they enter a product (blksprs/ops/flash_attention.py:1452, :1468, :1692).
@@ -102,8 +102,16 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
   walk.start(a, me.b, me.own, me.there, me.part, me.parts);
 
   OwnRows<Tr::kElem, SBS, NS, kHalves> qf, gf;
-  qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, (int)me.own, lane);
-  gf.load(a.d_o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, (int)me.own, lane);
+  acc_t dq[NS];
+  auto start_row = [&]() __attribute__((always_inline)) {
+    qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, (int)me.own, lane);
+    gf.load(a.d_o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, (int)me.own, lane);
+#pragma unroll
+    for (int h = 0; h < NS; ++h)
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) dq[h][r] = 0.f;
+  };
+  start_row();
   float delta = 0.f, neg_lse = -a.lse[stats + qi];
   if (neg_lse == INFINITY) neg_lse = -INFINITY;  // a query that sees nothing: p = 0
   {
@@ -114,77 +122,85 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
     delta = row_sum<SBS>(delta);
     if (me.there && me.part == 0 && kq == 0) a.delta[stats + qi] = delta;
   }
-  acc_t dq[NS];
-#pragma unroll
-  for (int h = 0; h < NS; ++h)
-#pragma unroll
-    for (int r = 0; r < kRegs; ++r) dq[h][r] = 0.f;
-
   const float qk_scale = a.scale * kLog2e;
   const float cc = a.bias ? 1.f : qk_scale;
   const uint32_t source = T::source_offset(lane);
   const char *const tensor_k = static_cast<const char *>(a.k), *const tensor_v = static_cast<const char *>(a.v);
   const typename T::RowReader k_rows(lds_k, lane), v_rows(lds_v, lane);
   const typename T::ColReader k_cols(lds_k, lane);
-  typename W::Step now, next;
-  walk.take(now, lane);
-  settle(qf);
-  settle(gf);
-  bool counted = false;  // exactly kCopies copies were issued after the tile that is needed next
-  if (now.count) {
-    walk.template copy<true>(now, tensor_v, lds_v, source, lane);
-    counted = walk.template copy<false>(now, tensor_k, lds_k, source, lane);
-  }
-  while (now.count) {
-    // ---- dP^T = V dO^T.  In flight at most: V and K of this step, in that order.
-    if (counted) wait_vmem<T::kCopies>();
-    else wait_vmem<0>();
-    acc_t dp[NB], sacc[NB];
-    W::template multiply_rows<Tr, true>(dp, now, v_rows, gf, lane);
-    wait_lds();
-    walk.take(next, lane);
-    counted = false;
-    if (next.count) counted = walk.template copy<true>(next, tensor_v, lds_v, source, lane);
-
-    // ---- S^T = K Q^T.  In flight at most: K of this step, V of the next.
-    if (counted) wait_vmem<T::kCopies>();
-    else wait_vmem<0>();
-    W::template multiply_rows<Tr, false>(sacc, now, k_rows, qf, lane);
-    float sv[kScores];
-#pragma unroll
-    for (int t = 0; t < NB; ++t)
-#pragma unroll
-      for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
-    if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, qi, kq);
-    apply_factor<Tr, kScores>(sv, cc);
-
-    // ---- dS = P (dP - delta)
-#pragma unroll
-    for (int x = 0; x < kScores; ++x)
-      sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), neg_lse)) * (dp[x / kRegs][x % kRegs] - delta);
-    if (now.special) {
-      const late_args_t p = late_args();
-      if (p->dbias) {  // every pair is visited once: plain stores
-#pragma unroll
-        for (int t = 0; t < NB; ++t)
-          if (now.bias[t] >= 0) {
-            constexpr int kSide = kHalves * SBS;
-            float *out = p->dbias + ((int64_t)now.bias[t] * kSide + (int)me.own % kHalves * SBS + qi) * kSide +
-                         now.other[t] % kHalves * SBS + 4 * kq;
-#pragma unroll
-            for (int r = 0; r < kRegs; r += 4) {
-              const float *v = sv + kRegs * t + r;
-              *reinterpret_cast<f32x4 *>(out + 2 * r) = f32x4{v[0], v[1], v[2], v[3]};
-            }
-          }
-      }
+  auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) {
+    using Ar = decltype(arithmetic);
+    typename W::Step now, next;
+    walk.take(now, lane);
+    settle(qf);
+    settle(gf);
+    const OwnOperand<Ar, SBS, NS, kHalves> q_operand(qf), g_operand(gf);
+    bool counted = false;  // exactly kCopies copies were issued after the tile that is needed next
+    if (now.count) {
+      walk.template copy<true>(now, tensor_v, lds_v, source, lane);
+      counted = walk.template copy<false>(now, tensor_k, lds_k, source, lane);
     }
-    // ---- dQ^T += K^T dS^T
-    W::template multiply_cols<Tr, false, kScores>(dq, now, k_cols, Weights<Tr, kScores>(sv));
-    wait_lds();
-    counted = false;
-    if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
-    now = next;
+    while (now.count) {
+      // ---- dP^T = V dO^T.  In flight at most: V and K of this step, in that order.
+      if (counted) wait_vmem<T::kCopies>();
+      else wait_vmem<0>();
+      acc_t dp[NB], sacc[NB];
+      W::template multiply_rows<Ar, true>(dp, now, v_rows, g_operand, lane);
+      wait_lds();
+      walk.take(next, lane);
+      counted = false;
+      if (next.count) counted = walk.template copy<true>(next, tensor_v, lds_v, source, lane);
+
+      // ---- S^T = K Q^T.  In flight at most: K of this step, V of the next.
+      if (counted) wait_vmem<T::kCopies>();
+      else wait_vmem<0>();
+      W::template multiply_rows<Ar, false>(sacc, now, k_rows, q_operand, lane);
+      float sv[kScores];
+#pragma unroll
+      for (int t = 0; t < NB; ++t)
+#pragma unroll
+        for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
+      if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, qi, kq);
+      apply_factor<Tr, kScores>(sv, cc);
+
+      // ---- dS = P (dP - delta)
+#pragma unroll
+      for (int x = 0; x < kScores; ++x)
+        sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), neg_lse)) * (dp[x / kRegs][x % kRegs] - delta);
+      if (now.special) {
+        const late_args_t p = late_args();
+        if (p->dbias) {  // every pair is visited once: plain stores
+#pragma unroll
+          for (int t = 0; t < NB; ++t)
+            if (now.bias[t] >= 0) {
+              constexpr int kSide = kHalves * SBS;
+              float *out = p->dbias + ((int64_t)now.bias[t] * kSide + (int)me.own % kHalves * SBS + qi) * kSide +
+                           now.other[t] % kHalves * SBS + 4 * kq;
+#pragma unroll
+              for (int r = 0; r < kRegs; r += 4) {
+                const float *v = sv + kRegs * t + r;
+                *reinterpret_cast<f32x4 *>(out + 2 * r) = f32x4{v[0], v[1], v[2], v[3]};
+              }
+            }
+        }
+      }
+      // ---- dQ^T += K^T dS^T
+      W::template multiply_cols<Ar, false, kScores>(dq, now, k_cols, Weights<Ar, kScores>(sv));
+      wait_lds();
+      counted = false;
+      if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
+      now = next;
+    }
+  };
+  if constexpr (in_parts<Tr, SBS, kSome>()) {
+    walk_list(SSplit{});
+    if (in_doubt<NS, kRegs>(dq)) {  // once more with the fp32 instruction
+      walk.start(a, me.b, me.own, me.there, me.part, me.parts);
+      start_row();
+      walk_list(Tr{});
+    }
+  } else {
+    walk_list(Tr{});
   }
   if (me.waves > 1) {
     float *mine = reinterpret_cast<float *>(lds_k);
@@ -221,13 +237,16 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
   walk.start(a, me.b, me.own, me.there, me.part, me.parts);
 
   OwnRows<Tr::kElem, SBS, NS, kHalves> kf, vf;
-  kf.load(a.k, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, (int)me.own, lane);
-  vf.load(a.v, a.pidx_v + row * a.nhv, (int)a.nhv, a.n_v_blocks, (int)me.own, lane);
   acc_t dk[NS], dv[NS];
+  auto start_row = [&]() __attribute__((always_inline)) {
+    kf.load(a.k, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, (int)me.own, lane);
+    vf.load(a.v, a.pidx_v + row * a.nhv, (int)a.nhv, a.n_v_blocks, (int)me.own, lane);
 #pragma unroll
-  for (int h = 0; h < NS; ++h)
+    for (int h = 0; h < NS; ++h)
 #pragma unroll
-    for (int r = 0; r < kRegs; ++r) dk[h][r] = dv[h][r] = 0.f;
+      for (int r = 0; r < kRegs; ++r) dk[h][r] = dv[h][r] = 0.f;
+  };
+  start_row();
 
   const float qk_scale = a.scale * kLog2e;
   const float cc = a.bias ? 1.f : qk_scale;
@@ -253,87 +272,107 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 
   const typename T::RowReader q_rows0(lds, lane), g_rows0(lds + T::kBytes, lane);
   const typename T::ColReader q_cols0(lds, lane), g_cols0(lds + T::kBytes, lane);
-  typename W::Step now, next;
-  walk.take(now, lane);
-  settle(kf);
-  settle(vf);
-  int buf = 0;
-  if (now.count) copy_all(now, lds);
-  while (now.count) {
-    const int at = kBufs == 2 ? buf * Shape::kKvBuf : 0;
-    if constexpr (kBufs == 2) {
-      // the next step's tiles into the other buffer, then wait for everything but them
-      wait_lds();
-      walk.take(next, lane);
-      bool counted = false;
-      if (next.count) counted = copy_all(next, lds + (buf ^ 1) * Shape::kKvBuf);
-      if (counted) wait_vmem<2 * T::kCopies + 1>();
-      else wait_vmem<0>();
-    } else {
-      wait_vmem<0>();
-    }
-    typename T::RowReader q_rows = q_rows0, g_rows = g_rows0;
-    typename T::ColReader q_cols = q_cols0, g_cols = g_cols0;
-    if constexpr (kBufs == 2) {
-      q_rows.shift(at), g_rows.shift(at);
-      q_cols.shift(at), g_cols.shift(at);
-    }
-    const float *lse = reinterpret_cast<const float *>(lds + at + 2 * T::kBytes), *delta = lse + 32;
-
-    // ---- S = Q K^T, P = exp2(S - lse)
-    acc_t sacc[NB], dp[NB];
-    W::template multiply_rows<Tr, false>(sacc, now, q_rows, kf, lane);
-    float sv[kScores], ls[kScores];
-#pragma unroll
-    for (int t = 0; t < NB; ++t)
-#pragma unroll
-      for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
-    if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, kj, kq);
-    apply_factor<Tr, kScores>(sv, cc);
-#pragma unroll
-    for (int x = 0; x < kScores; x += 4) {
-      const f32x4 l4 = *reinterpret_cast<const f32x4 *>(lse + (x / kRegs) * SBS + 2 * (x % kRegs) + 4 * kq);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ls[x + i] = l4[i];
-    }
-    W::template multiply_rows<Tr, true>(dp, now, g_rows, vf, lane);
-    float lowest = ls[0];
-#pragma unroll
-    for (int x = 1; x < kScores; ++x) lowest = fminf(lowest, ls[x]);
-    if (__any(lowest == -INFINITY)) {  // a query that sees nothing: p = 0
-#pragma unroll
-      for (int x = 0; x < kScores; ++x)
-        if (ls[x] == -INFINITY) ls[x] = INFINITY;
-    }
-#pragma unroll
-    for (int x = 0; x < kScores; ++x) sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), -ls[x]));
-    const Weights<Tr, kScores> pw(sv);
-
-    // ---- dS = P (dP - delta)
-#pragma unroll
-    for (int x = 0; x < kScores; x += 4) {
-      const f32x4 d4 = *reinterpret_cast<const f32x4 *>(delta + (x / kRegs) * SBS + 2 * (x % kRegs) + 4 * kq);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sv[x + i] *= dp[x / kRegs][x % kRegs + i] - d4[i];
-    }
-    // ---- dV^T += dO^T P
-    W::template multiply_cols<Tr, true, kScores>(dv, now, g_cols, pw);
-    if constexpr (kBufs == 1) {
-      wait_lds();
-      walk.take(next, lane);
-      if (next.count) {
-        walk.template copy<true>(next, tensor_g, lds + T::kBytes, source, lane);
-        copy_stats(next, lds + 2 * T::kBytes);
+  auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) {
+    using Ar = decltype(arithmetic);
+    typename W::Step now, next;
+    walk.take(now, lane);
+    settle(kf);
+    settle(vf);
+    const OwnOperand<Ar, SBS, NS, kHalves> k_operand(kf), v_operand(vf);
+    int buf = 0;
+    if (now.count) copy_all(now, lds);
+    while (now.count) {
+      const int at = kBufs == 2 ? buf * Shape::kKvBuf : 0;
+      if constexpr (kBufs == 2) {
+        // the next step's tiles into the other buffer, then wait for everything but them
+        wait_lds();
+        walk.take(next, lane);
+        bool counted = false;
+        if (next.count) counted = copy_all(next, lds + (buf ^ 1) * Shape::kKvBuf);
+        if (counted) wait_vmem<2 * T::kCopies + 1>();
+        else wait_vmem<0>();
+      } else {
+        wait_vmem<0>();
       }
+      typename T::RowReader q_rows = q_rows0, g_rows = g_rows0;
+      typename T::ColReader q_cols = q_cols0, g_cols = g_cols0;
+      if constexpr (kBufs == 2) {
+        q_rows.shift(at), g_rows.shift(at);
+        q_cols.shift(at), g_cols.shift(at);
+      }
+      const float *lse = reinterpret_cast<const float *>(lds + at + 2 * T::kBytes), *delta = lse + 32;
+
+      // ---- S = Q K^T, P = exp2(S - lse)
+      acc_t sacc[NB], dp[NB];
+      W::template multiply_rows<Ar, false>(sacc, now, q_rows, k_operand, lane);
+      float sv[kScores], ls[kScores];
+#pragma unroll
+      for (int t = 0; t < NB; ++t)
+#pragma unroll
+        for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
+      if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, kj, kq);
+      apply_factor<Tr, kScores>(sv, cc);
+#pragma unroll
+      for (int x = 0; x < kScores; x += 4) {
+        const f32x4 l4 = *reinterpret_cast<const f32x4 *>(lse + (x / kRegs) * SBS + 2 * (x % kRegs) + 4 * kq);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ls[x + i] = l4[i];
+      }
+      // in parts P is used up before dP is formed, for want of registers
+      constexpr bool kLateDp = std::is_same_v<Ar, SSplit>;
+      if constexpr (!kLateDp) W::template multiply_rows<Ar, true>(dp, now, g_rows, v_operand, lane);
+      float lowest = ls[0];
+#pragma unroll
+      for (int x = 1; x < kScores; ++x) lowest = fminf(lowest, ls[x]);
+      if (__any(lowest == -INFINITY)) {  // a query that sees nothing: p = 0
+#pragma unroll
+        for (int x = 0; x < kScores; ++x)
+          if (ls[x] == -INFINITY) ls[x] = INFINITY;
+      }
+#pragma unroll
+      for (int x = 0; x < kScores; ++x) sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), -ls[x]));
+      const Weights<Ar, kScores> pw(sv);
+      if constexpr (kLateDp) {
+        W::template multiply_cols<Ar, true, kScores>(dv, now, g_cols, pw);
+        W::template multiply_rows<Ar, true>(dp, now, g_rows, v_operand, lane);
+      }
+
+      // ---- dS = P (dP - delta)
+#pragma unroll
+      for (int x = 0; x < kScores; x += 4) {
+        const f32x4 d4 = *reinterpret_cast<const f32x4 *>(delta + (x / kRegs) * SBS + 2 * (x % kRegs) + 4 * kq);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sv[x + i] *= dp[x / kRegs][x % kRegs + i] - d4[i];
+      }
+      // ---- dV^T += dO^T P
+      if constexpr (!kLateDp) W::template multiply_cols<Ar, true, kScores>(dv, now, g_cols, pw);
+      if constexpr (kBufs == 1) {
+        wait_lds();
+        walk.take(next, lane);
+        if (next.count) {
+          walk.template copy<true>(next, tensor_g, lds + T::kBytes, source, lane);
+          copy_stats(next, lds + 2 * T::kBytes);
+        }
+      }
+      // ---- dK^T += Q^T dS
+      W::template multiply_cols<Ar, false, kScores>(dk, now, q_cols, Weights<Ar, kScores>(sv));
+      if constexpr (kBufs == 1) {
+        wait_lds();
+        if (next.count) walk.template copy<false>(next, tensor_q, lds, source, lane);
+      }
+      now = next;
+      buf ^= 1;
     }
-    // ---- dK^T += Q^T dS
-    W::template multiply_cols<Tr, false, kScores>(dk, now, q_cols, Weights<Tr, kScores>(sv));
-    if constexpr (kBufs == 1) {
-      wait_lds();
-      if (next.count) walk.template copy<false>(next, tensor_q, lds, source, lane);
+  };
+  if constexpr (in_parts<Tr, SBS, kSome>()) {
+    walk_list(SSplit{});
+    if (in_doubt<NS, kRegs>(dk) || in_doubt<NS, kRegs>(dv)) {  // once more with the fp32 instruction
+      walk.start(a, me.b, me.own, me.there, me.part, me.parts);
+      start_row();
+      walk_list(Tr{});
     }
-    now = next;
-    buf ^= 1;
+  } else {
+    walk_list(Tr{});
   }
   if (me.waves > 1) {
     float *mine = reinterpret_cast<float *>(lds);

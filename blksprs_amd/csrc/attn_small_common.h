@@ -7,14 +7,19 @@
 // dimension: one 128-bit read per fragment) and columns (contraction over the sequence: the transposing LDS read for
 // 16-bit elements, 32-bit reads for fp32).  Products: 32x32x16 (blocks of 32) and 16x16x32 (blocks of 16, where the 32
 // contracted values of a score product are two head slices and those of a value product two partner blocks) for 16-bit
-// elements, 32x32x2 and 16x16x4 for fp32, whose contracted values are taken in an order that suits the 128-bit reads.
+// elements; for fp32 32x32x16 of bf16 parts (blocks of 32) and 16x16x4 (blocks of 16; 32x32x2 where the parts do not hold the
+// values or slices are missing), whose contracted values are taken in an order that suits the 128-bit reads.
 #pragma once
+#include <type_traits>
+
 #include "attn_mfma_common.h"
+#include "split_f32.h"
 
 namespace bsa {
 namespace small {
 
 using namespace mfma;
+using namespace split;
 
 struct SBf16 : MBf16 {
   static constexpr int kElem = 2;
@@ -57,6 +62,15 @@ struct SF32 {
     return c;
   }
 };
+
+// fp32 products from bf16 parts: of blocks of 32 (and halves of blocks of 64) all of whose slices are there.  Blocks of 16, whose
+// fp32 products take half as long for the same values to split, are no faster with it (6 x 1040 queries, causal, head dimension
+// 32: forward 16.1 -> 16.6 us, dK / dV 20.0 -> 21.9).
+struct SSplit : SF32 {};
+template <typename Tr, int SBS, bool kSome>
+constexpr bool in_parts() {
+  return Tr::kElem == 4 && SBS == 32 && !kSome;
+}
 
 // Waits until at most N vector memory operations of the wave are outstanding.  The clobber keeps LDS reads behind it.
 template <int N>
@@ -314,6 +328,24 @@ struct OwnRows {
   }
 };
 
+// The own rows as the products of arithmetic Ar take them
+template <typename Ar, int SBS, int NS, int kHalves>
+struct OwnOperand {
+  const OwnRows<Ar::kElem, SBS, NS, kHalves> &rows;
+  __device__ inline explicit OwnOperand(const OwnRows<Ar::kElem, SBS, NS, kHalves> &own) : rows(own) {}
+};
+// in parts: fragments 2 p and 2 p + 1 in one, the second half zero behind an odd last one
+template <int SBS, int NS, int kHalves>
+struct OwnOperand<SSplit, SBS, NS, kHalves> {
+  static constexpr int kFrags = OwnRows<4, SBS, NS, kHalves>::T::kFrags, kParts = (kFrags + 1) / 2;
+  Parts parts[kParts];
+  __device__ inline explicit OwnOperand(const OwnRows<4, SBS, NS, kHalves> &own) {
+#pragma unroll
+    for (int p = 0; p < kParts; ++p)
+      parts[p] = Parts(own.fr[2 * p], 2 * p + 1 < kFrags ? own.fr[2 * p + 1] : u32x4{0u, 0u, 0u, 0u});
+  }
+};
+
 // Makes the compiler wait for the loads of the own rows here: left to their first use, the wait sits inside the loop and
 // is for every load in flight, each time round.
 template <int ES, int SBS, int NS, int kHalves>
@@ -324,17 +356,27 @@ __device__ static inline void settle(OwnRows<ES, SBS, NS, kHalves> &own) {
 
 // acc (per partner block t) = partner rows x own rows over all head slices: acc[t] belongs to this lane's own row
 // (lane % SBS) and partner rows 8 (r / 4) + 4 (lane / 32) + r % 4 (SBS 32) or 4 (lane / 16) + r (SBS 16).
-template <typename Tr, int SBS, int NS, int NB, int kHalves, typename Acc>
+// kOwnIsQuery: as in Walk; a score is the same bits wherever it is formed
+template <typename Tr, int SBS, int NS, int NB, int kHalves, bool kOwnIsQuery, typename Acc>
 __device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<Tr::kElem, SBS, NS, NB, kHalves>::RowReader &rows,
-                                           const OwnRows<Tr::kElem, SBS, NS, kHalves> &own) {
+                                           const OwnOperand<Tr, SBS, NS, kHalves> &own) {
+  constexpr int kFrags = Tile<Tr::kElem, SBS, NS, NB>::kFrags;
 #pragma unroll
   for (int t = 0; t < NB; ++t)
 #pragma unroll
     for (int r = 0; r < (SBS == 32 ? 16 : 4); ++r) acc[t][r] = 0.f;
+  if constexpr (std::is_same_v<Tr, SSplit>) {
 #pragma unroll
-  for (int f = 0; f < Tile<Tr::kElem, SBS, NS, NB>::kFrags; ++f)
+    for (int p = 0; p < OwnOperand<Tr, SBS, NS, kHalves>::kParts; ++p)
 #pragma unroll
-    for (int t = 0; t < NB; ++t) Tr::rows(acc[t], rows.frag(t, f), own.fr[f]);
+      for (int t = 0; t < NB; ++t)
+        multiply_parts<!kOwnIsQuery>(acc[t], Parts(rows.frag(t, 2 * p), 2 * p + 1 < kFrags ? rows.frag(t, 2 * p + 1) : u32x4{0u, 0u, 0u, 0u}), own.parts[p]);
+  } else {
+#pragma unroll
+    for (int f = 0; f < kFrags; ++f)
+#pragma unroll
+      for (int t = 0; t < NB; ++t) Tr::rows(acc[t], rows.frag(t, f), own.rows.fr[f]);
+  }
 }
 
 // The same over the slices in have[t] only: a slice that one of the two blocks does not have adds nothing, where its zeros
@@ -382,11 +424,31 @@ struct Weights<SF32, kScores> {
   }
 };
 
+template <int kScores>
+struct Weights<SSplit, kScores> : Weights<SF32, kScores> {
+  using Weights<SF32, kScores>::Weights;
+};
+
 // out[h] += partner columns^T x weights
 template <typename Tr, int SBS, int NS, int NB, int kHalves, int kScores, typename Acc>
 __device__ static inline void product_cols(Acc (&out)[NS], const typename Tile<Tr::kElem, SBS, NS, NB, kHalves>::ColReader &cols,
                                            const Weights<Tr, kScores> &w) {
-  if constexpr (Tr::kElem == 4) {
+  if constexpr (std::is_same_v<Tr, SSplit>) {
+    constexpr int kRegs = kScores / NB;
+#pragma unroll
+    for (int x = 0; x < kScores; x += 8) {
+      u32x4 v[2];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i / 4][i % 4] = __builtin_bit_cast(uint32_t, w.w[x + i]);
+      const Parts weights(v[0], v[1]);
+#pragma unroll
+      for (int h = 0; h < NS; ++h) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i / 4][i % 4] = __builtin_bit_cast(uint32_t, cols.value((x + i) / kRegs, h, (x + i) % kRegs));
+        multiply_parts(out[h], Parts(v[0], v[1]), weights);
+      }
+    }
+  } else if constexpr (Tr::kElem == 4) {
     constexpr int kRegs = kScores / NB;
 #pragma unroll
     for (int x = 0; x < kScores; ++x)
@@ -659,14 +721,14 @@ struct Walk {
   // acc = rows of the step's blocks of the first (second) tensor x own rows, and out += their columns^T x weights
   template <typename Tr, bool kSecond, typename Acc>
   __device__ static inline void multiply_rows(Acc (&acc)[NB], const Step &s, const typename T::RowReader &rows,
-                                              const OwnRows<ES, SBS, NS, kHalves> &own, int lane) {
+                                              const OwnOperand<Tr, SBS, NS, kHalves> &own, int lane) {
     if constexpr (kSome) {
       uint32_t have[NB];
 #pragma unroll
-      for (int t = 0; t < NB; ++t) have[t] = (kSecond ? s.have[t] >> 8 : s.have[t]) & own.there;
-      product_some_rows<Tr, SBS, NS, NB>(acc, rows, own, have, lane);
+      for (int t = 0; t < NB; ++t) have[t] = (kSecond ? s.have[t] >> 8 : s.have[t]) & own.rows.there;
+      product_some_rows<Tr, SBS, NS, NB>(acc, rows, own.rows, have, lane);
     } else {
-      product_rows<Tr, SBS, NS, NB, kHalves>(acc, rows, own);
+      product_rows<Tr, SBS, NS, NB, kHalves, kOwnIsQuery>(acc, rows, own);
     }
   }
   template <typename Tr, bool kSecond, int kScores, typename Acc>

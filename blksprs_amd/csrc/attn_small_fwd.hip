@@ -1,5 +1,5 @@
 // Block-sparse flash attention forward for blocks of 16 and 32 and head dimensions up to 128, fp16, bf16 and fp32, on the
-// matrix cores of the operand type.
+// matrix cores of the operand type, or bf16's for fp32 blocks of 32 (in_parts).
 //
 // A wave owns one query block (or a share of its key list, below) and walks the list alone: no barrier, no tile
 // shared between waves, so waves of a compute unit drift apart and fill each other's waits.  A step takes one key
@@ -17,11 +17,11 @@
 // What bounds it: a wave's chain per step (copies awaited, scores, softmax, value product) and the instructions of one
 // wave at a time.  Against the fp32 matrix-core kernel that ran these shapes before: 48 x 4096 queries, sbs 32, head
 // dimension 64, fp16, 33 key blocks per query block: 0.65 -> 0.072 ms (460 TFLOP/s, 18 % of the matrix cores' peak); 32
-// prompts of 1032 to 2064 tokens, sbs 16, bf16, causal: 0.54 -> 0.044 ms.  fp32, where the products take eight times as
-// long and hide the rest: 8 x 2048 queries, half of the blocks, head dimension 64: 0.089 -> 0.054 ms (80 TFLOP/s, half
-// of the fp32 matrix-core peak; 512 lists of 32 +- 4 blocks cut in four fill the chip once, so the launch waits for the
-// longest).  fp32 blocks of 64, whose halves walk alone like blocks of 32: 34 sequences of 480 to 960, head dimension 64,
-// causal: 0.100 -> 0.041 ms.
+// prompts of 1032 to 2064 tokens, sbs 16, bf16, causal: 0.54 -> 0.044 ms.  fp32, sbs 32, products from bf16 parts (split_f32.h):
+// 8 x 2048 queries, half of the blocks, head dimension 64: 51.1 -> 41.1 us (105 TFLOP/s) against the fp32 instruction; the 480
+// vector instructions of a step that split its values cost more than its 48 products, and 512 lists of 32 +- 4 blocks cut in
+// four fill the chip once, so the launch waits for the longest.  fp32 blocks of 64, whose halves walk alone like blocks of 32:
+// 20 x 960, causal, head dimension 64: 97.8 (eight waves to a tile) -> 27.4 us.
 //
 // Score pipeline (log2 domain), in the reference's order (blksprs/ops/flash_attention.py:1058-1224): scale * q k^T,
 // + bias, native causal predicate, explicit mask; probabilities are rounded to the operand type before they multiply
@@ -116,13 +116,17 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
   walk.start(a, me.b, me.own, me.there, me.part, me.parts);
 
   OwnRows<Tr::kElem, SBS, NS, kHalves> qf;
-  qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, (int)me.own, lane);
   acc_t oacc[NS];
+  float m_i, l_i;
+  auto start_row = [&]() __attribute__((always_inline)) {
+    qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, (int)me.own, lane);
 #pragma unroll
-  for (int h = 0; h < NS; ++h)
+    for (int h = 0; h < NS; ++h)
 #pragma unroll
-    for (int r = 0; r < kRegs; ++r) oacc[h][r] = 0.f;
-  float m_i = -INFINITY, l_i = 0.f;
+      for (int r = 0; r < kRegs; ++r) oacc[h][r] = 0.f;
+    m_i = -INFINITY, l_i = 0.f;
+  };
+  start_row();
 
   const float qk_scale = a.scale * kLog2e;
   const float cc = a.bias ? 1.f : qk_scale;
@@ -131,72 +135,86 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
 
   const typename T::RowReader k_rows(lds_k, lane);
   const typename T::ColReader v_cols(lds_v, lane);
-  typename W::Step now, next;
-  walk.take(now, lane);
-  settle(qf);
-  bool counted = false;  // exactly kCopies copies (the V tile's) were issued after the K tile's
-  if (now.count) {
-    walk.template copy<false>(now, tensor_k, lds_k, source, lane);
-    counted = walk.template copy<true>(now, tensor_v, lds_v, source, lane);
-  }
-  while (now.count) {
-    // ---- S^T = K Q^T.  In flight at most: K and V of this step, in that order.
-    if (counted) wait_vmem<T::kCopies>();
-    else wait_vmem<0>();
-    acc_t sacc[NB];
-    W::template multiply_rows<Tr, false>(sacc, now, k_rows, qf, lane);
-
-    // ---- K of the next step
-    wait_lds();
-    walk.take(next, lane);
-    counted = false;
-    if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
-
-    // ---- scores: sv holds them up to the positive factor cc, applied inside the exponential (16-bit)
-    float sv[kScores];
-#pragma unroll
-    for (int t = 0; t < NB; ++t)
-#pragma unroll
-      for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
-    if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, qi, kq);
-    apply_factor<Tr, kScores>(sv, cc);
-
-    // ---- online softmax of the row.  The reference is the exact running maximum: the largest probabilities then lie at
-    // and just below 1, where rounding to 16 bits costs least.  A maximum that follows in steps of up to 2^8 (as in
-    // attn_mfma.hip) saves most of the rescaling and lets them fall anywhere between two powers of two: errors of the output
-    // against 64 bits of 2.27e-3 instead of 2.09e-3 (bf16, 1024 keys, half of the blocks).
-    float m_blk = sv[0];
-#pragma unroll
-    for (int x = 1; x < kScores; ++x) m_blk = fmaxf(m_blk, sv[x]);
-    m_blk = row_max<SBS>(m_blk) * late_factor<Tr>(cc);
-    const float m_cand = fmaxf(m_i, m_blk);
-    if (__any(m_cand > m_i)) {
-      const float alpha = m_cand > m_i ? __builtin_amdgcn_exp2f(m_i - m_cand) : 1.f;
-      m_i = m_cand;
-      l_i *= alpha;
-#pragma unroll
-      for (int h = 0; h < NS; ++h)
-#pragma unroll
-        for (int r = 0; r < kRegs; ++r) oacc[h][r] *= alpha;
+  auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) {
+    using Ar = decltype(arithmetic);
+    typename W::Step now, next;
+    walk.take(now, lane);
+    settle(qf);
+    const OwnOperand<Ar, SBS, NS, kHalves> q_operand(qf);
+    bool counted = false;  // exactly kCopies copies (the V tile's) were issued after the K tile's
+    if (now.count) {
+      walk.template copy<false>(now, tensor_k, lds_k, source, lane);
+      counted = walk.template copy<true>(now, tensor_v, lds_v, source, lane);
     }
-    const float m_sub = (m_i == -INFINITY) ? 0.f : m_i;
-    float sum = 0.f;
-#pragma unroll
-    for (int x = 0; x < kScores; ++x) {
-      sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), -m_sub));
-      sum += sv[x];
-    }
-    l_i += sum;
-    const Weights<Tr, kScores> pf(sv);
+    while (now.count) {
+      // ---- S^T = K Q^T.  In flight at most: K and V of this step, in that order.
+      if (counted) wait_vmem<T::kCopies>();
+      else wait_vmem<0>();
+      acc_t sacc[NB];
+      W::template multiply_rows<Ar, false>(sacc, now, k_rows, q_operand, lane);
 
-    // ---- O^T += V^T P^T.  In flight at most: V of this step, K of the next.
-    if (counted) wait_vmem<T::kCopies>();
-    else wait_vmem<0>();
-    W::template multiply_cols<Tr, true, kScores>(oacc, now, v_cols, pf);
-    wait_lds();
-    counted = false;
-    if (next.count) counted = walk.template copy<true>(next, tensor_v, lds_v, source, lane);
-    now = next;
+      // ---- K of the next step
+      wait_lds();
+      walk.take(next, lane);
+      counted = false;
+      if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
+
+      // ---- scores: sv holds them up to the positive factor cc, applied inside the exponential (16-bit)
+      float sv[kScores];
+#pragma unroll
+      for (int t = 0; t < NB; ++t)
+#pragma unroll
+        for (int r = 0; r < kRegs; ++r) sv[kRegs * t + r] = sacc[t][r];
+      if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, qi, kq);
+      apply_factor<Tr, kScores>(sv, cc);
+
+      // ---- online softmax of the row.  The reference is the exact running maximum: the largest probabilities then lie at
+      // and just below 1, where rounding to 16 bits costs least.  A maximum that follows in steps of up to 2^8 (as in
+      // attn_mfma.hip) saves most of the rescaling and lets them fall anywhere between two powers of two: errors of the output
+      // against 64 bits of 2.27e-3 instead of 2.09e-3 (bf16, 1024 keys, half of the blocks).
+      float m_blk = sv[0];
+#pragma unroll
+      for (int x = 1; x < kScores; ++x) m_blk = fmaxf(m_blk, sv[x]);
+      m_blk = row_max<SBS>(m_blk) * late_factor<Tr>(cc);
+      const float m_cand = fmaxf(m_i, m_blk);
+      if (__any(m_cand > m_i)) {
+        const float alpha = m_cand > m_i ? __builtin_amdgcn_exp2f(m_i - m_cand) : 1.f;
+        m_i = m_cand;
+        l_i *= alpha;
+#pragma unroll
+        for (int h = 0; h < NS; ++h)
+#pragma unroll
+          for (int r = 0; r < kRegs; ++r) oacc[h][r] *= alpha;
+      }
+      const float m_sub = (m_i == -INFINITY) ? 0.f : m_i;
+      float sum = 0.f;
+#pragma unroll
+      for (int x = 0; x < kScores; ++x) {
+        sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), -m_sub));
+        sum += sv[x];
+      }
+      l_i += sum;
+      const Weights<Ar, kScores> pf(sv);
+
+      // ---- O^T += V^T P^T.  In flight at most: V of this step, K of the next.
+      if (counted) wait_vmem<T::kCopies>();
+      else wait_vmem<0>();
+      W::template multiply_cols<Ar, true, kScores>(oacc, now, v_cols, pf);
+      wait_lds();
+      counted = false;
+      if (next.count) counted = walk.template copy<true>(next, tensor_v, lds_v, source, lane);
+      now = next;
+    }
+  };
+  if constexpr (in_parts<Tr, SBS, kSome>()) {
+    walk_list(SSplit{});
+    if (in_doubt<NS, kRegs>(oacc, l_i)) {  // once more with the fp32 instruction
+      walk.start(a, me.b, me.own, me.there, me.part, me.parts);
+      start_row();
+      walk_list(Tr{});
+    }
+  } else {
+    walk_list(Tr{});
   }
 
   // ---- epilogue

@@ -1,0 +1,92 @@
+"""fp32 products formed from bf16 parts (split_f32.h): their error, values whose parts do not hold them (infinite, NaN, next to
+the largest number, far below one), and the fp32 instruction that forms such sums again."""
+
+import pytest
+import torch
+
+import blksprs_amd as bs
+from tests.helpers import rand_blocks
+
+pytestmark = pytest.mark.gpu
+
+
+def _dense(blocks, layout, sbs):
+    b, r, c = layout.shape
+    out = torch.zeros((b, r, c, sbs, sbs), dtype=torch.float64)
+    out[layout.nonzero(as_tuple=True)] = blocks.double()
+    return out.permute(0, 1, 3, 2, 4).reshape(b, r * sbs, c * sbs)
+
+
+def _compressed(dense, layout, sbs):
+    b, r, c = layout.shape
+    return dense.view(b, r, sbs, c, sbs).permute(0, 1, 3, 2, 4)[layout.nonzero(as_tuple=True)]
+
+
+def _assert_like(got, want, bound, what):
+    """Same infinities and NaN as ``want`` (64 bits, infinite from fp32's largest number on), elsewhere within ``bound``."""
+    got, want = got.detach().double().cpu(), want.float().double()
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[torch.isinf(want)], want[torch.isinf(want)]), what
+    assert ((got - want).abs() <= bound)[finite].all(), (what, float(((got - want).abs() / bound)[finite].max()))
+
+
+def _attention(device, sbs, nh, change=None, grad_scale=1.0):
+    B, n = 2, 5
+    la, full = torch.ones((B, n, n), dtype=torch.bool), torch.ones((B, n, nh), dtype=torch.bool)
+    q, k, v, go = (rand_blocks(B * n * nh, sbs, torch.float32, i) for i in range(4))
+    go = go * grad_scale
+    if change:
+        change(q, k, v, go)
+    ops = [t.to(device).requires_grad_(True) for t in (q, k, v)]
+    fd = full.to(device)
+    out = bs.ops.flash_attention(ops[0], fd, ops[1], fd, ops[2], fd, la.to(device), sbs)
+    grads = torch.autograd.grad(out, ops, go.to(device))
+    q, k, v, go = (_dense(t, full, sbs) for t in (q, k, v, go))
+    scale = (nh * sbs) ** -0.5
+    s = q @ k.transpose(1, 2) * scale
+    p = torch.softmax(s, dim=-1)
+    o = p @ v
+    dv = p.transpose(1, 2) @ go
+    ds = p * (go @ v.transpose(1, 2) - (go * o).sum(-1, keepdim=True)) * scale
+    want = (o, ds @ k, ds.transpose(1, 2) @ q, dv)
+    return (out, *grads), [_compressed(t, full, sbs) for t in want]
+
+
+@pytest.mark.parametrize("sbs,nh", [(32, 1), (32, 2), (32, 3), (32, 4), (64, 1), (64, 2)])
+@pytest.mark.parametrize("grad_scale", [1.0, 2.0 ** -112, 2.0 ** 100])
+def test_attention(device, sbs, nh, grad_scale):
+    """Relative errors (2-norm) against 64 bits; the largest seen is 4e-7.  Gradients of about 2^-112 have lost parts."""
+    got, want = _attention(device, sbs, nh, grad_scale=grad_scale)
+    for what, g, w in zip(("O", "dQ", "dK", "dV"), got, want):
+        g = g.detach().double().cpu()
+        assert float((g - w).norm() / w.norm()) < 1e-6, what
+
+
+@pytest.mark.parametrize("sbs,nh", [(32, 1), (32, 2), (32, 4), (64, 1), (64, 2)])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
+@pytest.mark.parametrize("where", ["v", "go"])
+def test_attention_of_single_values(device, sbs, nh, value, where):
+    """A value of V or of dO that its parts do not hold: what it reaches is what it is in 64 bits, the rest as exact as ever."""
+    def change(q, k, v, go):
+        (v if where == "v" else go)[3, 7, 11] = value
+
+    got, want = _attention(device, sbs, nh, change)
+    names = ("O", "dQ", "dK", "dV")
+    for what, g, w in zip(names, got, want):
+        g = g.detach().double().cpu()
+        if where == "go" and what in ("O", "dV") or where == "v" and what in ("O", "dV"):
+            _assert_like(g, w, 1e-4 + 1e-4 * w.abs(), what)
+        elif value != 3.4e38:
+            assert not torch.isfinite(g).all(), what
+            untouched = torch.isfinite(w)
+            assert torch.isfinite(g[untouched]).all(), what
+
+
+@pytest.mark.parametrize("sbs,nh", [(32, 2), (64, 1)])
+def test_attention_of_infinite_keys(device, sbs, nh):
+    """Scores of +inf make NaN of a query's row, scores of -inf leave a key out."""
+    def change(q, k, v, go):
+        k[2, 1, 3] = float("inf")
+
+    got, want = _attention(device, sbs, nh, change)
+    _assert_like(got[0], want[0], 1e-4 + 1e-4 * want[0].abs(), "O")
