@@ -1,8 +1,9 @@
 // Block-sparse GEMM: out[n] = sum over the contraction list of block n of x[px] @ y[py].
 //
 // Block sizes 16 and 32: a wave owns a run of consecutive output blocks and walks their pairs (matmul_small16_kernel,
-// matmul_small16_f32_kernel, matmul_runs32_kernel); larger blocks: a workgroup owns a 64 x 64 tile (matmul_quad_kernel).  Every
-// kernel walks a block's pairs in ascending k, so only non-zero K-blocks are touched and the fp32 accumulation order is fixed.
+// matmul_small16_f32_kernel, matmul_runs32_kernel); larger blocks: a workgroup owns a 64 x 64 tile (matmul_quad_kernel, and
+// matmul_split.hip for fp32).  Every kernel walks a block's pairs in ascending k, so only non-zero K-blocks are touched and the
+// fp32 accumulation order is fixed.
 //
 // An operand whose k index is contiguous in memory (x, or y read transposed) is read from LDS as it lies; one whose k index
 // is strided (y, or x read transposed) through the transposing LDS read for 16-bit types, and by 32-bit reads for fp32.
@@ -15,6 +16,13 @@
 #include <type_traits>
 
 #include "attn_mfma_common.h"
+
+namespace bsa {
+// matmul_split.hip
+int matmul_split_f32(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs,
+                     const int32_t *block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int sbs, int trans_x, int trans_y,
+                     hipStream_t s);
+}  // namespace bsa
 
 namespace {
 
@@ -268,46 +276,33 @@ __global__ __launch_bounds__(256, 5) void matmul_runs32_kernel(
   }
 }
 
-// ---- LDS chunks of the kernel whose workgroup shares a tile: 64 rows of 128 bytes (k contiguous, or 16-bit k rows), or
-// 32 k rows of 256 bytes (fp32, k strided)
+// ---- LDS chunks of the kernel whose workgroup shares a tile: 64 rows of 128 bytes (k contiguous, or k rows)
 
-// chunk index XOR of a 128-byte row, by row % 8: row reads of eight consecutive rows fall on eight chunks; for 16-bit
-// elements also the four rows of a transposing read on different halves of their rows
-template <int ES>
-__device__ inline int quad_swizzle(int r) {
-  return ES == 2 ? bsa::mfma::t_swizzle(r & 7) : r & 7;
-}
+// chunk index XOR of a 128-byte row, by row % 8: row reads of eight consecutive rows fall on eight chunks, and the four
+// rows of a transposing read on different halves of their rows
+__device__ inline int quad_swizzle(int r) { return bsa::mfma::t_swizzle(r & 7); }
 // 16 bytes of k of one row
-template <int ES>
 __device__ inline u32x4 quad_rows(const char *lds, int row, int chunk) {
-  return *reinterpret_cast<const u32x4 *>(lds + row * 128 + ((chunk ^ quad_swizzle<ES>(row)) << 4));
+  return *reinterpret_cast<const u32x4 *>(lds + row * 128 + ((chunk ^ quad_swizzle(row)) << 4));
 }
-// the same values of k (step s: 16-bit 16 s + 8 (lane / 32) .. + 7, fp32 8 s + 4 (lane / 32) .. + 3) of column
-// col0 + lane % 32, from k rows
-template <int ES>
+// the same values of k (step s: 16 s + 8 (lane / 32) .. + 7) of column col0 + lane % 32, from k rows
 __device__ inline u32x4 quad_cols(const char *lds, int col0, int s, int lane) {
-  const int kg = lane >> 5;
-  if constexpr (ES == 2) {
-    const int chunk = (col0 >> 3) + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-    u32x4 v;
+  const int kg = lane >> 5, chunk = (col0 >> 3) + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+  u32x4 v;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int r = 16 * s + 8 * kg + 4 * i + ((lane & 15) >> 2);
-      const char *p = lds + r * 128 + ((chunk ^ quad_swizzle<2>(r)) << 4) + ((lane & 1) << 3);
-      const auto t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4 *)p);
-      const u32x2 w = __builtin_bit_cast(u32x2, t);
-      v[2 * i] = w[0];
-      v[2 * i + 1] = w[1];
-    }
-    return v;
-  } else {
-    const uint32_t *p = reinterpret_cast<const uint32_t *>(lds) + (8 * s + 4 * kg) * 64 + col0 + (lane & 31);
-    return u32x4{p[0], p[64], p[128], p[192]};
+  for (int i = 0; i < 2; ++i) {
+    const int r = 16 * s + 8 * kg + 4 * i + ((lane & 15) >> 2);
+    const char *p = lds + r * 128 + ((chunk ^ quad_swizzle(r)) << 4) + ((lane & 1) << 3);
+    const auto t = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4 *)p);
+    const u32x2 w = __builtin_bit_cast(u32x2, t);
+    v[2 * i] = w[0];
+    v[2 * i + 1] = w[1];
   }
+  return v;
 }
 
-// sbs >= 64 on the tile path: fp32, and 16-bit elements at sbs 128 and above (or where neither the row nor the line kernel
-// applies).  A workgroup of four waves owns one 64 x 64 tile of an output block, each wave a 32 x 32 quadrant, and walks
+// 16-bit elements at sbs 128 and above, or at 64 where neither the row nor the line kernel applies (fp32: matmul_split.hip).
+// A workgroup of four waves owns one 64 x 64 tile of an output block, each wave a 32 x 32 quadrant, and walks
 // the block's pair list in chunks of 128 bytes of k; the chunk of x and the chunk of y lie in LDS for all four waves,
 // double buffered, copied asynchronously while the chunk before is multiplied, with one barrier per chunk.
 //
@@ -315,9 +310,7 @@ __device__ inline u32x4 quad_cols(const char *lds, int col0, int s, int lane) {
 // takes the whole difference: 2080 tiles of 4 to 16 pairs on 2048 places of a wave (two per SIMD, by registers and LDS) run
 // as long as the SIMD with the two longest, and a workgroup of four such tiles holds its LDS until the longest is done.
 // Here the four waves of a workgroup are equal, five workgroups share a compute unit, and tiles are handed out as places
-// become free.  fp32, 8 x 2048^3 at 25 %: 0.126 -> 0.103
-// ms forward, 0.134 and 0.125 -> 0.099 ms for the gradients (83 TFLOP/s; a dense layout 118, rocBLAS' fp32 product 154);
-// bf16, sbs 128, 8 x 2944 x 3968 x 2048 at 25 %: 0.064 -> 0.059, 0.061 -> 0.055, 0.064 -> 0.052 ms.  What is left is the
+// become free.  bf16, sbs 128, 8 x 2944 x 3968 x 2048 at 25 %: 0.064 -> 0.059, 0.061 -> 0.055, 0.064 -> 0.052 ms.  What is left is the
 // chain in front of a tile's first chunk (order, offsets, pairs, operands) and the last tiles of a launch.
 template <typename Tr, bool XT, bool YT>
 __global__ __launch_bounds__(256, 5) void matmul_quad_kernel(const char *__restrict__ x, const char *__restrict__ y,
@@ -327,7 +320,7 @@ __global__ __launch_bounds__(256, 5) void matmul_quad_kernel(const char *__restr
                                                              const int32_t *__restrict__ block_order, int64_t first,
                                                              int64_t end, int sbs, int side_log2, int64_t nnz_x,
                                                              int64_t nnz_y) {
-  constexpr int ES = Tr::kElem, KC = 128 / ES;  // k per chunk
+  constexpr int ES = 2, KC = 128 / ES;  // k per chunk
   constexpr int kOperand = 64 * 128, kBuffer = 2 * kOperand;
   __shared__ __attribute__((aligned(1024))) char smem[2 * kBuffer];
   const int lane = threadIdx.x & 63;
@@ -349,17 +342,13 @@ __global__ __launch_bounds__(256, 5) void matmul_quad_kernel(const char *__restr
   const int p_end = __builtin_amdgcn_readfirstlane(pair_offsets[n + 1]);
 
   // Copies: one instruction moves 1 KiB, lane l supplying the 16 bytes at position l; wave w takes KiB 2 w and 2 w + 1 of
-  // either chunk.  An operand whose k is contiguous: 64 rows of 128 bytes, eight to a KiB, chunk index swizzled by the row.
-  // Otherwise KC rows of k: 128 bytes each (16-bit, the same swizzle) or 256 (fp32, as they lie).
+  // either chunk: 64 rows (of k, unless k is contiguous) of 128 bytes, eight to a KiB, chunk index swizzled by the row.
   const int row8 = lane >> 3;
-  const uint32_t off128 = (uint32_t)row8 * ld + (uint32_t)(((lane & 7) ^ quad_swizzle<ES>(row8)) << 4);
-  const uint32_t off256 = (uint32_t)(lane >> 4) * ld + (uint32_t)((lane & 15) << 4);
-  auto copy_operand = [&](const char *base, bool k_strided, char *dst) {
-    const bool wide = ES == 4 && k_strided;
-    const int rows = wide ? 4 : 8;
+  const uint32_t off128 = (uint32_t)row8 * ld + (uint32_t)(((lane & 7) ^ quad_swizzle(row8)) << 4);
+  auto copy_operand = [&](const char *base, char *dst) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      bsa::mfma::copy_1k_to_lds(base + (int64_t)((2 * wave + i) * rows) * ld, wide ? off256 : off128, dst + (2 * wave + i) * 1024);
+      bsa::mfma::copy_1k_to_lds(base + (int64_t)((2 * wave + i) * 8) * ld, off128, dst + (2 * wave + i) * 1024);
   };
   // 64 entries of the pair list at a time, one per lane
   int win_base = p_begin, win_x = 0, win_y = 0;
@@ -387,8 +376,8 @@ __global__ __launch_bounds__(256, 5) void matmul_quad_kernel(const char *__restr
     const int64_t k_along = (int64_t)kc * 128, k_down = (int64_t)kc * KC * ld;
     const int64_t i_down = (int64_t)ti * 64 * ld, i_along = (int64_t)ti * 64 * ES;
     const int64_t j_down = (int64_t)tj * 64 * ld, j_along = (int64_t)tj * 64 * ES;
-    copy_operand(x + px * block_bytes + (XT ? k_down + i_along : i_down + k_along), XT, buf);
-    copy_operand(y + py * block_bytes + (YT ? j_down + k_along : k_down + j_along), !YT, buf + kOperand);
+    copy_operand(x + px * block_bytes + (XT ? k_down + i_along : i_down + k_along), buf);
+    copy_operand(y + py * block_bytes + (YT ? j_down + k_along : k_down + j_along), buf + kOperand);
     if (++kc == n_chunks) kc = 0, ++p;
   };
 
@@ -411,8 +400,8 @@ __global__ __launch_bounds__(256, 5) void matmul_quad_kernel(const char *__restr
     u32x4 fx[4], fy[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      fx[s] = XT ? quad_cols<ES>(bx, 32 * wi, s, lane) : quad_rows<ES>(bx, 32 * wi + li, 2 * s + kg);
-      fy[s] = YT ? quad_rows<ES>(by, 32 * wj + li, 2 * s + kg) : quad_cols<ES>(by, 32 * wj, s, lane);
+      fx[s] = XT ? quad_cols(bx, 32 * wi, s, lane) : quad_rows(bx, 32 * wi + li, 2 * s + kg);
+      fy[s] = YT ? quad_rows(by, 32 * wj + li, 2 * s + kg) : quad_cols(by, 32 * wj, s, lane);
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s) acc = Tr::mfma(fy[s], fx[s], acc);
@@ -427,11 +416,8 @@ __global__ __launch_bounds__(256, 5) void matmul_quad_kernel(const char *__restr
   for (int q = 0; q < 4; ++q) {
     const int at = (8 * q + 4 * kg) * ES;  // byte of the row
     char *dst = stage + li * kRow + ((((at >> 4) ^ li) & (kChunks - 1)) << 4) + (at & 15);
-    if constexpr (ES == 2)
-      *reinterpret_cast<uint2 *>(dst) = uint2{(uint32_t)Tr::round(acc[4 * q]) | ((uint32_t)Tr::round(acc[4 * q + 1]) << 16),
-                                              (uint32_t)Tr::round(acc[4 * q + 2]) | ((uint32_t)Tr::round(acc[4 * q + 3]) << 16)};
-    else
-      *reinterpret_cast<f32x4 *>(dst) = f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+    *reinterpret_cast<uint2 *>(dst) = uint2{(uint32_t)Tr::round(acc[4 * q]) | ((uint32_t)Tr::round(acc[4 * q + 1]) << 16),
+                                            (uint32_t)Tr::round(acc[4 * q + 2]) | ((uint32_t)Tr::round(acc[4 * q + 3]) << 16)};
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   char *ob = out + n * block_bytes + (int64_t)(64 * ti + 32 * wi) * ld + (64 * tj + 32 * wj) * ES;
@@ -765,7 +751,10 @@ int launch_any(const void *x, const void *y, void *out, const int32_t *pair_offs
   }
   if (sbs == 32)
     return launch_runs32<Tr>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, trans_x, trans_y, s);
-  return launch_quad<Tr>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, sbs, trans_x, trans_y, s);
+  if constexpr (std::is_same_v<Tr, F32Traits>)
+    return bsa::matmul_split_f32(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, sbs, trans_x, trans_y, s);
+  else
+    return launch_quad<Tr>(x, y, out, pair_offsets, pairs, block_order, nnz_o, nnz_x, nnz_y, sbs, trans_x, trans_y, s);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }

@@ -5,9 +5,11 @@ import pytest
 import torch
 
 import blksprs_amd as bs
-from tests.helpers import rand_blocks
+from tests.helpers import rand_blocks, rand_layout
 
 pytestmark = pytest.mark.gpu
+
+EPS = 2.0 ** -24
 
 
 def _dense(blocks, layout, sbs):
@@ -28,6 +30,70 @@ def _assert_like(got, want, bound, what):
     finite = torch.isfinite(want)
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[torch.isinf(want)], want[torch.isinf(want)]), what
     assert ((got - want).abs() <= bound)[finite].all(), (what, float(((got - want).abs() / bound)[finite].max()))
+
+
+def _matmul(device, sbs, R, K, C, density, change=None, x_scale=1.0, y_scale=1.0):
+    B = 2
+    lx, ly = rand_layout((B, R, K), density, 1, ensure_rows=True), rand_layout((B, K, C), density, 2, ensure_rows=True)
+    lo = torch.ones((B, R, C), dtype=torch.bool)
+    x, y = rand_blocks(int(lx.sum()), sbs, torch.float32, 3), rand_blocks(int(ly.sum()), sbs, torch.float32, 4)
+    go = rand_blocks(int(lo.sum()), sbs, torch.float32, 5)
+    x, y = x * x_scale, y * y_scale
+    if change:
+        change(x, y)
+    xd, yd = (t.to(device).requires_grad_(True) for t in (x, y))
+    out = bs.ops.matmul(xd, lx.to(device), yd, ly.to(device), lo.to(device), sbs)
+    dx, dy = torch.autograd.grad(out, (xd, yd), go.to(device))
+    x64, y64, g64 = _dense(x, lx, sbs), _dense(y, ly, sbs), _dense(go, lo, sbs)
+    # pairs of blocks that are not there add nothing, where 0 * inf would add NaN: block by block over k
+    o64 = torch.zeros_like(g64)
+    dx64, dy64 = torch.zeros_like(x64), torch.zeros_like(y64)
+    size_o, size_x, size_y = o64.clone(), dx64.clone(), dy64.clone()
+    for b in range(B):
+        for k in range(K):
+            ks = slice(k * sbs, (k + 1) * sbs)
+            for i in range(R):
+                rows = slice(i * sbs, (i + 1) * sbs)
+                for j in range(C):
+                    cols = slice(j * sbs, (j + 1) * sbs)
+                    if lx[b, i, k] and ly[b, k, j]:
+                        o64[b, rows, cols] += x64[b, rows, ks] @ y64[b, ks, cols]
+                        size_o[b, rows, cols] += x64[b, rows, ks].abs() @ y64[b, ks, cols].abs()
+                    if ly[b, k, j]:
+                        dx64[b, rows, ks] += g64[b, rows, cols] @ y64[b, ks, cols].T
+                        size_x[b, rows, ks] += g64[b, rows, cols].abs() @ y64[b, ks, cols].T.abs()
+                    if lx[b, i, k]:
+                        dy64[b, ks, cols] += x64[b, rows, ks].T @ g64[b, rows, cols]
+                        size_y[b, ks, cols] += x64[b, rows, ks].T.abs() @ g64[b, rows, cols].abs()
+    for what, got, want, size, layout, n in (("O", out, o64, size_o, lo, K), ("dX", dx, dx64, size_x, lx, C), ("dY", dy, dy64, size_y, ly, R)):
+        # six roundings for 16 values, three dropped products of 2^-26 together, and what underflows
+        roundings = 6 * n * sbs / 16 + 4
+        bound = roundings * 2 * EPS * _compressed(size, layout, sbs) + 1e-37
+        _assert_like(got, _compressed(want, layout, sbs), bound, what)
+
+
+@pytest.mark.parametrize("sbs", [64, 128])
+@pytest.mark.parametrize("R,K,C,density", [(1, 1, 1, 1.0), (3, 2, 5, 0.4), (1, 70, 2, 1.0)])
+def test_matmul(device, sbs, R, K, C, density):
+    _matmul(device, sbs, R, K if sbs == 64 else min(K, 34), C, density)
+
+
+@pytest.mark.parametrize("x_scale,y_scale", [(2.0 ** -115, 1.0), (1.0, 2.0 ** -118), (2.0 ** 100, 2.0 ** 10), (2.0 ** -60, 2.0 ** -50)])
+def test_matmul_of_small_and_large_operands(device, x_scale, y_scale):
+    _matmul(device, 64, 2, 3, 2, 0.7, x_scale=x_scale, y_scale=y_scale)
+
+
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan"), 3.4e38])
+def test_matmul_of_single_values(device, value):
+    """One value of x and one of y; 3.4e38 rounds to infinity in bf16."""
+    def change(x, y):
+        if value == 3.4e38:
+            x *= 2.0 ** -20
+            y *= 2.0 ** -20
+        x[0, 5, 40] = value
+        y[-1, 63, 0] = value
+
+    _matmul(device, 64, 2, 3, 2, 0.7, change)
 
 
 def _attention(device, sbs, nh, change=None, grad_scale=1.0):
