@@ -108,6 +108,8 @@ SIGNATURES = {
                                 c_int64, c_int64, c_int, c_int, c_void_p]),
     "bsa_attn_fwd_records": (c_int, [ctypes.POINTER(AttnArgs), c_void_p, c_void_p, c_void_p]),
     "bsa_attn_mask_dead": (c_int, [c_void_p, c_int64, ctypes.c_int32, c_void_p, c_void_p]),
+    "bsa_causal_lengths_range": (c_int, [c_void_p, c_int64, c_void_p, c_void_p]),
+    "bsa_causal_lengths_wait": (c_int, [c_void_p, c_int64, c_void_p]),
     "bsa_attn_bwd_scratch_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int64, c_int64]),
     "bsa_attn_bwd_ds_bytes": (c_size_t, [c_int64, ctypes.c_int32]),
     "bsa_attn_shares_piece": (c_int, [ctypes.POINTER(AttnArgs), c_int, c_int64, c_int64, ctypes.POINTER(c_int64),

@@ -120,6 +120,69 @@ extern "C" int bsa_attn_fwd_records(const bsa_attn_args *a, const int32_t *group
   return bsa::attn_fwd_records(*a, group_entries, records, bsa::as_stream(stream));
 }
 
+namespace {
+
+// One workgroup: a caller's sequences are few, and the launch in front of the attention kernels takes its 3 us anyway.  Written
+// by the kernel itself: a copy to the host passes a copy engine, and what follows in the stream waits for that.  range[2]: the
+// other two are there.
+__global__ __launch_bounds__(256) void causal_lengths_range_kernel(const int64_t *__restrict__ lengths, int64_t n, int64_t *range) {
+  __shared__ int64_t low[256], high[256];
+  int64_t lo = lengths[0], hi = lo;
+  for (int64_t i = threadIdx.x; i < n; i += 256) {
+    const int64_t v = lengths[i];
+    lo = v < lo ? v : lo;
+    hi = v > hi ? v : hi;
+  }
+  low[threadIdx.x] = lo;
+  high[threadIdx.x] = hi;
+  for (int step = 128; step > 0; step >>= 1) {
+    __syncthreads();
+    if (threadIdx.x < step) {
+      const int64_t l = low[threadIdx.x + step], h = high[threadIdx.x + step];
+      if (l < low[threadIdx.x]) low[threadIdx.x] = l;
+      if (h > high[threadIdx.x]) high[threadIdx.x] = h;
+    }
+  }
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(range, low[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(range + 1, high[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(range + 2, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+}  // namespace
+
+extern "C" int bsa_causal_lengths_range(const int64_t *lengths, int64_t n, int64_t *range, bsa_stream_t stream) {
+  const char *who = "bsa_causal_lengths_range";
+  BSA_REQUIRE(n >= 1, "%s: no lengths", who);
+  BSA_REQUIRE(lengths != nullptr && range != nullptr, "%s: NULL argument", who);
+  __atomic_store_n(range + 2, (int64_t)0, __ATOMIC_RELEASE);
+  causal_lengths_range_kernel<<<1, 256, 0, bsa::as_stream(stream)>>>(lengths, n, range);
+  return bsa::check_launch(who);
+}
+
+// Reads the flag rather than waiting for an event, which costs the host some 6 us more; a stream that is done, or that
+// failed, ends the wait as well.
+extern "C" int bsa_causal_lengths_wait(const int64_t *range, int64_t longest, bsa_stream_t stream) {
+  const char *who = "bsa_causal_lengths_wait";
+  BSA_REQUIRE(range != nullptr, "%s: NULL argument", who);
+  for (int turn = 1; __atomic_load_n(range + 2, __ATOMIC_ACQUIRE) == 0; ++turn) {
+    if ((turn & 0xfff) != 0) {
+      __builtin_ia32_pause();
+      continue;
+    }
+    turn = 0;
+    const hipError_t state = hipStreamQuery(bsa::as_stream(stream));
+    if (state == hipErrorNotReady) {
+      if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();  // not to be taken for a launch's
+      continue;
+    }
+    if (state != hipSuccess) return bsa::fail(BSA_ELAUNCH, "%s: %s", who, hipGetErrorString(state));
+    if (__atomic_load_n(range + 2, __ATOMIC_ACQUIRE) == 0) return bsa::fail(BSA_ELAUNCH, "%s: the search left no result", who);
+  }
+  return range[0] < 0 || range[1] > longest ? 1 : BSA_OK;
+}
+
 extern "C" int bsa_attn_mask_dead(const void *mask, int64_t n_mask_blocks, int32_t sbs, uint8_t *dead,
                                   bsa_stream_t stream) {
   const char *who = "bsa_attn_mask_dead";

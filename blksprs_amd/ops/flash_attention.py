@@ -265,8 +265,52 @@ def _smallest_and_largest(values: Tensor) -> tuple[int, int]:
     return smallest, largest
 
 
+# Up to this many values one workgroup finds their range in the time of a launch (bsa_causal_lengths_range).
+_RANGED_BY_ONE_WORKGROUP = 4096
+
+_RANGE_READERS = threading.local()
+_BEYOND_RANGE = "causal_lengths values must be between zero and {}"
+
+
+class _RangeOfLengths:
+    """The range check of causal lengths around the launch of the kernels that read them: ``start`` enqueues the search for
+    the smallest and the largest in front of it, ``finish`` waits for the two and raises as ever.  The kernels only compare
+    lengths with positions, so what they make of a length that is then refused is dropped, and the device does not idle
+    while the host reads: 8 prompts of 128 to 256 tokens, a new tensor of lengths for each, 43.9 -> 33.3 us a call.
+
+    Every ``start`` is followed by a ``finish``, which sees the device pass and gives the pinned words back to the thread: as
+    many as a thread has calls inside one another (hooks of saved tensors)."""
+
+    __slots__ = ("source", "key", "lengths", "longest", "words", "stream")
+
+    def __init__(self, source, key, lengths, longest):
+        self.source, self.key, self.lengths, self.longest = source, key, lengths, longest
+
+    def start(self) -> None:
+        device = self.lengths.device
+        free = getattr(_RANGE_READERS, "free", None)
+        if free is None:
+            free = _RANGE_READERS.free = []
+        self.words = free.pop() if free else torch.empty(3, dtype=torch.int64, pin_memory=True)
+        self.stream = _capi.stream(device)
+        with _capi.on_device(device):
+            _capi.call("bsa_causal_lengths_range", self.lengths.data_ptr(), self.lengths.numel(), self.words.data_ptr(),
+                       self.stream)
+
+    def finish(self) -> None:
+        rc = _capi.load().bsa_causal_lengths_wait(self.words.data_ptr(), self.longest, self.stream)
+        if rc != 1:
+            _capi.check(rc, "bsa_causal_lengths_wait")
+        _RANGE_READERS.free.append(self.words)
+        if rc == 1:
+            raise ValueError(_BEYOND_RANGE.format(self.longest))
+        _LENGTHS_SEEN.last = (self.source, self.key, self.lengths)
+
+
 def _normalise_causal_lengths(causal_lengths: Tensor | None, n_batches: int, q_length: int, k_length: int,
-                              device: torch.device) -> Tensor | None:
+                              device: torch.device, later: list | None = None) -> Tensor | None:
+    """The lengths as the kernels read them.  With a list ``later`` the check of their range may be left to the caller: it is
+    then the list's one entry."""
     if causal_lengths is None:
         return None
     if not isinstance(causal_lengths, Tensor):
@@ -287,9 +331,13 @@ def _normalise_causal_lengths(causal_lengths: Tensor | None, n_batches: int, q_l
     key = (causal_lengths._version, int(q_length)) if not torch.is_inference(causal_lengths) else None
     if seen is None or seen[0] is not causal_lengths or seen[1] != key or key is None:
         lengths = ensure_contiguous(causal_lengths.to(dtype=torch.int64))
+        if (later is not None and lengths.is_cuda and 0 < lengths.numel() <= _RANGED_BY_ONE_WORKGROUP
+                and not torch.cuda.is_current_stream_capturing()):
+            later.append(_RangeOfLengths(causal_lengths, key, lengths, int(q_length)))
+            return lengths
         smallest, largest = _smallest_and_largest(lengths)
         if smallest < 0 or largest > q_length:
-            raise ValueError(f"causal_lengths values must be between zero and {q_length}")
+            raise ValueError(_BEYOND_RANGE.format(q_length))
         _LENGTHS_SEEN.last = (causal_lengths, key, lengths)
     return _LENGTHS_SEEN.last[2]
 
@@ -698,8 +746,9 @@ def flash_attention(q: BlksprsTensor, sparsity_layout_q: Tensor,
 
     attention_shape = (n_batches, n_seq_blocks_q, n_seq_blocks_k)
     validate_shape(attention_layout, attention_shape, "attention_layout")
+    range_check: list[_RangeOfLengths] = []
     lengths = _normalise_causal_lengths(causal_lengths, n_batches, n_seq_blocks_q * sparsity_block_size,
-                                        n_seq_blocks_k * sparsity_block_size, q.device)
+                                        n_seq_blocks_k * sparsity_block_size, q.device, range_check)
 
     if sparsity_layout_o is not None:
         sparsity_layout_o = ensure_contiguous(sparsity_layout_o)
@@ -787,7 +836,13 @@ def flash_attention(q: BlksprsTensor, sparsity_layout_q: Tensor,
     needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad
                                               or (attention_bias is not None and attention_bias.requires_grad))
     meta.shares = _row_shares(meta, q.dtype, q.device, needs_grad)
-    if not needs_grad:
+    if range_check:
+        range_check[0].start()
+    try:
         # nothing to differentiate: the launch itself, without the autograd machinery around it
-        return BlksprsTensor.wrap(_forward_launch(q, k, v, attention_bias, mask_bytes, lengths, meta)[0])
-    return BlksprsTensor.wrap(_FlashAttention.apply(q, k, v, attention_bias, mask_bytes, lengths, meta))
+        out = (_FlashAttention.apply(q, k, v, attention_bias, mask_bytes, lengths, meta) if needs_grad
+               else _forward_launch(q, k, v, attention_bias, mask_bytes, lengths, meta)[0])
+    finally:
+        if range_check:
+            range_check[0].finish()
+    return BlksprsTensor.wrap(out)

@@ -478,6 +478,15 @@ int bsa_attn_fwd(const bsa_attn_args *args, bsa_stream_t stream);
  */
 int bsa_attn_mask_dead(const void *mask, int64_t n_mask_blocks, int32_t sbs, uint8_t *dead, bsa_stream_t stream);
 
+/*
+ * Range check of n >= 1 causal lengths around the launch of the kernels that read them (which only compare lengths with
+ * positions; the reference reads the range first, blksprs/ops/flash_attention.py:239-241).  The first call enqueues the
+ * search; range: three words of pinned host memory, the caller's until the second has returned, which waits for the
+ * search, not for what was enqueued behind it: BSA_OK, or 1 where some length is negative or above `longest`.
+ */
+int bsa_causal_lengths_range(const int64_t *lengths, int64_t n, int64_t *range, bsa_stream_t stream);
+int bsa_causal_lengths_wait(const int64_t *range, int64_t longest, bsa_stream_t stream);
+
 /* Size in bytes of bsa_attn_args.bwd_scratch for these sizes (16-byte aligned buffer). */
 size_t bsa_attn_bwd_scratch_bytes(int64_t B, int64_t nq, int64_t nk, int64_t n_layout_blocks, int64_t n_mask_blocks);
 /* Size in bytes of bsa_attn_args.bwd_ds for an attention layout of n_layout_blocks active blocks:

@@ -97,3 +97,45 @@ def test_range_check_of_causal_lengths_follows_changes_in_place(device):
     lengths.sub_(2 * sbs)
     shorter = call()
     assert torch.all(shorter[n - 1] == 0) and not torch.equal(shorter, first)
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 4096, 4097])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_lengths_beyond_the_range_are_refused_wherever_they_are(device, n, dtype):
+    """One workgroup looks for the range up to 4096 lengths, torch beyond; every sequence is one block of 16."""
+    sbs = 16
+    layout = torch.ones((n, 1, 1), dtype=torch.bool, device=device)
+    q = torch.randn((n, sbs, sbs), device=device)
+    lengths = (torch.arange(n, device=device) % (sbs + 1)).to(dtype)
+    call = lambda l: bs.ops.flash_attention(q, layout, q, layout, q, layout, layout, sbs, causal_lengths=l)
+    for l in (lengths, torch.full_like(lengths, sbs), torch.zeros_like(lengths)):
+        out = call(l)
+        assert torch.equal((out != 0).any(dim=2).sum(dim=1), l.long())
+    for place in {0, n // 3, n - 1}:
+        for value in (-1, sbs + 1, -(1 << 31), (1 << 31) - 1):
+            bad = lengths.clone()
+            bad[place] = value
+            with pytest.raises(ValueError, match="between zero and 16"):
+                call(bad)
+    assert torch.equal(call(lengths.clone()), call(lengths))
+
+
+def test_range_checks_inside_one_another(device):
+    """A hook of saved tensors that calls the operator itself, between the outer call's launch and its check."""
+    sbs, n = 16, 2
+    layout = torch.ones((1, n, 1), dtype=torch.bool, device=device)
+    la = torch.ones((1, n, n), dtype=torch.bool, device=device)
+    q = torch.randn((n, sbs, sbs), device=device, requires_grad=True)
+    call = lambda t, length: bs.ops.flash_attention(t, layout, t, layout, t, layout, la, sbs,
+                                                    causal_lengths=torch.tensor([length], device=device))
+    inner = []
+
+    def pack(t):
+        if not inner:
+            inner.append(call(q.detach(), 5))
+        return t
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+        with pytest.raises(ValueError, match="between zero and 32"):
+            call(q, 33)
+    assert len(inner) == 1
