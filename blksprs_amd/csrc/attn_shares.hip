@@ -156,9 +156,9 @@ static int least_parts(const bsa_attn_args &a, bool key_rows) {
 // waves: what the chip holds of these kernels at a time (their registers and LDS).  least: entries of a wave's walk that cost
 // about as much as its start and end, six steps (16-bit; four of fp32, whose products take longer).  Shares pay where the
 // longest share of waves_per_row is at least eight steps (fp32: four) and half a mean above the mean, or where a launch of more
-// than one round would start its longest lists, more than twice the mean, anywhere, and the walk of one takes 22 steps (fp32:
-// 12) or more: below, some 3 us of a launch (33 x 272, sbs 16, windows of 10 blocks, fp32: 15.1 -> 12.2), a new layout's first call
-// pays 70 us for them.
+// than one round would start its longest lists, more than twice the mean, anywhere, and the walk of one takes 22 steps (14 at
+// head dimensions above 64, fp32 8) or more: below, some 3 us of a launch (33 x 272, sbs 16, windows of 10 blocks, fp32: 15.1 ->
+// 12.2), a new layout's first call pays 70 us for them.
 int64_t attn_shares_piece(const bsa_attn_args &a, bool key_rows, int64_t n_entries, int64_t longest) {
   const int halves = halves_of(a);
   const bool wide = a.dtype == BSA_F32;
@@ -173,7 +173,8 @@ int64_t attn_shares_piece(const bsa_attn_args &a, bool key_rows, int64_t n_entri
   const int split = least_parts(a, key_rows);
   const int64_t share = halves * longest / split, worth = (wide ? 4 : 8) * per_step;
   const bool long_shares = 2 * share > 3 * piece && share >= piece + worth;
-  const bool order = rows * split > waves && halves * longest * rows > 2 * entries && share >= least + 2 * worth;
+  const bool order = rows * split > waves && halves * longest * rows > 2 * entries &&
+                     share >= least + (wide || !small_head ? worth : 2 * worth);
   return long_shares || order ? piece : 0;
 }
 
