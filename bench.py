@@ -75,7 +75,7 @@ PROFILE_STEMS = {
     "a1bwd": "attn_small_kernels_a1bwd_fp32_reference_benchmark_backward",
     "m32": "matmul_runs32_kernel_m32_bf16_sbs32",
     "m128": "matmul_quad_kernel_m128_bf16_sbs128",
-    "mf32": "matmul_quad_kernel_mf32_fp32_sbs64",
+    "mf32": "matmul_split_kernel_mf32_fp32_sbs64",
     "v1": "to_sparse_kernel_v1_bf16_to_sparse",
     "v2": "to_dense_kernel_v2_bf16_to_dense",
     "t1": "transpose_blocks16_kernel_t1_bf16_transpose",
@@ -399,7 +399,7 @@ def matmul_workload(name, B, n, sbs, dtype, density, ensure_rows, value_scale, d
                           f"torch matmul + to_sparse, {dt * reps:.1f} s"}
 
     dt_name = {torch.bfloat16: "bf16", torch.float16: "f16", torch.float32: "f32"}[dtype]
-    tile_kernel = ("matmul_quad_kernel" if sbs >= 64 else "matmul_runs32_kernel" if sbs == 32 else
+    tile_kernel = (("matmul_split_kernel" if dtype == torch.float32 else "matmul_quad_kernel") if sbs >= 64 else "matmul_runs32_kernel" if sbs == 32 else
                    "matmul_small16_kernel" if dtype != torch.float32 else "matmul_small16_f32_kernel")
     if backward:
         kernel = ("matmul_lines_kernel (two launches: dX by rows of dO, dY by its columns)"
