@@ -19,7 +19,7 @@
 // to overlap it.  Against the fp32 matrix-core kernels that ran these shapes before (48 x 4096 queries, sbs 32, head
 // dimension 64, fp16, 33 key blocks per query block): delta + zero fill 0.071 -> 0, dK / dV 1.89 -> 0.125 ms (530 TFLOP/s),
 // dQ 1.24 -> 0.090 ms (delta included); fp32, sbs 32, products from bf16 parts (split_f32.h), 8 x 2048 queries, half of the
-// blocks, head dimension 64: dK / dV 94.5 -> 73.0, dQ 74.8 -> 57.7 us (118 and 112 TFLOP/s) against the fp32 instruction.  fp32
+// blocks, head dimension 64: dK / dV 94.5 -> 75.5, dQ 74.8 -> 59.0 us (114 and 109 TFLOP/s) against the fp32 instruction.  fp32
 // blocks of 64, whose halves walk alone like blocks of 32: 20 x 960, causal, head dimension 64: delta + zero fill 19 -> 0, dK /
 // dV 129 (eight waves to a tile) -> 44, dQ 128 -> 37 us.
 //
@@ -128,13 +128,20 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
   const char *const tensor_k = static_cast<const char *>(a.k), *const tensor_v = static_cast<const char *>(a.v);
   const typename T::RowReader k_rows(lds_k, lane), v_rows(lds_v, lane);
   const typename T::ColReader k_cols(lds_k, lane);
-  auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) {
+  // whether the sums are what they should be (from parts they may not be)
+  auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) -> bool {
     using Ar = decltype(arithmetic);
     typename W::Step now, next;
     walk.take(now, lane);
     settle(qf);
     settle(gf);
-    const OwnOperand<Ar, SBS, NS, kHalves> q_operand(qf), g_operand(gf);
+    if constexpr (std::is_same_v<Ar, SSplit>) {
+      if (scores_in_doubt(qf, a.scale)) return false;
+    }
+    const OwnOperand<Ar, SBS, NS, kHalves, false> q_operand(qf);
+    const OwnOperand<Ar, SBS, NS, kHalves, true> g_operand(gf);
+    constexpr float kTimes = up_of<Ar>();
+    const float delta_up = delta * kTimes;
     bool counted = false;  // exactly kCopies copies were issued after the tile that is needed next
     if (now.count) {
       walk.template copy<true>(now, tensor_v, lds_v, source, lane);
@@ -163,10 +170,10 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
       if (now.special) walk.template finish_scores<Tr>(now, sv, qk_scale, qi, kq);
       apply_factor<Tr, kScores>(sv, cc);
 
-      // ---- dS = P (dP - delta)
+      // ---- dS = P (dP - delta), times up_of as a second operand (dP: up_of^2)
 #pragma unroll
       for (int x = 0; x < kScores; ++x)
-        sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), neg_lse)) * (dp[x / kRegs][x % kRegs] - delta);
+        sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), neg_lse)) * fmaf(dp[x / kRegs][x % kRegs], 1.f / kTimes, -delta_up);
       if (now.special) {
         const late_args_t p = late_args();
         if (p->dbias) {  // every pair is visited once: plain stores
@@ -179,7 +186,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 #pragma unroll
               for (int r = 0; r < kRegs; r += 4) {
                 const float *v = sv + kRegs * t + r;
-                *reinterpret_cast<f32x4 *>(out + 2 * r) = f32x4{v[0], v[1], v[2], v[3]};
+                *reinterpret_cast<f32x4 *>(out + 2 * r) = f32x4{v[0], v[1], v[2], v[3]} * (1.f / kTimes);
               }
             }
         }
@@ -191,10 +198,12 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
       if (next.count) counted = walk.template copy<false>(next, tensor_k, lds_k, source, lane);
       now = next;
     }
+    if constexpr (!std::is_same_v<Ar, SSplit>) return true;
+    scale_down<Ar, NS, kRegs>(dq);
+    return !not_finite<NS, kRegs>(dq);
   };
   if constexpr (in_parts<Tr, SBS, kSome>()) {
-    walk_list(SSplit{});
-    if (in_doubt<NS, kRegs>(dq)) {  // once more with the fp32 instruction
+    if (!walk_list(SSplit{})) {  // once more with the fp32 instruction
       walk.start(a, me.b, me.own, me.there, me.part, me.parts);
       start_row();
       walk_list(Tr{});
@@ -272,13 +281,18 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 
   const typename T::RowReader q_rows0(lds, lane), g_rows0(lds + T::kBytes, lane);
   const typename T::ColReader q_cols0(lds, lane), g_cols0(lds + T::kBytes, lane);
-  auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) {
+  auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) -> bool {  // as in the dQ kernel
     using Ar = decltype(arithmetic);
     typename W::Step now, next;
     walk.take(now, lane);
     settle(kf);
     settle(vf);
-    const OwnOperand<Ar, SBS, NS, kHalves> k_operand(kf), v_operand(vf);
+    if constexpr (std::is_same_v<Ar, SSplit>) {
+      if (scores_in_doubt(kf, a.scale)) return false;
+    }
+    const OwnOperand<Ar, SBS, NS, kHalves, false> k_operand(kf);
+    const OwnOperand<Ar, SBS, NS, kHalves, true> v_operand(vf);
+    constexpr float kTimes = up_of<Ar>();  // of P and dS as second operands; dP: the square
     int buf = 0;
     if (now.count) copy_all(now, lds);
     while (now.count) {
@@ -330,7 +344,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
           if (ls[x] == -INFINITY) ls[x] = INFINITY;
       }
 #pragma unroll
-      for (int x = 0; x < kScores; ++x) sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), -ls[x]));
+      for (int x = 0; x < kScores; ++x) sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), -ls[x])) * kTimes;
       const Weights<Ar, kScores> pw(sv);
       if constexpr (kLateDp) {
         W::template multiply_cols<Ar, true, kScores>(dv, now, g_cols, pw);
@@ -342,7 +356,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
       for (int x = 0; x < kScores; x += 4) {
         const f32x4 d4 = *reinterpret_cast<const f32x4 *>(delta + (x / kRegs) * SBS + 2 * (x % kRegs) + 4 * kq);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sv[x + i] *= dp[x / kRegs][x % kRegs + i] - d4[i];
+        for (int i = 0; i < 4; ++i) sv[x + i] *= fmaf(dp[x / kRegs][x % kRegs + i], 1.f / (kTimes * kTimes), -d4[i]);
       }
       // ---- dV^T += dO^T P
       if constexpr (!kLateDp) W::template multiply_cols<Ar, true, kScores>(dv, now, g_cols, pw);
@@ -363,10 +377,13 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
       now = next;
       buf ^= 1;
     }
+    if constexpr (!std::is_same_v<Ar, SSplit>) return true;
+    scale_down<Ar, NS, kRegs>(dk);
+    scale_down<Ar, NS, kRegs>(dv);
+    return !not_finite<NS, kRegs>(dk) && !not_finite<NS, kRegs>(dv);
   };
   if constexpr (in_parts<Tr, SBS, kSome>()) {
-    walk_list(SSplit{});
-    if (in_doubt<NS, kRegs>(dk) || in_doubt<NS, kRegs>(dv)) {  // once more with the fp32 instruction
+    if (!walk_list(SSplit{})) {  // once more with the fp32 instruction
       walk.start(a, me.b, me.own, me.there, me.part, me.parts);
       start_row();
       walk_list(Tr{});

@@ -67,6 +67,13 @@ struct SF32 {
 // fp32 products take half as long for the same values to split, are no faster with it (6 x 1040 queries, causal, head dimension
 // 32: forward 16.1 -> 16.6 us, dK / dV 20.0 -> 21.9).
 struct SSplit : SF32 {};
+template <int NS>
+constexpr bool kDotParts = NS > 2;  // Parts::of
+// What the partner's and the own values of a product other than the scores are multiplied by
+template <typename Ar>
+constexpr float up_of() {
+  return std::is_same_v<Ar, SSplit> ? kUp : 1.f;
+}
 template <typename Tr, int SBS, bool kSome>
 constexpr bool in_parts() {
   return Tr::kElem == 4 && SBS == 32 && !kSome;
@@ -328,21 +335,21 @@ struct OwnRows {
   }
 };
 
-// The own rows as the products of arithmetic Ar take them
-template <typename Ar, int SBS, int NS, int kHalves>
+// The own rows as the products of arithmetic Ar take them; kSecond: of the second tensor (Walk), otherwise for scores
+template <typename Ar, int SBS, int NS, int kHalves, bool kSecond>
 struct OwnOperand {
   const OwnRows<Ar::kElem, SBS, NS, kHalves> &rows;
   __device__ inline explicit OwnOperand(const OwnRows<Ar::kElem, SBS, NS, kHalves> &own) : rows(own) {}
 };
 // in parts: fragments 2 p and 2 p + 1 in one, the second half zero behind an odd last one
-template <int SBS, int NS, int kHalves>
-struct OwnOperand<SSplit, SBS, NS, kHalves> {
+template <int SBS, int NS, int kHalves, bool kSecond>
+struct OwnOperand<SSplit, SBS, NS, kHalves, kSecond> {
   static constexpr int kFrags = OwnRows<4, SBS, NS, kHalves>::T::kFrags, kParts = (kFrags + 1) / 2;
   Parts parts[kParts];
   __device__ inline explicit OwnOperand(const OwnRows<4, SBS, NS, kHalves> &own) {
 #pragma unroll
     for (int p = 0; p < kParts; ++p)
-      parts[p] = Parts(own.fr[2 * p], 2 * p + 1 < kFrags ? own.fr[2 * p + 1] : u32x4{0u, 0u, 0u, 0u});
+      parts[p] = Parts::of<kDotParts<NS>>(own.fr[2 * p], 2 * p + 1 < kFrags ? own.fr[2 * p + 1] : u32x4{0u, 0u, 0u, 0u}, kSecond ? kUp : 1.f);
   }
 };
 
@@ -354,12 +361,42 @@ __device__ static inline void settle(OwnRows<ES, SBS, NS, kHalves> &own) {
   for (int f = 0; f < OwnRows<ES, SBS, NS, kHalves>::T::kFrags; ++f) asm volatile("" : "+v"(own.fr[f]));
 }
 
+// Whether scores from parts, formed without kUp, could be off by more than 2^-30.  The own values are exact in their parts if they
+// are 0 or at least 2^-102; those of the partners are off by 2^-125 at most, and a score by 128 times that, the largest own value
+// and the scale.  (A score that overflows is as good as infinite, or leaves NaN in the sums.)
+template <int ES, int SBS, int NS, int kHalves>
+__device__ static inline bool scores_in_doubt(const OwnRows<ES, SBS, NS, kHalves> &own, float scale) {
+  constexpr int kFrags = OwnRows<ES, SBS, NS, kHalves>::T::kFrags;
+  float least = INFINITY, most = 0.f;
+#pragma unroll
+  for (int f = 0; f < kFrags; ++f)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float v = fabsf(as_float(own.fr[f][i]));
+      least = fminf(least, v), most = fmaxf(most, v);
+    }
+  bool small = __any(least < 0x1p-102f);
+  if (small) {  // or zero
+    least = INFINITY;
+#pragma unroll
+    for (int f = 0; f < kFrags; ++f)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = fabsf(as_float(own.fr[f][i]));
+        least = fminf(least, v > 0.f ? v : INFINITY);
+      }
+    small = __any(least < 0x1p-102f);
+  }
+  return small || __any(most > 0x1p70f) || scale > 0x1p17f;
+}
+
 // acc (per partner block t) = partner rows x own rows over all head slices: acc[t] belongs to this lane's own row
 // (lane % SBS) and partner rows 8 (r / 4) + 4 (lane / 32) + r % 4 (SBS 32) or 4 (lane / 16) + r (SBS 16).
-// kOwnIsQuery: as in Walk; a score is the same bits wherever it is formed
-template <typename Tr, int SBS, int NS, int NB, int kHalves, bool kOwnIsQuery, typename Acc>
+// kOwnIsQuery, kSecond: as in Walk; a score from parts is the same bits wherever it is formed; of the second tensor acc is
+// up_of^2 times the product
+template <typename Tr, int SBS, int NS, int NB, int kHalves, bool kOwnIsQuery, bool kSecond, typename Acc>
 __device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<Tr::kElem, SBS, NS, NB, kHalves>::RowReader &rows,
-                                           const OwnOperand<Tr, SBS, NS, kHalves> &own) {
+                                           const OwnOperand<Tr, SBS, NS, kHalves, kSecond> &own) {
   constexpr int kFrags = Tile<Tr::kElem, SBS, NS, NB>::kFrags;
 #pragma unroll
   for (int t = 0; t < NB; ++t)
@@ -367,10 +404,10 @@ __device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<T
     for (int r = 0; r < (SBS == 32 ? 16 : 4); ++r) acc[t][r] = 0.f;
   if constexpr (std::is_same_v<Tr, SSplit>) {
 #pragma unroll
-    for (int p = 0; p < OwnOperand<Tr, SBS, NS, kHalves>::kParts; ++p)
+    for (int p = 0; p < OwnOperand<Tr, SBS, NS, kHalves, kSecond>::kParts; ++p)
 #pragma unroll
       for (int t = 0; t < NB; ++t)
-        multiply_parts<!kOwnIsQuery>(acc[t], Parts(rows.frag(t, 2 * p), 2 * p + 1 < kFrags ? rows.frag(t, 2 * p + 1) : u32x4{0u, 0u, 0u, 0u}), own.parts[p]);
+        multiply_parts<!kOwnIsQuery>(acc[t], Parts::of<kDotParts<NS>>(rows.frag(t, 2 * p), 2 * p + 1 < kFrags ? rows.frag(t, 2 * p + 1) : u32x4{0u, 0u, 0u, 0u}, kSecond ? kUp : 1.f), own.parts[p]);
   } else {
 #pragma unroll
     for (int f = 0; f < kFrags; ++f)
@@ -429,7 +466,7 @@ struct Weights<SSplit, kScores> : Weights<SF32, kScores> {
   using Weights<SF32, kScores>::Weights;
 };
 
-// out[h] += partner columns^T x weights
+// out[h] += partner columns^T x weights, times up_of: weights that are up_of times theirs leave up_of^2 times the product
 template <typename Tr, int SBS, int NS, int NB, int kHalves, int kScores, typename Acc>
 __device__ static inline void product_cols(Acc (&out)[NS], const typename Tile<Tr::kElem, SBS, NS, NB, kHalves>::ColReader &cols,
                                            const Weights<Tr, kScores> &w) {
@@ -440,12 +477,12 @@ __device__ static inline void product_cols(Acc (&out)[NS], const typename Tile<T
       u32x4 v[2];
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[i / 4][i % 4] = __builtin_bit_cast(uint32_t, w.w[x + i]);
-      const Parts weights(v[0], v[1]);
+      const Parts weights = Parts::of<kDotParts<NS>>(v[0], v[1], 1.f);
 #pragma unroll
       for (int h = 0; h < NS; ++h) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i / 4][i % 4] = __builtin_bit_cast(uint32_t, cols.value((x + i) / kRegs, h, (x + i) % kRegs));
-        multiply_parts(out[h], Parts(v[0], v[1]), weights);
+        multiply_parts(out[h], Parts::of<kDotParts<NS>>(v[0], v[1], kUp), weights);
       }
     }
   } else if constexpr (Tr::kElem == 4) {
@@ -520,6 +557,16 @@ template <typename Tr>
 __device__ static inline void store4(char *p, float a, float b, float c, float d) {
   if constexpr (Tr::kElem == 4) *reinterpret_cast<f32x4 *>(p) = f32x4{a, b, c, d};
   else *reinterpret_cast<u32x2 *>(p) = u32x2{Tr::pack2(a, b), Tr::pack2(c, d)};
+}
+
+// Sums of products from parts (up_of) at their own size
+template <typename Ar, int NS, int kRegs, typename Acc>
+__device__ static inline void scale_down(Acc (&acc)[NS]) {
+  constexpr float kFactor = 1.f / (up_of<Ar>() * up_of<Ar>());
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
+#pragma unroll
+    for (int r = 0; r < kRegs; ++r) acc[h][r] *= kFactor;
 }
 
 // Maximum / sum over the lanes that hold the same own row (lanes l, l + SBS, ...)
@@ -721,14 +768,14 @@ struct Walk {
   // acc = rows of the step's blocks of the first (second) tensor x own rows, and out += their columns^T x weights
   template <typename Tr, bool kSecond, typename Acc>
   __device__ static inline void multiply_rows(Acc (&acc)[NB], const Step &s, const typename T::RowReader &rows,
-                                              const OwnOperand<Tr, SBS, NS, kHalves> &own, int lane) {
+                                              const OwnOperand<Tr, SBS, NS, kHalves, kSecond> &own, int lane) {
     if constexpr (kSome) {
       uint32_t have[NB];
 #pragma unroll
       for (int t = 0; t < NB; ++t) have[t] = (kSecond ? s.have[t] >> 8 : s.have[t]) & own.rows.there;
       product_some_rows<Tr, SBS, NS, NB>(acc, rows, own.rows, have, lane);
     } else {
-      product_rows<Tr, SBS, NS, NB, kHalves, kOwnIsQuery>(acc, rows, own);
+      product_rows<Tr, SBS, NS, NB, kHalves, kOwnIsQuery, kSecond>(acc, rows, own);
     }
   }
   template <typename Tr, bool kSecond, int kScores, typename Acc>

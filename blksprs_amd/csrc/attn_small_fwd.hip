@@ -18,7 +18,7 @@
 // wave at a time.  Against the fp32 matrix-core kernel that ran these shapes before: 48 x 4096 queries, sbs 32, head
 // dimension 64, fp16, 33 key blocks per query block: 0.65 -> 0.072 ms (460 TFLOP/s, 18 % of the matrix cores' peak); 32
 // prompts of 1032 to 2064 tokens, sbs 16, bf16, causal: 0.54 -> 0.044 ms.  fp32, sbs 32, products from bf16 parts (split_f32.h):
-// 8 x 2048 queries, half of the blocks, head dimension 64: 51.1 -> 41.1 us (105 TFLOP/s) against the fp32 instruction; the 480
+// 8 x 2048 queries, half of the blocks, head dimension 64: 51.1 -> 42.3 us (102 TFLOP/s) against the fp32 instruction; the 490
 // vector instructions of a step that split its values cost more than its 48 products, and 512 lists of 32 +- 4 blocks cut in
 // four fill the chip once, so the launch waits for the longest.  fp32 blocks of 64, whose halves walk alone like blocks of 32:
 // 20 x 960, causal, head dimension 64: 97.8 (eight waves to a tile) -> 27.4 us.
@@ -135,12 +135,16 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
 
   const typename T::RowReader k_rows(lds_k, lane);
   const typename T::ColReader v_cols(lds_v, lane);
-  auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) {
+  // whether the sums are what they should be (from parts they may not be)
+  auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) -> bool {
     using Ar = decltype(arithmetic);
     typename W::Step now, next;
     walk.take(now, lane);
     settle(qf);
-    const OwnOperand<Ar, SBS, NS, kHalves> q_operand(qf);
+    if constexpr (std::is_same_v<Ar, SSplit>) {
+      if (scores_in_doubt(qf, a.scale)) return false;
+    }
+    const OwnOperand<Ar, SBS, NS, kHalves, false> q_operand(qf);
     bool counted = false;  // exactly kCopies copies (the V tile's) were issued after the K tile's
     if (now.count) {
       walk.template copy<false>(now, tensor_k, lds_k, source, lane);
@@ -194,6 +198,10 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
         sum += sv[x];
       }
       l_i += sum;
+      if constexpr (up_of<Ar>() != 1.f) {
+#pragma unroll
+        for (int x = 0; x < kScores; ++x) sv[x] *= up_of<Ar>();
+      }
       const Weights<Ar, kScores> pf(sv);
 
       // ---- O^T += V^T P^T.  In flight at most: V of this step, K of the next.
@@ -205,10 +213,12 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
       if (next.count) counted = walk.template copy<true>(next, tensor_v, lds_v, source, lane);
       now = next;
     }
+    if constexpr (!std::is_same_v<Ar, SSplit>) return true;
+    scale_down<Ar, NS, kRegs>(oacc);
+    return !not_finite<NS, kRegs>(oacc, l_i);
   };
   if constexpr (in_parts<Tr, SBS, kSome>()) {
-    walk_list(SSplit{});
-    if (in_doubt<NS, kRegs>(oacc, l_i)) {  // once more with the fp32 instruction
+    if (!walk_list(SSplit{})) {  // once more with the fp32 instruction
       walk.start(a, me.b, me.own, me.there, me.part, me.parts);
       start_row();
       walk_list(Tr{});

@@ -8,12 +8,12 @@
 // operands.  The chunk of 24 KiB is not double buffered: six workgroups share a compute unit, and one splits or waits while
 // another multiplies.
 //
-// What bounds it: per chunk and wave 12 products of 32 cycles and 130 vector instructions of 4, 88 of them for the split (the two
+// What bounds it: per chunk and wave 12 products of 32 cycles and 114 vector instructions of 4, 72 of them for the split (the two
 // overlap by half, measured alone), on a card that lowers its clock for bf16 products of random values (1600 TFLOP/s of 2500
 // without anything beside them, where fp32 products run at 137 of 157); then tiles in the order in which places become free, the
 // last of which run alone.  Waves that multiply go first (s_setprio: dX 77 -> 71 us).  Two buffers with one barrier and the split
 // in the shadow of the wave's own products, which leaves three workgroups: 93 / 78 / 82 us where this takes 80 / 71 / 81 (8 x
-// 2048^3 at 25 %, sbs 64, forward / dX / dY).  The kernel before it, on the fp32 instruction, five workgroups of asynchronous
+// 2048^3 at 25 %, sbs 64, forward / dX / dY; 1 % more since the values are multiplied by kUp).  The kernel before it, on the fp32 instruction, five workgroups of asynchronous
 // copies: 103 / 99 / 99; 3 x 1920 x 2944 x 1664 at 30 %, sbs 128, all three: 199 -> 158.
 #include "split_f32.h"
 
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(256, 5) void matmul_split_kernel(const char *__rest
     load();
   }
   for (int it = 0; it < n_iter; ++it) {
-    const Parts px(ex.a, ex.b), py(ey.a, ey.b);
+    const Parts px = Parts::of<true>(ex.a, ex.b, kUp), py = Parts::of<true>(ey.a, ey.b, kUp);
     __syncthreads();  // nobody reads the chunk before any more
     *reinterpret_cast<u32x4 *>(x_put) = px.high;
     *reinterpret_cast<u32x4 *>(x_put + kPlane) = px.mid;
@@ -157,9 +157,10 @@ __global__ __launch_bounds__(256, 5) void matmul_split_kernel(const char *__rest
     __builtin_amdgcn_s_setprio(0);
   }
 
-  if (in_doubt<1, 16>(acc)) {  // once more with the fp32 instruction, from memory
+  const bool again = not_finite<1, 16>(acc);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[0][r] = 0.f;
+  for (int r = 0; r < 16; ++r) acc[0][r] = again ? 0.f : acc[0][r] * (kDown * kDown);
+  if (again) {  // with the fp32 instruction, from memory
     for (int q = p_begin; q < p_end; ++q) {
       const int2 v = *reinterpret_cast<const int2 *>(pairs + 2 * (int64_t)q);
       const int64_t bx = v.x < 0 || v.x >= nnz_x ? 0 : v.x, by = v.y < 0 || v.y >= nnz_y ? 0 : v.y;

@@ -10,29 +10,50 @@ using namespace mfma;
 __device__ static inline float as_float(uint32_t v) { return __builtin_bit_cast(float, v); }
 
 // fp32 values as three bf16 parts: the value rounded to 8 bits, what is left of it rounded to 8 bits, and the rest, which fits.
-// A product of two such values is six products of parts (what the other three are worth lies below 2^-26 of the product), each
+// A product of two such values is six products of parts, each
 // exact, added up in fp32 by matrix instructions of 16 times the fp32 instruction's rate: 2.7 times the products per second,
 // with one rounding per 16 (32) contracted values and part where the fp32 instruction rounds every 2 (4).  Sums of 64 / 512 / 2048
 // random products are 1.09e-7 / 3.4e-7 / 7.1e-7 from 64 bits, the fp32 instruction's 1.45e-7 / 4.1e-7 / 8.1e-7.
-// An infinite or NaN value (or one that rounds to infinity) has NaN among its parts, so it makes NaN of every sum it enters;
-// parts below bf16's range are lost.  in_doubt() finds both in the sums, which are then formed with the fp32 instruction.
+//
+// Range: bf16 has fp32's exponents, but the parts of a value below 2^-102 reach below its smallest normal number, and lose bits
+// there.  So a value is multiplied by kUp before it is split: every fp32 value below 2^104, subnormal ones included, is the sum of
+// its parts, and a sum of products is kUp^2 times what it should be (x = 2^-118 z, y = 2^60 z': without kUp 1e-5 from 64 bits).
+// What does not fit, an infinite or NaN value or one from 2^104 on, or a sum from 2^80 on, leaves a sum that is not finite:
+// not_finite() finds it, and the sums are formed again with the fp32 instruction.  Scores, which are told from one another
+// by their differences and may be masked afterwards, are formed without kUp (scores_in_doubt).
+constexpr float kUp = 0x1p24f, kDown = 0x1p-24f;
+
 struct Parts {
   u32x4 high, mid, low;
   __device__ inline Parts() {}
-  __device__ inline Parts(u32x4 a, u32x4 b) {  // eight values
+  // of eight values, times `up` (kUp or 1).  kDot: what is left of a value in one instruction, exact since it is a difference of
+  // fewer bits than either, instead of 1.5.  Fewer instructions and registers, but not faster ones: attention at head
+  // dimension 64, where two waves share a SIMD, is 3 to 7 % slower with it (dK / dV 82 -> 88 us), at 128 with one wave 2 to 15 %
+  // faster (forward 112 -> 110, dQ 153 -> 148, dK / dV 244 -> 208), products of blocks of 64 1 % (8 x 2048 queries, half of the blocks).
+  template <bool kDot>
+  __device__ static inline Parts of(u32x4 a, u32x4 b, float up) {
+    Parts p;
+    // held in registers: written into the instruction, 0x0000bf80 becomes the inline constant -1.0, and that is 0xbf800000
+    uint32_t minus_first = 0x0000bf80u, minus_second = 0xbf800000u;
+    if constexpr (kDot) asm("" : "+s"(minus_first), "+s"(minus_second));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      float x = as_float(i < 2 ? a[2 * i] : b[2 * i - 4]), y = as_float(i < 2 ? a[2 * i + 1] : b[2 * i - 3]);
-      uint32_t packed = MBf16::pack2(x, y);
-      asm("" : "+v"(packed));  // or each value is converted once more by itself for the subtraction
-      high[i] = packed;
-      x -= as_float(packed << 16), y -= as_float(packed & 0xffff0000u);
-      packed = MBf16::pack2(x, y);
-      asm("" : "+v"(packed));
-      mid[i] = packed;
-      x -= as_float(packed << 16), y -= as_float(packed & 0xffff0000u);
-      low[i] = MBf16::pack2(x, y);
+      float x = as_float(i < 2 ? a[2 * i] : b[2 * i - 4]) * up, y = as_float(i < 2 ? a[2 * i + 1] : b[2 * i - 3]) * up;
+      auto part = [&]() __attribute__((always_inline)) {
+        uint32_t packed = MBf16::pack2(x, y);
+        if constexpr (kDot) {
+          x = MBf16::dot2(packed, minus_first, x), y = MBf16::dot2(packed, minus_second, y);
+        } else {
+          asm("" : "+v"(packed));  // or each value is converted once more by itself for the subtraction
+          x -= as_float(packed << 16), y -= as_float(packed & 0xffff0000u);
+        }
+        return packed;
+      };
+      p.high[i] = part();
+      p.mid[i] = part();
+      p.low[i] = MBf16::pack2(x, y);
     }
+    return p;
   }
 };
 
@@ -52,19 +73,15 @@ __device__ static inline void multiply_parts(Acc &acc, const Parts &a, const Par
   multiply_part(acc, a.high, b.high);
 }
 
-// Whether sums of a wave formed from parts are to be formed again: one is infinite or NaN, or all are so small that parts of
-// what they were formed from may have been lost (a value below 2^-102 has less than 24 bits in its parts).
+// Whether one of a wave's sums is infinite or NaN
 template <int NS, int kRegs, typename Acc>
-__device__ static inline bool in_doubt(const Acc (&acc)[NS], float also = 0.f) {
-  float nan = also * 0.f, largest = 0.f;
+__device__ static inline bool not_finite(const Acc (&acc)[NS], float also = 0.f) {
+  float nan = also * 0.f;
 #pragma unroll
   for (int h = 0; h < NS; ++h)
 #pragma unroll
-    for (int r = 0; r < kRegs; ++r) {
-      nan = fmaf(acc[h][r], 0.f, nan);
-      largest = fmaxf(largest, fabsf(acc[h][r]));
-    }
-  return __any(nan != 0.f) || (!__any(largest >= 0x1p-80f) && __any(largest > 0.f));
+    for (int r = 0; r < kRegs; ++r) nan = fmaf(acc[h][r], 0.f, nan);
+  return __any(nan != 0.f);
 }
 
 }  // namespace split
