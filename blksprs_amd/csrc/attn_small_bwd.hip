@@ -103,7 +103,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 
   OwnRows<Tr::kElem, SBS, NS, kHalves> qf, gf;
   acc_t dq[NS];
-  auto start_row = [&]() __attribute__((always_inline)) {
+  auto start_row = [&](int lane) __attribute__((always_inline)) {
     qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, (int)me.own, lane);
     gf.load(a.d_o, a.pidx_o + row * a.nhv, (int)a.nhv, a.n_o_blocks, (int)me.own, lane);
 #pragma unroll
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 #pragma unroll
       for (int r = 0; r < kRegs; ++r) dq[h][r] = 0.f;
   };
-  start_row();
+  start_row(lane);
   float delta = 0.f, neg_lse = -a.lse[stats + qi];
   if (neg_lse == INFINITY) neg_lse = -INFINITY;  // a query that sees nothing: p = 0
   {
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
   if constexpr (in_parts<Tr, SBS, kSome>()) {
     if (!walk_list(SSplit{})) {  // once more with the fp32 instruction
       walk.start(a, me.b, me.own, me.there, me.part, me.parts);
-      start_row();
+      start_row(fresh_lane());
       walk_list(Tr{});
     }
   } else {
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 
   OwnRows<Tr::kElem, SBS, NS, kHalves> kf, vf;
   acc_t dk[NS], dv[NS];
-  auto start_row = [&]() __attribute__((always_inline)) {
+  auto start_row = [&](int lane) __attribute__((always_inline)) {
     kf.load(a.k, a.pidx_k + row * a.nh, (int)a.nh, a.n_k_blocks, (int)me.own, lane);
     vf.load(a.v, a.pidx_v + row * a.nhv, (int)a.nhv, a.n_v_blocks, (int)me.own, lane);
 #pragma unroll
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 #pragma unroll
       for (int r = 0; r < kRegs; ++r) dk[h][r] = dv[h][r] = 0.f;
   };
-  start_row();
+  start_row(lane);
 
   const float qk_scale = a.scale * kLog2e;
   const float cc = a.bias ? 1.f : qk_scale;
@@ -385,7 +385,7 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
   if constexpr (in_parts<Tr, SBS, kSome>()) {
     if (!walk_list(SSplit{})) {  // once more with the fp32 instruction
       walk.start(a, me.b, me.own, me.there, me.part, me.parts);
-      start_row();
+      start_row(fresh_lane());
       walk_list(Tr{});
     }
   } else {

@@ -559,6 +559,16 @@ __device__ static inline void store4(char *p, float a, float b, float c, float d
   else *reinterpret_cast<u32x2 *>(p) = u32x2{Tr::pack2(a, b), Tr::pack2(c, d)};
 }
 
+// The lane's number, of which the compiler knows nothing.  The loads of the own rows in front of a second walk over a list are
+// those in front of the first; with one lane number in both, their addresses stay in registers through the first walk, for the
+// second that is hardly ever made: the forward kernel of fp32 at head dimension 64 then needs 172 registers (with this 164,
+// which is a wave per SIMD more), dK / dV 12 more than the 256 there are.
+__device__ static inline int fresh_lane() {
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
 // Sums of products from parts (up_of) at their own size
 template <typename Ar, int NS, int kRegs, typename Acc>
 __device__ static inline void scale_down(Acc (&acc)[NS]) {

@@ -118,7 +118,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
   OwnRows<Tr::kElem, SBS, NS, kHalves> qf;
   acc_t oacc[NS];
   float m_i, l_i;
-  auto start_row = [&]() __attribute__((always_inline)) {
+  auto start_row = [&](int lane) __attribute__((always_inline)) {
     qf.load(a.q, a.pidx_q + row * a.nh, (int)a.nh, a.n_q_blocks, (int)me.own, lane);
 #pragma unroll
     for (int h = 0; h < NS; ++h)
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
       for (int r = 0; r < kRegs; ++r) oacc[h][r] = 0.f;
     m_i = -INFINITY, l_i = 0.f;
   };
-  start_row();
+  start_row(lane);
 
   const float qk_scale = a.scale * kLog2e;
   const float cc = a.bias ? 1.f : qk_scale;
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(64 * kWaves, (FwdShape<Tr::kElem, SBS, NS, kHalves>
   if constexpr (in_parts<Tr, SBS, kSome>()) {
     if (!walk_list(SSplit{})) {  // once more with the fp32 instruction
       walk.start(a, me.b, me.own, me.there, me.part, me.parts);
-      start_row();
+      start_row(fresh_lane());
       walk_list(Tr{});
     }
   } else {
