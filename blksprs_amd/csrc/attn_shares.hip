@@ -150,15 +150,36 @@ static int least_parts(const bsa_attn_args &a, bool key_rows) {
   return a.dtype == BSA_F32 ? waves_per_row<4>(rows, partners, per_step) : waves_per_row<2>(rows, partners, per_step);
 }
 
+// Entries from which a row is several workgroups'.  The scratch, the launch that adds the sums and its host work cost some
+// 15 us: as long as these many steps (head dimensions up to 64, beyond) by which a quarter of the list has to be longer than
+// a piece.
+static int64_t steps_of_a_scratch(const bsa_attn_args &a) {
+  const bool small_head = slices_of(a) * a.sbs <= 64;
+  return (a.dtype == BSA_F32 ? (small_head ? 6 : 3) : (small_head ? 24 : 16)) * (a.sbs == 16 ? 2 : 1);
+}
+static int64_t most_of_a_group(const bsa_attn_args &a, int64_t piece) {
+  const int64_t most = 4 * (piece + steps_of_a_scratch(a));
+  return most > 6 * piece ? most : 6 * piece;
+}
+
 // The longest share a wave should walk, in blocks of the kernels, or 0: the rows are even enough for waves_per_row, or not for
 // the kernels that read shares.
 //
 // waves: what the chip holds of these kernels at a time (their registers and LDS).  least: entries of a wave's walk that cost
-// about as much as its start and end, six steps (16-bit; four of fp32, whose products take longer).  Shares pay where the
-// longest share of waves_per_row is at least eight steps (fp32: four) and half a mean above the mean, or where a launch of more
-// than one round would start its longest lists, more than twice the mean, anywhere, and the walk of one takes 22 steps (14 at
-// head dimensions above 64, fp32 8) or more: below, some 3 us of a launch (33 x 272, sbs 16, windows of 10 blocks, fp32: 15.1 ->
-// 12.2), a new layout's first call pays 70 us for them.
+// about as much as its start and end, six steps (16-bit; four of fp32, whose products take longer).  Shares have to be long enough
+// for the host work of a call (7 us, 22 with a scratch) and the 70 us that a new layout's first call pays: eight steps (fp32: four)
+// and half a mean above the mean, and they have to change something.  Times are GPU times of forward + backward, without ->
+// with shares, us:
+//   cut    The longest rows become several workgroups'.  Where lengths fall off evenly (causal) those just below
+//          most_of_a_group stay, and the launch gets shorter by the difference only: fp32 causal, head dimension 64, sbs 32, 8 x 2048
+//          (64 blocks, cut from 61 on) 180 -> 197, 4 x 2048 (from 45 on) 162 -> 146, 2 x 4096 (128, from 61 on) 292 -> 206; bf16, 2 x
+//          4096 (128, from 121 on) 76 -> 84.  A few long ones among short ones: 2 x 4096 BigBird, fp32 331 -> 104, bf16 107 -> 49.
+//          6 x 1664 BigBird, fp32, sbs 64, head dimension 128 (52 halves, cut from 49 on) 382 -> 330.
+//   waves  The longest rows get more waves than waves_per_row gives them.  Longest share of 3.4 pieces (24 x 1536 causal, bf16, sbs
+//          32) 80 -> 63, 3.8 (8 x 2048, fp16, sbs 16) 95 -> 70; 1.7 (24 x 1536, bf16 at head dimension 128; fp16, sbs 16) 134 -> 137, 85 -> 87.
+//   order  A launch of more than one round would start its longest lists, more than twice the mean, anywhere: 24 x 1536 BigBird, fp32,
+//          sbs 32, head dimension 64 (share 12, piece 8) 275 -> 215; at 128 (piece 15, so no share is long) 630 -> 642.  The
+//          walk of one takes 22 steps (14 at head dimensions above 64, fp32 8) or more.
 int64_t attn_shares_piece(const bsa_attn_args &a, bool key_rows, int64_t n_entries, int64_t longest) {
   const int halves = halves_of(a);
   const bool wide = a.dtype == BSA_F32;
@@ -171,21 +192,13 @@ int64_t attn_shares_piece(const bsa_attn_args &a, bool key_rows, int64_t n_entri
   const int64_t least = (wide ? 4 : 6) * per_step, entries = (int64_t)halves * halves * n_entries;
   const int64_t mean = cdiv(entries, waves), piece = mean > least ? mean : least;
   const int split = least_parts(a, key_rows);
-  const int64_t share = halves * longest / split, worth = (wide ? 4 : 8) * per_step;
+  const int64_t most = most_of_a_group(a, piece), n = halves * longest, share = n / split, worth = (wide ? 4 : 8) * per_step;
   const bool long_shares = 2 * share > 3 * piece && share >= piece + worth;
-  const bool order = rows * split > waves && halves * longest * rows > 2 * entries &&
+  const bool cut = long_shares && n > most && (n * rows > 3 * entries || n - most > (wide ? 1 : 2) * steps_of_a_scratch(a));
+  const bool more_waves = long_shares && split < 4 && share >= 2 * piece;
+  const bool order = rows * split > waves && n * rows > 2 * entries && share >= piece &&
                      share >= least + (wide || !small_head ? worth : 2 * worth);
-  return long_shares || order ? piece : 0;
-}
-
-// Entries from which a row is several workgroups'.  The scratch, the launch that adds the sums and its host work cost some
-// 15 us: as long as these many steps (head dimensions up to 64, beyond) by which a quarter of the list has to be longer than
-// a piece.
-static int64_t most_of_a_group(const bsa_attn_args &a, int64_t piece) {
-  const bool small_head = slices_of(a) * a.sbs <= 64;
-  const int64_t steps = a.dtype == BSA_F32 ? (small_head ? 6 : 3) : (small_head ? 24 : 16);
-  const int64_t most = 4 * (piece + steps * (a.sbs == 16 ? 2 : 1));
-  return most > 6 * piece ? most : 6 * piece;
+  return cut || more_waves || order ? piece : 0;
 }
 
 int attn_shares_build(const bsa_attn_args &a, bool key_rows, int64_t piece, int64_t max_groups, int64_t max_merges, int32_t *groups,
