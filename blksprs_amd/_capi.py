@@ -59,6 +59,7 @@ class LinesArgs(ctypes.Structure):
 
 ATTN_RECORD_INTS = 16  # BSA_ATTN_RECORD_INTS
 SHARE_INTS = 12  # BSA_SHARE_INTS
+SHARES_FOR_ONE_CALL = 2  # BSA_SHARES_FOR_ONE_CALL
 ROWS_RECORD_INTS = 128  # BSA_ROWS_RECORD_INTS
 
 # name -> (restype, argtypes); must list every symbol of include/blksprs_amd.h

@@ -68,9 +68,11 @@ extern "C" int bsa_attn_fwd(const bsa_attn_args *args, bsa_stream_t stream) { re
 extern "C" int bsa_attn_shares_piece(const bsa_attn_args *a, int key_rows, int64_t n_entries, int64_t longest, int64_t *piece,
                                      int64_t *max_groups, int64_t *max_merges) {
   const char *who = "bsa_attn_shares_piece";
+  const bool for_one_call = (key_rows & BSA_SHARES_FOR_ONE_CALL) != 0;
+  key_rows &= ~BSA_SHARES_FOR_ONE_CALL;
   if (int rc = check_plan(who, a, key_rows)) return rc;
   BSA_REQUIRE(piece && max_groups && max_merges, "%s: NULL argument", who);
-  *piece = bsa::attn_shares_piece(*a, key_rows != 0, n_entries, longest);
+  *piece = bsa::attn_shares_piece(*a, key_rows != 0, for_one_call, n_entries, longest);
   *max_groups = *max_merges = 0;
   if (*piece > 0) bsa::attn_shares_limits(*a, key_rows != 0, n_entries, *piece, max_groups, max_merges);
   return BSA_OK;

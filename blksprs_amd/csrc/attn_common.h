@@ -50,7 +50,7 @@ int attn_bwd_generic(const bsa_attn_args &a, hipStream_t s);
 // MFMA paths; return 1 if the configuration is not covered (caller falls back to the generic kernels)
 int attn_fwd_mfma(const bsa_attn_args &a, hipStream_t s);
 int attn_fwd_small(const bsa_attn_args &a, const bsa_attn_shares *shares, hipStream_t s);
-int64_t attn_shares_piece(const bsa_attn_args &a, bool key_rows, int64_t n_entries, int64_t longest);
+int64_t attn_shares_piece(const bsa_attn_args &a, bool key_rows, bool for_one_call, int64_t n_entries, int64_t longest);
 void attn_shares_limits(const bsa_attn_args &a, bool key_rows, int64_t n_entries, int64_t piece, int64_t *max_groups, int64_t *max_merges);
 int attn_shares_build(const bsa_attn_args &a, bool key_rows, int64_t piece, int64_t max_groups, int64_t max_merges, int32_t *groups,
                       int32_t *merges, int64_t *stats, hipStream_t s);

@@ -180,7 +180,11 @@ static int64_t most_of_a_group(const bsa_attn_args &a, int64_t piece) {
 //   order  A launch of more than one round would start its longest lists, more than twice the mean, anywhere: 24 x 1536 BigBird, fp32,
 //          sbs 32, head dimension 64 (share 12, piece 8) 275 -> 215; at 128 (piece 15, so no share is long) 630 -> 642.  The
 //          walk of one takes 22 steps (14 at head dimensions above 64, fp32 8) or more.
-int64_t attn_shares_piece(const bsa_attn_args &a, bool key_rows, int64_t n_entries, int64_t longest) {
+// for_one_call: without a layout cache the tables and the wait for their size, some 50 us each, are this call's alone: only a
+// share that gets shorter by four times what pays for a scratch is worth them (fp32: one sequence of 6080, sbs 64, causal, forward
+// and backward, a call 600 without, 554 us with; 8 x 2048 causal 395 and 495, 14 x 1056 BigBird at 128 479 and 484; 16-bit: 7 x 3328
+// BigBird forward 237 and 265, 5 x 3152 causal 373 and 460).
+int64_t attn_shares_piece(const bsa_attn_args &a, bool key_rows, bool for_one_call, int64_t n_entries, int64_t longest) {
   const int halves = halves_of(a);
   const bool wide = a.dtype == BSA_F32;
   if ((a.sbs != 16 && a.sbs != 32 && !(a.sbs == 64 && wide)) || n_entries <= 0 || longest <= 0) return 0;
@@ -198,6 +202,7 @@ int64_t attn_shares_piece(const bsa_attn_args &a, bool key_rows, int64_t n_entri
   const bool more_waves = long_shares && split < 4 && share >= 2 * piece;
   const bool order = rows * split > waves && n * rows > 2 * entries && share >= piece &&
                      share >= least + (wide || !small_head ? worth : 2 * worth);
+  if (for_one_call && share < piece + 4 * steps_of_a_scratch(a)) return 0;
   return cut || more_waves || order ? piece : 0;
 }
 

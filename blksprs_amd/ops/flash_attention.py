@@ -413,13 +413,15 @@ class _Shares:
                                 scratch.data_ptr(), size), scratch
 
 
-def _row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool) -> tuple["_Shares | None", "_Shares | None"]:
-    """Shares of the query rows and, for a backward pass, of the key rows; ``None`` where the layout is even enough."""
+def _row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool,
+                for_one_call: bool) -> tuple["_Shares | None", "_Shares | None"]:
+    """Shares of the query rows and, for a backward pass, of the key rows; ``None`` where the layout is even enough.
+    ``for_one_call``: the tables are not kept in a layout cache."""
     shares = meta.tables.shares.get((meta.sbs, dtype, backward))
-    return _build_row_shares(meta, dtype, device, backward) if shares is None else shares
+    return _build_row_shares(meta, dtype, device, backward, for_one_call) if shares is None else shares
 
 
-def _build_row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool):
+def _build_row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool, for_one_call: bool):
     """Builds the shares at the first call that needs them, with one wait of the host for their sizes: they are complete
     when that call returns, whatever stream reads them next.  A call under graph capture may not wait: it goes without."""
     tables, lib = meta.tables, _capi.load()
@@ -431,7 +433,8 @@ def _build_row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool)
     shares, wanted = [None, None], []
     for key_rows in (0, 1) if backward else (0,):
         longest = tables.max_queries_per_key if key_rows else tables.max_keys_per_query
-        _capi.check(lib.bsa_attn_shares_piece(ctypes.byref(a), key_rows, tables.key_indices_i32.numel(), int(longest),
+        which = key_rows | (_capi.SHARES_FOR_ONE_CALL if for_one_call else 0)
+        _capi.check(lib.bsa_attn_shares_piece(ctypes.byref(a), which, tables.key_indices_i32.numel(), int(longest),
                                               ctypes.byref(piece), ctypes.byref(max_groups), ctypes.byref(max_merges)),
                     "bsa_attn_shares_piece")
         if piece.value:
@@ -801,6 +804,7 @@ def flash_attention(q: BlksprsTensor, sparsity_layout_q: Tensor,
     else:
         attention_bias = torch.empty(0, device=q.device, dtype=q.dtype)
 
+    for_one_call = layout_cache is None
     layout_cache = flash_attention_build_layout_cache(
         attention_layout, sparsity_layout_q, sparsity_layout_k, sparsity_layout_v,
         n_seq_blocks_q, n_seq_blocks_k, n_head_blocks_qk,
@@ -835,7 +839,7 @@ def flash_attention(q: BlksprsTensor, sparsity_layout_q: Tensor,
 
     needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad
                                               or (attention_bias is not None and attention_bias.requires_grad))
-    meta.shares = _row_shares(meta, q.dtype, q.device, needs_grad)
+    meta.shares = _row_shares(meta, q.dtype, q.device, needs_grad, for_one_call)
     if range_check:
         range_check[0].start()
     try:

@@ -509,10 +509,11 @@ typedef struct bsa_attn_shares {
 } bsa_attn_shares;
 
 #define BSA_SHARE_INTS 12
+#define BSA_SHARES_FOR_ONE_CALL 2
 
 /*
  * Whether shares pay for the query rows (key_rows 0: forward and dQ) or key rows (1: dK and dV) of a layout with n_entries active
- * blocks, at most `longest` in one row: *piece is 0 if not, else the number that bsa_attn_shares_build takes, and *max_groups and
+ * blocks, at most `longest` in one row (| BSA_SHARES_FOR_ONE_CALL: the tables are built for one call): *piece is 0 if not, else the number that bsa_attn_shares_build takes, and *max_groups and
  * *max_merges the sizes of its tables.  Reads B, nq, nk, nh, nhv, sbs and dtype of args.  Host only.
  */
 int bsa_attn_shares_piece(const bsa_attn_args *args, int key_rows, int64_t n_entries, int64_t longest, int64_t *piece,

@@ -49,12 +49,29 @@ def _layout(kind, heads, blocks):
     (torch.float16, 16, 64, 4, 2048, "bigbird", False),  # 74 -> 72
 ])
 def test_layouts_that_get_shares(dtype, sbs, head_dim, heads, seq, kind, wanted):
+    assert _wanted(dtype, sbs, head_dim, heads, seq, kind, 0) == wanted
+
+
+# a call without a cache, without -> with shares, us
+@pytest.mark.parametrize("dtype,sbs,head_dim,heads,seq,kind,wanted", [
+    (torch.float32, 64, 64, 1, 6080, "causal", True),  # 600 -> 554
+    (torch.float32, 32, 64, 8, 2048, "bigbird", False),
+    (torch.float32, 32, 128, 14, 1056, "bigbird", False),  # 479 -> 484
+    (torch.float16, 16, 64, 5, 3152, "causal", False),  # 373 -> 460
+    (torch.bfloat16, 32, 96, 7, 3328, "bigbird", False),  # 237 -> 265
+])
+def test_layouts_that_get_shares_for_one_call(dtype, sbs, head_dim, heads, seq, kind, wanted):
+    assert _wanted(dtype, sbs, head_dim, heads, seq, kind, _capi.SHARES_FOR_ONE_CALL) == wanted
+
+
+def _wanted(dtype, sbs, head_dim, heads, seq, kind, flag):
     blocks = seq // sbs
     layout = _layout(kind, heads, blocks)
     a = _capi.AttnArgs()
     a.B, a.nq, a.nk, a.nh, a.nhv = heads, blocks, blocks, head_dim // sbs, head_dim // sbs
     a.sbs, a.dtype = sbs, _capi.DTYPE_CODES[dtype]
     piece, most_groups, most_merges = _capi.c_int64(), _capi.c_int64(), _capi.c_int64()
-    rc = _capi.load().bsa_attn_shares_piece(ctypes.byref(a), 0, int(layout.sum()), int(layout.sum(2).max()), ctypes.byref(piece),
+    rc = _capi.load().bsa_attn_shares_piece(ctypes.byref(a), flag, int(layout.sum()), int(layout.sum(2).max()), ctypes.byref(piece),
                                             ctypes.byref(most_groups), ctypes.byref(most_merges))
-    assert rc == 0 and (piece.value > 0) == wanted
+    assert rc == 0
+    return piece.value > 0
