@@ -423,7 +423,8 @@ def _row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool,
 
 def _build_row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool, for_one_call: bool):
     """Builds the shares at the first call that needs them, with one wait of the host for their sizes: they are complete
-    when that call returns, whatever stream reads them next.  A call under graph capture may not wait: it goes without."""
+    when that call returns, whatever stream reads them next.  A call under graph capture may not wait: it goes without.
+    The query rows' are the same with and without a backward pass."""
     tables, lib = meta.tables, _capi.load()
     a = _capi.AttnArgs()
     a.B, a.nq, a.nk, a.nh, a.nhv = meta.dims
@@ -431,7 +432,10 @@ def _build_row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool,
     a.key_offsets, a.query_offsets = tables.key_offsets_i32.data_ptr(), tables.query_offsets_i32.data_ptr()
     piece, max_groups, max_merges = _capi.c_int64(), _capi.c_int64(), _capi.c_int64()
     shares, wanted = [None, None], []
-    for key_rows in (0, 1) if backward else (0,):
+    seen = tables.shares.get((meta.sbs, dtype, not backward))
+    if seen is not None:
+        shares[0] = seen[0]
+    for key_rows in range(0 if seen is None else 1, 2 if backward else 1):
         longest = tables.max_queries_per_key if key_rows else tables.max_keys_per_query
         which = key_rows | (_capi.SHARES_FOR_ONE_CALL if for_one_call else 0)
         _capi.check(lib.bsa_attn_shares_piece(ctypes.byref(a), which, tables.key_indices_i32.numel(), int(longest),
@@ -441,7 +445,7 @@ def _build_row_shares(meta: "_Meta", dtype: torch.dtype, device, backward: bool,
             wanted.append((key_rows, piece.value, max_groups.value, max_merges.value))
     if wanted:
         if torch.cuda.is_current_stream_capturing():
-            return None, None
+            return tuple(shares)
         stats = torch.zeros((len(wanted), 3), dtype=torch.int64, device=device)
         built = []
         with _capi.on_device(device):

@@ -1,4 +1,4 @@
-"""When the tables of shares (attn_shares.hip) are built: for a call without a cache only where that
+"""When the tables of shares (attn_shares.hip) are built: once per side of a layout, and for a call without a cache only where that
 call gains by it."""
 
 import pytest
@@ -31,6 +31,16 @@ def built(monkeypatch):
     monkeypatch.setattr(_capi, "call", lambda name, *args: (sides.append(args[1]) if name == "bsa_attn_shares_build" else None,
                                                             call(name, *args))[1])
     return sides
+
+
+@pytest.mark.parametrize("first", [False, True])
+def test_one_cache_for_inference_and_training(device, built, first):
+    layouts, cache = _long_rows(device, 260), {}  # a cache is for these tensors
+    for train in (first, not first, first):
+        _call(device, torch.bfloat16, 16, *layouts, cache, train)
+    assert sorted(built) == [0, 1]
+    shares = cache["tables"].shares
+    assert shares[(16, torch.bfloat16, True)][0] is shares[(16, torch.bfloat16, False)][0] is not None
 
 
 def test_calls_without_a_cache(device, built):
