@@ -273,10 +273,11 @@ _BEYOND_RANGE = "causal_lengths values must be between zero and {}"
 
 
 class _RangeOfLengths:
-    """The range check of causal lengths around the launch of the kernels that read them: ``start`` enqueues the search for
-    the smallest and the largest in front of it, ``finish`` waits for the two and raises as ever.  The kernels only compare
-    lengths with positions, so what they make of a length that is then refused is dropped, and the device does not idle
-    while the host reads: 8 prompts of 128 to 256 tokens, a new tensor of lengths for each, 43.9 -> 33.3 us a call.
+    """The range check of causal lengths around the rest of a call: ``start`` enqueues the search for the smallest and the
+    largest where the lengths are looked at, ``finish`` waits for the two behind the launch of the kernels that read them and
+    raises as ever, also where the rest of the call has been refused for something else by then: lengths come first.  The
+    kernels only compare lengths with positions, so what they make of a length that is then refused is dropped, and the device
+    does not idle while the host reads: 8 prompts of 128 to 256 tokens, a new tensor of lengths for each, 44.4 -> 38.1 us a call.
 
     Every ``start`` is followed by a ``finish``, which sees the device pass and gives the pinned words back to the thread: as
     many as a thread has calls inside one another (hooks of saved tensors)."""
@@ -757,96 +758,96 @@ def flash_attention(q: BlksprsTensor, sparsity_layout_q: Tensor,
     lengths = _normalise_causal_lengths(causal_lengths, n_batches, n_seq_blocks_q * sparsity_block_size,
                                         n_seq_blocks_k * sparsity_block_size, q.device, range_check)
 
-    if sparsity_layout_o is not None:
-        sparsity_layout_o = ensure_contiguous(sparsity_layout_o)
-        validate_dimensions(sparsity_layout_o)
-        validate_contiguous(sparsity_layout_o)
-        validate_device(sparsity_layout_o, q)
-        validate_sparsity_layout(sparsity_layout_o)
-        validate_shape(sparsity_layout_o, (n_batches, n_seq_blocks_q, n_head_blocks_v), "sparsity_layout_o")
-
-    if scale is None:
-        head_dimension = n_head_blocks_qk * sparsity_block_size
-        scale = 1.0 if head_dimension == 0 else 1.0 / math.sqrt(head_dimension)
-    elif not isinstance(scale, Real):
-        raise TypeError("Attention scale must be a real number or None")
-    else:
-        scale = float(scale)
-
-    if (attention_mask is None) != (sparsity_layout_mask is None):
-        raise ValueError("attention_mask and sparsity_layout_mask must be provided together")
-    mask_bytes = None
-    if attention_mask is not None:
-        attention_mask = ensure_contiguous(attention_mask)
-        sparsity_layout_mask = ensure_contiguous(sparsity_layout_mask)
-        validate_dimensions(attention_mask, sparsity_layout_mask)
-        validate_contiguous(attention_mask, sparsity_layout_mask)
-        validate_device(attention_mask, sparsity_layout_mask, q)
-        if attention_mask.dtype != torch.bool:
-            validate_dtype_float(attention_mask)
-        validate_binary(attention_mask)
-        validate_sparsity(sparsity_block_size, (attention_mask, sparsity_layout_mask))
-        validate_shape(sparsity_layout_mask, attention_shape, "sparsity_layout_mask")
-        base = as_base_tensor(attention_mask.detach())
-        # the kernels read one byte per mask element
-        mask_bytes = (base if base.dtype == torch.bool else base != 0).view(torch.uint8)
-
-    if (attention_bias is None) != (sparsity_layout_bias is None):
-        raise ValueError("attention_bias and sparsity_layout_bias must be provided together")
-    has_bias = attention_bias is not None
-    if has_bias:
-        attention_bias = ensure_contiguous(attention_bias)
-        sparsity_layout_bias = ensure_contiguous(sparsity_layout_bias)
-        validate_dimensions(attention_bias, sparsity_layout_bias)
-        validate_contiguous(attention_bias, sparsity_layout_bias)
-        validate_device(attention_bias, sparsity_layout_bias, q)
-        validate_dtype_float(attention_bias)
-        validate_sparsity(sparsity_block_size, (attention_bias, sparsity_layout_bias))
-        validate_shape(sparsity_layout_bias, attention_shape, "sparsity_layout_bias")
-        if attention_bias.dtype != q.dtype:
-            attention_bias = attention_bias.to(q.dtype)
-    else:
-        attention_bias = torch.empty(0, device=q.device, dtype=q.dtype)
-
-    for_one_call = layout_cache is None
-    layout_cache = flash_attention_build_layout_cache(
-        attention_layout, sparsity_layout_q, sparsity_layout_k, sparsity_layout_v,
-        n_seq_blocks_q, n_seq_blocks_k, n_head_blocks_qk,
-        sparsity_layout_o=sparsity_layout_o, n_head_blocks_v=n_head_blocks_v,
-        sparsity_layout_mask=sparsity_layout_mask, sparsity_layout_bias=sparsity_layout_bias,
-        layout_cache=layout_cache,
-    )
-    if "key_offsets_i32" not in layout_cache:
-        for name in ("key_offsets", "key_indices", "query_offsets", "query_indices"):
-            layout_cache[name + "_i32"] = _as_index(layout_cache[name], torch.int32)
-        if (n_seq_blocks_k < (1 << 28) and layout_cache["key_indices"].numel() < INT32_INDEX_MAX
-                and n_head_blocks_qk <= 2 and n_head_blocks_v <= 2 and sparsity_block_size == 64):
-            offsets, records, group_size = _build_forward_records(
-                layout_cache, attention_layout, int(n_batches), int(n_seq_blocks_q), int(n_seq_blocks_k),
-                int(n_head_blocks_qk), int(n_head_blocks_v), own_layout=True)
-            layout_cache["group_offsets"], layout_cache["group_records"] = offsets, records
-            layout_cache["group_size"] = group_size
-        layout_cache["tables"] = _Tables(layout_cache)
-        finalize_layout_cache(layout_cache)
-
-    meta = _Meta()
-    meta.tables = layout_cache["tables"]
-    meta.dims = (int(n_batches), int(n_seq_blocks_q), int(n_seq_blocks_k), int(n_head_blocks_qk),
-                 int(n_head_blocks_v))
-    meta.sbs = sparsity_block_size
-    meta.scale = scale
-    meta.has_bias = has_bias
-    # the default output layout: rows of a full V layout are there as a whole where a query block has a key block
-    meta.o_rows_whole = 1 if sparsity_layout_o is None else 0
-    meta.facts = _mask_facts(layout_cache, attention_layout, attention_mask, mask_bytes, lengths, meta.dims,
-                             sparsity_block_size)
-
-    needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad
-                                              or (attention_bias is not None and attention_bias.requires_grad))
-    meta.shares = _row_shares(meta, q.dtype, q.device, needs_grad, for_one_call)
     if range_check:
         range_check[0].start()
     try:
+        if sparsity_layout_o is not None:
+            sparsity_layout_o = ensure_contiguous(sparsity_layout_o)
+            validate_dimensions(sparsity_layout_o)
+            validate_contiguous(sparsity_layout_o)
+            validate_device(sparsity_layout_o, q)
+            validate_sparsity_layout(sparsity_layout_o)
+            validate_shape(sparsity_layout_o, (n_batches, n_seq_blocks_q, n_head_blocks_v), "sparsity_layout_o")
+
+        if scale is None:
+            head_dimension = n_head_blocks_qk * sparsity_block_size
+            scale = 1.0 if head_dimension == 0 else 1.0 / math.sqrt(head_dimension)
+        elif not isinstance(scale, Real):
+            raise TypeError("Attention scale must be a real number or None")
+        else:
+            scale = float(scale)
+
+        if (attention_mask is None) != (sparsity_layout_mask is None):
+            raise ValueError("attention_mask and sparsity_layout_mask must be provided together")
+        mask_bytes = None
+        if attention_mask is not None:
+            attention_mask = ensure_contiguous(attention_mask)
+            sparsity_layout_mask = ensure_contiguous(sparsity_layout_mask)
+            validate_dimensions(attention_mask, sparsity_layout_mask)
+            validate_contiguous(attention_mask, sparsity_layout_mask)
+            validate_device(attention_mask, sparsity_layout_mask, q)
+            if attention_mask.dtype != torch.bool:
+                validate_dtype_float(attention_mask)
+            validate_binary(attention_mask)
+            validate_sparsity(sparsity_block_size, (attention_mask, sparsity_layout_mask))
+            validate_shape(sparsity_layout_mask, attention_shape, "sparsity_layout_mask")
+            base = as_base_tensor(attention_mask.detach())
+            # the kernels read one byte per mask element
+            mask_bytes = (base if base.dtype == torch.bool else base != 0).view(torch.uint8)
+
+        if (attention_bias is None) != (sparsity_layout_bias is None):
+            raise ValueError("attention_bias and sparsity_layout_bias must be provided together")
+        has_bias = attention_bias is not None
+        if has_bias:
+            attention_bias = ensure_contiguous(attention_bias)
+            sparsity_layout_bias = ensure_contiguous(sparsity_layout_bias)
+            validate_dimensions(attention_bias, sparsity_layout_bias)
+            validate_contiguous(attention_bias, sparsity_layout_bias)
+            validate_device(attention_bias, sparsity_layout_bias, q)
+            validate_dtype_float(attention_bias)
+            validate_sparsity(sparsity_block_size, (attention_bias, sparsity_layout_bias))
+            validate_shape(sparsity_layout_bias, attention_shape, "sparsity_layout_bias")
+            if attention_bias.dtype != q.dtype:
+                attention_bias = attention_bias.to(q.dtype)
+        else:
+            attention_bias = torch.empty(0, device=q.device, dtype=q.dtype)
+
+        for_one_call = layout_cache is None
+        layout_cache = flash_attention_build_layout_cache(
+            attention_layout, sparsity_layout_q, sparsity_layout_k, sparsity_layout_v,
+            n_seq_blocks_q, n_seq_blocks_k, n_head_blocks_qk,
+            sparsity_layout_o=sparsity_layout_o, n_head_blocks_v=n_head_blocks_v,
+            sparsity_layout_mask=sparsity_layout_mask, sparsity_layout_bias=sparsity_layout_bias,
+            layout_cache=layout_cache,
+        )
+        if "key_offsets_i32" not in layout_cache:
+            for name in ("key_offsets", "key_indices", "query_offsets", "query_indices"):
+                layout_cache[name + "_i32"] = _as_index(layout_cache[name], torch.int32)
+            if (n_seq_blocks_k < (1 << 28) and layout_cache["key_indices"].numel() < INT32_INDEX_MAX
+                    and n_head_blocks_qk <= 2 and n_head_blocks_v <= 2 and sparsity_block_size == 64):
+                offsets, records, group_size = _build_forward_records(
+                    layout_cache, attention_layout, int(n_batches), int(n_seq_blocks_q), int(n_seq_blocks_k),
+                    int(n_head_blocks_qk), int(n_head_blocks_v), own_layout=True)
+                layout_cache["group_offsets"], layout_cache["group_records"] = offsets, records
+                layout_cache["group_size"] = group_size
+            layout_cache["tables"] = _Tables(layout_cache)
+            finalize_layout_cache(layout_cache)
+
+        meta = _Meta()
+        meta.tables = layout_cache["tables"]
+        meta.dims = (int(n_batches), int(n_seq_blocks_q), int(n_seq_blocks_k), int(n_head_blocks_qk),
+                     int(n_head_blocks_v))
+        meta.sbs = sparsity_block_size
+        meta.scale = scale
+        meta.has_bias = has_bias
+        # the default output layout: rows of a full V layout are there as a whole where a query block has a key block
+        meta.o_rows_whole = 1 if sparsity_layout_o is None else 0
+        meta.facts = _mask_facts(layout_cache, attention_layout, attention_mask, mask_bytes, lengths, meta.dims,
+                                 sparsity_block_size)
+
+        needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad
+                                                  or (attention_bias is not None and attention_bias.requires_grad))
+        meta.shares = _row_shares(meta, q.dtype, q.device, needs_grad, for_one_call)
         # nothing to differentiate: the launch itself, without the autograd machinery around it
         out = (_FlashAttention.apply(q, k, v, attention_bias, mask_bytes, lengths, meta) if needs_grad
                else _forward_launch(q, k, v, attention_bias, mask_bytes, lengths, meta)[0])
