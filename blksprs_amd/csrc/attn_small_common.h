@@ -341,15 +341,16 @@ struct OwnOperand {
   const OwnRows<Ar::kElem, SBS, NS, kHalves> &rows;
   __device__ inline explicit OwnOperand(const OwnRows<Ar::kElem, SBS, NS, kHalves> &own) : rows(own) {}
 };
-// in parts: fragments 2 p and 2 p + 1 in one, the second half zero behind an odd last one
+// in parts: fragments 2 p and 2 p + 1 in one
 template <int SBS, int NS, int kHalves, bool kSecond>
 struct OwnOperand<SSplit, SBS, NS, kHalves, kSecond> {
-  static constexpr int kFrags = OwnRows<4, SBS, NS, kHalves>::T::kFrags, kParts = (kFrags + 1) / 2;
+  static constexpr int kFrags = OwnRows<4, SBS, NS, kHalves>::T::kFrags, kParts = kFrags / 2;
+  static_assert(kFrags % 2 == 0, "whole pairs of fragments");
   Parts parts[kParts];
   __device__ inline explicit OwnOperand(const OwnRows<4, SBS, NS, kHalves> &own) {
 #pragma unroll
     for (int p = 0; p < kParts; ++p)
-      parts[p] = Parts::of<kDotParts<NS>>(own.fr[2 * p], 2 * p + 1 < kFrags ? own.fr[2 * p + 1] : u32x4{0u, 0u, 0u, 0u}, kSecond ? kUp : 1.f);
+      parts[p] = Parts::of<kDotParts<NS>>(own.fr[2 * p], own.fr[2 * p + 1], kSecond ? kUp : 1.f);
   }
 };
 
@@ -407,7 +408,8 @@ __device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<T
     for (int p = 0; p < OwnOperand<Tr, SBS, NS, kHalves, kSecond>::kParts; ++p)
 #pragma unroll
       for (int t = 0; t < NB; ++t)
-        multiply_parts<!kOwnIsQuery>(acc[t], Parts::of<kDotParts<NS>>(rows.frag(t, 2 * p), 2 * p + 1 < kFrags ? rows.frag(t, 2 * p + 1) : u32x4{0u, 0u, 0u, 0u}, kSecond ? kUp : 1.f), own.parts[p]);
+        multiply_parts<!kOwnIsQuery>(acc[t], Parts::of<kDotParts<NS>>(rows.frag(t, 2 * p), rows.frag(t, 2 * p + 1), kSecond ? kUp : 1.f),
+                                     own.parts[p]);
   } else {
 #pragma unroll
     for (int f = 0; f < kFrags; ++f)

@@ -58,19 +58,15 @@ struct Parts {
 };
 
 // acc += a x b, the small products first
-__device__ static inline void multiply_part(f32x16 &acc, u32x4 a, u32x4 b) { acc = MBf16::mfma(a, b, acc); }
-__device__ static inline void multiply_part(f32x4 &acc, u32x4 a, u32x4 b) {
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
-}
 // kExchanged: in the order of the exchanged operands, so that a x b and b x a are the same bits in two kernels
-template <bool kExchanged = false, typename Acc>
-__device__ static inline void multiply_parts(Acc &acc, const Parts &a, const Parts &b) {
-  multiply_part(acc, kExchanged ? a.high : a.low, kExchanged ? b.low : b.high);
-  multiply_part(acc, kExchanged ? a.low : a.high, kExchanged ? b.high : b.low);
-  multiply_part(acc, a.mid, b.mid);
-  multiply_part(acc, kExchanged ? a.high : a.mid, kExchanged ? b.mid : b.high);
-  multiply_part(acc, kExchanged ? a.mid : a.high, kExchanged ? b.high : b.mid);
-  multiply_part(acc, a.high, b.high);
+template <bool kExchanged = false>
+__device__ static inline void multiply_parts(f32x16 &acc, const Parts &a, const Parts &b) {
+  acc = MBf16::mfma(kExchanged ? a.high : a.low, kExchanged ? b.low : b.high, acc);
+  acc = MBf16::mfma(kExchanged ? a.low : a.high, kExchanged ? b.high : b.low, acc);
+  acc = MBf16::mfma(a.mid, b.mid, acc);
+  acc = MBf16::mfma(kExchanged ? a.high : a.mid, kExchanged ? b.mid : b.high, acc);
+  acc = MBf16::mfma(kExchanged ? a.mid : a.high, kExchanged ? b.high : b.mid, acc);
+  acc = MBf16::mfma(a.high, b.high, acc);
 }
 
 // Whether one of a wave's sums is infinite or NaN
