@@ -808,6 +808,10 @@ struct Walk {
   // multiplied by qk_scale and complete, and cc is 1.  me: this lane's own row; group: lane / SBS.
   template <typename Tr>
   __device__ inline void finish_scores(const Step &s, float *sv, float qk_scale, int me, int group) const {
+    // fp32 up to head dimension 64: what the lane's addresses in a mask or bias block have in common is formed here and not in front
+    // of the walk, where it takes registers that dK / dV does not have (BigBird: 53.4 -> 51.9 us; dK / dV at 128, which spills
+    // others then, 134 -> 140)
+    if constexpr (ES == 4 && NS <= 2) asm volatile("" : "+v"(me), "+v"(group));
     constexpr int kRegs = SBS == 32 ? 16 : 4;
     constexpr int kSide = kHalves * SBS;  // of a block of the layout, for mask and bias
     const late_args_t p = late_args();

@@ -40,11 +40,11 @@ def kernels():
 @pytest.mark.parametrize("kernel", ["fwd", "dq", "dkv"])
 @pytest.mark.parametrize("slices,halves", [(1, 1), (2, 1), (3, 1), (4, 1), (2, 2), (4, 2)])
 def test_fp32_attention_keeps_its_registers(kernels, kernel, slices, halves):
-    """Blocks of 32 (halves 1) and of 64 (2).  dK / dV: up to four at head dimension 64, stored once in front of the walk; at 128
+    """Blocks of 32 (halves 1) and of 64 (2).  dK / dV: up to two at head dimension 64 in halves, stored once in front of the walk; at 128
     operands in parts and sums take 320 of 512 registers and up to 28 of the rest are stored and loaded in a step of 3100
     instructions."""
     found = [k for name, k in kernels.items()
              if f"attn_small_{kernel}_kernelI" in name and f"SF32ELi32ELi{slices}ELb0ELi{halves}EE" in name]
     assert len(found) == 1
     spilled = found[0][".vgpr_spill_count"]
-    assert spilled <= ({2: 4, 4: 28}.get(slices, 0) if kernel == "dkv" else 0)
+    assert spilled <= ({(2, 2): 2, (4, 1): 28, (4, 2): 28}.get((slices, halves), 0) if kernel == "dkv" else 0)
