@@ -1,7 +1,8 @@
 // C ABI of block-sparse flash attention: argument checks and the choice of kernels: 16-bit operands in 64 x 64 blocks
 // with at most two head slices (attn_mfma.hip, attn_bwd_mfma.hip), blocks of 16 and 32 and fp32 blocks of 64 with head
 // dimensions up to 128 (attn_small_fwd.hip, attn_small_bwd.hip), the rest on the fp32 matrix-core instruction
-// (attn_f32mma.hip: fp32 blocks of 64 with missing slices, longer head dimensions, scales that are not positive, tensors that do not start on 16 bytes), and the generic
+// (attn_f32mma.hip: fp32 blocks of 64 with missing slices, longer head dimensions, scales that are not positive, tensors that
+// do not start on 16 bytes), and the generic
 // kernels for more head slices than fit LDS.
 #include "attn_common.h"
 

@@ -10,9 +10,9 @@
 // than four waves are several workgroups', whose sums a small launch adds up, in order.  Long rows come first, then the others
 // by the waves they get, each kind in the order of RowOfWave.
 //
-// 7 sequences of 3328, sbs 32, head dimension 96, BigBird, bf16, forward: 28.9 us with, 74.8 without; 14 of 1056, sbs 32, head
-// dimension 128, BigBird, fp32, forward and backward: 245 with, 347 without; one of 6080, sbs 64, head dimension 64, causal,
-// fp32, the same: 324 with, 478 without.
+// 7 sequences of 3328, sbs 32, head dimension 96, BigBird, bf16, forward: 27 us with, 76 without; 14 of 1056, sbs 32, head
+// dimension 128, BigBird, fp32, forward and backward: 248 with, 340 without; one of 6080, sbs 64, head dimension 64, causal,
+// fp32, the same: 279 with, 429 without.
 #include "attn_small_common.h"
 
 namespace bsa {

@@ -19,7 +19,7 @@
 // to overlap it.  Against the fp32 matrix-core kernels that ran these shapes before (48 x 4096 queries, sbs 32, head
 // dimension 64, fp16, 33 key blocks per query block): delta + zero fill 0.071 -> 0, dK / dV 1.89 -> 0.125 ms (530 TFLOP/s),
 // dQ 1.24 -> 0.090 ms (delta included); fp32, sbs 32, products from bf16 parts (split_f32.h), 8 x 2048 queries, half of the
-// blocks, head dimension 64: dK / dV 94.5 -> 75.5, dQ 74.8 -> 59.0 us (114 and 109 TFLOP/s) against the fp32 instruction.  fp32
+// blocks, head dimension 64: dK / dV 94.5 -> 73.1, dQ 74.8 -> 55.8 us (118 and 115 TFLOP/s) against the fp32 instruction.  fp32
 // blocks of 64, whose halves walk alone like blocks of 32: 20 x 960, causal, head dimension 64: delta + zero fill 19 -> 0, dK /
 // dV 129 (eight waves to a tile) -> 44, dQ 128 -> 37 us.
 //

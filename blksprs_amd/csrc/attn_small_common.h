@@ -65,7 +65,12 @@ struct SF32 {
 
 // fp32 products from bf16 parts: of blocks of 32 (and halves of blocks of 64) all of whose slices are there.  Blocks of 16, whose
 // fp32 products take half as long for the same values to split, are no faster with it (6 x 1040 queries, causal, head dimension
-// 32: forward 16.1 -> 16.6 us, dK / dV 20.0 -> 21.9).
+// 32: forward 16.1 -> 16.6 us, dK / dV 20.0 -> 21.9).  Blocks of 32, fp32 instruction -> parts, us (8 x 2048, half of the blocks):
+//     head dimension     32             64             96             128
+//     forward       32.4 -> 29.8   55.2 -> 46.5   96.5 -> 83.7   122 -> 105
+//     dQ            42.8 -> 38.4   76.7 -> 63.2    128 -> 110    166 -> 140
+//     dK / dV       54.1 -> 47.8   97.6 -> 81.0    170 -> 152    219 -> 198
+// causal and BigBird layouts 4 to 24 % less (dK / dV of BigBird at 128: 138 -> 132), blocks of 64 at 128 2 to 12 %.
 struct SSplit : SF32 {};
 template <int NS>
 constexpr bool kDotParts = NS > 2;  // Parts::of
@@ -393,7 +398,8 @@ __device__ static inline bool scores_in_doubt(const OwnRows<ES, SBS, NS, kHalves
 
 // acc (per partner block t) = partner rows x own rows over all head slices: acc[t] belongs to this lane's own row
 // (lane % SBS) and partner rows 8 (r / 4) + 4 (lane / 32) + r % 4 (SBS 32) or 4 (lane / 16) + r (SBS 16).
-// kOwnIsQuery, kSecond: as in Walk; a score from parts is the same bits wherever it is formed; of the second tensor acc is
+// kOwnIsQuery, kSecond: as in Walk; a score from parts is the same bits wherever it is formed, but forward and backward kernels
+// look at blocks of their own before they form one from parts (scores_in_doubt) and may differ there by its rounding; of the second tensor acc is
 // up_of^2 times the product
 template <typename Tr, int SBS, int NS, int NB, int kHalves, bool kOwnIsQuery, bool kSecond, typename Acc>
 __device__ static inline void product_rows(Acc (&acc)[NB], const typename Tile<Tr::kElem, SBS, NS, NB, kHalves>::RowReader &rows,
@@ -976,7 +982,7 @@ struct RowOfWave {
   __device__ inline RowOfWave(const Shares &shares, int halves, int64_t batches, int64_t rows_per_batch, bool last_first, int wave,
                               int waves_of_group, int split) {
     if (shares.groups) {
-      // groups of an XCD are BSA_SHARE_XCDS apart, also with two halves each
+      // groups of an XCD are eight (XCDs) apart, also with two halves each
       const uint32_t xcd = blockIdx.x & 7, turn = blockIdx.x >> 3;
       const int32_t *g = shares.groups + (int64_t)((turn / halves) * 8 + xcd) * BSA_SHARE_INTS;
       own = first_lane(g[wave]);

@@ -18,7 +18,7 @@
 // wave at a time.  Against the fp32 matrix-core kernel that ran these shapes before: 48 x 4096 queries, sbs 32, head
 // dimension 64, fp16, 33 key blocks per query block: 0.65 -> 0.072 ms (460 TFLOP/s, 18 % of the matrix cores' peak); 32
 // prompts of 1032 to 2064 tokens, sbs 16, bf16, causal: 0.54 -> 0.044 ms.  fp32, sbs 32, products from bf16 parts (split_f32.h):
-// 8 x 2048 queries, half of the blocks, head dimension 64: 51.1 -> 42.3 us (102 TFLOP/s) against the fp32 instruction; the 490
+// 8 x 2048 queries, half of the blocks, head dimension 64: 51.1 -> 41.0 us (105 TFLOP/s) against the fp32 instruction; the 490
 // vector instructions of a step that split its values cost more than its 48 products, and 512 lists of 32 +- 4 blocks cut in
 // four fill the chip once, so the launch waits for the longest.  fp32 blocks of 64, whose halves walk alone like blocks of 32:
 // 20 x 960, causal, head dimension 64: 97.8 (eight waves to a tile) -> 27.4 us.

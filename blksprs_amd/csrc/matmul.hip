@@ -16,13 +16,7 @@
 #include <type_traits>
 
 #include "attn_mfma_common.h"
-
-namespace bsa {
-// matmul_split.hip
-int matmul_split_f32(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs,
-                     const int32_t *block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int sbs, int trans_x, int trans_y,
-                     hipStream_t s);
-}  // namespace bsa
+#include "split_f32.h"
 
 namespace {
 

@@ -14,7 +14,7 @@
 // last of which run alone.  Waves that multiply go first (s_setprio: dX 77 -> 71 us).  Two buffers with one barrier and the split
 // in the shadow of the wave's own products, which leaves three workgroups: 93 / 78 / 82 us where this takes 80 / 71 / 81 (8 x
 // 2048^3 at 25 %, sbs 64, forward / dX / dY; 1 % more since the values are multiplied by kUp).  The kernel before it, on the fp32 instruction, five workgroups of asynchronous
-// copies: 103 / 99 / 99; 3 x 1920 x 2944 x 1664 at 30 %, sbs 128, all three: 199 -> 158.
+// copies: 103 / 99 / 99; 3 x 1920 x 2944 x 1664 at 30 %, sbs 128, all three: 199 -> 173.
 #include "split_f32.h"
 
 namespace bsa {

@@ -9,9 +9,11 @@ using namespace mfma;
 
 __device__ static inline float as_float(uint32_t v) { return __builtin_bit_cast(float, v); }
 
-// fp32 values as three bf16 parts: the value rounded to 8 bits, what is left of it rounded to 8 bits, and the rest, which fits.
-// A product of two such values is six products of parts, each
-// exact, added up in fp32 by matrix instructions of 16 times the fp32 instruction's rate: 2.7 times the products per second,
+// fp32 values as three bf16 parts: the value rounded to 8 bits, what is left of it rounded to 8 bits, and the rest, which fits
+// (G. Henry, P. T. P. Tang and A. Heinecke, Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations, 2019).  A product of two such values is six products of parts, each exact, added up in fp32 by matrix instructions
+// of 16 times the fp32 instruction's rate: 2.7 times the products per second.  The other three are worth up to 2^-24 of the
+// product (the second part is up to 2^-8 of a value, the third 2^-17), 0.1 of that in the mean square.  The sums come
 // with one rounding per 16 (32) contracted values and part where the fp32 instruction rounds every 2 (4).  Sums of 64 / 512 / 2048
 // random products are 1.09e-7 / 3.4e-7 / 7.1e-7 from 64 bits, the fp32 instruction's 1.45e-7 / 4.1e-7 / 8.1e-7.
 //
@@ -81,4 +83,9 @@ __device__ static inline bool not_finite(const Acc (&acc)[NS], float also = 0.f)
 }
 
 }  // namespace split
+
+// matmul_split.hip: fp32, sbs 64 and above
+int matmul_split_f32(const void *x, const void *y, void *out, const int32_t *pair_offsets, const int32_t *pairs,
+                     const int32_t *block_order, int64_t nnz_o, int64_t nnz_x, int64_t nnz_y, int sbs, int trans_x, int trans_y,
+                     hipStream_t s);
 }  // namespace bsa

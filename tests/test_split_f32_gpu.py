@@ -1,5 +1,5 @@
 """fp32 products formed from bf16 parts (split_f32.h): their error, values whose parts do not hold them (infinite, NaN, next to
-the largest number, far below one), and the fp32 instruction that forms such sums again."""
+the largest number), and the fp32 instruction that forms such sums again; values far below one."""
 
 import pytest
 import torch
@@ -66,7 +66,8 @@ def _matmul(device, sbs, R, K, C, density, change=None, x_scale=1.0, y_scale=1.0
                         dy64[b, ks, cols] += x64[b, rows, ks].T @ g64[b, rows, cols]
                         size_y[b, ks, cols] += x64[b, rows, ks].T.abs() @ g64[b, rows, cols].abs()
     for what, got, want, size, layout, n in (("O", out, o64, size_o, lo, K), ("dX", dx, dx64, size_x, lx, C), ("dY", dy, dy64, size_y, ly, R)):
-        # six roundings for 16 values, three dropped products of 2^-26 together, and what underflows
+        # six roundings for 16 values, three dropped products of up to EPS together, and what underflows.  A bound for the worst
+        # case: tests/test_split_f32_range_gpu.py holds the mean square, which tells whether all six products are there
         roundings = 6 * n * sbs / 16 + 4
         bound = roundings * 2 * EPS * _compressed(size, layout, sbs) + 1e-37
         _assert_like(got, _compressed(want, layout, sbs), bound, what)
@@ -121,7 +122,7 @@ def _attention(device, sbs, nh, change=None, grad_scale=1.0):
 @pytest.mark.parametrize("sbs,nh", [(32, 1), (32, 2), (32, 3), (32, 4), (64, 1), (64, 2)])
 @pytest.mark.parametrize("grad_scale", [1.0, 2.0 ** -112, 2.0 ** 100])
 def test_attention(device, sbs, nh, grad_scale):
-    """Relative errors (2-norm) against 64 bits; the largest seen is 4e-7.  Gradients of about 2^-112 have lost parts."""
+    """Relative errors (2-norm) against 64 bits; the largest seen is 4e-7."""
     got, want = _attention(device, sbs, nh, grad_scale=grad_scale)
     for what, g, w in zip(("O", "dQ", "dK", "dV"), got, want):
         g = g.detach().double().cpu()
