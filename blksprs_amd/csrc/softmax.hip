@@ -3,26 +3,33 @@
 // The blocks of one block row are consecutive in the compressed tensor (row-major
 // block order), so a row is `count` whole blocks starting at row_offsets[r].  One
 // wavefront owns a group of element rows of one block row and reads them with one
-// float4 per lane: for sbs <= 256 the 64 lanes cover 256 consecutive floats of a
-// block (256/sbs element rows), so every wave load is one contiguous KiB.  The max /
-// sum reductions stay inside the sbs/4 lanes of an element row (xor shuffles).
-// Rows of up to 32 float4 units per lane stay in registers between the reduction
-// and the write (one HBM read + one write); longer rows make two read passes.
+// float4 per lane.  sbs/4 lanes cover an element row of one block; where rows are long,
+// 2, 4 or 8 such groups of lanes share it, each taking every second, fourth or eighth
+// block (make_geom), so that it fits their registers: rows of up to 16 float4 units per
+// lane (32 in the forward pass of sbs >= 128) stay there between the reduction and the
+// write (one HBM read + one write), longer rows make two read passes.  The reductions stay inside the lanes of a row.
+//
+// Bound by HBM.  Block-causal rows of n = 2048 elements and 10 % more blocks, us forward +
+// backward, a row on sbs/4 lanes (32 units in registers) -> shared: sbs 16, 16 matrices
+// 87 + 165 -> 62 + 83; sbs 32 77 + 125 -> 57 + 82; sbs 64, 32 matrices 114 + 165 -> 106 + 153
+// (5.7 and 5.9 TB/s); three matrices of 37 blocks of 32 a side 13.3 + 16.0 -> 6.6 + 7.9.
 #include "common.h"
 
 namespace {
 
-constexpr int kMaxUnits = 32;
+constexpr int kBwdUnits = 16;  // float4 units per lane in registers, of either tensor
 constexpr int kWaves = 4;  // waves (tasks) per workgroup
 
 struct RowGeom {
   int sbs_log2;
-  int lpr;       // lanes per element row = min(64, sbs/4)
-  int nq_log2;   // float4 units per lane per block = max(1, sbs/256), as log2
-  int groups_log2;  // wave tasks per block row = sbs * lpr / 64, as log2
+  int lpr;          // lanes on one block of an element row = min(64, sbs/4)
+  int nq_log2;      // float4 units per lane per block = max(1, sbs/256), as log2
+  int split_log2;   // lane groups that share an element row, each taking every 2^split_log2-th block of it
+  int lanes;        // lanes of an element row = lpr << split_log2
+  int groups_log2;  // wave tasks per block row = sbs * lanes / 64, as log2
 };
 
-// The reductions over the lpr lanes of an element row, without a trip through LDS (a shuffle computes a lane
+// The reductions over the lanes of an element row, without a trip through LDS (a shuffle computes a lane
 // address, goes through LDS and waits for it).  Steps 1 and 2 exchange inside a group of four lanes (DPP quad_perm);
 // after them the four lanes of a group agree, so mirroring a half row (lane i <-> 7 - i) pairs every group with its
 // neighbour and mirroring a row (i <-> 15 - i) pairs the two halves of 16 lanes: partners other than those of an
@@ -62,16 +69,21 @@ __device__ inline float lanes_sum(float v, int lpr) {
 // float offset of unit u, relative to the first block of the row and to the lane's own offset (the same for every
 // lane: the compiler keeps it in scalar registers)
 __device__ inline int64_t unit_offset(int u, const RowGeom &g) {
-  const int t = u >> g.nq_log2;
+  const int t = (u >> g.nq_log2) << g.split_log2;
   const int q = u & ((1 << g.nq_log2) - 1);
   return ((int64_t)t << (2 * g.sbs_log2)) + q * 256;
 }
 
-// What this wave works on: `first` (float offset of the row's first block), `units` (float4 units per lane) and the
-// task index are the same for all lanes and are computed from values the compiler knows to be wave-uniform, so
-// the loops over units branch on scalar registers instead of masking lanes.
-__device__ inline bool wave_task(const RowGeom &g, const int32_t *row_offsets, int64_t n_tasks, int64_t &first,
-                                 int &units, int &lane_base) {
+// What this wave works on: `first` (float offset of the row's first block) and `units` (rounds of float4 units per lane)
+// are the same for all lanes and are computed from values the compiler knows to be wave-uniform, so the loops over units
+// branch on scalar registers instead of masking lanes.  A lane group whose part of the row has no unit in the last round
+// (in_last) reads the first group's there (its tail_base), which changes no maximum, and leaves it out of sums and results.
+struct RowTask {
+  int64_t first;
+  int units, lane_base, tail_base;
+  bool in_last;
+};
+__device__ inline bool wave_task(const RowGeom &g, const int32_t *row_offsets, int64_t n_tasks, RowTask &task) {
   // Workgroup b runs on XCD b % 8: each XCD takes a contiguous eighth of the tasks, so the waves that read
   // neighbouring KiB of the same blocks (the tasks of one block row) share one L2.
   const int64_t n_groups = (n_tasks + kWaves - 1) / kWaves, per_xcd = (n_groups + 7) >> 3;
@@ -84,11 +96,15 @@ __device__ inline bool wave_task(const RowGeom &g, const int32_t *row_offsets, i
   const int start = row_offsets[r];
   const int count = row_offsets[r + 1] - start;
   if (count <= 0) return false;
-  first = (int64_t)start << (2 * g.sbs_log2);
-  units = count << g.nq_log2;
-  const int rows_per_wave = 64 / g.lpr;
-  const int row_in_block = grp * rows_per_wave + lane / g.lpr;
-  lane_base = (row_in_block << g.sbs_log2) + (lane % g.lpr) * 4;
+  task.first = (int64_t)start << (2 * g.sbs_log2);
+  const int split = 1 << g.split_log2, rounds = (count + split - 1) >> g.split_log2;
+  task.units = rounds << g.nq_log2;
+  const int part = lane / g.lpr & (split - 1);
+  const int row_in_block = grp * (64 / g.lanes) + lane / g.lanes;
+  task.tail_base = (row_in_block << g.sbs_log2) + (lane % g.lpr) * 4;
+  task.lane_base = task.tail_base + (part << (2 * g.sbs_log2));
+  task.in_last = part < count - ((rounds - 1) << g.split_log2);
+  if (task.in_last) task.tail_base = task.lane_base;
   return true;
 }
 
@@ -117,19 +133,28 @@ __device__ inline float max_with(float m, float4 v) {
   return t;
 }
 
+// This lane's part of a row of a tensor
+struct RowPart {
+  const float *row, *tail;  // where its units are read from, in all rounds and in the last
+  int last;                 // the last round
+  __device__ inline RowPart(const float *tensor, const RowTask &task)
+      : row(tensor + task.first + task.lane_base), tail(tensor + task.first + task.tail_base), last(task.units - 1) {}
+  __device__ inline float4 unit(int u, const RowGeom &g) const {
+    // with several units per block (blocks wider than 256) no row is split and tail is row
+    return *reinterpret_cast<const float4 *>((u == last ? tail : row) + unit_offset(u, g));
+  }
+};
+
 // Loads units [0, units) of a row into v, four at a time: within a group of four the index is clamped to the last
 // unit (a repeated load of a line just fetched) so that the group has no branch, and no load is followed by its
 // use: all loads of the row are in flight together.  Entries at and beyond `units` hold copies of the last unit.
 template <int N>
-__device__ inline void load_row(float4 (&v)[N], const float *row, int units, const RowGeom &g) {
+__device__ inline void load_row(float4 (&v)[N], const RowPart &part, const RowGeom &g) {
 #pragma unroll
   for (int c = 0; c < N; c += 4) {
-    if (c < units) {
+    if (c <= part.last) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int u = c + j < units ? c + j : units - 1;
-        v[c + j] = *reinterpret_cast<const float4 *>(row + unit_offset(u, g));
-      }
+      for (int j = 0; j < 4; ++j) v[c + j] = part.unit(c + j < part.last ? c + j : part.last, g);
     }
   }
 }
@@ -138,39 +163,39 @@ __device__ inline void load_row(float4 (&v)[N], const float *row, int units, con
 // branch between them; entries at and beyond `count` hold copies of the last unit.
 constexpr int kChunk = 8;
 template <int N>
-__device__ inline void load_chunk(float4 (&v)[N], const float *row, int u0, int count, const RowGeom &g) {
+__device__ inline void load_chunk(float4 (&v)[N], const RowPart &part, int u0, int count, const RowGeom &g) {
 #pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const int u = u0 + (j < count ? j : count - 1);
-    v[j] = *reinterpret_cast<const float4 *>(row + unit_offset(u, g));
-  }
+  for (int j = 0; j < N; ++j) v[j] = part.unit(u0 + (j < count ? j : count - 1), g);
 }
 
+// kUnits: float4 units per lane in registers
+template <int kUnits>
 __global__ __launch_bounds__(64 * kWaves) void softmax_fwd_kernel(const float *__restrict__ x, float *__restrict__ out,
                                                           const int32_t *__restrict__ row_offsets, int64_t n_tasks,
                                                           RowGeom g) {
-  int64_t first;
-  int units, lane_base;
-  if (!wave_task(g, row_offsets, n_tasks, first, units, lane_base)) return;
-  const float *xr = x + first + lane_base;
-  float *orow = out + first + lane_base;
+  RowTask task;
+  if (!wave_task(g, row_offsets, n_tasks, task)) return;
+  const int units = task.units;
+  const RowPart xr(x, task);
+  float *orow = out + task.first + task.lane_base;
+  auto mine = [&](int u) { return u < units - 1 || task.in_last; };  // of u < units
 
-  if (units <= kMaxUnits) {
-    float4 v[kMaxUnits];
-    load_row(v, xr, units, g);
+  if (units <= kUnits) {
+    float4 v[kUnits];
+    load_row(v, xr, g);
     float m = -INFINITY;
 #pragma unroll
-    for (int c = 0; c < kMaxUnits; c += 4) {
+    for (int c = 0; c < kUnits; c += 4) {
       if (c < units) {  // the copies of the last unit change no maximum
 #pragma unroll
         for (int j = 0; j < 4; ++j) m = max_with(m, v[c + j]);
       }
     }
-    const float m2 = lanes_max(m, g.lpr) * kLog2e;
+    const float m2 = lanes_max(m, g.lanes) * kLog2e;
     float s = 0.f;
 #pragma unroll
-    for (int u = 0; u < kMaxUnits; ++u) {
-      if (u < units) {
+    for (int u = 0; u < kUnits; ++u) {
+      if (u < units && mine(u)) {
         v[u].x = exp_rel(v[u].x, m2);
         v[u].y = exp_rel(v[u].y, m2);
         v[u].z = exp_rel(v[u].z, m2);
@@ -178,11 +203,11 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_fwd_kernel(const float *_
         s += (v[u].x + v[u].y) + (v[u].z + v[u].w);
       }
     }
-    s = lanes_sum(s, g.lpr);
+    s = lanes_sum(s, g.lanes);
     const float inv = 1.f / s;  // one division per row, then products
 #pragma unroll
-    for (int u = 0; u < kMaxUnits; ++u) {
-      if (u < units) {
+    for (int u = 0; u < kUnits; ++u) {
+      if (u < units && mine(u)) {
         float4 o;
         o.x = v[u].x * inv;
         o.y = v[u].y * inv;
@@ -209,7 +234,7 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_fwd_kernel(const float *_
       float add = 0.f;
 #pragma unroll
       for (int j = 0; j < kChunk; ++j)
-        if (j < count)
+        if (j < count && mine(u0 + j))
           add += (exp_rel(v[j].x, mn2) + exp_rel(v[j].y, mn2)) + (exp_rel(v[j].z, mn2) + exp_rel(v[j].w, mn2));
       s = s * exp2_of(m * kLog2e - mn2) + add;
     } else {
@@ -221,10 +246,10 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_fwd_kernel(const float *_
     }
     m = mn;
   }
-  const float mall = lanes_max(m, g.lpr);
+  const float mall = lanes_max(m, g.lanes);
   const float mall2 = mall * kLog2e;
   float part = (m == -INFINITY) ? ((s != s) ? s : 0.f) : s * exp2_of(m * kLog2e - mall2);
-  const float sall = lanes_sum(part, g.lpr);
+  const float sall = lanes_sum(part, g.lanes);
   const float inv_all = 1.f / sall;
   for (int u0 = 0; u0 < units; u0 += kChunk) {
     const int count = units - u0 < kChunk ? units - u0 : kChunk;
@@ -232,7 +257,7 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_fwd_kernel(const float *_
     load_chunk(v, xr, u0, count, g);
 #pragma unroll
     for (int j = 0; j < kChunk; ++j) {
-      if (j < count) {
+      if (j < count && mine(u0 + j)) {
         float4 o;
         o.x = exp_rel(v[j].x, mall2) * inv_all;
         o.y = exp_rel(v[j].y, mall2) * inv_all;
@@ -248,27 +273,26 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *_
                                                           const float *__restrict__ y, float *__restrict__ grad_in,
                                                           const int32_t *__restrict__ row_offsets, int64_t n_tasks,
                                                           RowGeom g) {
-  int64_t first;
-  int units, lane_base;
-  if (!wave_task(g, row_offsets, n_tasks, first, units, lane_base)) return;
-  const float *gr = grad_out + first + lane_base;
-  const float *yr = y + first + lane_base;
-  float *dr = grad_in + first + lane_base;
+  RowTask task;
+  if (!wave_task(g, row_offsets, n_tasks, task)) return;
+  const int units = task.units;
+  const RowPart gr(grad_out, task), yr(y, task);
+  float *dr = grad_in + task.first + task.lane_base;
+  auto mine = [&](int u) { return u < units - 1 || task.in_last; };  // of u < units
 
-  if (units <= kMaxUnits / 2) {
-    constexpr int kU = kMaxUnits / 2;
-    float4 yv[kU], gv[kU];
-    load_row(yv, yr, units, g);
-    load_row(gv, gr, units, g);
+  if (units <= kBwdUnits) {
+    float4 yv[kBwdUnits], gv[kBwdUnits];
+    load_row(yv, yr, g);
+    load_row(gv, gr, g);
     float s = 0.f;
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (u < units) s += (yv[u].x * gv[u].x + yv[u].y * gv[u].y) + (yv[u].z * gv[u].z + yv[u].w * gv[u].w);
+    for (int u = 0; u < kBwdUnits; ++u) {
+      if (u < units && mine(u)) s += (yv[u].x * gv[u].x + yv[u].y * gv[u].y) + (yv[u].z * gv[u].z + yv[u].w * gv[u].w);
     }
-    s = lanes_sum(s, g.lpr);
+    s = lanes_sum(s, g.lanes);
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (u < units) {
+    for (int u = 0; u < kBwdUnits; ++u) {
+      if (u < units && mine(u)) {
         float4 o;
         o.x = yv[u].x * (gv[u].x - s);
         o.y = yv[u].y * (gv[u].y - s);
@@ -280,34 +304,34 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *_
     return;
   }
 
-  if (units <= kMaxUnits) {
+  if (units <= 2 * kBwdUnits) {
     // middle rows: y stays in registers, the gradient passes twice in chunks (once for the row's sum, once for the
     // result): 1.5 instead of 2 reads of the row's 2 x 16 bytes per element
-    float4 yv[kMaxUnits];
-    load_row(yv, yr, units, g);
+    float4 yv[2 * kBwdUnits];
+    load_row(yv, yr, g);
     float s = 0.f;
 #pragma unroll
-    for (int c = 0; c < kMaxUnits; c += kChunk) {
+    for (int c = 0; c < 2 * kBwdUnits; c += kChunk) {
       if (c < units) {
         const int count = units - c < kChunk ? units - c : kChunk;
         float4 gv[kChunk];
         load_chunk(gv, gr, c, count, g);
 #pragma unroll
         for (int j = 0; j < kChunk; ++j)
-          if (j < count)
+          if (j < count && mine(c + j))
             s += (yv[c + j].x * gv[j].x + yv[c + j].y * gv[j].y) + (yv[c + j].z * gv[j].z + yv[c + j].w * gv[j].w);
       }
     }
-    s = lanes_sum(s, g.lpr);
+    s = lanes_sum(s, g.lanes);
 #pragma unroll
-    for (int c = 0; c < kMaxUnits; c += kChunk) {
+    for (int c = 0; c < 2 * kBwdUnits; c += kChunk) {
       if (c < units) {
         const int count = units - c < kChunk ? units - c : kChunk;
         float4 gv[kChunk];
         load_chunk(gv, gr, c, count, g);
 #pragma unroll
         for (int j = 0; j < kChunk; ++j) {
-          if (j < count) {
+          if (j < count && mine(c + j)) {
             float4 o;
             o.x = yv[c + j].x * (gv[j].x - s);
             o.y = yv[c + j].y * (gv[j].y - s);
@@ -330,9 +354,9 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *_
     load_chunk(gv, gr, u0, count, g);
 #pragma unroll
     for (int j = 0; j < kChunk; ++j)
-      if (j < count) s += (yv[j].x * gv[j].x + yv[j].y * gv[j].y) + (yv[j].z * gv[j].z + yv[j].w * gv[j].w);
+      if (j < count && mine(u0 + j)) s += (yv[j].x * gv[j].x + yv[j].y * gv[j].y) + (yv[j].z * gv[j].z + yv[j].w * gv[j].w);
   }
-  s = lanes_sum(s, g.lpr);
+  s = lanes_sum(s, g.lanes);
   for (int u0 = 0; u0 < units; u0 += kChunk) {
     const int count = units - u0 < kChunk ? units - u0 : kChunk;
     float4 yv[kChunk], gv[kChunk];
@@ -340,7 +364,7 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *_
     load_chunk(gv, gr, u0, count, g);
 #pragma unroll
     for (int j = 0; j < kChunk; ++j) {
-      if (j < count) {
+      if (j < count && mine(u0 + j)) {
         float4 o;
         o.x = yv[j].x * (gv[j].x - s);
         o.y = yv[j].y * (gv[j].y - s);
@@ -352,7 +376,7 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *_
   }
 }
 
-int make_geom(const char *who, int sbs, RowGeom &g) {
+int make_geom(const char *who, int sbs, int64_t n_rows, int64_t nnz, int units, RowGeom &g) {
   BSA_REQUIRE(sbs >= 16 && bsa::is_pow2(sbs), "%s: sbs must be a power of two >= 16 (got %d)", who, sbs);
   int l = 0;
   while ((1 << l) < sbs) ++l;
@@ -361,8 +385,15 @@ int make_geom(const char *who, int sbs, RowGeom &g) {
   int nq = sbs / 256 > 1 ? sbs / 256 : 1;
   g.nq_log2 = 0;
   while ((1 << g.nq_log2) < nq) ++g.nq_log2;
+  // As many groups of lanes on a row as bring one 5/3 times as long as the mean (a block-causal layout's longest is twice the
+  // mean) down to `units` rounds.  Blocks of 16 keep two rows per wave, whole lines of 128 bytes (forward, sbs 16, above: 62
+  // us so, 74 with a row per wave).  The launch stays below 2^31 threads.
+  const int most = sbs == 16 ? 32 : 64;
+  g.split_log2 = 0, g.lanes = g.lpr;
+  while (2 * g.lanes <= most && 5 * (nnz >> g.split_log2) > 3 * units * n_rows && n_rows * sbs * 2 * g.lanes < ((int64_t)1 << 31))
+    ++g.split_log2, g.lanes *= 2;
   g.groups_log2 = 0;
-  while ((1 << g.groups_log2) < sbs * g.lpr / 64) ++g.groups_log2;
+  while ((1 << g.groups_log2) < sbs * g.lanes / 64) ++g.groups_log2;
   return BSA_OK;
 }
 
@@ -370,10 +401,13 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 }  // namespace
 
+// Forward, eight units per lane leave seven waves per SIMD: sbs 64, above, 106 us, 114 with 16 to 32 units.  Rows of wider
+// blocks stay whole up to 32 units: sbs 128 110 us so, 119 with 16 units in registers, 113 with two groups of lanes on a row.
+// Backward, 16 units of both tensors: 153 us either way, but fewer, longer rounds at sbs 16 (83 against 92).
 extern "C" int bsa_softmax_fwd(const float *x, float *out, const int32_t *row_offsets, int64_t n_rows, int64_t nnz,
                                int sbs, bsa_stream_t stream) {
   RowGeom g;
-  if (int rc = make_geom("bsa_softmax_fwd", sbs, g)) return rc;
+  if (int rc = make_geom("bsa_softmax_fwd", sbs, n_rows, nnz, sbs < 128 ? 8 : 32, g)) return rc;
   BSA_REQUIRE(n_rows >= 0 && nnz >= 0, "bsa_softmax_fwd: negative size");
   if (n_rows == 0 || nnz == 0) return BSA_OK;
   BSA_REQUIRE(x && out && row_offsets, "bsa_softmax_fwd: NULL pointer");
@@ -382,14 +416,15 @@ extern "C" int bsa_softmax_fwd(const float *x, float *out, const int32_t *row_of
   const int64_t n_tasks = n_rows << g.groups_log2;
   const int64_t blocks = bsa::cdiv(bsa::cdiv(n_tasks, kWaves), 8) * 8;  // a whole number of workgroups per XCD
   if (blocks > 0x7fffffffLL) return bsa::fail(BSA_ELIMIT, "bsa_softmax_fwd: too many rows");
-  softmax_fwd_kernel<<<(unsigned)blocks, 64 * kWaves, 0, bsa::as_stream(stream)>>>(x, out, row_offsets, n_tasks, g);
+  auto kernel = sbs < 128 ? &softmax_fwd_kernel<16> : &softmax_fwd_kernel<32>;
+  kernel<<<(unsigned)blocks, 64 * kWaves, 0, bsa::as_stream(stream)>>>(x, out, row_offsets, n_tasks, g);
   return bsa::check_launch("softmax_fwd_kernel");
 }
 
 extern "C" int bsa_softmax_bwd(const float *grad_out, const float *y, float *grad_in, const int32_t *row_offsets,
                                int64_t n_rows, int64_t nnz, int sbs, bsa_stream_t stream) {
   RowGeom g;
-  if (int rc = make_geom("bsa_softmax_bwd", sbs, g)) return rc;
+  if (int rc = make_geom("bsa_softmax_bwd", sbs, n_rows, nnz, kBwdUnits, g)) return rc;
   BSA_REQUIRE(n_rows >= 0 && nnz >= 0, "bsa_softmax_bwd: negative size");
   if (n_rows == 0 || nnz == 0) return BSA_OK;
   BSA_REQUIRE(grad_out && y && grad_in && row_offsets, "bsa_softmax_bwd: NULL pointer");
