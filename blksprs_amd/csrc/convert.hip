@@ -18,7 +18,10 @@ __device__ inline uint4 load_streaming(const uint4 *p) {
   return uint4{v[0], v[1], v[2], v[3]};
 }
 
-// results that are written once and not read back by the kernel bypass the caches
+// results that are written once and not read back by the kernel bypass the caches; not the compressed blocks of to_sparse,
+// which the caller is about to compute on: kept in the caches they come back faster (layout, to_sparse and to_dense of 16 x
+// 4096 x 4096 bf16 at 25 %: to_sparse 48.9 -> 44.4 us, the to_dense behind it 110 -> 98; 6 x 4096 x 2048 fp32, sbs 16, half of
+// the blocks: 45 -> 42 and 57 -> 42)
 __device__ inline void store_streaming(uint4 *p, uint4 v) {
   __builtin_nontemporal_store(u32x4_t{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4_t *>(p));
 }
@@ -40,7 +43,7 @@ __global__ __launch_bounds__(256) void to_sparse_kernel(const uint4 *__restrict_
     const int64_t r = coords[n * 3 + 1];
     const int64_t c = coords[n * 3 + 2];
     const int64_t src = b * dense_batch_vecs + ((r << sbs_log2) + e) * dense_row_vecs + (c << vec_per_row_log2) + q;
-    store_streaming(blocks + g, dense[src]);
+    blocks[g] = dense[src];
   }
 }
 
