@@ -164,25 +164,10 @@ extern "C" int bsa_causal_lengths_range(const int64_t *lengths, int64_t n, int64
   return bsa::check_launch(who);
 }
 
-// Reads the flag rather than waiting for an event, which costs the host some 6 us more; a stream that is done, or that
-// failed, ends the wait as well.
 extern "C" int bsa_causal_lengths_wait(const int64_t *range, int64_t longest, bsa_stream_t stream) {
   const char *who = "bsa_causal_lengths_wait";
   BSA_REQUIRE(range != nullptr, "%s: NULL argument", who);
-  for (int turn = 1; __atomic_load_n(range + 2, __ATOMIC_ACQUIRE) == 0; ++turn) {
-    if ((turn & 0xfff) != 0) {
-      __builtin_ia32_pause();
-      continue;
-    }
-    turn = 0;
-    const hipError_t state = hipStreamQuery(bsa::as_stream(stream));
-    if (state == hipErrorNotReady) {
-      if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();  // not to be taken for a launch's
-      continue;
-    }
-    if (state != hipSuccess) return bsa::fail(BSA_ELAUNCH, "%s: %s", who, hipGetErrorString(state));
-    if (__atomic_load_n(range + 2, __ATOMIC_ACQUIRE) == 0) return bsa::fail(BSA_ELAUNCH, "%s: the search left no result", who);
-  }
+  if (!bsa::wait_for_word(who, range + 2, 0, stream)) return BSA_ELAUNCH;
   return range[0] < 0 || range[1] > longest ? 1 : BSA_OK;
 }
 

@@ -1,4 +1,4 @@
-// Error reporting of the C ABI.
+// Error reporting of the C ABI, waits of the host.
 #include "common.h"
 
 namespace bsa {
@@ -14,6 +14,30 @@ int fail(int code, const char *fmt, ...) {
   vsnprintf(error_buffer(), 512, fmt, ap);
   va_end(ap);
   return code;
+}
+
+bool wait_for_word(const char *who, const int64_t *word, int64_t before, bsa_stream_t stream) {
+  for (int turn = 1; __atomic_load_n(word, __ATOMIC_ACQUIRE) == before; ++turn) {
+    if ((turn & 0xfff) != 0) {
+      __builtin_ia32_pause();
+      continue;
+    }
+    turn = 0;
+    const hipError_t state = hipStreamQuery(as_stream(stream));
+    if (state == hipErrorNotReady) {
+      if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();  // not to be taken for a launch's
+      continue;
+    }
+    if (state != hipSuccess) {
+      fail(BSA_ELAUNCH, "%s: %s", who, hipGetErrorString(state));
+      return false;
+    }
+    if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == before) {
+      fail(BSA_ELAUNCH, "%s: the kernel left no result", who);
+      return false;
+    }
+  }
+  return true;
 }
 
 }  // namespace bsa

@@ -61,6 +61,11 @@ __global__ __launch_bounds__(kScanThreads) void tile_counts_kernel(const In *__r
   if (threadIdx.x == 0) tile_counts[blockIdx.x] = total;
 }
 
+// The host may be looking for the total (bsa_lut_counted_wait)
+__device__ inline void publish_total(int64_t *stats, int64_t total) {
+  __hip_atomic_store(stats, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // One block: exclusive scan of the tile counts (int64 results), total -> stats[0],
 // stats[1] = 0, and the closing entries of the optional outputs.
 __global__ __launch_bounds__(kScanThreads) void scan_tiles_kernel(const int32_t *__restrict__ tile_counts,
@@ -78,8 +83,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_tiles_kernel(const int32_t 
     carry += total;
   }
   if (threadIdx.x == 0) {
-    stats[0] = carry;
     stats[1] = 0;
+    publish_total(stats, carry);
     if (last_i32) *last_i32 = (int32_t)carry;
   }
 }
@@ -126,8 +131,8 @@ __device__ inline int64_t sum_in_front(const int64_t *tile_offsets, const int32_
 // what scan_tiles_kernel writes besides the offsets
 __device__ inline void write_totals(int64_t total, int64_t *stats, int32_t *last_i32) {
   if (blockIdx.x != gridDim.x - 1 || threadIdx.x != 0) return;
-  stats[0] = total;
   stats[1] = 0;
+  publish_total(stats, total);
   if (last_i32) *last_i32 = (int32_t)total;
 }
 
@@ -420,6 +425,24 @@ extern "C" int bsa_lut_packed(const uint8_t *layout, int64_t n, int64_t row_len,
   ScanWorkspace w = carve(workspace, n);
   return lut_packed_launch("bsa_lut_packed", layout, n, row_len, packed, row_offsets, stats_dev, stats_host,
                            n > 0 ? w.tile_counts : nullptr, n > 0 ? w.tile_offsets : nullptr, bsa::as_stream(stream));
+}
+
+extern "C" int bsa_lut_packed_counted(const uint8_t *layout, int64_t n, int64_t *packed, int64_t *words, void *workspace,
+                                      size_t workspace_bytes, bsa_stream_t stream) {
+  const char *who = "bsa_lut_packed_counted";
+  BSA_REQUIRE(words != nullptr, "%s: words is NULL", who);
+  BSA_REQUIRE(n > 0, "%s: no layout", who);
+  BSA_REQUIRE(workspace && workspace_bytes >= scan_workspace_bytes(n), "%s: workspace too small", who);
+  ScanWorkspace w = carve(workspace, n);
+  __atomic_store_n(words, (int64_t)-1, __ATOMIC_RELEASE);
+  return lut_packed_launch(who, layout, n, 0, packed, nullptr, words, nullptr, w.tile_counts, w.tile_offsets,
+                           bsa::as_stream(stream));
+}
+
+extern "C" int64_t bsa_lut_counted_wait(const int64_t *words, bsa_stream_t stream) {
+  const char *who = "bsa_lut_counted_wait";
+  BSA_REQUIRE(words != nullptr, "%s: words is NULL", who);
+  return bsa::wait_for_word(who, words, -1, stream) ? __atomic_load_n(words, __ATOMIC_ACQUIRE) : BSA_ELAUNCH;
 }
 
 // ---------------------------------------------------------------------------------------------------

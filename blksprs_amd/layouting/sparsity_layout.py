@@ -37,8 +37,8 @@ def build_sparsity_layout(x: Tensor, sparsity_block_size: int) -> Tensor:
     B, R, C = x.size(0), x.size(1) // sparsity_block_size, x.size(2) // sparsity_block_size
     out = torch.zeros((B, R, C), dtype=torch.bool, device=x.device)
     if out.numel():
-        with torch.no_grad(), torch.cuda.device(x.device):
-            _capi.call("bsa_layout_from_dense", _capi.ptr(x.detach()), out.view(torch.uint8).data_ptr(), B, R, C,
+        with _capi.on_device(x.device):
+            _capi.call("bsa_layout_from_dense", _capi.ptr(x), out.data_ptr(), B, R, C,
                        sparsity_block_size, x.element_size(), int(x.dtype.is_floating_point), _capi.stream(x.device))
     return as_base_tensor(out)
 

@@ -10,8 +10,8 @@ from torch import Tensor
 
 from .. import _capi
 from ..utils.blksprs_tensor import BlksprsTensor
-from ..utils.tools import (build_packed_indices, eager_only, finalize_layout_cache, nonzero_from_packed, pack_layout,
-                           pack_layouts, prepare_layout_cache)
+from ..utils.tools import (build_packed_indices, counts_while_enqueued, eager_only, finalize_layout_cache,
+                           nonzero_for_one_call, nonzero_from_packed, pack_layout, pack_layouts, prepare_layout_cache)
 from ..utils.validation import (ensure_contiguous, validate_contiguous, validate_device, validate_dimensions,
                                 validate_dtype_supported, validate_sparsity, validate_sparsity_block_size,
                                 validate_sparsity_dense)
@@ -19,6 +19,8 @@ from ..utils.validation import (ensure_contiguous, validate_contiguous, validate
 
 def _fill_bits(fill_value, dtype: torch.dtype) -> int:
     """Bit pattern of ``fill_value`` converted to ``dtype`` the way ``torch.full`` converts it."""
+    if type(fill_value) is int and fill_value == 0:  # the default: all bits clear in every type
+        return 0
     scalar = torch.full((1,), fill_value, dtype=dtype)
     width = {1: torch.uint8, 2: torch.int16, 4: torch.int32, 8: torch.int64}[scalar.element_size()]
     return int(scalar.view(width).item()) & ((1 << (8 * scalar.element_size())) - 1)
@@ -121,14 +123,18 @@ def to_sparse(x: Tensor, sparsity_layout: Tensor,
     validate_sparsity_dense(sparsity_block_size, (x, sparsity_layout))
     validate_sparsity_block_size(sparsity_block_size, x)
 
-    layout_cache = to_sparse_build_layout_cache(layout_cache, sparsity_layout)
+    if layout_cache is None and counts_while_enqueued(sparsity_layout):
+        validate_contiguous(sparsity_layout)
+        layout_indices, n_sparse_blocks = nonzero_for_one_call(sparsity_layout)
+    else:
+        layout_cache = to_sparse_build_layout_cache(layout_cache, sparsity_layout)
+        layout_indices, n_sparse_blocks = layout_cache["layout_indices"], layout_cache["n_sparse_blocks"]
 
     # a single all-active block is its own compressed form: hand the storage back
     if _single_full_block(sparsity_layout):
         return BlksprsTensor.wrap(x)
 
-    return BlksprsTensor.wrap(_ToSparse.apply(x, sparsity_layout, layout_cache["layout_indices"],
-                                              sparsity_block_size, layout_cache["n_sparse_blocks"]))
+    return BlksprsTensor.wrap(_ToSparse.apply(x, sparsity_layout, layout_indices, sparsity_block_size, n_sparse_blocks))
 
 
 @eager_only

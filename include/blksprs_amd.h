@@ -72,6 +72,16 @@ int bsa_lut_packed(const uint8_t *layout, int64_t n, int64_t row_len, int64_t *p
                    void *workspace, size_t workspace_bytes, bsa_stream_t stream);
 
 /*
+ * bsa_lut_packed without row offsets, for a caller that goes on enqueuing while the blocks are counted.  words: two words of
+ * pinned host memory, the caller's until bsa_lut_counted_wait has returned, which waits for the count, not for what was
+ * enqueued behind the scan, and returns it, or a negative BSA_E* code.  The reference reads the count first
+ * (blksprs/ops/conversion.py:286-288).
+ */
+int bsa_lut_packed_counted(const uint8_t *layout, int64_t n, int64_t *packed, int64_t *words, void *workspace,
+                           size_t workspace_bytes, bsa_stream_t stream);
+int64_t bsa_lut_counted_wait(const int64_t *words, bsa_stream_t stream);
+
+/*
  * bsa_lut_packed for callers that cannot allocate device memory (code under HIP graph capture, serving loops,
  * harnesses that forbid hipMalloc): the same launches and the same results, but the scan's scratch (one int32
  * count and one int64 offset per tile of 2048 layout entries) lives in a file-scope device array of 96 KiB that

@@ -1,0 +1,47 @@
+"""to_sparse of a layout that is used once: the host looks for the block count while the coordinates are enqueued."""
+
+import pytest
+import torch
+
+import blksprs_amd as bs
+from blksprs_amd.utils import tools
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape,density", [
+    ((1, 1, 2), 1.0), ((1, 3, 5), 0.0), ((2, 9, 13), 0.4), ((1, 1, 2048), 0.5), ((3, 683, 1), 0.5), ((4, 64, 128), 0.1),
+    ((8, 128, 128), 0.05),  # 2^17 entries: the last that takes this way
+    ((1, 131, 1001), 0.02),  # beyond
+])
+def test_to_sparse_without_a_cache_counts_while_it_enqueues(device, shape, density):
+    layout = (torch.rand(shape, generator=torch.Generator().manual_seed(sum(shape))) < density).to(device)
+    assert tools.counts_while_enqueued(layout) == (layout.numel() <= 1 << 17)
+    B, R, C = shape
+    x = torch.randn((B, 16 * R, 16 * C), device=device)
+    want = x.view(B, R, 16, C, 16).permute(0, 1, 3, 2, 4)[layout]
+    for _ in range(3):
+        assert torch.equal(torch.Tensor(bs.ops.to_sparse(x, layout, 16)), want)
+    assert torch.equal(torch.Tensor(bs.ops.to_sparse(x, layout, 16, layout_cache={})), want)
+
+
+def test_coordinates_of_a_layout_that_does_not_start_on_16_bytes(device):
+    whole = torch.rand((1, 5000), device=device) < 0.3
+    layout = whole.view(-1)[3:4995].view(2, 48, 52)
+    coords, count = tools.nonzero_for_one_call(layout)
+    assert count == int(layout.sum()) and torch.equal(coords, layout.nonzero()) and coords.is_contiguous()
+
+
+def test_to_sparse_behind_queued_work_of_another_stream(device):
+    stream = torch.cuda.Stream()
+    x = torch.zeros((2, 256, 256), device=device)
+    layout = torch.zeros((2, 16, 16), dtype=torch.bool, device=device)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(20_000_000)
+        x.add_(1)
+        layout[:, ::3, 1::2] = True
+        out = bs.ops.to_sparse(x, layout, 16)
+        n = out.size(0)
+    stream.synchronize()
+    assert n == 2 * 6 * 8 and bool((out == 1).all())
