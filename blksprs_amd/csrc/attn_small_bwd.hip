@@ -45,16 +45,21 @@ struct BwdShape {
   static constexpr int kPartial = SBS * SBS * NS * 4;
   static constexpr int kSlot = SBS * SBS * NS;  // floats of a slot of the scratch, twice for dK and dV
   static constexpr int kStats = 256;  // lse and delta of the 32 queries of a step
-  // dK / dV kernel: Q and dO of two steps where registers allow two waves per SIMD anyway (sbs 32: 133 against 137 us);
-  // at sbs 16 one step's tiles and twice the waves are faster (67 against 92 us)
-  static constexpr int kBufs = ES == 2 && SBS == 32 && NS <= 2 ? 2 : 1;
-  static constexpr int kKvBuf = 2 * T::kBytes + kStats;
   // the last row fragment of an odd number of slices of 16 reads (and drops) a slice beyond its tile
   static constexpr int kPad = T::kHalfLast ? T::kPiece : 0;
-  static constexpr int kKvLds = kPad + (kBufs * kKvBuf > 2 * kPartial ? kBufs * kKvBuf : 2 * kPartial);
+  // dK / dV kernel of 16-bit blocks of 32.  What limits its waves is LDS and registers: with room for a wave's own dK and dV (twice
+  // the tiles of a step) a SIMD holds one wave at head dimensions 96 and 128 and two at 64; these sums now go through the tiles of
+  // all waves of a row once they are done, and P is used up before dP is formed, which leaves two, one and three.  A second tile
+  // for Q, which is read first and last in a step, lets a step's copies go out a step ahead; at 64 its addresses are more than three
+  // waves' registers hold (a fragment of K spilled in the loop), and three waves without it are as fast as two with it.
+  // Forward + backward of bf16: 24 x 4096, windows of 1024, head dimension 96: 240 -> 208 us; causal, 128: 516 -> 503; 16 x 1024, 40 %,
+  // 64: 53 -> 50; 24 x 2048, 30 %, 64: 80 -> 79; 48 x 4096, windows of 1024, 64: 273 -> 272.
+  static constexpr bool kTwoQ = ES == 2 && SBS == 32 && NS != 2;
+  static constexpr int kKvLds = kPad + (kTwoQ ? 3 : 2) * T::kBytes + (kTwoQ ? 2 : 1) * kStats;
   static constexpr int kQLds = kPad + (2 * T::kBytes > kPartial ? 2 * T::kBytes : kPartial);
   static constexpr int kQMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS <= 2 ? 3 : 2) : (NS <= 4 ? 4 : 2);
-  static constexpr int kKvMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS <= 3 ? 2 : 1) : (NS <= 4 ? 3 : 2);
+  template <bool kSome>
+  static constexpr int kKvMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS + kSome <= 2 ? 3 : NS <= 3 ? 2 : 1) : (NS <= 4 ? 3 : 2);
 };
 
 // 4 bytes per lane, global -> LDS: lane l's value lands at dst + 4 l
@@ -228,16 +233,17 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 }
 
 template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
-__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>::kKvMinWaves)) void attn_small_dkv_kernel(bsa_attn_args a, int split, Shares shares) {
+__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>::template kKvMinWaves<kSome>)) void attn_small_dkv_kernel(bsa_attn_args a, int split, Shares shares) {
   using Shape = BwdShape<Tr::kElem, SBS, NS, kHalves>;
   using T = typename Shape::T;
   using W = Walk<Tr::kElem, SBS, NS, Shape::NB, false, kSome, kHalves>;
-  constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs, kBufs = Shape::kBufs;
+  constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs;
+  constexpr bool kTwoQ = Shape::kTwoQ;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
   const int lane = threadIdx.x & 63;
   const int wave = first_lane(threadIdx.x >> 6);
-  char *lds = small_smem + wave * Shape::kKvLds;  // per buffer: Q tile, dO tile, lse and delta
+  char *lds = small_smem + wave * Shape::kKvLds;  // Q tile, dO tile, a second Q tile, lse and delta of one or two steps
 
   const RowOfWave me(shares, kHalves, a.B, kHalves * a.nk, false, wave, kWaves, split);
   const int64_t row = me.b * a.nk + me.own / kHalves;  // of the layout
@@ -262,25 +268,34 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
   const uint32_t source = T::source_offset(lane);
   const char *const tensor_q = static_cast<const char *>(a.q), *const tensor_g = static_cast<const char *>(a.d_o);
   // this lane's share of the statistics copy: lanes 0 .. 31 lse, 32 .. 63 delta of the step's 32 queries
-  const float *const stats = (lane < 32 ? a.lse : a.delta) + me.b * a.nq * (kHalves * SBS) + lane % SBS;
+  const int64_t queries = me.b * a.nq * (kHalves * SBS);
+  const float *const stats = (lane < 32 ? a.lse : a.delta) + queries + lane % SBS;
   const int stats_block = SBS == 16 ? (lane >> 4) & 1 : 0;
+  // 16-bit blocks of 32: addresses are formed where they are used, since registers are what limits the waves
+  constexpr bool kLateAddresses = Tr::kElem == 2 && SBS == 32;
   auto copy_stats = [&](const typename W::Step &s, char *dst) {
     int other = __builtin_amdgcn_readlane(walk.other, s.slot[0]);
+    if constexpr (kLateAddresses) {
+      const late_args_t p = late_args();
+      const int l = fresh_lane();
+      const float *lse = p->lse + queries, *delta = p->delta + queries;
+      lse += (int64_t)other * SBS, delta += (int64_t)other * SBS;
+      copy_words_to_lds((l < 32 ? lse : delta) + l % SBS, dst);
+      return;
+    }
     if constexpr (NB > 1) {
       const int second = s.count > 1 ? __builtin_amdgcn_readlane(walk.other, s.slot[1]) : other;
       other = stats_block ? second : other;
     }
     copy_words_to_lds(stats + (int64_t)other * SBS, dst);
   };
-  auto copy_all = [&](typename W::Step &s, char *buf) {
-    const bool q_whole = walk.template copy<false>(s, tensor_q, buf, source, lane);
-    const bool g_whole = walk.template copy<true>(s, tensor_g, buf + T::kBytes, source, lane);
-    copy_stats(s, buf + 2 * T::kBytes);
-    return q_whole && g_whole;
+  auto source_now = [&]() -> uint32_t {
+    if constexpr (kLateAddresses && NS == 2) return T::source_offset(fresh_lane());
+    else return source;
   };
-
-  const typename T::RowReader q_rows0(lds, lane), g_rows0(lds + T::kBytes, lane);
-  const typename T::ColReader q_cols0(lds, lane), g_cols0(lds + T::kBytes, lane);
+  constexpr int kStatsAt = (kTwoQ ? 3 : 2) * T::kBytes;
+  const typename T::RowReader q_rows0(lds, lane), g_rows(lds + T::kBytes, lane);
+  const typename T::ColReader q_cols0(lds, lane), g_cols(lds + T::kBytes, lane);
   auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) -> bool {  // as in the dQ kernel
     using Ar = decltype(arithmetic);
     typename W::Step now, next;
@@ -293,28 +308,31 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
     const OwnOperand<Ar, SBS, NS, kHalves, false> k_operand(kf);
     const OwnOperand<Ar, SBS, NS, kHalves, true> v_operand(vf);
     constexpr float kTimes = up_of<Ar>();  // of P and dS as second operands; dP: the square
-    int buf = 0;
-    if (now.count) copy_all(now, lds);
+    // kTwoQ: Q and the statistics of a step are requested a step ahead, dO as soon as this step has used its own
+    int q_at = 0;  // 0 or 1: which Q tile and statistics
+    bool g_counted = false;  // dO of this step: exactly kCopies copies
+    typename T::RowReader q_rows = q_rows0;
+    typename T::ColReader q_cols = q_cols0;
+    const float *lse = reinterpret_cast<const float *>(lds + kStatsAt);
+    if (now.count) {
+      walk.template copy<false>(now, tensor_q, lds, source, lane);
+      copy_stats(now, lds + kStatsAt);
+      g_counted = walk.template copy<true>(now, tensor_g, lds + T::kBytes, source, lane);
+    }
     while (now.count) {
-      const int at = kBufs == 2 ? buf * Shape::kKvBuf : 0;
-      if constexpr (kBufs == 2) {
-        // the next step's tiles into the other buffer, then wait for everything but them
-        wait_lds();
+      bool q_counted = false;  // Q and the statistics of the next step: exactly kCopies + 1 copies
+      if constexpr (kTwoQ) {
         walk.take(next, lane);
-        bool counted = false;
-        if (next.count) counted = copy_all(next, lds + (buf ^ 1) * Shape::kKvBuf);
-        if (counted) wait_vmem<2 * T::kCopies + 1>();
+        if (next.count) {
+          q_counted = walk.template copy<false>(next, tensor_q, lds + (q_at ^ 1) * 2 * T::kBytes, source_now(), lane);
+          copy_stats(next, lds + kStatsAt + (q_at ^ 1) * Shape::kStats);
+        }
+        if (q_counted && g_counted) wait_vmem<2 * T::kCopies + 1>();
         else wait_vmem<0>();
       } else {
         wait_vmem<0>();
       }
-      typename T::RowReader q_rows = q_rows0, g_rows = g_rows0;
-      typename T::ColReader q_cols = q_cols0, g_cols = g_cols0;
-      if constexpr (kBufs == 2) {
-        q_rows.shift(at), g_rows.shift(at);
-        q_cols.shift(at), g_cols.shift(at);
-      }
-      const float *lse = reinterpret_cast<const float *>(lds + at + 2 * T::kBytes), *delta = lse + 32;
+      const float *const delta = lse + 32;
 
       // ---- S = Q K^T, P = exp2(S - lse)
       acc_t sacc[NB], dp[NB];
@@ -332,8 +350,8 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 #pragma unroll
         for (int i = 0; i < 4; ++i) ls[x + i] = l4[i];
       }
-      // in parts P is used up before dP is formed, for want of registers
-      constexpr bool kLateDp = std::is_same_v<Ar, SSplit>;
+      // in parts, and in 16-bit blocks of 32, P is used up before dP is formed, for want of registers
+      constexpr bool kLateDp = std::is_same_v<Ar, SSplit> || (Tr::kElem == 2 && SBS == 32);
       if constexpr (!kLateDp) W::template multiply_rows<Ar, true>(dp, now, g_rows, v_operand, lane);
       float lowest = ls[0];
 #pragma unroll
@@ -346,6 +364,10 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 #pragma unroll
       for (int x = 0; x < kScores; ++x) sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), -ls[x])) * kTimes;
       const Weights<Ar, kScores> pw(sv);
+      if constexpr (kTwoQ) {
+        if (q_counted) wait_vmem<T::kCopies + 1>();
+        else wait_vmem<0>();
+      }
       if constexpr (kLateDp) {
         W::template multiply_cols<Ar, true, kScores>(dv, now, g_cols, pw);
         W::template multiply_rows<Ar, true>(dp, now, g_rows, v_operand, lane);
@@ -360,22 +382,24 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
       }
       // ---- dV^T += dO^T P
       if constexpr (!kLateDp) W::template multiply_cols<Ar, true, kScores>(dv, now, g_cols, pw);
-      if constexpr (kBufs == 1) {
-        wait_lds();
-        walk.take(next, lane);
-        if (next.count) {
-          walk.template copy<true>(next, tensor_g, lds + T::kBytes, source, lane);
-          copy_stats(next, lds + 2 * T::kBytes);
-        }
+      wait_lds();
+      if constexpr (!kTwoQ) walk.take(next, lane);
+      if (next.count) {
+        g_counted = walk.template copy<true>(next, tensor_g, lds + T::kBytes, source_now(), lane);
+        if constexpr (!kTwoQ) copy_stats(next, lds + kStatsAt);
       }
       // ---- dK^T += Q^T dS
       W::template multiply_cols<Ar, false, kScores>(dk, now, q_cols, Weights<Ar, kScores>(sv));
-      if constexpr (kBufs == 1) {
-        wait_lds();
-        if (next.count) walk.template copy<false>(next, tensor_q, lds, source, lane);
+      wait_lds();
+      if constexpr (kTwoQ) {
+        const int turn = q_at ? -1 : 1;
+        q_rows.shift(turn * 2 * T::kBytes), q_cols.shift(turn * 2 * T::kBytes);
+        lse += turn * (Shape::kStats / 4);
+        q_at ^= 1;
+      } else if (next.count) {
+        walk.template copy<false>(next, tensor_q, lds, source_now(), lane);
       }
       now = next;
-      buf ^= 1;
     }
     if constexpr (!std::is_same_v<Ar, SSplit>) return true;
     scale_down<Ar, NS, kRegs>(dk);
@@ -392,16 +416,40 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
     walk_list(Tr{});
   }
   if (me.waves > 1) {
-    float *mine = reinterpret_cast<float *>(lds);
-    if (me.place != 0) {
-      leave_partial<NS, kRegs>(dk, mine, lane);
-      leave_partial<NS, kRegs>(dv, mine + Shape::kPartial / 4, lane);
-    }
-    __syncthreads();
-    if (me.place != 0) return;
-    for (int p = 1; p < me.waves; ++p) {
-      add_partial<NS, kRegs>(dk, mine + p * (Shape::kKvLds / 4), lane);
-      add_partial<NS, kRegs>(dv, mine + p * (Shape::kKvLds / 4) + Shape::kPartial / 4, lane);
+    if constexpr (Shape::kKvLds >= 2 * Shape::kPartial) {
+      float *mine = reinterpret_cast<float *>(lds);
+      if (me.place != 0) {
+        leave_partial<NS, kRegs>(dk, mine, lane);
+        leave_partial<NS, kRegs>(dv, mine + Shape::kPartial / 4, lane);
+      }
+      __syncthreads();
+      if (me.place != 0) return;
+      for (int p = 1; p < me.waves; ++p) {
+        add_partial<NS, kRegs>(dk, mine + p * (Shape::kKvLds / 4), lane);
+        add_partial<NS, kRegs>(dv, mine + p * (Shape::kKvLds / 4) + Shape::kPartial / 4, lane);
+      }
+    } else {
+      // sums that are larger than a wave's tiles (16-bit blocks of 32): the tiles of all waves of the row take in as many sums at
+      // a time as they hold, once the walks are over
+      static_assert(Shape::kKvLds >= Shape::kPartial, "the sums of a wave in the tiles of two");
+      float *const sums = reinterpret_cast<float *>(lds - me.place * Shape::kKvLds);
+      const int fit = me.waves * Shape::kKvLds / (2 * Shape::kPartial);
+      for (int first = 1; first < me.waves; first += fit) {
+        __syncthreads();
+        if (me.place >= first && me.place < first + fit) {
+          float *mine = sums + (me.place - first) * (Shape::kPartial / 2);
+          leave_partial<NS, kRegs>(dk, mine, lane);
+          leave_partial<NS, kRegs>(dv, mine + Shape::kPartial / 4, lane);
+        }
+        __syncthreads();
+        if (me.place != 0) continue;
+        for (int p = first; p < me.waves && p < first + fit; ++p) {
+          const float *other = sums + (p - first) * (Shape::kPartial / 2);
+          add_partial<NS, kRegs>(dk, other, lane);
+          add_partial<NS, kRegs>(dv, other + Shape::kPartial / 4, lane);
+        }
+      }
+      if (me.place != 0) return;
     }
   }
   if (!me.there) return;

@@ -44,6 +44,16 @@ def test_rows_of_a_launch(device, dtype, sbs, B, n, use_causal):
               seed=B + n, use_causal=use_causal)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("nh", [1, 2, 3, 4])
+@pytest.mark.parametrize("B,n", [(1, 3), (2, 9), (33, 16)])
+def test_sums_of_waves_that_share_a_key_block(device, dtype, nh, B, n):
+    """dK and dV of 16-bit blocks of 32 are larger than the tiles of the wave that has them: lists of one step and of several
+    for each of four waves (3 and 18 key blocks) and of two (528)."""
+    _run_case(device, dtype, 32, B=B, nq=n, nk=n, nh=nh, nhv=nh, density=0.8, seed=10 * nh + n, use_mask=True)
+    _run_case(device, dtype, 32, B=B, nq=n, nk=n, nh=nh, nhv=nh, density=0.3, seed=nh + n, use_causal=True)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("B,n", [(2, 1), (7, 7), (8, 8), (8, 9), (13, 17), (16, 3), (20, 11)])
 def test_rows_over_xcds(device, dtype, B, n):
