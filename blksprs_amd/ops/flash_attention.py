@@ -398,7 +398,8 @@ class _Tables:
     def new_argument(self, dims) -> _capi.AttnArgs:
         """An argument block with the sizes and the tables filled in, which are the same for every call: a copy (0.1 us; field by
         field 3; with the short way through a complete cache 8 prompts of 128 to 256 tokens take 38.0 -> 29.1 us a call)."""
-        if self.argument is None or self.argument[0] != dims:
+        kept = self.argument  # read once: another thread may replace it
+        if kept is None or kept[0] != dims:
             a = _capi.AttnArgs()
             a.B, a.nq, a.nk, a.nh, a.nhv = dims
             a.n_o_blocks = self.n_sparse_blocks_o
@@ -413,8 +414,8 @@ class _Tables:
                 a.group_offsets = self.group_offsets.data_ptr()
                 a.group_records = _capi.ptr(self.group_records)
                 a.group_size = self.group_size
-            self.argument = dims, a
-        return _capi.AttnArgs.from_buffer_copy(self.argument[1])
+            self.argument = kept = dims, a
+        return _capi.AttnArgs.from_buffer_copy(kept[1])
 
 
 class _Shares:
