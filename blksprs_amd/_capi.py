@@ -169,7 +169,10 @@ def ptr(t) -> int:
 
 
 def stream(device) -> int:
-    """The current torch stream of ``device`` as a raw hipStream_t."""
+    """The current torch stream of ``device`` as a raw hipStream_t.  Every launch asks for one, so this is where memory that is
+    not the GPU's is refused, with argument validation off too (``on_device`` has nothing to do for such a device)."""
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import blksprs_amd as bs
+from blksprs_amd import _capi
 from blksprs_amd.utils import tools, validation
 
 
@@ -47,6 +48,28 @@ def test_operators_refuse_cpu_tensors():
     finally:
         bs.utils.enable_validation()
 
+
+
+@pytest.mark.parametrize("launch", [
+    lambda x, lay: bs.layouting.build_sparsity_layout(x, 16),
+    lambda x, lay: bs.layouting.build_sparsity_layout_matmul(lay, lay.transpose(1, 2).contiguous()),
+    lambda x, lay: bs.ops.transpose(x, lay, 16),
+    lambda x, lay: bs.ops.to_dense(x, lay, 16),
+], ids=["build_sparsity_layout", "build_sparsity_layout_matmul", "transpose", "to_dense"])
+def test_no_launch_on_host_memory_without_validation(monkeypatch, launch):
+    """Nothing reaches the library with the address of a CPU tensor, whatever the device that is current."""
+    launched = []
+    monkeypatch.setattr(_capi, "call", lambda name, *args: launched.append(name))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0)
+    validation.disable_validation()
+    try:
+        with pytest.raises((ValueError, RuntimeError), match="Expected a cuda device|needs GPU tensors"):
+            launch(torch.ones((2, 16, 16)), torch.ones((2, 1, 1), dtype=torch.bool))
+    finally:
+        validation.enable_validation()
+    assert launched == []
 
 def test_validation_messages():
     v = validation
