@@ -395,6 +395,10 @@ class _Tables:
         self.shares = {}  # (block size, dtype, backward) -> shares of the query rows, of the key rows, added on demand
         self.argument = None  # the part of the argument block that says where these tables are, for one set of sizes
 
+    def __reduce__(self):
+        """A copy (of a module that keeps its cache, say) has tensors of its own, so nothing that says where they lie goes along."""
+        return _Tables, ({name: getattr(self, name) for name in self._NAMES},)
+
     def new_argument(self, dims) -> _capi.AttnArgs:
         """An argument block with the sizes and the tables filled in, which are the same for every call: a copy (0.1 us; field by
         field 3; with the short way through a complete cache 8 prompts of 128 to 256 tokens take 38.0 -> 29.1 us a call)."""

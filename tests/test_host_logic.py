@@ -1,6 +1,8 @@
 """Host-side behaviour that needs no GPU: validation switches and messages, the layout cache rules, the
 shape helpers, and that the operators refuse CPU tensors instead of computing somewhere else."""
 
+import copy
+import pickle
 import threading
 
 import pytest
@@ -8,6 +10,7 @@ import torch
 
 import blksprs_amd as bs
 from blksprs_amd import _capi
+from blksprs_amd.ops.flash_attention import _Shares, _Tables
 from blksprs_amd.utils import tools, validation
 
 
@@ -334,3 +337,26 @@ def test_long_lists_of_blocks_of_32_follow_the_work_order():
     finally:
         mm._launch = launch
     assert seen == ["order", None, None, "order", "order"]
+
+
+@pytest.mark.parametrize("copy_of", [copy.deepcopy, lambda value: pickle.loads(pickle.dumps(value))], ids=["deepcopy", "pickle"])
+def test_used_attention_tables_can_be_copied(copy_of):
+    """A layout cache is copied with the module that keeps it; a call has left addresses in its tables."""
+    def tables(cache):
+        return _Tables({**cache, "n_sparse_blocks_o": 4, "group_size": 2, "max_keys_per_query": 2, "max_queries_per_key": 2})
+
+    names = ("packed_indices_q", "packed_indices_k", "packed_indices_v", "packed_indices_o", "group_offsets", "group_records",
+             *(f"{side}_{what}_i32" for side in ("key", "query") for what in ("offsets", "indices")))
+    original = tables({name: torch.full((8,), i) for i, name in enumerate(names)})
+    dims = (1, 2, 2, 1, 1)
+    original.new_argument(dims)
+    original.shares[(32, torch.float16, False)] = (_Shares(torch.zeros(4), torch.zeros(4), 1, 1, 0, [0, 0, 0]), None)
+    copied = copy_of({"tables": original})["tables"]
+    argument = copied.new_argument(dims)
+    for name in names:
+        mine, theirs = getattr(copied, name), getattr(original, name)
+        assert torch.equal(mine, theirs) and mine.data_ptr() != theirs.data_ptr()
+    assert (copied.n_sparse_blocks_o, copied.group_size, copied.max_keys_per_query) == (4, 2, 2)
+    assert argument.pidx_q == copied.packed_indices_q.data_ptr() and argument.key_offsets == copied.key_offsets_i32.data_ptr()
+    assert argument.group_records == copied.group_records.data_ptr()
+    assert copied.shares == {}  # made again when a call needs them
