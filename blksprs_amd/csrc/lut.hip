@@ -61,18 +61,22 @@ __global__ __launch_bounds__(kScanThreads) void tile_counts_kernel(const In *__r
   if (threadIdx.x == 0) tile_counts[blockIdx.x] = total;
 }
 
-// The host may be looking for the total (bsa_lut_counted_wait)
-__device__ inline void publish_total(int64_t *stats, int64_t total) {
-  __hip_atomic_store(stats, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
+// What a scan leaves besides its tables; by one thread.  count may be a word of the host's, which takes it back as soon as it sees
+// the total (bsa_lut_counted_wait): nothing else is written there.
+struct Totals {
+  int64_t *count, *longest_row;  // the second, where there is one, is cleared for row_max_kernel
+  int32_t *last_i32;             // the closing entry of offsets, where there are some
+  __device__ inline void write(int64_t total) const {
+    if (longest_row) *longest_row = 0;
+    if (last_i32) *last_i32 = (int32_t)total;
+    __hip_atomic_store(count, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+};
 
-// One block: exclusive scan of the tile counts (int64 results), total -> stats[0],
-// stats[1] = 0, and the closing entries of the optional outputs.
+// One block: exclusive scan of the tile counts (int64 results), and the totals.
 __global__ __launch_bounds__(kScanThreads) void scan_tiles_kernel(const int32_t *__restrict__ tile_counts,
                                                                   int64_t n_tiles,
-                                                                  int64_t *__restrict__ tile_offsets,
-                                                                  int64_t *__restrict__ stats,
-                                                                  int32_t *__restrict__ last_i32) {
+                                                                  int64_t *__restrict__ tile_offsets, Totals totals) {
   int64_t carry = 0;
   for (int64_t start = 0; start < n_tiles; start += kScanThreads) {
     int64_t p = start + threadIdx.x;
@@ -82,11 +86,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_tiles_kernel(const int32_t 
     if (p < n_tiles) tile_offsets[p] = carry + excl;
     carry += total;
   }
-  if (threadIdx.x == 0) {
-    stats[1] = 0;
-    publish_total(stats, carry);
-    if (last_i32) *last_i32 = (int32_t)carry;
-  }
+  if (threadIdx.x == 0) totals.write(carry);
 }
 
 // Where a tile's workgroup finds the sum of the entries in front of its tile.
@@ -128,14 +128,6 @@ __device__ inline int64_t sum_in_front(const int64_t *tile_offsets, const int32_
   return total;
 }
 
-// what scan_tiles_kernel writes besides the offsets
-__device__ inline void write_totals(int64_t total, int64_t *stats, int32_t *last_i32) {
-  if (blockIdx.x != gridDim.x - 1 || threadIdx.x != 0) return;
-  stats[1] = 0;
-  publish_total(stats, total);
-  if (last_i32) *last_i32 = (int32_t)total;
-}
-
 // Per tile: writes the reverse index and, when row_len > 0, the CSR offset of
 // every row that starts inside the tile.
 template <Prefix kPrefix>
@@ -144,8 +136,7 @@ __global__ __launch_bounds__(kScanThreads) void write_packed_kernel(const uint8_
                                                                     const int32_t *__restrict__ tile_counts,
                                                                     int64_t row_len, int64_t *__restrict__ packed,
                                                                     int32_t *__restrict__ row_offsets,
-                                                                    int64_t *__restrict__ stats,
-                                                                    int32_t *__restrict__ last_i32) {
+                                                                    Totals totals) {
   const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
   int flags[kScanItems];
   int s = 0;
@@ -158,7 +149,9 @@ __global__ __launch_bounds__(kScanThreads) void write_packed_kernel(const uint8_
   int total;
   const int64_t front = sum_in_front<kPrefix>(tile_offsets, tile_counts, layout);
   int64_t prefix = front + block_exclusive_scan(s, total);
-  if constexpr (kPrefix != kFromOffsets) write_totals(front + total, stats, last_i32);
+  if constexpr (kPrefix != kFromOffsets) {  // else scan_tiles_kernel has written them
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) totals.write(front + total);
+  }
 #pragma unroll
   for (int i = 0; i < kScanItems; ++i) {
     int64_t p = base + i;
@@ -375,10 +368,11 @@ extern "C" size_t bsa_lut_workspace_bytes(int64_t n) { return scan_workspace_byt
 namespace {
 
 // The launches of the scan; tile_counts (int32) and tile_offsets (int64) hold one entry per tile of kScanTile
-// layout entries and are written before they are read.
+// layout entries and are written before they are read.  stats_words: how many of the two words of stats_dev are the scan's
+// (one: without row offsets only).
 int lut_packed_launch(const char *who, const uint8_t *layout, int64_t n, int64_t row_len, int64_t *packed,
-                      int32_t *row_offsets, int64_t *stats_dev, int64_t *stats_host, int32_t *tile_counts,
-                      int64_t *tile_offsets, hipStream_t s) {
+                      int32_t *row_offsets, int64_t *stats_dev, int stats_words, int64_t *stats_host,
+                      int32_t *tile_counts, int64_t *tile_offsets, hipStream_t s) {
   BSA_REQUIRE(n >= 0 && row_len >= 0, "%s: negative size", who);
   BSA_REQUIRE(stats_dev != nullptr, "%s: stats_dev is NULL", who);
   BSA_REQUIRE(row_len == 0 || row_offsets != nullptr, "%s: row_len given without row_offsets", who);
@@ -394,10 +388,10 @@ int lut_packed_launch(const char *who, const uint8_t *layout, int64_t n, int64_t
   BSA_REQUIRE(tile_counts && tile_offsets, "%s: no workspace", who);
   const int64_t tiles = bsa::cdiv(n, kScanTile);
   const int64_t n_rows = row_len > 0 ? n / row_len : 0;
-  int32_t *last = row_len > 0 ? row_offsets + n_rows : nullptr;
+  const Totals totals{stats_dev, stats_words > 1 ? stats_dev + 1 : nullptr, row_len > 0 ? row_offsets + n_rows : nullptr};
 #define BSA_WRITE_PACKED(PREFIX)                                                                                       \
   write_packed_kernel<PREFIX><<<(unsigned)tiles, kScanThreads, 0, s>>>(layout, n, tile_offsets, tile_counts, row_len, \
-                                                                       packed, row_offsets, stats_dev, last)
+                                                                       packed, row_offsets, totals)
   if (n <= kMaxRecounted && (reinterpret_cast<uintptr_t>(layout) & 15) == 0) {
     BSA_WRITE_PACKED(kFromLayout);
   } else {
@@ -405,7 +399,7 @@ int lut_packed_launch(const char *who, const uint8_t *layout, int64_t n, int64_t
     if (tiles <= kMaxCountedTiles) {
       BSA_WRITE_PACKED(kFromCounts);
     } else {
-      scan_tiles_kernel<<<1, kScanThreads, 0, s>>>(tile_counts, tiles, tile_offsets, stats_dev, last);
+      scan_tiles_kernel<<<1, kScanThreads, 0, s>>>(tile_counts, tiles, tile_offsets, totals);
       BSA_WRITE_PACKED(kFromOffsets);
     }
   }
@@ -423,26 +417,26 @@ extern "C" int bsa_lut_packed(const uint8_t *layout, int64_t n, int64_t row_len,
   BSA_REQUIRE(n <= 0 || (workspace && workspace_bytes >= scan_workspace_bytes(n)),
               "bsa_lut_packed: workspace too small");
   ScanWorkspace w = carve(workspace, n);
-  return lut_packed_launch("bsa_lut_packed", layout, n, row_len, packed, row_offsets, stats_dev, stats_host,
+  return lut_packed_launch("bsa_lut_packed", layout, n, row_len, packed, row_offsets, stats_dev, 2, stats_host,
                            n > 0 ? w.tile_counts : nullptr, n > 0 ? w.tile_offsets : nullptr, bsa::as_stream(stream));
 }
 
-extern "C" int bsa_lut_packed_counted(const uint8_t *layout, int64_t n, int64_t *packed, int64_t *words, void *workspace,
+extern "C" int bsa_lut_packed_counted(const uint8_t *layout, int64_t n, int64_t *packed, int64_t *word, void *workspace,
                                       size_t workspace_bytes, bsa_stream_t stream) {
   const char *who = "bsa_lut_packed_counted";
-  BSA_REQUIRE(words != nullptr, "%s: words is NULL", who);
+  BSA_REQUIRE(word != nullptr, "%s: word is NULL", who);
   BSA_REQUIRE(n > 0, "%s: no layout", who);
   BSA_REQUIRE(workspace && workspace_bytes >= scan_workspace_bytes(n), "%s: workspace too small", who);
   ScanWorkspace w = carve(workspace, n);
-  __atomic_store_n(words, (int64_t)-1, __ATOMIC_RELEASE);
-  return lut_packed_launch(who, layout, n, 0, packed, nullptr, words, nullptr, w.tile_counts, w.tile_offsets,
+  __atomic_store_n(word, (int64_t)-1, __ATOMIC_RELEASE);
+  return lut_packed_launch(who, layout, n, 0, packed, nullptr, word, 1, nullptr, w.tile_counts, w.tile_offsets,
                            bsa::as_stream(stream));
 }
 
-extern "C" int64_t bsa_lut_counted_wait(const int64_t *words, bsa_stream_t stream) {
+extern "C" int64_t bsa_lut_counted_wait(const int64_t *word, bsa_stream_t stream) {
   const char *who = "bsa_lut_counted_wait";
-  BSA_REQUIRE(words != nullptr, "%s: words is NULL", who);
-  return bsa::wait_for_word(who, words, -1, stream) ? __atomic_load_n(words, __ATOMIC_ACQUIRE) : BSA_ELAUNCH;
+  BSA_REQUIRE(word != nullptr, "%s: word is NULL", who);
+  return bsa::wait_for_word(who, word, -1, stream) ? __atomic_load_n(word, __ATOMIC_ACQUIRE) : BSA_ELAUNCH;
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -498,7 +492,7 @@ extern "C" int bsa_lut_packed_static(const uint8_t *layout, int64_t n, int64_t r
   // call, so what an earlier call left in the array does not matter.
   int32_t *tile_counts = static_cast<int32_t *>(ws);
   int64_t *tile_offsets = reinterpret_cast<int64_t *>(static_cast<char *>(ws) + kStaticMaxTiles * 4);
-  return lut_packed_launch("bsa_lut_packed_static", layout, n, row_len, packed, row_offsets, stats_dev, nullptr,
+  return lut_packed_launch("bsa_lut_packed_static", layout, n, row_len, packed, row_offsets, stats_dev, 2, nullptr,
                            tile_counts, tile_offsets, bsa::as_stream(stream));
 }
 
@@ -617,7 +611,8 @@ extern "C" int bsa_lut_contraction_offsets(const int64_t *pidx_x, const int64_t 
   pair_counts_kernel<<<grid_for(n, 256), 256, 0, s>>>(pidx_o, B, R, C, W, mask_x, mask_y, w.counts);
   const int64_t tiles = bsa::cdiv(n, kScanTile);
   tile_counts_kernel<int32_t><<<(unsigned)tiles, kScanThreads, 0, s>>>(w.counts, n, w.tile_counts);
-  scan_tiles_kernel<<<1, kScanThreads, 0, s>>>(w.tile_counts, tiles, w.tile_offsets, stats_dev, pos_offsets + n);
+  scan_tiles_kernel<<<1, kScanThreads, 0, s>>>(w.tile_counts, tiles, w.tile_offsets,
+                                              Totals{stats_dev, stats_dev + 1, pos_offsets + n});
   write_prefix_kernel<<<(unsigned)tiles, kScanThreads, 0, s>>>(w.counts, n, w.tile_offsets, pos_offsets);
   if (int rc = bsa::check_launch("bsa_lut_contraction_offsets")) return rc;
   return fetch_stats(stats_dev, stats_host, s);

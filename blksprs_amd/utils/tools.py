@@ -162,22 +162,22 @@ def nonzero_for_one_call(sparsity_layout: Tensor) -> tuple[Tensor, int]:
     free = getattr(_COUNT_WORDS, "free", None)
     if free is None:
         free = _COUNT_WORDS.free = []
-    words = free.pop() if free else torch.empty(2, dtype=torch.int64, pin_memory=True)
+    word = free.pop() if free else torch.empty(1, dtype=torch.int64, pin_memory=True)
     ws_bytes = lib.bsa_lut_workspace_bytes(n)
     packed = torch.empty(n, dtype=torch.int64, device=dev)
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     stream = _capi.stream(dev)
     with _capi.on_device(dev):
-        _capi.call("bsa_lut_packed_counted", lay.data_ptr(), n, packed.data_ptr(), words.data_ptr(), workspace.data_ptr(),
+        _capi.call("bsa_lut_packed_counted", lay.data_ptr(), n, packed.data_ptr(), word.data_ptr(), workspace.data_ptr(),
                    ws_bytes, stream)
         try:
             coords = torch.empty((n, 3), dtype=torch.int64, device=dev)
             _capi.call("bsa_lut_nonzero", packed.data_ptr(), B, R, C, coords.data_ptr(), stream)
-        finally:  # the words are the scan's until it has written them
-            count = lib.bsa_lut_counted_wait(words.data_ptr(), stream)
+        finally:  # the word is the scan's until it has written it
+            count = lib.bsa_lut_counted_wait(word.data_ptr(), stream)
     if count < 0:
         _capi.check(int(count), "bsa_lut_counted_wait")
-    free.append(words)
+    free.append(word)
     return coords[:count], int(count)
 
 

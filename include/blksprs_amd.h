@@ -72,14 +72,14 @@ int bsa_lut_packed(const uint8_t *layout, int64_t n, int64_t row_len, int64_t *p
                    void *workspace, size_t workspace_bytes, bsa_stream_t stream);
 
 /*
- * bsa_lut_packed without row offsets, for a caller that goes on enqueuing while the blocks are counted.  words: two words of
- * pinned host memory, the caller's until bsa_lut_counted_wait has returned, which waits for the count, not for what was
- * enqueued behind the scan, and returns it, or a negative BSA_E* code.  The reference reads the count first
+ * bsa_lut_packed without row offsets, for a caller that goes on enqueuing while the blocks are counted.  word: a word of pinned
+ * host memory, the scan's until bsa_lut_counted_wait has returned, which waits for the count, not for what was enqueued behind
+ * the scan, and returns it, or a negative BSA_E* code; the count is all that is written there.  The reference reads the count first
  * (blksprs/ops/conversion.py:286-288).
  */
-int bsa_lut_packed_counted(const uint8_t *layout, int64_t n, int64_t *packed, int64_t *words, void *workspace,
+int bsa_lut_packed_counted(const uint8_t *layout, int64_t n, int64_t *packed, int64_t *word, void *workspace,
                            size_t workspace_bytes, bsa_stream_t stream);
-int64_t bsa_lut_counted_wait(const int64_t *words, bsa_stream_t stream);
+int64_t bsa_lut_counted_wait(const int64_t *word, bsa_stream_t stream);
 
 /*
  * bsa_lut_packed for callers that cannot allocate device memory (code under HIP graph capture, serving loops,

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import blksprs_amd as bs
+from blksprs_amd import _capi
 from blksprs_amd.utils import tools
 
 pytestmark = pytest.mark.gpu
@@ -45,3 +46,22 @@ def test_to_sparse_behind_queued_work_of_another_stream(device):
         n = out.size(0)
     stream.synchronize()
     assert n == 2 * 6 * 8 and bool((out == 1).all())
+
+
+@pytest.mark.parametrize("entries,first", [(2048, 0), (1 << 17, 0), (5000, 3), ((1 << 21) + 2049, 0)])
+def test_the_count_is_all_that_the_host_is_left(device, entries, first):
+    """Counted from the layout, from the tiles' counts and by a scan of them: the host takes its word back as soon as it has seen
+    the count, so nothing may be written beside it or after it."""
+    whole = torch.rand(first + entries, device=device, generator=torch.Generator(device).manual_seed(entries)) < 0.3
+    layout = whole[first:].view(torch.uint8)
+    packed = torch.empty(entries, dtype=torch.int64, device=device)
+    workspace = torch.empty(_capi.load().bsa_lut_workspace_bytes(entries), dtype=torch.uint8, device=device)
+    words = torch.full((3,), 1 << 40, dtype=torch.int64, device="cpu").pin_memory()
+    stream = _capi.stream(device)
+    _capi.call("bsa_lut_packed_counted", layout.data_ptr(), entries, packed.data_ptr(), words[1:].data_ptr(), workspace.data_ptr(),
+               workspace.numel(), stream)
+    count = _capi.load().bsa_lut_counted_wait(words[1:].data_ptr(), stream)
+    torch.cuda.synchronize()
+    assert words.tolist() == [1 << 40, count, 1 << 40] and count == int(whole[first:].sum())
+    expected = torch.where(layout != 0, layout.cumsum(0, dtype=torch.int64) - 1, -1)
+    assert torch.equal(packed, expected)
