@@ -294,7 +294,7 @@ class _RangeOfLengths:
         free = getattr(_RANGE_READERS, "free", None)
         if free is None:
             free = _RANGE_READERS.free = []
-        self.words = free.pop() if free else torch.empty(3, dtype=torch.int64, pin_memory=True)
+        self.words = free.pop() if free else torch.empty(3, dtype=torch.int64, device="cpu", pin_memory=True)
         self.stream = _capi.stream(device)
         with _capi.on_device(device):
             _capi.call("bsa_causal_lengths_range", self.lengths.data_ptr(), self.lengths.numel(), self.words.data_ptr(),

@@ -162,7 +162,7 @@ def nonzero_for_one_call(sparsity_layout: Tensor) -> tuple[Tensor, int]:
     free = getattr(_COUNT_WORDS, "free", None)
     if free is None:
         free = _COUNT_WORDS.free = []
-    word = free.pop() if free else torch.empty(1, dtype=torch.int64, pin_memory=True)
+    word = free.pop() if free else torch.empty(1, dtype=torch.int64, device="cpu", pin_memory=True)
     ws_bytes = lib.bsa_lut_workspace_bytes(n)
     packed = torch.empty(n, dtype=torch.int64, device=dev)
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
