@@ -197,6 +197,13 @@ def call(name: str, *args) -> None:
         check(rc, name)
 
 
+def wait(name: str, *args) -> int:
+    """Calls an entry point that waits for what a kernel leaves in pinned memory; returns its result."""
+    global host_waits
+    host_waits += 1
+    return getattr(load(), name)(*args)
+
+
 class on_device:
     """``with on_device(device):`` makes ``device`` the current one for the launches inside, and does nothing at
     all when it already is (the common case; torch's own context manager costs two microseconds either way)."""

@@ -301,7 +301,7 @@ class _RangeOfLengths:
                        self.stream)
 
     def finish(self) -> None:
-        rc = _capi.load().bsa_causal_lengths_wait(self.words.data_ptr(), self.longest, self.stream)
+        rc = _capi.wait("bsa_causal_lengths_wait", self.words.data_ptr(), self.longest, self.stream)
         if rc != 1:
             _capi.check(rc, "bsa_causal_lengths_wait")
         _RANGE_READERS.free.append(self.words)

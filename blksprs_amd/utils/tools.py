@@ -174,7 +174,7 @@ def nonzero_for_one_call(sparsity_layout: Tensor) -> tuple[Tensor, int]:
             coords = torch.empty((n, 3), dtype=torch.int64, device=dev)
             _capi.call("bsa_lut_nonzero", packed.data_ptr(), B, R, C, coords.data_ptr(), stream)
         finally:  # the word is the scan's until it has written it
-            count = lib.bsa_lut_counted_wait(word.data_ptr(), stream)
+            count = _capi.wait("bsa_lut_counted_wait", word.data_ptr(), stream)
     if count < 0:
         _capi.check(int(count), "bsa_lut_counted_wait")
     free.append(word)

@@ -65,3 +65,26 @@ def test_the_count_is_all_that_the_host_is_left(device, entries, first):
     assert words.tolist() == [1 << 40, count, 1 << 40] and count == int(whole[first:].sum())
     expected = torch.where(layout != 0, layout.cumsum(0, dtype=torch.int64) - 1, -1)
     assert torch.equal(packed, expected)
+
+
+def test_every_look_at_pinned_memory_is_a_counted_wait(device):
+    """torch's own report of waits (sync debug mode) does not see them."""
+    layout = torch.ones((1, 2, 2), dtype=torch.bool, device=device)
+    x, cache = torch.zeros((1, 32, 32), device=device), {}
+    full = torch.ones((1, 2, 1), dtype=torch.bool, device=device)
+    blocks, attention_cache = torch.zeros((2, 16, 16), device=device), {}
+    lengths = torch.tensor([32], device=device)
+
+    def waits(call):
+        before = _capi.host_waits
+        call()
+        return _capi.host_waits - before
+
+    def attend():
+        bs.ops.flash_attention(blocks, full, blocks, full, blocks, full, layout, 16, causal_lengths=lengths,
+                               layout_cache=attention_cache)
+
+    bs.ops.to_sparse(x, layout, 16, layout_cache=cache)
+    assert [waits(lambda: bs.ops.to_sparse(x, layout, 16)) for _ in range(2)] == [1, 1]
+    assert waits(lambda: bs.ops.to_sparse(x, layout, 16, layout_cache=cache)) == 0
+    assert [waits(attend) for _ in range(2)] == [1, 0]  # the range of lengths that were seen before is known
