@@ -34,3 +34,17 @@ def test_softmax_of_rows_shared_by_groups_of_lanes(device, sbs, lengths):
     # dx = y (g - s): s = sum y g is off by those 64 EPS and the additions of its terms, all below sum y |g| <= max |g| of a row
     dx = orc.softmax_backward(go.double(), y, layout.numpy(), sbs)
     assert ((xd.grad.double().cpu() - dx).abs() <= 256 * EPS * y * float(go.abs().max()) + 1e-37).all()
+
+
+@pytest.mark.parametrize("sbs,blocks", [(16, 300), (16, 1200), (64, 300)])
+@pytest.mark.parametrize("largest", [13.3, 15.7, 30.1])
+def test_a_maximum_that_stays_through_a_long_row(device, sbs, blocks, largest):
+    """A row of several hundred blocks among rows of one: its sum is carried through 38 to 150 chunks that bring no larger value."""
+    layout = torch.zeros((1, 401, blocks), dtype=torch.bool)
+    layout[0, 0] = layout[0, :, 0] = True
+    x = torch.randn((blocks + 400, sbs, sbs), generator=torch.Generator().manual_seed(blocks))
+    x[0, :, 0] = largest
+    out = torch.Tensor(bs.ops.softmax(x.to(device), layout.to(device), sbs)).double().cpu()
+    y = orc.softmax(x.double(), layout.numpy(), sbs)
+    # as above: 64 EPS of an exponential and its sum, whose few hundred additions per lane are of positive terms
+    assert ((out - y).abs() <= (64 + blocks / 4) * EPS * y + 1e-37).all()
