@@ -6,13 +6,18 @@
 // float4 per lane.  sbs/4 lanes cover an element row of one block; where rows are long,
 // 2, 4 or 8 such groups of lanes share it, each taking every second, fourth or eighth
 // block (make_geom), so that it fits their registers: rows of up to 16 float4 units per
-// lane (32 in the forward pass of sbs >= 128) stay there between the reduction and the
+// lane (32 in the forward pass where no row is shared, and of sbs >= 128) stay there between the reduction and the
 // write (one HBM read + one write), longer rows make two read passes.  The reductions stay inside the lanes of a row.
 //
 // Bound by HBM.  Block-causal rows of n = 2048 elements and 10 % more blocks, us forward +
 // backward, a row on sbs/4 lanes (32 units in registers) -> shared: sbs 16, 16 matrices
 // 87 + 165 -> 62 + 83; sbs 32 77 + 125 -> 57 + 82; sbs 64, 32 matrices 114 + 165 -> 106 + 153
 // (5.7 and 5.9 TB/s); three matrices of 37 blocks of 32 a side 13.3 + 16.0 -> 6.6 + 7.9.
+// Which rows are shared follows from the mean, so a few long rows among short ones are not: the kernels without kShared keep 32
+// units forward and have nothing to do with lanes that leave a unit out.  128 matrices of 32 blocks a side, a diagonal and the
+// one beside it with two whole rows, forward + backward with (16 units) -> without: sbs 64 95 + 145 -> 76 + 144, sbs 32
+// 36.6 + 35.8 -> 26.4 + 35.1, sbs 16 (256 matrices) 19.3 + 19.9 -> 16.2 + 18.3; 24 blocks of 64, windows of four, where no row is
+// long: 53.3 + 98.5 -> 54.8 + 96.1.
 #include "common.h"
 
 namespace {
@@ -68,8 +73,9 @@ __device__ inline float lanes_sum(float v, int lpr) {
 
 // float offset of unit u, relative to the first block of the row and to the lane's own offset (the same for every
 // lane: the compiler keeps it in scalar registers)
+template <bool kShared>
 __device__ inline int64_t unit_offset(int u, const RowGeom &g) {
-  const int t = (u >> g.nq_log2) << g.split_log2;
+  const int t = kShared ? (u >> g.nq_log2) << g.split_log2 : u >> g.nq_log2;
   const int q = u & ((1 << g.nq_log2) - 1);
   return ((int64_t)t << (2 * g.sbs_log2)) + q * 256;
 }
@@ -83,6 +89,7 @@ struct RowTask {
   int units, lane_base, tail_base;
   bool in_last;
 };
+template <bool kShared>
 __device__ inline bool wave_task(const RowGeom &g, const int32_t *row_offsets, int64_t n_tasks, RowTask &task) {
   // Workgroup b runs on XCD b % 8: each XCD takes a contiguous eighth of the tasks, so the waves that read
   // neighbouring KiB of the same blocks (the tasks of one block row) share one L2.
@@ -97,6 +104,12 @@ __device__ inline bool wave_task(const RowGeom &g, const int32_t *row_offsets, i
   const int count = row_offsets[r + 1] - start;
   if (count <= 0) return false;
   task.first = (int64_t)start << (2 * g.sbs_log2);
+  if constexpr (!kShared) {
+    task.units = count << g.nq_log2;
+    task.lane_base = task.tail_base = ((grp * (64 / g.lpr) + lane / g.lpr) << g.sbs_log2) + (lane % g.lpr) * 4;
+    task.in_last = true;
+    return true;
+  }
   const int split = 1 << g.split_log2, rounds = (count + split - 1) >> g.split_log2;
   task.units = rounds << g.nq_log2;
   const int part = lane / g.lpr & (split - 1);
@@ -133,23 +146,23 @@ __device__ inline float max_with(float m, float4 v) {
   return t;
 }
 
-// This lane's part of a row of a tensor
+// This lane's part of a row of a tensor.  kShared: several groups of lanes share the row
+template <bool kShared>
 struct RowPart {
   const float *row, *tail;  // where its units are read from, in all rounds and in the last
   int last;                 // the last round
   __device__ inline RowPart(const float *tensor, const RowTask &task)
       : row(tensor + task.first + task.lane_base), tail(tensor + task.first + task.tail_base), last(task.units - 1) {}
   __device__ inline float4 unit(int u, const RowGeom &g) const {
-    // with several units per block (blocks wider than 256) no row is split and tail is row
-    return *reinterpret_cast<const float4 *>((u == last ? tail : row) + unit_offset(u, g));
+    return *reinterpret_cast<const float4 *>((kShared && u == last ? tail : row) + unit_offset<kShared>(u, g));
   }
 };
 
 // Loads units [0, units) of a row into v, four at a time: within a group of four the index is clamped to the last
 // unit (a repeated load of a line just fetched) so that the group has no branch, and no load is followed by its
 // use: all loads of the row are in flight together.  Entries at and beyond `units` hold copies of the last unit.
-template <int N>
-__device__ inline void load_row(float4 (&v)[N], const RowPart &part, const RowGeom &g) {
+template <int N, bool kShared>
+__device__ inline void load_row(float4 (&v)[N], const RowPart<kShared> &part, const RowGeom &g) {
 #pragma unroll
   for (int c = 0; c < N; c += 4) {
     if (c <= part.last) {
@@ -162,23 +175,38 @@ __device__ inline void load_row(float4 (&v)[N], const RowPart &part, const RowGe
 // Units [u0, u0 + count) of a row, count <= N: the index is clamped to the last of them, so the loads have no
 // branch between them; entries at and beyond `count` hold copies of the last unit.
 constexpr int kChunk = 8;
-template <int N>
-__device__ inline void load_chunk(float4 (&v)[N], const RowPart &part, int u0, int count, const RowGeom &g) {
+template <int N, bool kShared>
+__device__ inline void load_chunk(float4 (&v)[N], const RowPart<kShared> &part, int u0, int count, const RowGeom &g) {
 #pragma unroll
   for (int j = 0; j < N; ++j) v[j] = part.unit(u0 + (j < count ? j : count - 1), g);
 }
 
+// use(j) for the units [u0, u0 + count) of a chunk that are this lane's (mine).  A whole chunk in front of the last unit is used
+// without tests: with them alone the compiler moves loads behind them, each with a wait of its own (backward, 64 matrices of 128
+// blocks of 16 a side, a window of 3 blocks and one whole row: 65 us, 37 so).
+template <typename Mine, typename Use>
+__device__ inline void each_of_chunk(int u0, int count, int units, Mine mine, Use use) {
+  if (u0 + kChunk < units) {
+#pragma unroll
+    for (int j = 0; j < kChunk; ++j) use(j);
+  } else {
+#pragma unroll
+    for (int j = 0; j < kChunk; ++j)
+      if (j < count && mine(u0 + j)) use(j);
+  }
+}
+
 // kUnits: float4 units per lane in registers
-template <int kUnits>
+template <int kUnits, bool kShared>
 __global__ __launch_bounds__(64 * kWaves) void softmax_fwd_kernel(const float *__restrict__ x, float *__restrict__ out,
                                                           const int32_t *__restrict__ row_offsets, int64_t n_tasks,
                                                           RowGeom g) {
   RowTask task;
-  if (!wave_task(g, row_offsets, n_tasks, task)) return;
+  if (!wave_task<kShared>(g, row_offsets, n_tasks, task)) return;
   const int units = task.units;
-  const RowPart xr(x, task);
+  const RowPart<kShared> xr(x, task);
   float *orow = out + task.first + task.lane_base;
-  auto mine = [&](int u) { return u < units - 1 || task.in_last; };  // of u < units
+  auto mine = [&](int u) { return !kShared || u < units - 1 || task.in_last; };  // of u < units
 
   if (units <= kUnits) {
     float4 v[kUnits];
@@ -213,7 +241,7 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_fwd_kernel(const float *_
         o.y = v[u].y * inv;
         o.z = v[u].z * inv;
         o.w = v[u].w * inv;
-        store_streaming(orow + unit_offset(u, g), o);
+        store_streaming(orow + unit_offset<kShared>(u, g), o);
       }
     }
     return;
@@ -235,10 +263,9 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_fwd_kernel(const float *_
     if (mn != -INFINITY) {
       const float mn2 = mn * kLog2e;
       float add = 0.f;
-#pragma unroll
-      for (int j = 0; j < kChunk; ++j)
-        if (j < count && mine(u0 + j))
-          add += (exp_rel(v[j].x, mn2) + exp_rel(v[j].y, mn2)) + (exp_rel(v[j].z, mn2) + exp_rel(v[j].w, mn2));
+      each_of_chunk(u0, count, units, mine, [&](int j) {
+        add += (exp_rel(v[j].x, mn2) + exp_rel(v[j].y, mn2)) + (exp_rel(v[j].z, mn2) + exp_rel(v[j].w, mn2));
+      });
       s = s * exp2_of(m2 - mn2) + add;
       m2 = mn2;
     } else {
@@ -259,30 +286,28 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_fwd_kernel(const float *_
     const int count = units - u0 < kChunk ? units - u0 : kChunk;
     float4 v[kChunk];
     load_chunk(v, xr, u0, count, g);
-#pragma unroll
-    for (int j = 0; j < kChunk; ++j) {
-      if (j < count && mine(u0 + j)) {
-        float4 o;
-        o.x = exp_rel(v[j].x, mall2) * inv_all;
-        o.y = exp_rel(v[j].y, mall2) * inv_all;
-        o.z = exp_rel(v[j].z, mall2) * inv_all;
-        o.w = exp_rel(v[j].w, mall2) * inv_all;
-        store_streaming(orow + unit_offset(u0 + j, g), o);
-      }
-    }
+    each_of_chunk(u0, count, units, mine, [&](int j) {
+      float4 o;
+      o.x = exp_rel(v[j].x, mall2) * inv_all;
+      o.y = exp_rel(v[j].y, mall2) * inv_all;
+      o.z = exp_rel(v[j].z, mall2) * inv_all;
+      o.w = exp_rel(v[j].w, mall2) * inv_all;
+      store_streaming(orow + unit_offset<kShared>(u0 + j, g), o);
+    });
   }
 }
 
+template <bool kShared>
 __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *__restrict__ grad_out,
                                                           const float *__restrict__ y, float *__restrict__ grad_in,
                                                           const int32_t *__restrict__ row_offsets, int64_t n_tasks,
                                                           RowGeom g) {
   RowTask task;
-  if (!wave_task(g, row_offsets, n_tasks, task)) return;
+  if (!wave_task<kShared>(g, row_offsets, n_tasks, task)) return;
   const int units = task.units;
-  const RowPart gr(grad_out, task), yr(y, task);
+  const RowPart<kShared> gr(grad_out, task), yr(y, task);
   float *dr = grad_in + task.first + task.lane_base;
-  auto mine = [&](int u) { return u < units - 1 || task.in_last; };  // of u < units
+  auto mine = [&](int u) { return !kShared || u < units - 1 || task.in_last; };  // of u < units
 
   if (units <= kBwdUnits) {
     float4 yv[kBwdUnits], gv[kBwdUnits];
@@ -302,7 +327,7 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *_
         o.y = yv[u].y * (gv[u].y - s);
         o.z = yv[u].z * (gv[u].z - s);
         o.w = yv[u].w * (gv[u].w - s);
-        store_streaming(dr + unit_offset(u, g), o);
+        store_streaming(dr + unit_offset<kShared>(u, g), o);
       }
     }
     return;
@@ -320,10 +345,9 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *_
         const int count = units - c < kChunk ? units - c : kChunk;
         float4 gv[kChunk];
         load_chunk(gv, gr, c, count, g);
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j)
-          if (j < count && mine(c + j))
-            s += (yv[c + j].x * gv[j].x + yv[c + j].y * gv[j].y) + (yv[c + j].z * gv[j].z + yv[c + j].w * gv[j].w);
+        each_of_chunk(c, count, units, mine, [&](int j) {
+          s += (yv[c + j].x * gv[j].x + yv[c + j].y * gv[j].y) + (yv[c + j].z * gv[j].z + yv[c + j].w * gv[j].w);
+        });
       }
     }
     s = lanes_sum(s, g.lanes);
@@ -333,17 +357,14 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *_
         const int count = units - c < kChunk ? units - c : kChunk;
         float4 gv[kChunk];
         load_chunk(gv, gr, c, count, g);
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
-          if (j < count && mine(c + j)) {
-            float4 o;
-            o.x = yv[c + j].x * (gv[j].x - s);
-            o.y = yv[c + j].y * (gv[j].y - s);
-            o.z = yv[c + j].z * (gv[j].z - s);
-            o.w = yv[c + j].w * (gv[j].w - s);
-            store_streaming(dr + unit_offset(c + j, g), o);
-          }
-        }
+        each_of_chunk(c, count, units, mine, [&](int j) {
+          float4 o;
+          o.x = yv[c + j].x * (gv[j].x - s);
+          o.y = yv[c + j].y * (gv[j].y - s);
+          o.z = yv[c + j].z * (gv[j].z - s);
+          o.w = yv[c + j].w * (gv[j].w - s);
+          store_streaming(dr + unit_offset<kShared>(c + j, g), o);
+        });
       }
     }
     return;
@@ -356,9 +377,9 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *_
     float4 yv[kChunk], gv[kChunk];
     load_chunk(yv, yr, u0, count, g);
     load_chunk(gv, gr, u0, count, g);
-#pragma unroll
-    for (int j = 0; j < kChunk; ++j)
-      if (j < count && mine(u0 + j)) s += (yv[j].x * gv[j].x + yv[j].y * gv[j].y) + (yv[j].z * gv[j].z + yv[j].w * gv[j].w);
+    each_of_chunk(u0, count, units, mine, [&](int j) {
+      s += (yv[j].x * gv[j].x + yv[j].y * gv[j].y) + (yv[j].z * gv[j].z + yv[j].w * gv[j].w);
+    });
   }
   s = lanes_sum(s, g.lanes);
   for (int u0 = 0; u0 < units; u0 += kChunk) {
@@ -366,17 +387,14 @@ __global__ __launch_bounds__(64 * kWaves) void softmax_bwd_kernel(const float *_
     float4 yv[kChunk], gv[kChunk];
     load_chunk(yv, yr, u0, count, g);
     load_chunk(gv, gr, u0, count, g);
-#pragma unroll
-    for (int j = 0; j < kChunk; ++j) {
-      if (j < count && mine(u0 + j)) {
-        float4 o;
-        o.x = yv[j].x * (gv[j].x - s);
-        o.y = yv[j].y * (gv[j].y - s);
-        o.z = yv[j].z * (gv[j].z - s);
-        o.w = yv[j].w * (gv[j].w - s);
-        store_streaming(dr + unit_offset(u0 + j, g), o);
-      }
-    }
+    each_of_chunk(u0, count, units, mine, [&](int j) {
+      float4 o;
+      o.x = yv[j].x * (gv[j].x - s);
+      o.y = yv[j].y * (gv[j].y - s);
+      o.z = yv[j].z * (gv[j].z - s);
+      o.w = yv[j].w * (gv[j].w - s);
+      store_streaming(dr + unit_offset<kShared>(u0 + j, g), o);
+    });
   }
 }
 
@@ -405,8 +423,8 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 }  // namespace
 
-// Forward, eight units per lane leave seven waves per SIMD: sbs 64, above, 106 us, 114 with 16 to 32 units.  Rows of wider
-// blocks stay whole up to 32 units: sbs 128 110 us so, 119 with 16 units in registers, 113 with two groups of lanes on a row.
+// Forward, shared rows of eight units per lane leave seven waves per SIMD: sbs 64, above, 106 us, 114 with 16 to 32 units.  Rows
+// of wider blocks stay whole up to 32 units: sbs 128 110 us so, 119 with 16 units in registers, 113 with two groups of lanes on a row.
 // Backward, 16 units of both tensors: 153 us either way, but fewer, longer rounds at sbs 16 (83 against 92).
 extern "C" int bsa_softmax_fwd(const float *x, float *out, const int32_t *row_offsets, int64_t n_rows, int64_t nnz,
                                int sbs, bsa_stream_t stream) {
@@ -420,7 +438,7 @@ extern "C" int bsa_softmax_fwd(const float *x, float *out, const int32_t *row_of
   const int64_t n_tasks = n_rows << g.groups_log2;
   const int64_t blocks = bsa::cdiv(bsa::cdiv(n_tasks, kWaves), 8) * 8;  // a whole number of workgroups per XCD
   if (blocks > 0x7fffffffLL) return bsa::fail(BSA_ELIMIT, "bsa_softmax_fwd: too many rows");
-  auto kernel = sbs < 128 ? &softmax_fwd_kernel<16> : &softmax_fwd_kernel<32>;
+  auto kernel = g.split_log2 == 0 ? &softmax_fwd_kernel<32, false> : sbs < 128 ? &softmax_fwd_kernel<16, true> : &softmax_fwd_kernel<32, true>;
   kernel<<<(unsigned)blocks, 64 * kWaves, 0, bsa::as_stream(stream)>>>(x, out, row_offsets, n_tasks, g);
   return bsa::check_launch("softmax_fwd_kernel");
 }
@@ -438,7 +456,7 @@ extern "C" int bsa_softmax_bwd(const float *grad_out, const float *y, float *gra
   const int64_t n_tasks = n_rows << g.groups_log2;
   const int64_t blocks = bsa::cdiv(bsa::cdiv(n_tasks, kWaves), 8) * 8;  // a whole number of workgroups per XCD
   if (blocks > 0x7fffffffLL) return bsa::fail(BSA_ELIMIT, "bsa_softmax_bwd: too many rows");
-  softmax_bwd_kernel<<<(unsigned)blocks, 64 * kWaves, 0, bsa::as_stream(stream)>>>(grad_out, y, grad_in, row_offsets,
-                                                                           n_tasks, g);
+  auto kernel = g.split_log2 == 0 ? &softmax_bwd_kernel<false> : &softmax_bwd_kernel<true>;
+  kernel<<<(unsigned)blocks, 64 * kWaves, 0, bsa::as_stream(stream)>>>(grad_out, y, grad_in, row_offsets, n_tasks, g);
   return bsa::check_launch("softmax_bwd_kernel");
 }

@@ -1,5 +1,6 @@
 """Softmax of rows that several groups of lanes share: row lengths around the rounds of a group, rows that leave some groups
-without a block in the last round, and rows much longer than the mean, whose lanes read them twice."""
+without a block in the last round, and rows much longer than the mean, whose lanes read them twice; and long rows that are not
+shared, since the mean is short."""
 
 import pytest
 import torch
@@ -48,3 +49,10 @@ def test_a_maximum_that_stays_through_a_long_row(device, sbs, blocks, largest):
     y = orc.softmax(x.double(), layout.numpy(), sbs)
     # as above: 64 EPS of an exponential and its sum, whose few hundred additions per lane are of positive terms
     assert ((out - y).abs() <= (64 + blocks / 4) * EPS * y + 1e-37).all()
+
+
+@pytest.mark.parametrize("sbs", [16, 32, 64])
+@pytest.mark.parametrize("long_rows", [[15, 16, 17], [24, 25, 31], [32, 33, 40], [8, 9, 65], [41, 47, 48, 49]])
+def test_softmax_of_long_rows_among_short_ones(device, sbs, long_rows):
+    """Means below 4.8 blocks: whole chunks of eight units, and ends of one to eight, in registers (up to 16 and 32) and beyond."""
+    test_softmax_of_rows_shared_by_groups_of_lanes(device, sbs, [1, 2, 3] * 24 + long_rows)
