@@ -15,8 +15,8 @@
 //     S = Q K^T, dP = dO V^T        rows of Q, dO from LDS, K and V in registers
 //     dV^T += dO^T P, dK^T += Q^T dS columns of dO, Q from LDS
 //
-// What bounds it: the chain of a step (tiles awaited, products, exponentials, products) with two to four waves per SIMD
-// to overlap it.  Against the fp32 matrix-core kernels that ran these shapes before (48 x 4096 queries, sbs 32, head
+// What bounds it: the chain of a step (tiles awaited, products, exponentials, products) with one (dK / dV at head dimension 128)
+// to seven waves per SIMD to overlap it, two or three for blocks of 32 at 64.  Against the fp32 matrix-core kernels that ran these shapes before (48 x 4096 queries, sbs 32, head
 // dimension 64, fp16, 33 key blocks per query block): delta + zero fill 0.071 -> 0, dK / dV 1.89 -> 0.125 ms (530 TFLOP/s),
 // dQ 1.24 -> 0.090 ms (delta included); fp32, sbs 32, products from bf16 parts (split_f32.h), 8 x 2048 queries, half of the
 // blocks, head dimension 64: dK / dV 94.5 -> 73.1, dQ 74.8 -> 55.8 us (118 and 115 TFLOP/s) against the fp32 instruction.  fp32
@@ -47,19 +47,20 @@ struct BwdShape {
   static constexpr int kStats = 256;  // lse and delta of the 32 queries of a step
   // the last row fragment of an odd number of slices of 16 reads (and drops) a slice beyond its tile
   static constexpr int kPad = T::kHalfLast ? T::kPiece : 0;
-  // dK / dV kernel of 16-bit blocks of 32.  What limits its waves is LDS and registers: with room for a wave's own dK and dV (twice
-  // the tiles of a step) a SIMD holds one wave at head dimensions 96 and 128 and two at 64; these sums now go through the tiles of
-  // all waves of a row once they are done, and P is used up before dP is formed, which leaves two, one and three.  A second tile
-  // for Q, which is read first and last in a step, lets a step's copies go out a step ahead; at 64 its addresses are more than three
-  // waves' registers hold (a fragment of K spilled in the loop), and three waves without it are as fast as two with it.
-  // Forward + backward of bf16: 24 x 4096, windows of 1024, head dimension 96: 240 -> 208 us; causal, 128: 516 -> 503; 16 x 1024, 40 %,
-  // 64: 53 -> 50; 24 x 2048, 30 %, 64: 80 -> 79; 48 x 4096, windows of 1024, 64: 273 -> 272.
-  static constexpr bool kTwoQ = ES == 2 && SBS == 32 && NS != 2;
-  static constexpr int kKvLds = kPad + (kTwoQ ? 3 : 2) * T::kBytes + (kTwoQ ? 2 : 1) * kStats;
+  // dK / dV kernel of 16-bit blocks of 32: tiles of two steps, so that a step's copies go out a step ahead.  Up to head dimension 64 a
+  // wave has LDS for both tiles twice, which its own dK and dV need anyway once it is done.  Beyond, that (twice the tiles of a step)
+  // left a SIMD one wave: there the sums go through the tiles of all waves of a row, P is used up before dP is formed, and only Q,
+  // which is read first and last in a step, has a second tile: two waves at 96, one and shorter waits at 128.  Forward + backward of
+  // bf16: 24 x 4096, windows of 1024, head dimension 96: 243 -> 213 us; causal, 128: 530 -> 512.  The same at 64, with one tile of
+  // each and three waves (five registers spilled), is faster where three are there to be run and lists are even, 24 x 2048, 30 %
+  // of the blocks, 84 -> 81, and slower elsewhere: 12 x 3008, causal, 108 -> 118, 24 x 1536 65 -> 70, 4 x 1024 34.3 -> 36.3;
+  // at 32 (four waves for three) backward of 24 x 2048, 30 %, 39.0 -> 40.9, of 8 x 1024 15.1 -> 16.1.
+  static constexpr bool kTwoQ = ES == 2 && SBS == 32, kTwoG = kTwoQ && NS <= 2;
+  static constexpr int kTiles = kTwoG ? 4 : kTwoQ ? 3 : 2;
+  static constexpr int kKvLds = kPad + kTiles * T::kBytes + (kTwoQ ? 2 : 1) * kStats;
   static constexpr int kQLds = kPad + (2 * T::kBytes > kPartial ? 2 * T::kBytes : kPartial);
   static constexpr int kQMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS <= 2 ? 3 : 2) : (NS <= 4 ? 4 : 2);
-  template <bool kSome>
-  static constexpr int kKvMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS + kSome <= 2 ? 3 : NS <= 3 ? 2 : 1) : (NS <= 4 ? 3 : 2);
+  static constexpr int kKvMinWaves = ES == 4 ? (NS * SBS <= 64 ? 2 : 1) : SBS == 32 ? (NS <= 3 ? 2 : 1) : (NS <= 4 ? 3 : 2);
 };
 
 // 4 bytes per lane, global -> LDS: lane l's value lands at dst + 4 l
@@ -233,17 +234,17 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 }
 
 template <typename Tr, int SBS, int NS, bool kSome, int kHalves>
-__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>::template kKvMinWaves<kSome>)) void attn_small_dkv_kernel(bsa_attn_args a, int split, Shares shares) {
+__global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>::kKvMinWaves)) void attn_small_dkv_kernel(bsa_attn_args a, int split, Shares shares) {
   using Shape = BwdShape<Tr::kElem, SBS, NS, kHalves>;
   using T = typename Shape::T;
   using W = Walk<Tr::kElem, SBS, NS, Shape::NB, false, kSome, kHalves>;
   constexpr int NB = Shape::NB, kScores = Shape::kScores, kRegs = Shape::kRegs;
-  constexpr bool kTwoQ = Shape::kTwoQ;
+  constexpr bool kTwoQ = Shape::kTwoQ, kTwoG = Shape::kTwoG;
   using acc_t = std::conditional_t<SBS == 32, f32x16, f32x4>;
   extern __shared__ __attribute__((aligned(1024))) char small_smem[];
   const int lane = threadIdx.x & 63;
   const int wave = first_lane(threadIdx.x >> 6);
-  char *lds = small_smem + wave * Shape::kKvLds;  // Q tile, dO tile, a second Q tile, lse and delta of one or two steps
+  char *lds = small_smem + wave * Shape::kKvLds;  // a Q and a dO tile, the second ones, lse and delta of one or two steps
 
   const RowOfWave me(shares, kHalves, a.B, kHalves * a.nk, false, wave, kWaves, split);
   const int64_t row = me.b * a.nk + me.own / kHalves;  // of the layout
@@ -271,8 +272,8 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
   const int64_t queries = me.b * a.nq * (kHalves * SBS);
   const float *const stats = (lane < 32 ? a.lse : a.delta) + queries + lane % SBS;
   const int stats_block = SBS == 16 ? (lane >> 4) & 1 : 0;
-  // 16-bit blocks of 32: addresses are formed where they are used, since registers are what limits the waves
-  constexpr bool kLateAddresses = Tr::kElem == 2 && SBS == 32;
+  // 16-bit blocks of 32 beyond head dimension 64: addresses are formed where they are used, since registers are what limits the waves
+  constexpr bool kLateAddresses = kTwoQ && !kTwoG;
   auto copy_stats = [&](const typename W::Step &s, char *dst) {
     int other = __builtin_amdgcn_readlane(walk.other, s.slot[0]);
     if constexpr (kLateAddresses) {
@@ -289,13 +290,9 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
     }
     copy_words_to_lds(stats + (int64_t)other * SBS, dst);
   };
-  auto source_now = [&]() -> uint32_t {
-    if constexpr (kLateAddresses && NS == 2) return T::source_offset(fresh_lane());
-    else return source;
-  };
-  constexpr int kStatsAt = (kTwoQ ? 3 : 2) * T::kBytes;
-  const typename T::RowReader q_rows0(lds, lane), g_rows(lds + T::kBytes, lane);
-  const typename T::ColReader q_cols0(lds, lane), g_cols(lds + T::kBytes, lane);
+  constexpr int kStatsAt = Shape::kTiles * T::kBytes;
+  const typename T::RowReader q_rows0(lds, lane), g_rows0(lds + T::kBytes, lane);
+  const typename T::ColReader q_cols0(lds, lane), g_cols0(lds + T::kBytes, lane);
   auto walk_list = [&](auto arithmetic) __attribute__((always_inline)) -> bool {  // as in the dQ kernel
     using Ar = decltype(arithmetic);
     typename W::Step now, next;
@@ -308,26 +305,29 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
     const OwnOperand<Ar, SBS, NS, kHalves, false> k_operand(kf);
     const OwnOperand<Ar, SBS, NS, kHalves, true> v_operand(vf);
     constexpr float kTimes = up_of<Ar>();  // of P and dS as second operands; dP: the square
-    // kTwoQ: Q and the statistics of a step are requested a step ahead, dO as soon as this step has used its own
-    int q_at = 0;  // 0 or 1: which Q tile and statistics
-    bool g_counted = false;  // dO of this step: exactly kCopies copies
-    typename T::RowReader q_rows = q_rows0;
-    typename T::ColReader q_cols = q_cols0;
+    // kTwoQ: Q and the statistics of a step are requested a step ahead; dO as well (kTwoG), or as soon as this step has used its own
+    int at = 0;  // 0 or 1: which of two tiles and statistics
+    bool g_counted = kTwoG;  // dO of this step: exactly kCopies copies (kTwoG: in place with Q)
+    typename T::RowReader q_rows = q_rows0, g_rows = g_rows0;
+    typename T::ColReader q_cols = q_cols0, g_cols = g_cols0;
     const float *lse = reinterpret_cast<const float *>(lds + kStatsAt);
     if (now.count) {
       walk.template copy<false>(now, tensor_q, lds, source, lane);
       copy_stats(now, lds + kStatsAt);
-      g_counted = walk.template copy<true>(now, tensor_g, lds + T::kBytes, source, lane);
+      const bool counted = walk.template copy<true>(now, tensor_g, lds + T::kBytes, source, lane);
+      if constexpr (!kTwoG) g_counted = counted;
     }
     while (now.count) {
-      bool q_counted = false;  // Q and the statistics of the next step: exactly kCopies + 1 copies
+      bool counted = false;  // what is requested here for the next step: exactly kCopies + 1 copies (kTwoG: 2 kCopies + 1)
       if constexpr (kTwoQ) {
         walk.take(next, lane);
         if (next.count) {
-          q_counted = walk.template copy<false>(next, tensor_q, lds + (q_at ^ 1) * 2 * T::kBytes, source_now(), lane);
-          copy_stats(next, lds + kStatsAt + (q_at ^ 1) * Shape::kStats);
+          char *const to = lds + (at ^ 1) * 2 * T::kBytes;
+          counted = walk.template copy<false>(next, tensor_q, to, source, lane);
+          if constexpr (kTwoG) counted = walk.template copy<true>(next, tensor_g, to + T::kBytes, source, lane) && counted;
+          copy_stats(next, lds + kStatsAt + (at ^ 1) * Shape::kStats);
         }
-        if (q_counted && g_counted) wait_vmem<2 * T::kCopies + 1>();
+        if (counted && g_counted) wait_vmem<2 * T::kCopies + 1>();
         else wait_vmem<0>();
       } else {
         wait_vmem<0>();
@@ -350,8 +350,8 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 #pragma unroll
         for (int i = 0; i < 4; ++i) ls[x + i] = l4[i];
       }
-      // in parts, and in 16-bit blocks of 32, P is used up before dP is formed, for want of registers
-      constexpr bool kLateDp = std::is_same_v<Ar, SSplit> || (Tr::kElem == 2 && SBS == 32);
+      // in parts, and where only Q has two tiles, P is used up before dP is formed, for want of registers
+      constexpr bool kLateDp = std::is_same_v<Ar, SSplit> || (kTwoQ && !kTwoG);
       if constexpr (!kLateDp) W::template multiply_rows<Ar, true>(dp, now, g_rows, v_operand, lane);
       float lowest = ls[0];
 #pragma unroll
@@ -364,8 +364,8 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
 #pragma unroll
       for (int x = 0; x < kScores; ++x) sv[x] = __builtin_amdgcn_exp2f(fmaf(sv[x], late_factor<Tr>(cc), -ls[x])) * kTimes;
       const Weights<Ar, kScores> pw(sv);
-      if constexpr (kTwoQ) {
-        if (q_counted) wait_vmem<T::kCopies + 1>();
+      if constexpr (kTwoQ && !kTwoG) {
+        if (counted) wait_vmem<T::kCopies + 1>();
         else wait_vmem<0>();
       }
       if constexpr (kLateDp) {
@@ -382,22 +382,25 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
       }
       // ---- dV^T += dO^T P
       if constexpr (!kLateDp) W::template multiply_cols<Ar, true, kScores>(dv, now, g_cols, pw);
-      wait_lds();
-      if constexpr (!kTwoQ) walk.take(next, lane);
-      if (next.count) {
-        g_counted = walk.template copy<true>(next, tensor_g, lds + T::kBytes, source_now(), lane);
-        if constexpr (!kTwoQ) copy_stats(next, lds + kStatsAt);
+      if constexpr (!kTwoG) {
+        wait_lds();
+        if constexpr (!kTwoQ) walk.take(next, lane);
+        if (next.count) {
+          g_counted = walk.template copy<true>(next, tensor_g, lds + T::kBytes, source, lane);
+          if constexpr (!kTwoQ) copy_stats(next, lds + kStatsAt);
+        }
       }
       // ---- dK^T += Q^T dS
       W::template multiply_cols<Ar, false, kScores>(dk, now, q_cols, Weights<Ar, kScores>(sv));
       wait_lds();
       if constexpr (kTwoQ) {
-        const int turn = q_at ? -1 : 1;
+        const int turn = at ? -1 : 1;
         q_rows.shift(turn * 2 * T::kBytes), q_cols.shift(turn * 2 * T::kBytes);
+        if constexpr (kTwoG) g_rows.shift(turn * 2 * T::kBytes), g_cols.shift(turn * 2 * T::kBytes);
         lse += turn * (Shape::kStats / 4);
-        q_at ^= 1;
+        at ^= 1;
       } else if (next.count) {
-        walk.template copy<false>(next, tensor_q, lds, source_now(), lane);
+        walk.template copy<false>(next, tensor_q, lds, source, lane);
       }
       now = next;
     }
@@ -429,8 +432,8 @@ __global__ __launch_bounds__(64 * kWaves, (BwdShape<Tr::kElem, SBS, NS, kHalves>
         add_partial<NS, kRegs>(dv, mine + p * (Shape::kKvLds / 4) + Shape::kPartial / 4, lane);
       }
     } else {
-      // sums that are larger than a wave's tiles (16-bit blocks of 32): the tiles of all waves of the row take in as many sums at
-      // a time as they hold, once the walks are over
+      // sums that are larger than a wave's tiles (16-bit blocks of 32 beyond head dimension 64): the tiles of all waves of the row
+      // take in as many sums at a time as they hold, once the walks are over
       static_assert(Shape::kKvLds >= Shape::kPartial, "the sums of a wave in the tiles of two");
       float *const sums = reinterpret_cast<float *>(lds - me.place * Shape::kKvLds);
       const int fit = me.waves * Shape::kKvLds / (2 * Shape::kPartial);

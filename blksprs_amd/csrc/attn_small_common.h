@@ -816,8 +816,8 @@ struct Walk {
   __device__ inline void finish_scores(const Step &s, float *sv, float qk_scale, int me, int group) const {
     // fp32 up to head dimension 64: what the lane's addresses in a mask or bias block have in common is formed here and not in front
     // of the walk, where it takes registers that dK / dV does not have (BigBird: 53.4 -> 51.9 us; dK / dV at 128, which spills
-    // others then, 134 -> 140); likewise for 16-bit blocks of 32 (14 registers of dK / dV at 64)
-    if constexpr ((ES == 4 || SBS == 32) && NS <= 2) asm volatile("" : "+v"(me), "+v"(group));
+    // others then, 134 -> 140)
+    if constexpr (ES == 4 && NS <= 2) asm volatile("" : "+v"(me), "+v"(group));
     constexpr int kRegs = SBS == 32 ? 16 : 4;
     constexpr int kSide = kHalves * SBS;  // of a block of the layout, for mask and bias
     const late_args_t p = late_args();

@@ -48,3 +48,12 @@ def test_fp32_attention_keeps_its_registers(kernels, kernel, slices, halves):
     assert len(found) == 1
     spilled = found[0][".vgpr_spill_count"]
     assert spilled <= ({(2, 2): 2, (4, 1): 28, (4, 2): 28}.get((slices, halves), 0) if kernel == "dkv" else 0)
+
+
+@pytest.mark.parametrize("kernel", ["fwd", "dq", "dkv"])
+@pytest.mark.parametrize("sbs,most", [(16, 8), (32, 4)])
+def test_16_bit_attention_of_small_blocks_keeps_its_registers(kernels, kernel, sbs, most):
+    """Every head dimension, with and without slices that may be missing."""
+    found = [k for name, k in kernels.items() if f"attn_small_{kernel}_kernelI" in name and f"ELi{sbs}ELi" in name and "SF32" not in name]
+    assert len(found) == 2 * 2 * most
+    assert all(k[".vgpr_spill_count"] == 0 for k in found)
