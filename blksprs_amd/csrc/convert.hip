@@ -18,15 +18,22 @@ __device__ inline uint4 load_streaming(const uint4 *p) {
   return uint4{v[0], v[1], v[2], v[3]};
 }
 
-// results that are written once and not read back by the kernel bypass the caches; not the compressed blocks of to_sparse,
-// which the caller is about to compute on: kept in the caches they come back faster (layout, to_sparse and to_dense of 16 x
-// 4096 x 4096 bf16 at 25 %: to_sparse 48.9 -> 44.4 us, the to_dense behind it 110 -> 98; 6 x 4096 x 2048 fp32, sbs 16, half of
-// the blocks: 45 -> 42 and 57 -> 42)
+// results that are written once and not read back by the kernel bypass the caches
 __device__ inline void store_streaming(uint4 *p, uint4 v) {
   __builtin_nontemporal_store(u32x4_t{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4_t *>(p));
 }
 
 // blocks[n][e][:] <- dense[b][r*sbs + e][c*sbs : (c+1)*sbs]
+//
+// kKeep: the compressed blocks, which the caller is about to compute on, stay in the caches and come back faster from there, as
+// long as they fit the memory-side cache of 256 MiB.  to_sparse + to_dense, us, past the caches -> kept (two dense tensors in
+// turn): sbs 64 fp32, 134 MB of 537 compressed 159 -> 134, 189 of 268 144 -> 125, 214 of 537 199 -> 188, 256 of 268 177 -> 172, 294 of
+// 537 242 -> 240, 375 of 537 288 -> 293, 965 of 1074 700 -> 724; sbs 16 bf16, 34 MB of 134 52 -> 44, 121 of 268 140 -> 126, 188 of 268
+// 172 -> 174, 255 of 268 201 -> 207, 296 of 537 304 -> 312.  to_sparse alone, whose stores wait for others to leave: 133 MB
+// 41 -> 42, 189 62 -> 70, 375 130 -> 142.
+constexpr int64_t kKeptBytes = (int64_t)256 << 20;
+
+template <bool kKeep>
 __global__ __launch_bounds__(256) void to_sparse_kernel(const uint4 *__restrict__ dense,
                                                         const int64_t *__restrict__ coords,
                                                         uint4 *__restrict__ blocks, int64_t n_vec,
@@ -43,7 +50,8 @@ __global__ __launch_bounds__(256) void to_sparse_kernel(const uint4 *__restrict_
     const int64_t r = coords[n * 3 + 1];
     const int64_t c = coords[n * 3 + 2];
     const int64_t src = b * dense_batch_vecs + ((r << sbs_log2) + e) * dense_row_vecs + (c << vec_per_row_log2) + q;
-    blocks[g] = dense[src];
+    if constexpr (kKeep) blocks[g] = dense[src];
+    else store_streaming(blocks + g, dense[src]);
   }
 }
 
@@ -265,7 +273,8 @@ extern "C" int bsa_to_sparse(const void *dense, const int64_t *coords, void *blo
   const int vec_per_row = sbs * elem_size / 16;
   const int64_t n_vec = nnz * sbs * vec_per_row;
   const int64_t dense_row_vecs = cols * elem_size / 16;
-  to_sparse_kernel<<<copy_grid(n_vec), 256, 0, bsa::as_stream(stream)>>>(
+  auto kernel = n_vec <= kKeptBytes / 16 ? &to_sparse_kernel<true> : &to_sparse_kernel<false>;
+  kernel<<<copy_grid(n_vec), 256, 0, bsa::as_stream(stream)>>>(
       static_cast<const uint4 *>(dense), coords, static_cast<uint4 *>(blocks), n_vec, ilog2(vec_per_row),
       ilog2(sbs), dense_row_vecs, rows * dense_row_vecs);
   return bsa::check_launch("to_sparse_kernel");

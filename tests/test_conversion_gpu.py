@@ -130,3 +130,16 @@ def test_validation_errors(device):
         bs.ops.to_dense(torch.randn((4, 16, 16), device=device), layout.to(torch.complex64), 16)
     with pytest.raises(ValueError, match="not supported"):
         bs.ops.to_sparse(torch.randn((1, 32, 32), device=device).to(torch.complex64), layout, 16)
+
+
+@pytest.mark.parametrize("count", [16383, 16384, 16385, 16512])
+def test_compressed_blocks_up_to_and_beyond_what_the_caches_keep(device, count):
+    """fp32 blocks of 64: 16384 of them are 256 MiB, from where on they are stored past the caches."""
+    layout = torch.zeros(128 * 129, dtype=torch.bool, device=device)
+    layout[torch.randperm(128 * 129, generator=torch.Generator().manual_seed(count))[:count].to(device)] = True
+    layout = layout.view(1, 128, 129)
+    x = torch.rand((1, 128 * 64, 129 * 64), device=device)
+    blocks = torch.Tensor(bs.ops.to_sparse(x, layout, 64))
+    assert torch.equal(blocks, x.view(1, 128, 64, 129, 64).transpose(2, 3)[layout])
+    dense = bs.ops.to_dense(blocks, layout, 64)
+    assert torch.equal(dense.view(1, 128, 64, 129, 64), x.view(1, 128, 64, 129, 64) * layout[:, :, None, :, None])
