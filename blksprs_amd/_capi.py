@@ -170,11 +170,14 @@ def ptr(t) -> int:
 
 def stream(device) -> int:
     """The current torch stream of ``device`` as a raw hipStream_t.  Every launch asks for one, so this is where memory that is
-    not the GPU's is refused, with argument validation off too (``on_device`` has nothing to do for such a device)."""
-    if device.type != "cuda":
-        raise ValueError(f"Expected a cuda device, but got: {device}")
+    not the GPU's is refused, with argument validation off too (``on_device`` has nothing to do for such a device).  Its
+    tensors' devices have no index, so that a launch on the GPU is not asked for the type (0.2 us)."""
     index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    if index is None:
+        if device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 # entry points that wait for the stream when their `stats_host` argument (at the given position) is not NULL
