@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256, 5) void matmul_runs32_kernel(
     for (int s = 0; s < B::kFrags; ++s) fx[s] = rx.frag(slot, s), fy[s] = ry.frag(slot + B::kBytes, s);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next blocks are copied over them
     // the products at one place: with a copy of them behind each test the sums travelled from registers to registers, 32 moves
-    // a pair that wait for the products (8 x 2976 x 4064 x 2080 at 25 %, bf16: 292 -> 281 us for the three; fp32 900 -> 868)
+    // a pair that wait for the products (8 x 2976 x 4064 x 2080 at 25 %: bf16 280 -> 274 us for the three, fp32 855 -> 827)
     const bool last = p + 1 >= block_end;
     if (!last && next < p_last) request(slot);
 #pragma unroll
